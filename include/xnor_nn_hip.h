@@ -29,6 +29,19 @@ extern "C" {
  * share its stream and, for host pointers, its staging buffers). */
 xnor_nn_status_t xnor_nn_hip_set_stream(const xnor_nn_convolution_t *c, void *stream);
 
+/* One forward pass in one call: binarize_data, calculate_k and forward of the reference's
+ * wrapper (reference include/xnor_nn.hpp:45-53) on `src` and `dst`; slots user_src and user_dst
+ * are left null after success.  Same results and the same rules as the three executors called
+ * in that order, for less host work per pass.  flags:
+ *   XNOR_NN_HIP_DEVICE_POINTERS  src and dst are device pointers (the caller knows; otherwise
+ *                                the driver is asked);
+ *   XNOR_NN_HIP_ON_STREAM        xnor_nn_hip_set_stream(c, stream) first; without it `stream`
+ *                                is not looked at. */
+#define XNOR_NN_HIP_DEVICE_POINTERS 1
+#define XNOR_NN_HIP_ON_STREAM 2
+xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
+        xnor_nn_resources_t res, const void *src, void *dst, void *stream, int flags);
+
 /* Stage fusion, on by default.  The reference's three per-forward stages each make a full
  * pass of their own (reference src/bcast_binarize_data.cpp:43-73,
  * src/bcast_calculate_k.cpp:42-85).  Here binarize_data also leaves mean|x| in res[a], and

@@ -50,6 +50,9 @@ ConvolutionDesc._fields_ = [
     ("state", C.c_void_p),
 ]
 
+# flags of xnor_nn_hip_forward_pass
+DEVICE_POINTERS, ON_STREAM = 1, 2
+
 # Symbols of include/xnor_nn.h: name -> (restype, argtypes)
 CORE_SYMBOLS = {
     "xnor_nn_get_status_message": (None, [C.c_char_p, C.c_int]),
@@ -63,6 +66,8 @@ CORE_SYMBOLS = {
 # Symbols of include/xnor_nn_hip.h
 HIP_SYMBOLS = {
     "xnor_nn_hip_set_stream": (C.c_int, [C.POINTER(ConvolutionDesc), C.c_void_p]),
+    # (addresses, not pointer objects: the call is made once per forward pass)
+    "xnor_nn_hip_forward_pass": (C.c_int, [C.c_void_p] * 5 + [C.c_int]),
     "xnor_nn_hip_set_stage_fusion": (C.c_int, [C.POINTER(ConvolutionDesc), C.c_int]),
     "xnor_nn_hip_plain_read": (C.c_int, [C.c_void_p, C.c_size_t, C.c_void_p]),
     "xnor_nn_hip_mfma_only": (C.c_int, [C.c_int, C.c_int, C.c_void_p]),

@@ -23,6 +23,8 @@ class Convolution:
         self.lib = capi.load()
         self.desc = capi.ConvolutionDesc()
         self.res = capi.Resources()
+        self._desc_at, self._res_at = C.addressof(self.desc), C.addressof(self.res)
+        self._forward_pass = self.lib.xnor_nn_hip_forward_pass
         self._check(self.lib.xnor_nn_init_convolution(
             C.byref(self.desc), algorithm, src_fmt, weights_fmt, dst_fmt,
             MB, OC, IC, IH, IW, KH, KW, SH, SW, PH, PW))
@@ -45,13 +47,23 @@ class Convolution:
             C.byref(self.desc), capi.as_pointer(src), capi.as_pointer(dst))
 
     def forward(self, src, dst):
-        self.res[capi.RES_USER_SRC] = capi.as_pointer(src)
-        self.res[capi.RES_USER_DST] = capi.as_pointer(dst)
-        self._check(self.desc.binarize_data(C.byref(self.desc), self.res))
-        self._check(self.desc.calculate_k(C.byref(self.desc), self.res))
-        self._check(self.desc.forward(C.byref(self.desc), self.res))
-        self.res[capi.RES_USER_SRC] = None
-        self.res[capi.RES_USER_DST] = None
+        """binarize_data, calculate_k and forward in one library call (torch knows where its
+        tensors live; for anything else the library asks the driver)."""
+        if getattr(src, "is_cuda", False) and getattr(dst, "is_cuda", False):
+            status = self._forward_pass(self._desc_at, self._res_at, src.data_ptr(),
+                                        dst.data_ptr(), None, capi.DEVICE_POINTERS)
+        else:
+            status = self._forward_pass(self._desc_at, self._res_at, capi.as_pointer(src),
+                                        capi.as_pointer(dst), None, 0)
+        if status:
+            self._check(status)
+
+    def forward_on_stream(self, src, dst, stream):
+        """The same on torch tensors on the GPU, on a stream given by its handle."""
+        status = self._forward_pass(self._desc_at, self._res_at, src.data_ptr(), dst.data_ptr(),
+                                    stream, capi.DEVICE_POINTERS | capi.ON_STREAM)
+        if status:
+            self._check(status)
 
     # -- stage-level access (what C callers do through the descriptor) -----------------
     def stage(self, name, src=None, dst=None, check=True):

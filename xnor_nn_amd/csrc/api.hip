@@ -368,6 +368,50 @@ xnor_nn_status_t exec_forward(const xnor_nn_convolution_t *c, xnor_nn_resources_
     return run_convolution(c, res, res[xnor_nn_resource_user_dst], false);
 }
 
+// A forward pass on device buffers in one call: what the three executors do one after the
+// other, without the records that hand mean|x| from one to the next (nothing can come between
+// the stages).  Two launches on the descriptor's stream.  Called with st->mu held.
+xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const float *x,
+        float *y) {
+    float *a = static_cast<float *>(res[xnor_nn_resource_a]);
+    float *k = static_cast<float *>(res[xnor_nn_resource_k]);
+    bool others = false; // box filters of other K planes that still have to read `a`
+    {
+        std::lock_guard<std::mutex> lock(handover_mu);
+        if (!ready_by_a.empty()) ready_by_a.erase(a);
+        if (!owed_by_k.empty()) {
+            owed_by_k.erase(k); // superseded: the plane is written below
+            for (const auto &e : owed_by_k) others = others || e.second.a == a;
+        }
+    }
+    if (others) {
+        const xnor_nn_status_t rc = settle_readers_of(st, a, k);
+        if (rc != xnor_nn_success) return rc;
+    }
+    uint32_t *xbits = static_cast<uint32_t *>(res[xnor_nn_resource_bin_src]);
+    if (launch_binarize_data(st->g, x, xbits, a, st->stream, st->time_binarize.next())
+            != hipSuccess)
+        return xnor_nn_error_memory;
+    const uint32_t *wfrag = reinterpret_cast<const uint32_t *>(
+            static_cast<const char *>(res[xnor_nn_resource_bin_weights]) + st->g.wfrag_offset);
+    return launch_convolution_mfma(st->g, xbits, wfrag,
+                   static_cast<const float *>(res[xnor_nn_resource_alpha]), k, y, nullptr, a, k,
+                   st->stream, st->time_convolution.next()) == hipSuccess
+        ? xnor_nn_success : xnor_nn_error_memory;
+}
+
+// The descriptor's stream, with st->mu held.
+xnor_nn_status_t change_stream(State *st, hipStream_t to) {
+    // xnor_nn_binarize_weights_float keeps its partial sums with the descriptor: kernels of an
+    // earlier call that are still under way on the old stream must be through with them
+    // before a call on the new stream may overwrite them
+    if (to != st->stream && st->float_parts != nullptr
+            && hipStreamSynchronize(st->stream) != hipSuccess)
+        return xnor_nn_error_memory;
+    st->stream = to;
+    return xnor_nn_success;
+}
+
 xnor_nn_status_t to_host(const xnor_nn_convolution_t *c, const void *dev, void *dst,
         size_t bytes) {
     State *st = state_of(c);
@@ -493,6 +537,7 @@ xnor_nn_status_t xnor_nn_init_convolution(xnor_nn_convolution_t *c,
             (void)hipGetLastError();
         }
     }
+    binarize_plan(g);
     mfma_plan(g);
     g.wfrag_offset = (bit_bytes + 255) / 256 * 256;
     c->resource_size[xnor_nn_resource_bin_weights] =
@@ -633,15 +678,45 @@ xnor_nn_status_t xnor_nn_hip_set_stream(const xnor_nn_convolution_t *c, void *st
     if (!bcast_descriptor(c)) return xnor_nn_error_invalid_input;
     State *st = state_of(c);
     std::lock_guard<std::mutex> call(st->mu);
-    hipStream_t to = static_cast<hipStream_t>(stream);
-    // xnor_nn_binarize_weights_float keeps its partial sums with the descriptor: kernels of an
-    // earlier call that are still under way on the old stream must be through with them
-    // before a call on the new stream may overwrite them
-    if (to != st->stream && st->float_parts != nullptr
-            && hipStreamSynchronize(st->stream) != hipSuccess)
-        return xnor_nn_error_memory;
-    st->stream = to;
-    return xnor_nn_success;
+    return change_stream(st, static_cast<hipStream_t>(stream));
+}
+
+// The three executors of a forward pass in one call (include/xnor_nn_hip.h).  With device
+// buffers and the matrix-core convolution the pass is two launches and nothing else on the
+// host: one lock, no pointer query where the caller vouches for the buffers (a query is
+// 0.4 us, an executor call through ctypes as much again), no hand-over records.  Everything
+// else goes through the executors.
+xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
+        xnor_nn_resources_t res, const void *src, void *dst, void *stream, int flags) {
+    if (c == nullptr || res == nullptr) return xnor_nn_error_invalid_input;
+    if (bcast_descriptor(c)) {
+        State *st = state_of(c);
+        std::lock_guard<std::mutex> call(st->mu);
+        if (flags & XNOR_NN_HIP_ON_STREAM) {
+            const xnor_nn_status_t rc = change_stream(st, static_cast<hipStream_t>(stream));
+            if (rc != xnor_nn_success) return rc;
+        }
+        bool complete = src != nullptr && dst != nullptr && is_data_format(c->src_format)
+            && is_data_format(c->dst_format);
+        for (int i = xnor_nn_resource_internal; i < xnor_nn_resource_number; i++)
+            complete = complete && res[i] != nullptr;
+        if (complete && st->g.use_mfma && fusion_on(st) && !st->verbose
+                && ((flags & XNOR_NN_HIP_DEVICE_POINTERS) || (on_device(src) && on_device(dst)))) {
+            const xnor_nn_status_t rc = forward_on_device(st, res, static_cast<const float *>(src),
+                    static_cast<float *>(dst));
+            if (rc == xnor_nn_success)
+                res[xnor_nn_resource_user_src] = res[xnor_nn_resource_user_dst] = nullptr;
+            return rc;
+        }
+    }
+    res[xnor_nn_resource_user_src] = const_cast<void *>(src);
+    res[xnor_nn_resource_user_dst] = dst;
+    xnor_nn_status_t rc = c->binarize_data(c, res);
+    if (rc == xnor_nn_success) rc = c->calculate_k(c, res);
+    if (rc == xnor_nn_success) rc = c->forward(c, res);
+    if (rc == xnor_nn_success)
+        res[xnor_nn_resource_user_src] = res[xnor_nn_resource_user_dst] = nullptr;
+    return rc;
 }
 
 xnor_nn_status_t xnor_nn_hip_set_stage_fusion(const xnor_nn_convolution_t *c, int on) {

@@ -347,13 +347,8 @@ void launch_tiled(const Geometry &g, const float *x, uint32_t *bits, float *a, h
     // waves the hand-over chain of one workgroup gets long and too few workgroups are
     // resident to cover it (512 input channels: 14.1 us with 16 waves, 10.4 us with 2 x 8;
     // 384 channels: 12 x 1 and 6 x 2 are equal at MB 256, 12 x 1 is 5% faster at MB 1024).
-    // XNOR_NN_HIP_BIN_WAVES overrides the cap for measurements.
     const int need = g.xw;
-    int cap = MAX_WAVES;
-    if (const char *e = getenv("XNOR_NN_HIP_BIN_WAVES")) {
-        const int v = atoi(e);
-        if (v >= 1 && v <= 16) cap = v;
-    }
+    const int cap = g.bin_waves;
     const int rounds = (need + cap - 1) / cap;
     const int nw = (need + rounds - 1) / rounds;
     const uint32_t ntiles = (g.npix_in + TILE - 1) / TILE;
@@ -369,11 +364,9 @@ void launch_tiled(const Geometry &g, const float *x, uint32_t *bits, float *a, h
 }
 
 // NHWC input runs the tiled kernel unless its LDS (chain, packed words, turn-around rows) would
-// not fit 64 KB (more than about a thousand channels); XNOR_NN_HIP_NHWC=lane forces the
-// one-lane-per-pixel kernel (for measurements).
+// not fit 64 KB (more than about a thousand channels).
 bool nhwc_by_lane(const Geometry &g) {
-    const char *e = getenv("XNOR_NN_HIP_NHWC");
-    if (e && e[0] == 'l') return true;
+    if (g.bin_nhwc_lane) return true;
     const int rounds = (g.xw + MAX_WAVES - 1) / MAX_WAVES;
     const int nw = (g.xw + rounds - 1) / rounds;
     return sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw) + 16
@@ -398,6 +391,19 @@ static bool tiled_nchw(const Geometry &g) {
 static bool vector_nhwc(const Geometry &g) {
     return g.src_fmt == xnor_nn_data_format_nhwc && (g.ic & 3) == 0
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET;
+}
+
+// The measurement switches of this stage, read once when a descriptor is initialised (a launch
+// asks the environment for nothing): XNOR_NN_HIP_BIN_WAVES caps the waves of a workgroup,
+// XNOR_NN_HIP_NHWC=lane forces the one-lane-per-pixel kernel for NHWC input.
+void binarize_plan(Geometry &g) {
+    g.bin_waves = MAX_WAVES;
+    if (const char *e = getenv("XNOR_NN_HIP_BIN_WAVES")) {
+        const int v = atoi(e);
+        if (v >= 1 && v <= 16) g.bin_waves = v;
+    }
+    const char *e = getenv("XNOR_NN_HIP_NHWC");
+    g.bin_nhwc_lane = e && e[0] == 'l' ? 1 : 0;
 }
 
 const char *binarize_kernel_name(const Geometry &g) {

@@ -65,6 +65,8 @@ struct Geometry {
     int ocb;      // ceil(oc/q)
     int ihw, ohw; // ih*iw, oh*ow
     uint32_t npix_in, npix_out; // mb*ihw, mb*ohw
+    int bin_waves;              // waves per workgroup of the binarize kernel at most
+    int bin_nhwc_lane;          // 1: NHWC input by the one-lane-per-pixel kernel
     int cus;                    // compute units of the device (256 if it cannot be asked)
     int use_mfma;               // 1: stage 3 runs the FP4 matrix-core kernel
     int mfma_ps;                // its tile size in 32-pixel blocks (1..4)
@@ -167,6 +169,7 @@ inline State *state_of(const xnor_nn_convolution_t *c) {
 }
 
 // Kernel launchers (one per stage); each returns the hipError_t of the launch.
+void binarize_plan(Geometry &g); // bin_waves, bin_nhwc_lane
 hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bits,
         float *a_or_null, hipStream_t s, const KernelEvents &ev = KernelEvents{});
 hipError_t launch_mean_abs(const Geometry &g, const float *x, float *a, hipStream_t s);
