@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from test_gpu_boundary import make, same_bits, second_table
+from test_gpu_parity import run_and_compare
 from util import oracle_shape
 from xnor_nn_amd import capi, synth
 
@@ -59,3 +60,48 @@ def test_forward_pass_in_one_call(oracle, gpu, where, separate_k):
         other[capi.RES_A] = own_a
         conv.lib.xnor_nn_free_resources(other)
         conv.close()
+
+
+def problem(t, zeros=False):
+    """Dimensions and synthetic tensors (NCHW, OIHW) of
+    (mb, ic, oc, ih, iw, kh, kw, sh, sw, ph, pw)."""
+    d = dict(zip(("mb", "ic", "oc", "ih", "iw", "kh", "kw", "sh", "sw", "ph", "pw"), t))
+    x = synth.normal(77, d["mb"] * d["ic"] * d["ih"] * d["iw"])
+    if zeros:
+        x[synth.zero_mask(5, x.size, 3)] = np.float32(0)
+    w = synth.normal(78, d["oc"] * d["ic"] * d["kh"] * d["kw"], 0.05)
+    return d, x.reshape(d["mb"], d["ic"], d["ih"], d["iw"]), \
+        w.reshape(d["oc"], d["ic"], d["kh"], d["kw"])
+
+
+def in_layout(x, w, fmts):
+    if fmts[0] == capi.FMT_NHWC:
+        x = np.ascontiguousarray(x.transpose(0, 2, 3, 1))
+    if fmts[1] == capi.FMT_HWIO:
+        w = np.ascontiguousarray(w.transpose(2, 3, 1, 0))
+    return x, w
+
+
+NCHW = (capi.FMT_NCHW, capi.FMT_OIHW, capi.FMT_NCHW)
+NHWC = (capi.FMT_NHWC, capi.FMT_HWIO, capi.FMT_NHWC)
+
+
+@pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
+@pytest.mark.parametrize("t", [
+    (1, 1, 1, 5, 5, 5, 5, 1, 1, 0, 0),       # one pixel, one filter
+    (3, 1, 32, 28, 28, 5, 5, 1, 1, 0, 0),    # a byte of codes per kernel row
+    (2, 3, 96, 61, 61, 11, 11, 4, 4, 0, 0),  # 33 products per kernel row
+    (2, 16, 33, 9, 11, 5, 5, 1, 1, 2, 2),    # dword-aligned rows, filters past a block
+    (5, 5, 70, 13, 13, 7, 7, 2, 2, 3, 3),    # uneven shifts, a tile's worth minus some
+    (3, 11, 6, 7, 5, 5, 4, 1, 2, 2, 2),      # kernel nearly as large as the image, uneven
+    (2, 8, 130, 10, 10, 7, 7, 1, 1, 3, 3),   # filters over several workgroups
+    (3, 2, 8, 183, 183, 3, 3, 1, 1, 1, 1),   # tiles of 128 pixels, one step
+    (12, 3, 32, 150, 150, 9, 9, 1, 1, 4, 4), # tiles of 128 pixels, eight waves
+    (2, 16, 64, 40, 150, 9, 9, 1, 1, 4, 4),  # more than 64 KB of LDS
+    (1, 16, 24, 30, 600, 13, 13, 1, 1, 6, 6), # rows too many for the LDS: another kernel
+], ids=str)
+def test_few_channels(oracle, monkeypatch, t, fmts, separate_k):
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, *in_layout(x, w, fmts), fmts)

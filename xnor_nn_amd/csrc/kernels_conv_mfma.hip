@@ -1403,7 +1403,27 @@ size_t mfma_weight_bytes(const Geometry &g) {
     return (size_t)oc_subblocks(g) * units * steps_per_tap(g) * 1024;
 }
 
+// Output stores stream past the caches when the input of the next forward pass and this
+// output cannot both stay in the 256 MB Infinity Cache, and the runs of one filter start
+// on 64-byte boundaries: with ragged planes (13 x 13, 27 x 27) streaming stores leave
+// partial lines behind and cost the kernel 15 to 25 %, more than the next pass gains.
+// XNOR_NN_HIP_STREAM_DST=0|1 overrides, for measurements.
+static int stream_output(const Geometry &g) {
+    if (const char *e = getenv("XNOR_NN_HIP_STREAM_DST")) return e[0] == '1' ? 1 : 0;
+    const uint64_t in_bytes = (uint64_t)g.npix_in * g.ic * 4u;
+    const uint64_t out_bytes = (uint64_t)g.npix_out * g.oc * 4u;
+    const uint32_t run_bytes = g.dst_fmt == xnor_nn_data_format_nchw ? (uint32_t)g.ohw * 4u
+                                                                     : (uint32_t)g.oc * 4u;
+    return in_bytes + out_bytes > (200ull << 20) && run_bytes % 64 == 0 ? 1 : 0;
+}
+
 void mfma_plan(Geometry &g) {
+    g.stream_dst = stream_output(g);
+    g.mfma_parts = g.mfma_groups = 1;
+    if (shallow_plan(g)) { // (every other mfma_* field stays zero)
+        g.use_mfma = 1;
+        return;
+    }
     // as many pixel groups as idle waves, fewer if even a one-block tile would not fit the LDS
     for (g.mfma_groups = pixel_groups(g); g.mfma_groups > 1; g.mfma_groups /= 2)
         if (lds_bytes(g, 1) <= (size_t)LDS_LIMIT) break;
@@ -1416,21 +1436,9 @@ void mfma_plan(Geometry &g) {
     g.mfma_small_lds = 0;
     g.mfma_persist = g.mfma_reverse = 0;
     g.mfma_tiles_per_round = g.mfma_rounds = g.mfma_stagger = 0;
-    g.stream_dst = 0;
     g.mfma_parts = 1;
     g.mfma_lds = g.mfma_wbytes = 0;
     if (!g.use_mfma) return;
-    // Output stores stream past the caches when the input of the next forward pass and this
-    // output cannot both stay in the 256 MB Infinity Cache, and the runs of one filter start
-    // on 64-byte boundaries: with ragged planes (13 x 13, 27 x 27) streaming stores leave
-    // partial lines behind and cost the kernel 15 to 25 %, more than the next pass gains.
-    // XNOR_NN_HIP_STREAM_DST=0|1 overrides, for measurements.
-    const uint64_t in_bytes = (uint64_t)g.npix_in * g.ic * 4u;
-    const uint64_t out_bytes = (uint64_t)g.npix_out * g.oc * 4u;
-    const uint32_t run_bytes = g.dst_fmt == xnor_nn_data_format_nchw ? (uint32_t)g.ohw * 4u
-                                                                     : (uint32_t)g.oc * 4u;
-    g.stream_dst = in_bytes + out_bytes > (200ull << 20) && run_bytes % 64 == 0 ? 1 : 0;
-    if (const char *e = getenv("XNOR_NN_HIP_STREAM_DST")) g.stream_dst = e[0] == '1' ? 1 : 0;
     g.mfma_steps = steps_per_tap(g);
     g.mfma_pair = pair_taps(g) ? 1 : 0;
     g.mfma_parts = channel_parts(g);
@@ -1550,6 +1558,7 @@ hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s) {
 
 hipError_t launch_pack_weights_fp4(const Geometry &g, const float *w, uint32_t *frag,
         hipStream_t s) {
+    if (g.mfma_shallow) return launch_pack_weights_shallow(g, w, frag, s);
     const size_t dwords = g.mfma_wbytes / 4;
     hipLaunchKernelGGL(pack_weights_fp4_kernel, dim3((unsigned)((dwords + 255) / 256)),
             dim3(256), 0, s, w, frag, g, g.mfma_steps, oc_subblocks(g), g.mfma_pair, g.mfma_parts);
@@ -1558,7 +1567,10 @@ hipError_t launch_pack_weights_fp4(const Geometry &g, const float *w, uint32_t *
 
 const char *mfma_kernel_name(const Geometry &g) {
     static thread_local char name[80];
-    if (g.mfma_small)
+    if (g.mfma_shallow)
+        snprintf(name, sizeof name, "conv_mfma_fp4_shallow_kernel<P=%d,STEPS=%d>", g.mfma_shallow,
+                g.mfma_steps);
+    else if (g.mfma_small)
         snprintf(name, sizeof name, "conv_mfma_fp4_small_kernel<KS=%d>", g.mfma_steps);
     else if (g.mfma_parts > 1)
         snprintf(name, sizeof name, "conv_mfma_fp4_kernel<KS=%d,PS=%d,PARTS=%d>",
@@ -1581,6 +1593,9 @@ const char *mfma_kernel_name(const Geometry &g) {
 hipError_t launch_convolution_mfma(const Geometry &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k,
         float *dst, int32_t *popc, const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
+    if (g.mfma_shallow)
+        return launch_convolution_shallow(g, xbits, wfrag, alpha, k, dst, popc, a_or_null, k_out,
+                s, ev);
     if (g.mfma_small && popc == nullptr)
         return launch_convolution_small(g, xbits, wfrag, alpha, k, dst, a_or_null, k_out, s, ev);
     if (g.mfma_pair) {

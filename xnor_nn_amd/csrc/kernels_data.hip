@@ -202,6 +202,55 @@ void binarize_nhwc_tiled_kernel(const float *__restrict__ x, uint32_t *__restric
             tiles_per_xcd);
 }
 
+// NCHW input of at most 32 channels (one packed word per pixel): a lane takes all channels of U
+// pixels 256 apart, so nothing is handed over between waves and nothing goes through LDS.  CH is
+// the channel count rounded up to a power of two (4 to 32), U = 32 / CH, so that a lane has up to
+// 32 loads in flight whatever the channel count: with one wave per 64 pixels and three channels
+// the tiled kernel above kept 768 bytes in flight per wave and was bound by the rate at which
+// workgroups start (AlexNet's first layer, minibatch 64: 40 MB in 32 us, here 17).
+template <int CH, int U, bool WRITE_BITS, bool WRITE_A>
+__global__ __launch_bounds__(256)
+void binarize_nchw_shallow_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
+        float *__restrict__ a, const uint32_t npix, const int ic, const uint32_t ihw,
+        const FastDiv div_ihw, const float inv_ic, const uint32_t groups,
+        const uint32_t groups_per_xcd) {
+    // each XCD takes one contiguous range of the pixels (shared cache lines meet in one L2)
+    const uint32_t group = (blockIdx.x & 7) * groups_per_xcd + (blockIdx.x >> 3);
+    if (group >= groups) return;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(x), 0, (int)(npix * (uint32_t)ic * 4u), 0x00020000);
+    const uint32_t p0 = group * (256u * U) + threadIdx.x;
+    float t[U][CH];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t p = p0 + u * 256u, pc = p < npix ? p : npix - 1;
+        const uint32_t img = div_ihw.div(pc);
+        const uint32_t off = (img * ((uint32_t)ic * ihw) + (pc - img * ihw)) * 4u;
+#pragma unroll
+        for (int c = 0; c < CH; c++)
+            if (c < ic) // uniform
+                t[u][c] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                        src, off, (uint32_t)c * ihw * 4u, 0));
+            else
+                t[u][c] = 0.f; // bit masked out below, |+0| leaves the sum as it is
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t p = p0 + u * 256u;
+        uint32_t neg = 0; // sign bits, first channel ends up in the MSB of CH bits
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            neg = __builtin_amdgcn_alignbit(neg, fbits(t[u][c]), 31);
+            acc = __fadd_rn(acc, __fmul_rn(__builtin_fabsf(t[u][c]), inv_ic));
+        }
+        if (p < npix) {
+            if (WRITE_BITS) bits[p] = (~(neg << (32 - CH))) & top_bits(ic);
+            if (WRITE_A) a[p] = acc;
+        }
+    }
+}
+
 // Any source layout, one lane per pixel, channels visited in order.  Used for NHWC input
 // (reference src/bcast_binarize_data.cpp:56-57, src/bcast_calculate_k.cpp:59-60).
 template <bool WRITE_BITS, bool WRITE_A>
@@ -363,6 +412,29 @@ void launch_tiled(const Geometry &g, const float *x, uint32_t *bits, float *a, h
                 dim3(nw * TILE), lds, s, ev, x, bits, a, g, 1.f / g.ic, rounds, ntiles, per_xcd);
 }
 
+template <int CH, bool WRITE_BITS, bool WRITE_A>
+void launch_shallow(const Geometry &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
+        const KernelEvents &ev) {
+    constexpr int U = 32 / CH;
+    // several pixels per lane only where that still leaves every compute unit two workgroups
+    const bool many = U > 1 && g.npix_in >= 2u * (uint32_t)g.cus * 256u * U;
+    const uint32_t groups = (g.npix_in + 256u * (many ? U : 1) - 1) / (256u * (many ? U : 1));
+    const uint32_t per_xcd = (groups + 7) / 8;
+    const auto kernel = many ? binarize_nchw_shallow_kernel<CH, U, WRITE_BITS, WRITE_A>
+                             : binarize_nchw_shallow_kernel<CH, 1, WRITE_BITS, WRITE_A>;
+    launch_kernel(kernel, dim3(per_xcd * 8), dim3(256), 0, s, ev, x, bits, a, g.npix_in, g.ic,
+            (uint32_t)g.ihw, g.div_ihw, 1.f / g.ic, groups, per_xcd);
+}
+
+template <bool WRITE_BITS, bool WRITE_A>
+void launch_shallow_any(const Geometry &g, const float *x, uint32_t *bits, float *a,
+        hipStream_t s, const KernelEvents &ev) {
+    if (g.ic <= 4) launch_shallow<4, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
+    else if (g.ic <= 8) launch_shallow<8, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
+    else if (g.ic <= 16) launch_shallow<16, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
+    else launch_shallow<32, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
+}
+
 // NHWC input runs the tiled kernel unless its LDS (chain, packed words, turn-around rows) would
 // not fit 64 KB (more than about a thousand channels).
 bool nhwc_by_lane(const Geometry &g) {
@@ -386,6 +458,12 @@ static bool tiled_nchw(const Geometry &g) {
         && sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw) <= 64 * 1024;
 }
 
+// Few channels: pixel numbers (rounded up to a workgroup's) and byte offsets stay below 2^31.
+static bool shallow_nchw(const Geometry &g) {
+    return g.ic <= 32 && tiled_nchw(g)
+        && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < (1ull << 31);
+}
+
 // The NHWC kernel reads 16 bytes per load at 32-bit byte offsets (and drops pieces past the
 // last channel the same way).
 static bool vector_nhwc(const Geometry &g) {
@@ -407,7 +485,8 @@ void binarize_plan(Geometry &g) {
 }
 
 const char *binarize_kernel_name(const Geometry &g) {
-    return tiled_nchw(g) ? "binarize_nchw_kernel"
+    return shallow_nchw(g) ? "binarize_nchw_shallow_kernel"
+        : tiled_nchw(g) ? "binarize_nchw_kernel"
         : !vector_nhwc(g) ? "binarize_generic_kernel"
         : nhwc_by_lane(g) ? "binarize_nhwc_kernel" : "binarize_nhwc_tiled_kernel";
 }
@@ -415,7 +494,10 @@ const char *binarize_kernel_name(const Geometry &g) {
 hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bits,
         float *a_or_null, hipStream_t s, const KernelEvents &ev) {
     const float inv_ic = 1.f / g.ic;
-    if (tiled_nchw(g)) {
+    if (shallow_nchw(g)) {
+        if (a_or_null) launch_shallow_any<true, true>(g, x, bits, a_or_null, s, ev);
+        else launch_shallow_any<true, false>(g, x, bits, nullptr, s, ev);
+    } else if (tiled_nchw(g)) {
         if (a_or_null) launch_tiled<false, true, true>(g, x, bits, a_or_null, s, ev);
         else launch_tiled<false, true, false>(g, x, bits, nullptr, s, ev);
     } else if (vector_nhwc(g) && !nhwc_by_lane(g)) {
@@ -443,7 +525,9 @@ hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bit
 
 hipError_t launch_mean_abs(const Geometry &g, const float *x, float *a, hipStream_t s) {
     const float inv_ic = 1.f / g.ic;
-    if (tiled_nchw(g)) {
+    if (shallow_nchw(g)) {
+        launch_shallow_any<false, true>(g, x, nullptr, a, s, KernelEvents{});
+    } else if (tiled_nchw(g)) {
         launch_tiled<false, false, true>(g, x, nullptr, a, s, KernelEvents{});
     } else if (vector_nhwc(g) && !nhwc_by_lane(g)) {
         launch_tiled<true, false, true>(g, x, nullptr, a, s, KernelEvents{});

@@ -11,6 +11,7 @@
 #include <hip/hip_ext.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -89,6 +90,10 @@ struct Geometry {
     int mfma_small;             // 1: few tiles: the small-problem kernel (kernels_conv_small.hip),
     int mfma_small_rows;        // the input pixels one of its blocks stages at most
     uint32_t mfma_small_lds;    // and its LDS bytes per workgroup
+    int mfma_shallow;           // > 0: few channels: the kernel of kernels_conv_shallow.hip with
+                                // tiles of this many output pixels,
+    int mfma_shallow_rows;      // padded input rows per tile at most
+    int mfma_shallow_blocks;    // and 32-filter blocks per workgroup
     int stream_dst;             // 1: the matrix-core kernel stores its output with the nt bit
     uint32_t mfma_lds, mfma_wbytes;
     FastDiv div_ihw, div_iw, div_ohw, div_ow;
@@ -130,6 +135,22 @@ inline void launch_kernel(K kernel, dim3 grid, dim3 block, size_t lds, hipStream
     else
         hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
 }
+
+// More than 64 KB of dynamic LDS has to be asked for: once per kernel, device and size.  One
+// static object per kernel remembers what has been granted.
+struct LdsGrant {
+    std::atomic<size_t> have[64];
+    hipError_t ask(const void *kernel, size_t lds) {
+        if (lds <= 64 * 1024) return hipSuccess;
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+        if (lds <= have[dev].load(std::memory_order_acquire)) return hipSuccess;
+        const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                (int)lds);
+        if (e == hipSuccess) have[dev].store(lds, std::memory_order_release);
+        return e;
+    }
+};
 
 // Event pairs for xnor_nn_hip_time_kernels: one ring per timed stage.
 struct KernelTimer {
@@ -211,6 +232,14 @@ const char *convolution_kernel_name(const Geometry &g);
 bool small_kernel_applies(const Geometry &g, int *rows, uint32_t *lds);
 hipError_t launch_convolution_small(const Geometry &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
+        const float *a_or_null, float *k_out, hipStream_t s,
+        const KernelEvents &ev = KernelEvents{});
+// The matrix-core kernel for few input channels (chosen by mfma_plan: g.mfma_shallow).
+bool shallow_plan(Geometry &g);
+hipError_t launch_pack_weights_shallow(const Geometry &g, const float *w, uint32_t *frag,
+        hipStream_t s);
+hipError_t launch_convolution_shallow(const Geometry &g, const uint32_t *xbits,
+        const uint32_t *wfrag, const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
 const char *binarize_kernel_name(const Geometry &g);
