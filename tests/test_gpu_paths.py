@@ -98,7 +98,7 @@ NHWC = (capi.FMT_NHWC, capi.FMT_HWIO, capi.FMT_NHWC)
     (3, 2, 8, 183, 183, 3, 3, 1, 1, 1, 1),   # tiles of 128 pixels, one step
     (12, 3, 32, 150, 150, 9, 9, 1, 1, 4, 4), # tiles of 128 pixels, eight waves
     (2, 16, 64, 40, 150, 9, 9, 1, 1, 4, 4),  # more than 64 KB of LDS
-    (1, 16, 24, 30, 600, 13, 13, 1, 1, 6, 6), # rows too many for the LDS: another kernel
+    (1, 16, 24, 20, 1600, 13, 13, 1, 1, 6, 6), # rows too many for the LDS: another kernel
 ], ids=str)
 def test_few_channels(oracle, monkeypatch, t, fmts, separate_k):
     if separate_k:

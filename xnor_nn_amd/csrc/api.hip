@@ -28,9 +28,9 @@ bool is_weights_format(int f) {
     return f == xnor_nn_weights_format_oihw || f == xnor_nn_weights_format_hwio;
 }
 
-size_t src_elems(const Geometry &g) { return (size_t)g.mb * g.ic * g.ih * g.iw; }
-size_t weights_elems(const Geometry &g) { return (size_t)g.oc * g.ic * g.kh * g.kw; }
-size_t dst_elems(const Geometry &g) { return (size_t)g.mb * g.oc * g.oh * g.ow; }
+size_t src_elems(const Plan &g) { return (size_t)g.mb * g.ic * g.ih * g.iw; }
+size_t weights_elems(const Plan &g) { return (size_t)g.oc * g.ic * g.kh * g.kw; }
+size_t dst_elems(const Plan &g) { return (size_t)g.mb * g.oc * g.oh * g.ow; }
 
 // True when a kernel can dereference p (device or managed allocation).
 bool on_device(const void *p) {
@@ -445,7 +445,7 @@ bool make_timer(KernelTimer &t, int capacity) {
     return true;
 }
 
-int canonical_bici(const Geometry &g) { return (g.ic * g.kh * g.kw < 32767) ? 2 : 4; }
+int canonical_bici(const Plan &g) { return (g.ic * g.kh * g.kw < 32767) ? 2 : 4; }
 int div_up(int a, int b) { return (a + b - 1) / b; }
 
 bool bcast_descriptor(const xnor_nn_convolution_t *c) {
@@ -499,7 +499,7 @@ xnor_nn_status_t xnor_nn_init_convolution(xnor_nn_convolution_t *c,
 
     State *st = new (std::nothrow) State();
     if (!st) return xnor_nn_success; // executors stay "unimplemented", like a failed match
-    Geometry &g = st->g;
+    Plan &g = st->g;
     g.mb = mb; g.ic = ic; g.ih = ih; g.iw = iw; g.oc = oc; g.oh = c->oh; g.ow = c->ow;
     g.kh = kh; g.kw = kw; g.sh = sh; g.sw = sw; g.ph = ph; g.pw = pw;
     g.src_fmt = src_fmt; g.w_fmt = weights_fmt; g.dst_fmt = dst_fmt;
@@ -778,7 +778,7 @@ xnor_nn_status_t xnor_nn_hip_export_bin_src(const xnor_nn_convolution_t *c,
         xnor_nn_resources_t res, void *dst, size_t dst_bytes) {
     if (!bcast_descriptor(c) || !res[xnor_nn_resource_bin_src] || !dst)
         return xnor_nn_error_invalid_input;
-    const Geometry &g = state_of(c)->g;
+    const Plan &g = state_of(c)->g;
     const int bici = canonical_bici(g);
     const int abic = div_up(div_up(g.ic, 8), bici) * bici;
     if (dst_bytes != (size_t)g.npix_in * abic) return xnor_nn_error_invalid_input;
@@ -800,7 +800,7 @@ xnor_nn_status_t xnor_nn_hip_export_bin_weights(const xnor_nn_convolution_t *c,
         xnor_nn_resources_t res, int oci, void *dst, size_t dst_bytes) {
     if (!bcast_descriptor(c) || !res[xnor_nn_resource_bin_weights] || !dst || oci <= 0)
         return xnor_nn_error_invalid_input;
-    const Geometry &g = state_of(c)->g;
+    const Plan &g = state_of(c)->g;
     if (g.oc % oci != 0) return xnor_nn_error_invalid_input;
     const int bici = canonical_bici(g);
     const int ico = div_up(div_up(g.ic, bici), 8);
@@ -893,7 +893,7 @@ xnor_nn_status_t xnor_nn_hip_device_info(int *compute_units, int *clock_khz) {
 int xnor_nn_hip_kernel_name(const xnor_nn_convolution_t *c, int stage, char *buf,
         size_t buf_bytes) {
     if (!bcast_descriptor(c) || !buf || buf_bytes == 0) return 0;
-    const Geometry &g = state_of(c)->g;
+    const Plan &g = state_of(c)->g;
     const char *name = "";
     switch (stage) {
     case xnor_nn_operation_convolution_forward: name = convolution_kernel_name(g); break;

@@ -137,17 +137,17 @@ void conv_xnor_popc_kernel(const uint32_t *__restrict__ xbits,
 }
 
 template <int XW, int Q>
-hipError_t launch_variant(const Geometry &g, const uint32_t *xbits, const uint32_t *wbits,
+hipError_t launch_variant(const Plan &g, const uint32_t *xbits, const uint32_t *wbits,
         const float *alpha, const float *k, const int32_t *opc, float *dst, int32_t *popc,
         hipStream_t s, const KernelEvents &ev) {
     const dim3 grid((g.npix_out + 63) / 64, (g.ocb + WAVES - 1) / WAVES);
     const dim3 block(64 * WAVES);
     if (popc)
         launch_kernel(conv_xnor_popc_kernel<XW, Q, true>, grid, block, 0, s, ev, xbits,
-                wbits, alpha, k, opc, dst, popc, g);
+                wbits, alpha, k, opc, dst, popc, geometry(g));
     else
         launch_kernel(conv_xnor_popc_kernel<XW, Q, false>, grid, block, 0, s, ev, xbits,
-                wbits, alpha, k, opc, dst, popc, g);
+                wbits, alpha, k, opc, dst, popc, geometry(g));
     return hipGetLastError();
 }
 
@@ -160,7 +160,7 @@ int pick_q(int oc, int xw) {
     return oc >= 16 ? 16 : 8;
 }
 
-const char *convolution_kernel_name(const Geometry &g) {
+const char *convolution_kernel_name(const Plan &g) {
     static thread_local char name[64];
     if (g.use_mfma) return mfma_kernel_name(g);
     const int xw = (g.xw == 3 || g.xw == 8 || g.xw == 12 || g.xw == 16) ? g.xw : 0;
@@ -168,7 +168,7 @@ const char *convolution_kernel_name(const Geometry &g) {
     return name;
 }
 
-hipError_t launch_convolution(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution(const Plan &g, const uint32_t *xbits,
         const uint32_t *wbits, const float *alpha, const float *k, const int32_t *opc,
         float *dst, int32_t *popc, hipStream_t s, const KernelEvents &ev) {
 #define XNOR_CASE(XW_, Q_) \

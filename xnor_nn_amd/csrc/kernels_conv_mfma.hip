@@ -1077,7 +1077,7 @@ void pack_weights_fp4_kernel(const float *__restrict__ w, uint32_t *__restrict__
 // counts above 8 rounded up to 12 or 16 (the extra steps multiply FP4 zeros).
 // Pairing two taps per KS = ceil(IC/32) steps pays when the number of 32-channel words is odd
 // (otherwise every tap ends on a half-empty step) and small enough for the register file.
-bool pair_taps(const Geometry &g) {
+bool pair_taps(const Plan &g) {
     const int taps = g.kh * g.kw;
     if ((g.xw & 1) == 0 || g.xw > 5 || taps < 2) return false;
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_PAIR")) return e[0] == '1';
@@ -1086,7 +1086,7 @@ bool pair_taps(const Geometry &g) {
 // More than 1024 channels: parts of 12 or 16 steps, as few padded steps as possible (the
 // fewer parts on a tie).  Sets the steps per part; returns the number of parts, 1 if the
 // channels fit one part.
-int channel_parts(const Geometry &g, int *steps = nullptr) {
+int channel_parts(const Plan &g, int *steps = nullptr) {
     const int ks = (g.ic + 63) / 64;
     int best_parts = 1, best_steps = 16;
     if (ks > 16) {
@@ -1102,7 +1102,7 @@ int channel_parts(const Geometry &g, int *steps = nullptr) {
     if (steps) *steps = best_steps;
     return best_parts;
 }
-int steps_per_tap(const Geometry &g) {
+int steps_per_tap(const Plan &g) {
     if (pair_taps(g)) return g.xw; // per pair of taps
     const int ks = (g.ic + 63) / 64;
     if (ks > 16) {
@@ -1113,13 +1113,13 @@ int steps_per_tap(const Geometry &g) {
     if (ks > 8) return (ks + 3) / 4 * 4; // 12 or 16
     return ks > 4 && (ks & 1) ? ks + 1 : ks;
 }
-int oc_subblocks(const Geometry &g) { return ((g.oc + NT - 1) / NT) * (NT / 32); }
+int oc_subblocks(const Plan &g) { return ((g.oc + NT - 1) / NT) * (NT / 32); }
 
 // Largest number of input pixels any tile of mt output pixels touches.  Tiles start at
 // multiples of `step` pixels (their own size for a launch with one tile size, 32 for a launch
 // with two); the offset of a tile within its image repeats after at most OHW starts, so that
 // many (plus the last, possibly short, tile) are enough to look at.
-int max_tile_rows(const Geometry &g, uint32_t mt, uint32_t step = 0) {
+int max_tile_rows(const Plan &g, uint32_t mt, uint32_t step = 0) {
     if (step == 0) step = mt;
     const uint32_t starts = (g.npix_out + step - 1) / step;
     const uint32_t look = starts < (uint32_t)g.ohw + 1 ? starts : (uint32_t)g.ohw + 1;
@@ -1139,7 +1139,7 @@ int max_tile_rows(const Geometry &g, uint32_t mt, uint32_t step = 0) {
 // have filters, with 64 or fewer only one; the others then take the same filters on further
 // pixel blocks (see conv_tile).  Not with channel parts.  XNOR_NN_HIP_MFMA_GROUPS=1|2|4
 // overrides (for measurements; more groups than idle waves are not taken).
-int pixel_groups(const Geometry &g) {
+int pixel_groups(const Plan &g) {
     if (channel_parts(g) > 1) return 1;
     // two tile sizes in one launch or persistent workgroups asked for by name: one group
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_MIX"))
@@ -1153,7 +1153,7 @@ int pixel_groups(const Geometry &g) {
     return groups;
 }
 
-size_t lds_bytes_for(const Geometry &g, size_t rows, int ps, bool persist = false) {
+size_t lds_bytes_for(const Plan &g, size_t rows, int ps, bool persist = false) {
     const size_t row_bytes = pair_taps(g) ? g.xw * 16
         : channel_parts(g) * steps_per_tap(g) * 32 + ROW_PAD;
     // persistent workgroups: two staging areas for packed words and for mean|x| (conv_tile)
@@ -1165,7 +1165,7 @@ size_t lds_bytes_for(const Geometry &g, size_t rows, int ps, bool persist = fals
         bytes = ((bytes + 15) & ~(size_t)15) + 4 * 32 * TURN_ROW * sizeof(float);
     return bytes;
 }
-size_t lds_bytes(const Geometry &g, int ps) {
+size_t lds_bytes(const Plan &g, int ps) {
     return lds_bytes_for(g, (size_t)max_tile_rows(g, 32 * ps * g.mfma_groups), ps);
 }
 
@@ -1197,7 +1197,7 @@ size_t lds_bytes(const Geometry &g, int ps) {
 // fastest tile on 50 of them and within 3.2 % on the rest.
 // Four pixel blocks do not fit the register file with 16 steps per tap or with tap pairing
 // over five words (those variants spill), and are not instantiated for channel parts.
-bool tile_fits_registers(const Geometry &g, int ps) {
+bool tile_fits_registers(const Plan &g, int ps) {
     if (ps < 4) return true;
     if (channel_parts(g) > 1) return false;
     return pair_taps(g) ? g.xw < 5 : steps_per_tap(g) < 16;
@@ -1208,7 +1208,7 @@ bool tile_fits_registers(const Geometry &g, int ps) {
 // tap and 184 or more otherwise, two 119 with one step per tap, 135 to 167 with two to four or
 // twelve steps and 188 or more otherwise, one 70 to 118 up to four steps and from twelve, 139
 // or 149 with five or six, 181 with eight; a SIMD holds 512 per lane) and by LDS.
-int resident_workgroups(const Geometry &g, int ps) {
+int resident_workgroups(const Plan &g, int ps) {
     const int ks = steps_per_tap(g);
     int by_regs = 2;
     if (ps == 3) by_regs = ks == 1 ? 3 : 2;
@@ -1219,7 +1219,7 @@ int resident_workgroups(const Geometry &g, int ps) {
     return fit < 2 ? 2 : fit; // a tile that runs alone is priced separately
 }
 
-int pick_ps(const Geometry &g) {
+int pick_ps(const Plan &g) {
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_PS")) {
         const int v = atoi(e);
         if (v >= 1 && v <= 4 && lds_bytes(g, v) <= (size_t)LDS_LIMIT && tile_fits_registers(g, v))
@@ -1258,7 +1258,7 @@ int pick_ps(const Geometry &g) {
 }
 
 template <int KS, int PS, bool PAIR, bool DEEP = false, int PSB = 0>
-hipError_t launch_mfma(const Geometry &g, const uint32_t *xbits, const uint32_t *wfrag,
+hipError_t launch_mfma(const Plan &g, const uint32_t *xbits, const uint32_t *wfrag,
         const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     const int chunks = (g.oc + NT - 1) / NT;
@@ -1297,19 +1297,19 @@ hipError_t launch_mfma(const Geometry &g, const uint32_t *xbits, const uint32_t 
     }
     if (popc)
         launch_kernel(conv_mfma_fp4_kernel<KS, PS, PSB, true, PAIR, DEEP>, grid, block, lds, s,
-                ev, xbits, wf, alpha, k, dst, popc, g, rows, chunks, units, per_xcd,
+                ev, xbits, wf, alpha, k, dst, popc, geometry(g), rows, chunks, units, per_xcd,
                 FastDiv::make((uint32_t)g.xw), a_or_null, k_out, 1.f / g.kh / g.kw, parts,
                 g.mfma_wbytes, big, blocks);
     else
         launch_kernel(conv_mfma_fp4_kernel<KS, PS, PSB, false, PAIR, DEEP>, grid, block, lds, s,
-                ev, xbits, wf, alpha, k, dst, popc, g, rows, chunks, units, per_xcd,
+                ev, xbits, wf, alpha, k, dst, popc, geometry(g), rows, chunks, units, per_xcd,
                 FastDiv::make((uint32_t)g.xw), a_or_null, k_out, 1.f / g.kh / g.kw, parts,
                 g.mfma_wbytes, big, blocks);
     return hipGetLastError();
 }
 
 template <int KS, bool PAIR>
-hipError_t launch_mfma_persistent(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_mfma_persistent(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
         const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     const int chunks = (g.oc + NT - 1) / NT;
@@ -1329,7 +1329,7 @@ hipError_t launch_mfma_persistent(const Geometry &g, const uint32_t *xbits,
         }
     }
     launch_kernel(kernel, grid, block, lds, s, ev, xbits, reinterpret_cast<const v4i *>(wfrag),
-            alpha, k, dst, g, g.mfma_rows, chunks, g.mfma_tiles_per_round,
+            alpha, k, dst, geometry(g), g.mfma_rows, chunks, g.mfma_tiles_per_round,
             FastDiv::make((uint32_t)g.xw), a_or_null, k_out, 1.f / g.kh / g.kw, g.mfma_wbytes,
             g.mfma_big_per_xcd, g.mfma_blocks_per_xcd, g.mfma_rounds, g.mfma_reverse,
             g.mfma_stagger);
@@ -1337,7 +1337,7 @@ hipError_t launch_mfma_persistent(const Geometry &g, const uint32_t *xbits,
 }
 
 template <int KS>
-hipError_t launch_mfma_deep(const Geometry &g, const uint32_t *xbits, const uint32_t *wfrag,
+hipError_t launch_mfma_deep(const Plan &g, const uint32_t *xbits, const uint32_t *wfrag,
         const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     switch (g.mfma_ps) {
@@ -1349,7 +1349,7 @@ hipError_t launch_mfma_deep(const Geometry &g, const uint32_t *xbits, const uint
 }
 
 template <int KS, bool PAIR = false>
-hipError_t launch_mfma_ps(const Geometry &g, const uint32_t *xbits, const uint32_t *wfrag,
+hipError_t launch_mfma_ps(const Plan &g, const uint32_t *xbits, const uint32_t *wfrag,
         const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     if (g.mfma_ps_small > 0) { // two tile sizes: four blocks, and two or three
@@ -1387,7 +1387,7 @@ hipError_t launch_mfma_ps(const Geometry &g, const uint32_t *xbits, const uint32
 // tile of input rows fits the 160 KB of LDS; everything else runs the XNOR/popcount kernel.
 // XNOR_NN_HIP_CONV=valu forces the latter (used to profile the two side by side).
 // Returns the tile size (32-pixel blocks per workgroup, 1..4) or 0 when not applicable.
-static int mfma_tile_blocks(const Geometry &g) {
+static int mfma_tile_blocks(const Plan &g) {
     if (const char *e = getenv("XNOR_NN_HIP_CONV"))
         if (e[0] == 'v') return 0;
     if ((g.ic + 63) / 64 > 64) return 0;
@@ -1398,7 +1398,7 @@ static int mfma_tile_blocks(const Geometry &g) {
     return pick_ps(g);
 }
 
-size_t mfma_weight_bytes(const Geometry &g) {
+size_t mfma_weight_bytes(const Plan &g) {
     const int units = pair_taps(g) ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw * channel_parts(g);
     return (size_t)oc_subblocks(g) * units * steps_per_tap(g) * 1024;
 }
@@ -1408,7 +1408,7 @@ size_t mfma_weight_bytes(const Geometry &g) {
 // on 64-byte boundaries: with ragged planes (13 x 13, 27 x 27) streaming stores leave
 // partial lines behind and cost the kernel 15 to 25 %, more than the next pass gains.
 // XNOR_NN_HIP_STREAM_DST=0|1 overrides, for measurements.
-static int stream_output(const Geometry &g) {
+static int stream_output(const Plan &g) {
     if (const char *e = getenv("XNOR_NN_HIP_STREAM_DST")) return e[0] == '1' ? 1 : 0;
     const uint64_t in_bytes = (uint64_t)g.npix_in * g.ic * 4u;
     const uint64_t out_bytes = (uint64_t)g.npix_out * g.oc * 4u;
@@ -1417,7 +1417,7 @@ static int stream_output(const Geometry &g) {
     return in_bytes + out_bytes > (200ull << 20) && run_bytes % 64 == 0 ? 1 : 0;
 }
 
-void mfma_plan(Geometry &g) {
+void mfma_plan(Plan &g) {
     g.stream_dst = stream_output(g);
     g.mfma_parts = g.mfma_groups = 1;
     if (shallow_plan(g)) { // (every other mfma_* field stays zero)
@@ -1556,16 +1556,16 @@ hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_pack_weights_fp4(const Geometry &g, const float *w, uint32_t *frag,
+hipError_t launch_pack_weights_fp4(const Plan &g, const float *w, uint32_t *frag,
         hipStream_t s) {
     if (g.mfma_shallow) return launch_pack_weights_shallow(g, w, frag, s);
     const size_t dwords = g.mfma_wbytes / 4;
     hipLaunchKernelGGL(pack_weights_fp4_kernel, dim3((unsigned)((dwords + 255) / 256)),
-            dim3(256), 0, s, w, frag, g, g.mfma_steps, oc_subblocks(g), g.mfma_pair, g.mfma_parts);
+            dim3(256), 0, s, w, frag, geometry(g), g.mfma_steps, oc_subblocks(g), g.mfma_pair, g.mfma_parts);
     return hipGetLastError();
 }
 
-const char *mfma_kernel_name(const Geometry &g) {
+const char *mfma_kernel_name(const Plan &g) {
     static thread_local char name[80];
     if (g.mfma_shallow)
         snprintf(name, sizeof name, "conv_mfma_fp4_shallow_kernel<P=%d,STEPS=%d>", g.mfma_shallow,
@@ -1590,7 +1590,7 @@ const char *mfma_kernel_name(const Geometry &g) {
     return name;
 }
 
-hipError_t launch_convolution_mfma(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution_mfma(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k,
         float *dst, int32_t *popc, const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     if (g.mfma_shallow)

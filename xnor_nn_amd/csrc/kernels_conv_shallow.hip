@@ -422,9 +422,9 @@ void pack_weights_shallow_kernel(const float *__restrict__ w, uint32_t *__restri
     frag[i] = out;
 }
 
-int row_codes_of(const Geometry &g) { return (g.kw * g.ic + 7) / 8; }
+int row_codes_of(const Plan &g) { return (g.kw * g.ic + 7) / 8; }
 
-ShallowPlan make_plan(const Geometry &g) {
+ShallowPlan make_plan(const Plan &g) {
     ShallowPlan s{};
     s.npix_out = g.npix_out; s.npix_in = g.npix_in;
     s.ic = g.ic; s.ih = g.ih; s.iw = g.iw; s.oc = g.oc; s.oh = g.oh; s.ow = g.ow; s.ohw = g.ohw;
@@ -480,7 +480,7 @@ size_t set_tile(ShallowPlan &s, int pixels, int per_wg, int rows) {
 }
 
 // Output pixels per tile and filter blocks per workgroup.
-size_t choose_tile(const Geometry &g, ShallowPlan &s, int *pixels) {
+size_t choose_tile(const Plan &g, ShallowPlan &s, int *pixels) {
     
     for (int p : {128, 64}) {
         // below two tiles of 128 per compute unit the smaller ones fill the chip better (100 images
@@ -507,7 +507,7 @@ size_t choose_tile(const Geometry &g, ShallowPlan &s, int *pixels) {
 // against 16.7 us) unless the steps are a quarter (1 to 3 channels: equal or a little ahead).
 // Only where a tile's padded input rows fit the LDS; a tile shape or variant of another kernel
 // asked for by name means that kernel.
-bool shallow_plan(Geometry &g) {
+bool shallow_plan(Plan &g) {
     for (const char *e : {"XNOR_NN_HIP_CONV", "XNOR_NN_HIP_MFMA_PS", "XNOR_NN_HIP_MFMA_PAIR",
                  "XNOR_NN_HIP_MFMA_MIX", "XNOR_NN_HIP_MFMA_SMALL", "XNOR_NN_HIP_MFMA_GROUPS",
                  "XNOR_NN_HIP_MFMA_PERSIST"})
@@ -534,7 +534,7 @@ bool shallow_plan(Geometry &g) {
     return true;
 }
 
-hipError_t launch_convolution_shallow(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t stream, const KernelEvents &ev) {
     ShallowPlan s = make_plan(g);
@@ -567,11 +567,11 @@ hipError_t launch_convolution_shallow(const Geometry &g, const uint32_t *xbits,
     return hipGetLastError();
 }
 
-hipError_t launch_pack_weights_shallow(const Geometry &g, const float *w, uint32_t *frag,
+hipError_t launch_pack_weights_shallow(const Plan &g, const float *w, uint32_t *frag,
         hipStream_t s) {
     const uint32_t dwords = g.mfma_wbytes / 4;
     hipLaunchKernelGGL(pack_weights_shallow_kernel, dim3((dwords + 255) / 256), dim3(256), 0, s,
-            w, frag, g, g.mfma_steps, row_codes_of(g), dwords);
+            w, frag, geometry(g), g.mfma_steps, row_codes_of(g), dwords);
     return hipGetLastError();
 }
 

@@ -233,7 +233,7 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
 // paired taps is walked differently), and few enough (pixel block, filter block) pairs that
 // the large-launch kernel would leave most of the chip idle.  XNOR_NN_HIP_MFMA_SMALL=0|1
 // overrides the size rule (for measurements).
-bool small_kernel_applies(const Geometry &g, int *rows_out, uint32_t *lds_out) {
+bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     if (!g.use_mfma || g.mfma_pair || g.mfma_parts > 1) return false;
     const uint32_t blocks = (g.npix_out + 31) / 32;
     const uint32_t subs = (uint32_t)(g.oc + 31) / 32;
@@ -274,14 +274,14 @@ bool small_kernel_applies(const Geometry &g, int *rows_out, uint32_t *lds_out) {
     return true;
 }
 
-hipError_t launch_convolution_small(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
         const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
     const uint32_t blocks = (g.npix_out + 31) / 32;
     const int subs = (g.oc + 31) / 32;
     launch_kernel(conv_mfma_fp4_small_kernel, dim3(blocks * (uint32_t)subs), dim3(256),
             (size_t)g.mfma_small_lds, s, ev, xbits, reinterpret_cast<const v4i *>(wfrag), alpha, k,
-            dst, g, g.mfma_small_rows, g.mfma_steps, subs, g.mfma_wbytes, a_or_null, k_out,
+            dst, geometry(g), g.mfma_small_rows, g.mfma_steps, subs, g.mfma_wbytes, a_or_null, k_out,
             1.f / g.kh / g.kw, FastDiv::make((uint32_t)g.xw));
     return hipGetLastError();
 }

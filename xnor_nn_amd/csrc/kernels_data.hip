@@ -390,7 +390,7 @@ void plain_read_kernel(const v4u *__restrict__ x, const size_t n16) {
 }
 
 template <bool NHWC, bool WRITE_BITS, bool WRITE_A>
-void launch_tiled(const Geometry &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
+void launch_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
         const KernelEvents &ev) {
     // At most twelve waves per workgroup, the slices split evenly over the rounds: with more
     // waves the hand-over chain of one workgroup gets long and too few workgroups are
@@ -406,14 +406,14 @@ void launch_tiled(const Geometry &g, const float *x, uint32_t *bits, float *a, h
     if (NHWC) lds = ((lds + 15) & ~(size_t)15) + sizeof(float) * nw * 32 * TURN_ROW;
     if (NHWC)
         launch_kernel(binarize_nhwc_tiled_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
-                dim3(nw * TILE), lds, s, ev, x, bits, a, g, 1.f / g.ic, rounds, ntiles, per_xcd);
+                dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
     else
         launch_kernel(binarize_nchw_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
-                dim3(nw * TILE), lds, s, ev, x, bits, a, g, 1.f / g.ic, rounds, ntiles, per_xcd);
+                dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
 }
 
 template <int CH, bool WRITE_BITS, bool WRITE_A>
-void launch_shallow(const Geometry &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
+void launch_shallow(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
         const KernelEvents &ev) {
     constexpr int U = 32 / CH;
     // several pixels per lane only where that still leaves every compute unit two workgroups
@@ -427,7 +427,7 @@ void launch_shallow(const Geometry &g, const float *x, uint32_t *bits, float *a,
 }
 
 template <bool WRITE_BITS, bool WRITE_A>
-void launch_shallow_any(const Geometry &g, const float *x, uint32_t *bits, float *a,
+void launch_shallow_any(const Plan &g, const float *x, uint32_t *bits, float *a,
         hipStream_t s, const KernelEvents &ev) {
     if (g.ic <= 4) launch_shallow<4, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
     else if (g.ic <= 8) launch_shallow<8, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
@@ -437,7 +437,7 @@ void launch_shallow_any(const Geometry &g, const float *x, uint32_t *bits, float
 
 // NHWC input runs the tiled kernel unless its LDS (chain, packed words, turn-around rows) would
 // not fit 64 KB (more than about a thousand channels).
-bool nhwc_by_lane(const Geometry &g) {
+bool nhwc_by_lane(const Plan &g) {
     if (g.bin_nhwc_lane) return true;
     const int rounds = (g.xw + MAX_WAVES - 1) / MAX_WAVES;
     const int nw = (g.xw + rounds - 1) / rounds;
@@ -452,21 +452,21 @@ bool nhwc_by_lane(const Geometry &g) {
 // generic kernel.  A channel past the end of a ragged slice is read through the byte offset
 // 0xFFFFFFF0, which has to lie outside the buffer for the load to return +0: the input must
 // end below that offset.
-static bool tiled_nchw(const Geometry &g) {
+static bool tiled_nchw(const Plan &g) {
     return g.src_fmt == xnor_nn_data_format_nchw
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET
         && sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw) <= 64 * 1024;
 }
 
 // Few channels: pixel numbers (rounded up to a workgroup's) and byte offsets stay below 2^31.
-static bool shallow_nchw(const Geometry &g) {
+static bool shallow_nchw(const Plan &g) {
     return g.ic <= 32 && tiled_nchw(g)
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < (1ull << 31);
 }
 
 // The NHWC kernel reads 16 bytes per load at 32-bit byte offsets (and drops pieces past the
 // last channel the same way).
-static bool vector_nhwc(const Geometry &g) {
+static bool vector_nhwc(const Plan &g) {
     return g.src_fmt == xnor_nn_data_format_nhwc && (g.ic & 3) == 0
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET;
 }
@@ -474,7 +474,7 @@ static bool vector_nhwc(const Geometry &g) {
 // The measurement switches of this stage, read once when a descriptor is initialised (a launch
 // asks the environment for nothing): XNOR_NN_HIP_BIN_WAVES caps the waves of a workgroup,
 // XNOR_NN_HIP_NHWC=lane forces the one-lane-per-pixel kernel for NHWC input.
-void binarize_plan(Geometry &g) {
+void binarize_plan(Plan &g) {
     g.bin_waves = MAX_WAVES;
     if (const char *e = getenv("XNOR_NN_HIP_BIN_WAVES")) {
         const int v = atoi(e);
@@ -484,14 +484,14 @@ void binarize_plan(Geometry &g) {
     g.bin_nhwc_lane = e && e[0] == 'l' ? 1 : 0;
 }
 
-const char *binarize_kernel_name(const Geometry &g) {
+const char *binarize_kernel_name(const Plan &g) {
     return shallow_nchw(g) ? "binarize_nchw_shallow_kernel"
         : tiled_nchw(g) ? "binarize_nchw_kernel"
         : !vector_nhwc(g) ? "binarize_generic_kernel"
         : nhwc_by_lane(g) ? "binarize_nhwc_kernel" : "binarize_nhwc_tiled_kernel";
 }
 
-hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bits,
+hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
         float *a_or_null, hipStream_t s, const KernelEvents &ev) {
     const float inv_ic = 1.f / g.ic;
     if (shallow_nchw(g)) {
@@ -507,23 +507,23 @@ hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bit
         const unsigned blocks = (g.npix_in + 255) / 256;
         if (a_or_null)
             launch_kernel(binarize_nhwc_kernel<true, true>, dim3(blocks), dim3(256), 0, s, ev,
-                    x, bits, a_or_null, g, inv_ic);
+                    x, bits, a_or_null, geometry(g), inv_ic);
         else
             launch_kernel(binarize_nhwc_kernel<true, false>, dim3(blocks), dim3(256), 0, s, ev,
-                    x, bits, a_or_null, g, inv_ic);
+                    x, bits, a_or_null, geometry(g), inv_ic);
     } else {
         const unsigned blocks = (g.npix_in + 255) / 256;
         if (a_or_null)
             launch_kernel(binarize_generic_kernel<true, true>, dim3(blocks), dim3(256), 0, s,
-                    ev, x, bits, a_or_null, g, inv_ic);
+                    ev, x, bits, a_or_null, geometry(g), inv_ic);
         else
             launch_kernel(binarize_generic_kernel<true, false>, dim3(blocks), dim3(256), 0, s,
-                    ev, x, bits, a_or_null, g, inv_ic);
+                    ev, x, bits, a_or_null, geometry(g), inv_ic);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_mean_abs(const Geometry &g, const float *x, float *a, hipStream_t s) {
+hipError_t launch_mean_abs(const Plan &g, const float *x, float *a, hipStream_t s) {
     const float inv_ic = 1.f / g.ic;
     if (shallow_nchw(g)) {
         launch_shallow_any<false, true>(g, x, nullptr, a, s, KernelEvents{});
@@ -534,11 +534,11 @@ hipError_t launch_mean_abs(const Geometry &g, const float *x, float *a, hipStrea
     } else if (vector_nhwc(g)) {
         const unsigned blocks = (g.npix_in + 255) / 256;
         hipLaunchKernelGGL((binarize_nhwc_kernel<false, true>), dim3(blocks), dim3(256), 0, s,
-                x, nullptr, a, g, inv_ic);
+                x, nullptr, a, geometry(g), inv_ic);
     } else {
         const unsigned blocks = (g.npix_in + 255) / 256;
         hipLaunchKernelGGL((binarize_generic_kernel<false, true>), dim3(blocks), dim3(256),
-                0, s, x, nullptr, a, g, inv_ic);
+                0, s, x, nullptr, a, geometry(g), inv_ic);
     }
     return hipGetLastError();
 }
@@ -550,10 +550,10 @@ hipError_t launch_plain_read(const void *buf, size_t bytes, hipStream_t s,
     return hipGetLastError();
 }
 
-hipError_t launch_box_filter(const Geometry &g, const float *a, float *k, hipStream_t s) {
+hipError_t launch_box_filter(const Plan &g, const float *a, float *k, hipStream_t s) {
     const float inv_khw = 1.f / g.kh / g.kw; // two divisions, like the reference
     const unsigned blocks = (g.npix_out + 255) / 256;
-    hipLaunchKernelGGL(box_filter_kernel, dim3(blocks), dim3(256), 0, s, a, k, g, inv_khw);
+    hipLaunchKernelGGL(box_filter_kernel, dim3(blocks), dim3(256), 0, s, a, k, geometry(g), inv_khw);
     return hipGetLastError();
 }
 

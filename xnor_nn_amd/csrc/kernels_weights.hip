@@ -253,11 +253,11 @@ void sign_times_mean_kernel(const float *__restrict__ from, float *__restrict__ 
 
 } // namespace
 
-hipError_t launch_binarize_weights(const Geometry &g, const float *w, uint32_t *bits,
+hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits,
         float *alpha, int32_t *opc, hipStream_t s) {
     const size_t words = (size_t)g.ocb * g.kh * g.kw * g.xw * g.q;
     hipLaunchKernelGGL(pack_weights_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256),
-            0, s, w, bits, g);
+            0, s, w, bits, geometry(g));
     const float chw = 1.f / (g.ic * g.kh * g.kw);
     if (g.w_fmt == xnor_nn_weights_format_oihw)
         hipLaunchKernelGGL(alpha_oihw_kernel, dim3((g.oc + ALPHA_F - 1) / ALPHA_F), dim3(64), 0,
@@ -265,9 +265,9 @@ hipError_t launch_binarize_weights(const Geometry &g, const float *w, uint32_t *
                 g.oc, g.ic * g.kh * g.kw, chw);
     else
         hipLaunchKernelGGL(alpha_strided_kernel, dim3((g.oc + 63) / 64), dim3(512), 0, s, w,
-                alpha, g, chw, FastDiv::make((uint32_t)(g.kh * g.kw)),
+                alpha, geometry(g), chw, FastDiv::make((uint32_t)(g.kh * g.kw)),
                 FastDiv::make((uint32_t)g.kw));
-    hipLaunchKernelGGL(op_count_kernel, dim3((g.ohw + 255) / 256), dim3(256), 0, s, opc, g);
+    hipLaunchKernelGGL(op_count_kernel, dim3((g.ohw + 255) / 256), dim3(256), 0, s, opc, geometry(g));
     return hipGetLastError();
 }
 

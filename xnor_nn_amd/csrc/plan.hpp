@@ -66,6 +66,16 @@ struct Geometry {
     int ocb;      // ceil(oc/q)
     int ihw, ohw; // ih*iw, oh*ow
     uint32_t npix_in, npix_out; // mb*ihw, mb*ohw
+    int mfma_groups;            // pixel groups per tile (1, 2, 4): with 128 / 64 filters or fewer
+                                // the waves without filters take further pixel blocks instead
+    int stream_dst;             // 1: the matrix-core kernel stores its output with the nt bit
+    FastDiv div_ihw, div_iw, div_ohw, div_ow;
+};
+
+// What the host adds to it when a descriptor is initialised: which kernels run and with what
+// tiles.  Kernels get the Geometry part only (geometry() below): the argument block is copied on
+// every launch and read by every workgroup.
+struct Plan : Geometry {
     int bin_waves;              // waves per workgroup of the binarize kernel at most
     int bin_nhwc_lane;          // 1: NHWC input by the one-lane-per-pixel kernel
     int cus;                    // compute units of the device (256 if it cannot be asked)
@@ -73,8 +83,6 @@ struct Geometry {
     int mfma_ps;                // its tile size in 32-pixel blocks (1..4)
     int mfma_ps_small;          // > 0: a launch with two tile sizes; the later workgroups of an
                                 // XCD take this many blocks (see the kernel)
-    int mfma_groups;            // pixel groups per tile (1, 2, 4): with 128 / 64 filters or fewer
-                                // the waves without filters take further pixel blocks instead
     uint32_t mfma_big_per_xcd;  // ... after this many workgroups with mfma_ps blocks,
     uint32_t mfma_blocks_per_xcd; // out of this many pixel blocks per XCD
     int mfma_persist;           // 1: two workgroups per CU stay and walk over the tiles, taking
@@ -94,10 +102,9 @@ struct Geometry {
                                 // tiles of this many output pixels,
     int mfma_shallow_rows;      // padded input rows per tile at most
     int mfma_shallow_blocks;    // and 32-filter blocks per workgroup
-    int stream_dst;             // 1: the matrix-core kernel stores its output with the nt bit
     uint32_t mfma_lds, mfma_wbytes;
-    FastDiv div_ihw, div_iw, div_ohw, div_ow;
 };
+inline const Geometry &geometry(const Plan &p) { return p; }
 
 // First and last input pixel (flattened index) that a tile of the output pixels
 // [p_first, p_end) can touch with an in-bounds tap: from the start of the first input row of
@@ -163,7 +170,7 @@ struct KernelTimer {
 };
 
 struct State {
-    Geometry g;
+    Plan g;
     hipStream_t stream = nullptr;
     // Held for the length of every executor call: two host threads may share one descriptor
     // (each with a resource table of its own), and the staging buffers below, the stream and
@@ -190,17 +197,17 @@ inline State *state_of(const xnor_nn_convolution_t *c) {
 }
 
 // Kernel launchers (one per stage); each returns the hipError_t of the launch.
-void binarize_plan(Geometry &g); // bin_waves, bin_nhwc_lane
-hipError_t launch_binarize_data(const Geometry &g, const float *x, uint32_t *bits,
+void binarize_plan(Plan &g); // bin_waves, bin_nhwc_lane
+hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
         float *a_or_null, hipStream_t s, const KernelEvents &ev = KernelEvents{});
-hipError_t launch_mean_abs(const Geometry &g, const float *x, float *a, hipStream_t s);
-hipError_t launch_box_filter(const Geometry &g, const float *a, float *k, hipStream_t s);
+hipError_t launch_mean_abs(const Plan &g, const float *x, float *a, hipStream_t s);
+hipError_t launch_box_filter(const Plan &g, const float *a, float *k, hipStream_t s);
 // calibration: one pass of plain 16-byte reads over bytes / 16 * 16 bytes of device memory
 hipError_t launch_plain_read(const void *buf, size_t bytes, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
-hipError_t launch_binarize_weights(const Geometry &g, const float *w, uint32_t *bits,
+hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits,
         float *alpha, int32_t *opc, hipStream_t s);
-hipError_t launch_convolution(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution(const Plan &g, const uint32_t *xbits,
         const uint32_t *wbits, const float *alpha, const float *k, const int32_t *opc,
         float *dst, int32_t *popc_or_null, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
@@ -213,36 +220,36 @@ hipError_t launch_weights_float(const float *from, float *to, size_t n, float *p
 hipError_t weights_float_scratch(float **out);
 // Decides whether the matrix-core kernel takes the problem and fills use_mfma, mfma_ps and
 // the mfma_* fields (everything the launch needs, so that a forward call computes nothing).
-void mfma_plan(Geometry &g);
-const char *mfma_kernel_name(const Geometry &g);
-size_t mfma_weight_bytes(const Geometry &g);
-hipError_t launch_pack_weights_fp4(const Geometry &g, const float *w, uint32_t *frag,
+void mfma_plan(Plan &g);
+const char *mfma_kernel_name(const Plan &g);
+size_t mfma_weight_bytes(const Plan &g);
+hipError_t launch_pack_weights_fp4(const Plan &g, const float *w, uint32_t *frag,
         hipStream_t s);
 // With a_or_null set, the kernel ignores k, computes the K plane itself from mean|x| (the
 // box filter of stage 2) and also stores it to k_out.
-hipError_t launch_convolution_mfma(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution_mfma(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k,
         float *dst, int32_t *popc_or_null, const float *a_or_null, float *k_out,
         hipStream_t s, const KernelEvents &ev = KernelEvents{});
 // calibration: `workgroups` x 4 waves, each issuing 8 * iterations FP4 matrix instructions
 // (32x32x64) on register-resident +-1 operands
 hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s);
-const char *convolution_kernel_name(const Geometry &g);
+const char *convolution_kernel_name(const Plan &g);
 // The matrix-core kernel for launches of few tiles (filled in by mfma_plan: g.mfma_small).
-bool small_kernel_applies(const Geometry &g, int *rows, uint32_t *lds);
-hipError_t launch_convolution_small(const Geometry &g, const uint32_t *xbits,
+bool small_kernel_applies(const Plan &g, int *rows, uint32_t *lds);
+hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
         const float *a_or_null, float *k_out, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
 // The matrix-core kernel for few input channels (chosen by mfma_plan: g.mfma_shallow).
-bool shallow_plan(Geometry &g);
-hipError_t launch_pack_weights_shallow(const Geometry &g, const float *w, uint32_t *frag,
+bool shallow_plan(Plan &g);
+hipError_t launch_pack_weights_shallow(const Plan &g, const float *w, uint32_t *frag,
         hipStream_t s);
-hipError_t launch_convolution_shallow(const Geometry &g, const uint32_t *xbits,
+hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
-const char *binarize_kernel_name(const Geometry &g);
+const char *binarize_kernel_name(const Plan &g);
 
 int pick_q(int oc, int xw);
 
