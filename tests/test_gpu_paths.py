@@ -105,3 +105,69 @@ def test_few_channels(oracle, monkeypatch, t, fmts, separate_k):
         monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
     d, x, w = problem(t, zeros=True)
     run_and_compare(oracle, d, *in_layout(x, w, fmts), fmts)
+
+
+@pytest.mark.parametrize("t", [
+    (1, 1, 1, 3, 3, 1, 1, 1, 1, 0, 0),        # one value
+    (1, 7, 5, 4, 4, 3, 3, 1, 1, 1, 1),        # 63 values: one short of a row of the sum
+    (1, 257, 33, 4, 4, 1, 1, 1, 1, 0, 0),     # 257: one more than it holds; channels past a word
+    (1, 160, 40, 5, 5, 3, 3, 1, 1, 1, 1),     # paired taps, odd number of taps
+    (1, 1100, 17, 4, 4, 3, 3, 1, 1, 1, 1),    # channel parts
+    (1, 5000, 9, 3, 3, 1, 1, 1, 1, 0, 0),     # no matrix-core layout
+    (1, 1612, 8, 4, 4, 2, 5, 1, 1, 2, 2),     # 16120 values: as many as fit
+    (1, 1613, 8, 4, 4, 2, 5, 1, 1, 2, 2),     # too many for one launch
+    (2, 6, 40, 40, 30, 5, 5, 1, 1, 0, 2),     # kernel rows back to back, many operation counts
+], ids=str)
+def test_weight_stage(oracle, t):
+    d, x, w = problem(t)
+    w[np.abs(w) < 0.01] = np.float32(-0.0)
+    run_and_compare(oracle, d, x, w)
+
+
+@pytest.mark.parametrize("kind", ["ties", "zeros", "tiny", "huge", "mixed", "late"])
+def test_scale_of_weights_the_sum_rounds_oddly(oracle, kind):
+    """alpha is one chain of rounded additions: values halfway between two units of the running
+    sum, sums that stay at or near zero, values that outgrow the sum and values it swallows."""
+    d, x, w = problem((1, 64, 16, 3, 3, 4, 4, 1, 1, 1, 1))
+    n = 1024
+    flat = w.reshape(16, n)
+    u = np.float32(2.0) ** np.arange(-14, 2, dtype=np.float32)
+    if kind == "ties": # small multiples of a power of two: most additions end halfway
+        flat[:] = (np.round(flat * 60) * 2.0 ** -11 + 2.0 ** -24).astype(np.float32)
+        flat[:, 0] = u
+    elif kind == "zeros":
+        flat[:8] = 0
+        flat[8:, :900] = 0
+    elif kind == "tiny":
+        flat *= np.float32(1e-38)
+        flat[3:6, 700] = np.float32(1e-30)
+    elif kind == "huge":
+        flat *= np.float32(1e37)
+    elif kind == "mixed":
+        flat *= np.float32(2.0) ** (np.arange(n) % 37 - 18).astype(np.float32)
+    else:
+        flat[:, 1000] = np.float32(5000.0) * u
+    run_and_compare(oracle, d, x, w)
+
+
+@pytest.mark.parametrize("n,shift", [(1, 0), (255, 0), (1025, 1), (4096, 0), (600001, 0),
+                                     (600001, 3)])
+def test_float_weights_at_any_length_and_alignment(oracle, gpu, n, shift):
+    import torch
+    d, _, _ = problem((1, n, 1, 1, 1, 1, 1, 1, 1, 0, 0))
+    w = synth.normal(3, n, 0.05)
+    conv = make(d, None)
+    try:
+        from_t = torch.zeros(n + shift, device=gpu)
+        from_t[shift:] = torch.from_numpy(w).to(gpu)
+        to_t = torch.full((n + 8,), 7.0, device=gpu)
+        torch.cuda.synchronize()
+        conv.binarizeWeightsFloat(from_t[shift:], to_t)
+        conv.synchronize()
+        got = to_t.cpu().numpy()
+        assert np.all(got[n:] == 7.0)
+        mean = float(np.mean(w.astype(np.float64)))
+        assert np.array_equal(np.sign(got[:n]), np.sign(np.where(w >= 0, mean, -mean)))
+        assert np.all(np.abs(np.abs(got[:n]) - abs(mean)) <= 1e-6 * np.mean(np.abs(w)))
+    finally:
+        conv.close()

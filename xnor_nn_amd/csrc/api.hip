@@ -284,15 +284,12 @@ xnor_nn_status_t exec_binarize_weights(const xnor_nn_convolution_t *c,
             weights_elems(st->g) * sizeof(float), &w);
     if (rc != xnor_nn_success) return rc;
     if (st->verbose) printf("xnor_nn exec binarize_weights: pack/alpha/op_count kernels\n");
+    char *packed = static_cast<char *>(res[xnor_nn_resource_bin_weights]);
     if (launch_binarize_weights(st->g, static_cast<const float *>(w),
-                static_cast<uint32_t *>(res[xnor_nn_resource_bin_weights]),
+                reinterpret_cast<uint32_t *>(packed),
+                st->g.use_mfma ? reinterpret_cast<uint32_t *>(packed + st->g.wfrag_offset) : nullptr,
                 static_cast<float *>(res[xnor_nn_resource_alpha]),
                 static_cast<int32_t *>(res[xnor_nn_resource_operations_count]), st->stream)
-            != hipSuccess)
-        return xnor_nn_error_memory;
-    if (st->g.use_mfma && launch_pack_weights_fp4(st->g, static_cast<const float *>(w),
-                reinterpret_cast<uint32_t *>(static_cast<char *>(
-                        res[xnor_nn_resource_bin_weights]) + st->g.wfrag_offset), st->stream)
             != hipSuccess)
         return xnor_nn_error_memory;
     return xnor_nn_success;

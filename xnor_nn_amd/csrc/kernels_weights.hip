@@ -2,7 +2,7 @@
 // and the per-output-pixel operation counts
 // (reference src/bcast_binarize_weights.cpp:54-142), plus the float sign(w)*mean(w)
 // helper (reference src/binarize_weights_float.cpp:3-25).  None of this is on the
-// per-forward path, so the kernels favour exact reference order over speed.
+// per-forward path, but a training iteration runs it every time.
 #include <mutex>
 
 #include "plan.hpp"
@@ -21,6 +21,247 @@ __device__ __forceinline__ size_t w_index(const Geometry &g, int oc, int ic, int
     if (g.w_fmt == xnor_nn_weights_format_oihw)
         return (((size_t)oc * g.ic + ic) * g.kh + kh) * g.kw + kw;
     return (((size_t)kh * g.kw + kw) * g.ic + ic) * g.oc + oc;
+}
+
+// Everything of a weight set in one launch, for OIHW weights whose filters fit the LDS: a
+// workgroup is one filter.  It reads the filter once, coalesced, and keeps it in LDS as
+// fl(|w| * chw) with the sign of w; then wave 0 adds the magnitudes in order (alpha) while the
+// other three pack the signs, as words for the XNOR/popcount kernel and the export helper and as
+// FP4 fragments for the matrix-core kernels.  The workgroups after the last filter compute the
+// operation counts.
+// The sum has to round after every addition like the reference's loop, one chain of IC*KH*KW
+// dependent additions: eight cycles each, 13 of this kernel's 17.6 us on the 256 x 384 x 3 x 3
+// weights of AlexNet's conv4 when it was walked that way.  ordered_sum below takes most of it 64
+// values at a time with the same roundings: 14.8 us.  The four kernels this one replaces
+// (three passes over the weights, two of them uncoalesced) took 12.9 + 32.2 + 4.7 + 5.7 us.
+constexpr int FILTER_WAVES = 4, FILTER_THREADS = 64 * FILTER_WAVES;
+constexpr int FILTER_CHUNK = 256;        // values the sum holds at a time, four per lane
+constexpr size_t FILTER_LDS = 64 * 1024; // of one filter at most
+
+struct FilterPlan {
+    int n, taps;               // values of a filter, kernel taps
+    int filters;               // workgroups that have a filter (padding filters included)
+    int frag_filters;          // filters of the fragment layout (0: no fragments)
+    int units, ks, pair, parts; // as pack_weights_fp4_kernel walks them
+    int row_codes;             // > 0: the layout of kernels_conv_shallow.hip instead
+    float chw;
+};
+
+// fl(...fl(fl(0 + |v[0]|) + |v[1]|)... + |v[n-1]|) by one wave, n a multiple of FILTER_CHUNK,
+// v in LDS; every lane returns the result.
+// While the running sum stays inside one binade, with units of u in its last place, adding x
+// moves it by exactly rint(x / u) units, whatever it is (x / u is exact: u is a power of two),
+// except when x / u lies halfway between two integers, where the sum's own last bit decides.
+// The moves are integers, so those of 64 values can be added in any order.  A row of 64 values
+// that has such a tie, or that carries the sum into the next binade (each binade once), is added
+// one by one.
+__device__ __forceinline__ float ordered_sum(const float *v, const int n, const int lane) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    uint32_t sum = 0; // bits of the running sum; adding m to them moves it by m units
+    auto one_by_one = [&](const float *row) {
+        float acc = __uint_as_float(sum);
+        v4f t[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = reinterpret_cast<const v4f *>(row)[i];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = __fadd_rn(acc, __builtin_fabsf(t[i][e]));
+        sum = (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(acc));
+    };
+    v4f x = reinterpret_cast<const v4f *>(v)[lane]; // lanes 16r .. 16r+15 hold row r
+    for (int base = 0; base < n; base += FILTER_CHUNK) {
+        const v4f next = reinterpret_cast<const v4f *>(
+                v + (base + FILTER_CHUNK < n ? base + FILTER_CHUNK : 0))[lane];
+        for (int row = 0; row < 4;) { // uniform
+            const uint32_t exponent = sum >> 23;
+            if (exponent >= 24) {
+                const float per_unit = __uint_as_float((277u - exponent) << 23); // 1 / u
+                uint32_t moves = 0;
+                bool tie = false;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    // more than a binade's worth is as good as exactly that
+                    const float units = fminf(__builtin_fabsf(x[e]) * per_unit, 8388608.f);
+                    const float whole = __builtin_rintf(units);
+                    moves += (uint32_t)whole;
+                    tie = tie || __builtin_fabsf(units - whole) == 0.5f;
+                }
+                // totals of the four rows of 16 lanes (row_shr 1, 2, 4, 8), in their last lanes
+                moves += __builtin_amdgcn_update_dpp(0, (int)moves, 0x111, 0xF, 0xF, true);
+                moves += __builtin_amdgcn_update_dpp(0, (int)moves, 0x112, 0xF, 0xF, true);
+                moves += __builtin_amdgcn_update_dpp(0, (int)moves, 0x114, 0xF, 0xF, true);
+                moves += __builtin_amdgcn_update_dpp(0, (int)moves, 0x118, 0xF, 0xF, true);
+                const uint64_t ties = __ballot(tie);
+                bool more = true;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)moves, 16 * r + 15);
+                    if (more && r == row) {
+                        more = ((ties >> (16 * r)) & 0xFFFFu) == 0
+                            && (uint64_t)(sum & 0x7FFFFFu) + m < 0x800000u;
+                        if (more) {
+                            sum += m;
+                            row++;
+                        }
+                    }
+                }
+            }
+            if (row < 4) one_by_one(v + base + 64 * row++);
+        }
+        x = next;
+    }
+    return __uint_as_float(sum);
+}
+
+__global__ __launch_bounds__(FILTER_THREADS)
+void binarize_filter_kernel(const float *__restrict__ w, uint32_t *__restrict__ bits,
+        uint32_t *__restrict__ frag, float *__restrict__ alpha, int32_t *__restrict__ opc,
+        const Geometry g, const FilterPlan f) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    extern __shared__ __attribute__((aligned(16))) float row[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int oc = blockIdx.x;
+    if (oc >= f.filters) { // operation counts (reference src/bcast_binarize_weights.cpp:126-142)
+        const int p = (oc - f.filters) * FILTER_THREADS + tid;
+        if (p >= g.ohw) return;
+        const int oh = p / g.ow, ow = p - oh * g.ow;
+        const int y = oh * g.sh - g.ph, x = ow * g.sw - g.pw;
+        const int ny = min(y + g.kh, g.ih) - max(y, 0), nx = min(x + g.kw, g.iw) - max(x, 0);
+        opc[p] = ny > 0 && nx > 0 ? ny * nx * g.ic : 0;
+        return;
+    }
+    const bool real = oc < g.oc; // uniform; a padding filter is written as ones / FP4 zeros
+    const int padded = (f.n + FILTER_CHUNK - 1) / FILTER_CHUNK * FILTER_CHUNK;
+    if (real) {
+        const float *src = w + (size_t)oc * f.n;
+        auto scaled = [&](float v) {
+            return __builtin_copysignf(__fmul_rn(__builtin_fabsf(v), f.chw), v);
+        };
+        if ((f.n & 3) == 0 && ((size_t)w & 15) == 0) { // rows start on 16-byte boundaries
+            const v4f *src4 = reinterpret_cast<const v4f *>(src);
+            for (int i0 = tid; i0 < padded / 4; i0 += 4 * FILTER_THREADS) {
+                v4f v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int i = i0 + u * FILTER_THREADS;
+                    v[u] = i < f.n / 4 ? src4[i] : v4f{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int i = i0 + u * FILTER_THREADS;
+                    if (i < padded / 4)
+                        reinterpret_cast<v4f *>(row)[i] = v4f{scaled(v[u][0]), scaled(v[u][1]),
+                                                              scaled(v[u][2]), scaled(v[u][3])};
+                }
+            }
+        } else {
+            for (int i0 = tid; i0 < padded; i0 += 8 * FILTER_THREADS) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int i = i0 + u * FILTER_THREADS;
+                    v[u] = i < f.n ? src[i] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int i = i0 + u * FILTER_THREADS;
+                    if (i < padded) row[i] = scaled(v[u]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        if (!real) return;
+        // reference src/bcast_binarize_weights.cpp:95-115; the +0 past the filter's end changes
+        // no sum
+        const float acc = ordered_sum(row, padded, tid);
+        if (tid == 0) alpha[oc] = acc;
+        return;
+    }
+    // sign bits (set: clear sign) of the 32 channels of word j at a tap; channels >= IC are ones
+    auto word_of = [&](int tap, int j) {
+        uint32_t word = 0xFFFFFFFFu;
+        if (real) {
+            const int c_n = min(32, g.ic - 32 * j);
+            const float *at = row + 32 * j * f.taps + tap;
+            for (int c0 = 0; c0 < c_n; c0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = at[min(c0 + u, c_n - 1) * f.taps];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (c0 + u < c_n && (__float_as_uint(v[u]) >> 31))
+                        word &= ~(0x80000000u >> (c0 + u));
+            }
+        }
+        return word;
+    };
+    const int ob = oc / g.q, qi = oc - ob * g.q;
+    auto put_word = [&](int tap, int j, uint32_t word) {
+        if (ob < g.ocb) bits[(((size_t)ob * f.taps + tap) * g.xw + j) * g.q + qi] = word;
+    };
+    // FP4 codes of the eight channels in a byte of sign bits (bit 7 = first channel = low nibble)
+    auto codes = [&](uint32_t byte) {
+        uint32_t x = __brev(byte) >> 24; // bit i -> bit 4i
+        x = (x | x << 12) & 0x000F000Fu;
+        x = (x | x << 6) & 0x03030303u;
+        x = (x | x << 3) & 0x11111111u;
+        return 0xAAAAAAAAu ^ (x << 3);
+    };
+    constexpr int PACKERS = FILTER_THREADS - 64;
+    const int me = tid - 64;
+    const bool has_frag = oc < f.frag_filters;
+    if (f.row_codes > 0) { // few channels: kernel rows back to back
+        for (int i = me; i < f.taps * g.xw; i += PACKERS) put_word(i / g.xw, i % g.xw, word_of(i / g.xw, i % g.xw));
+        const int steps = f.ks;
+        for (int i = me; has_frag && i < steps * 8; i += PACKERS) { // dword i of the filter
+            const int kh = i / f.row_codes;
+            uint32_t out = 0;
+            for (int k = 0; k < 8; k++) {
+                const int b = (i - kh * f.row_codes) * 8 + k, kw = b / g.ic, c = b - kw * g.ic;
+                if (real && kh < g.kh && kw < g.kw)
+                    out |= ((__float_as_uint(row[c * f.taps + kh * g.kw + kw]) >> 31) ? 0xAu : 0x2u)
+                        << (4 * k);
+            }
+            const int step = i >> 3, half = (i >> 2) & 1;
+            frag[((((size_t)(oc >> 5) * steps + step) * 64) + (oc & 31) + 32 * half) * 4 + (i & 3)]
+                = out;
+        }
+        return;
+    }
+    const int positions = f.frag_filters ? 2 * f.ks : g.xw;
+    for (int i = me; i < f.units * positions; i += PACKERS) {
+        const int u = i / positions, s = i - u * positions;
+        int tap = u, j = s;
+        if (f.pair) {
+            tap = 2 * u + (s >= f.ks ? 1 : 0);
+            j = s >= f.ks ? s - f.ks : s;
+        } else if (f.parts > 1) {
+            tap = u / f.parts;
+            j = (u - tap * f.parts) * positions + s;
+        }
+        const bool source = tap < f.taps && j < g.xw;
+        uint32_t word = 0;
+        if (source) {
+            word = word_of(tap, j);
+            put_word(tap, j, word);
+        }
+        if (!has_frag) continue;
+        uint4 q = {0u, 0u, 0u, 0u};
+        if (source && real) {
+            const int c_n = g.ic - 32 * j; // codes of channels >= IC are zero
+            auto part = [&](int d) {
+                const int left = c_n - 8 * d;
+                return left <= 0 ? 0u : left >= 8 ? codes((word >> (24 - 8 * d)) & 0xFF)
+                    : codes((word >> (24 - 8 * d)) & 0xFF) & (0xFFFFFFFFu >> (32 - 4 * left));
+            };
+            q = uint4{part(0), part(1), part(2), part(3)};
+        }
+        reinterpret_cast<uint4 *>(frag)[(((size_t)(oc >> 5) * f.units + u) * f.ks + (s >> 1)) * 64
+            + (oc & 31) + 32 * (s & 1)] = q;
+    }
 }
 
 // One thread per packed word of the device layout [OCB][KH*KW][XW][Q].
@@ -214,16 +455,14 @@ void op_count_kernel(int32_t *__restrict__ opc, const Geometry g) {
 // partial sums in the same fixed tree, so all of them multiply by the same mean.
 constexpr int PARTS = 256; // also the length of `scratch` above
 
-__device__ __forceinline__ float tree_sum_256(float v, float *lds) {
-    const int t = threadIdx.x;
-    lds[t] = v;
-    __syncthreads();
+// Sum of 256 values in a fixed tree (v[t] + v[t + 128], then 64, 32, ... apart), by one wave that
+// holds them as v[lane], v[lane + 64], v[lane + 128], v[lane + 192]; the result is in lane 0.
+__device__ __forceinline__ float tree_sum_256(const float v0, const float v1, const float v2,
+        const float v3) {
+    float v = __fadd_rn(__fadd_rn(v0, v2), __fadd_rn(v1, v3));
 #pragma unroll
-    for (int half = 128; half >= 1; half >>= 1) {
-        if (t < half) lds[t] = __fadd_rn(lds[t], lds[t + half]);
-        __syncthreads();
-    }
-    return lds[0];
+    for (int half = 32; half >= 1; half >>= 1) v = __fadd_rn(v, __shfl_down(v, half));
+    return v;
 }
 
 __global__ __launch_bounds__(256)
@@ -234,27 +473,83 @@ void partial_sum_kernel(const float *__restrict__ from, float *__restrict__ part
     const size_t lo = (size_t)blockIdx.x * per;
     const size_t hi = lo + per < n ? lo + per : n;
     float acc = 0.f;
-    for (size_t i = lo + threadIdx.x; i < hi; i += 256) acc = __fadd_rn(acc, from[i]);
-    const float sum = tree_sum_256(acc, lds);
-    if (threadIdx.x == 0) parts[blockIdx.x] = sum;
+    for (size_t i0 = lo + threadIdx.x; i0 < hi; i0 += 8 * 256) {
+        float v[8]; // eight loads under way together; +0 past the end changes no sum
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = i0 + u * 256 < hi ? from[i0 + u * 256] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc = __fadd_rn(acc, v[u]);
+    }
+    lds[threadIdx.x] = acc;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int t = threadIdx.x;
+    const float sum = tree_sum_256(lds[t], lds[t + 64], lds[t + 128], lds[t + 192]);
+    if (t == 0) parts[blockIdx.x] = sum;
 }
 
+// Every wave adds the partial sums for itself (no barrier).  VEC: both tensors lie on 16-byte
+// boundaries.
+template <bool VEC>
 __global__ __launch_bounds__(256)
 void sign_times_mean_kernel(const float *__restrict__ from, float *__restrict__ to,
         const float *__restrict__ parts, const size_t n, const float inv_n) {
-    __shared__ float lds[256];
-    const float mean = __fmul_rn(tree_sum_256(parts[threadIdx.x], lds), inv_n);
-    // four consecutive elements per thread
-    const size_t i0 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    const size_t i0 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; // four consecutive elements
+    const bool whole = VEC && i0 + 4 <= n;
+    v4f v = {0.f, 0.f, 0.f, 0.f};
+    if (whole) {
+        v = *reinterpret_cast<const v4f *>(from + i0);
+    } else {
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (i0 + u < n) to[i0 + u] = from[i0 + u] >= 0.f ? mean : -mean;
+        for (int u = 0; u < 4; u++)
+            if (i0 + u < n) v[u] = from[i0 + u];
+    }
+    const int lane = threadIdx.x & 63;
+    const float sum = tree_sum_256(parts[lane], parts[lane + 64], parts[lane + 128],
+            parts[lane + 192]);
+    const float mean = __fmul_rn(__uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(
+                                         (int)__float_as_uint(sum))), inv_n);
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = v[u] >= 0.f ? mean : -mean;
+    if (whole) {
+        *reinterpret_cast<v4f *>(to + i0) = v;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i0 + u < n) to[i0 + u] = v[u];
+    }
 }
 
 } // namespace
 
 hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits,
-        float *alpha, int32_t *opc, hipStream_t s) {
+        uint32_t *frag, float *alpha, int32_t *opc, hipStream_t s) {
+    const int taps = g.kh * g.kw;
+    const uint64_t n = (uint64_t)g.ic * taps;
+    if (g.w_fmt == xnor_nn_weights_format_oihw
+            && (n + FILTER_CHUNK) * sizeof(float) <= FILTER_LDS) {
+        FilterPlan f{};
+        f.n = (int)n;
+        f.taps = taps;
+        f.chw = 1.f / (g.ic * g.kh * g.kw);
+        f.units = taps;
+        f.parts = 1;
+        if (frag != nullptr) {
+            f.ks = g.mfma_steps;
+            f.pair = g.mfma_pair;
+            f.parts = g.mfma_parts;
+            f.row_codes = g.mfma_shallow ? (g.kw * g.ic + 7) / 8 : 0;
+            f.units = g.mfma_shallow ? 1 : f.pair ? (taps + 1) / 2 : taps * f.parts;
+            f.frag_filters = (int)(g.mfma_wbytes / ((size_t)f.units * f.ks * 1024)) * 32;
+        }
+        f.filters = g.ocb * g.q > f.frag_filters ? g.ocb * g.q : f.frag_filters;
+        const size_t lds = (n + FILTER_CHUNK - 1) / FILTER_CHUNK * FILTER_CHUNK * sizeof(float);
+        const unsigned count_blocks = (unsigned)(g.ohw + FILTER_THREADS - 1) / FILTER_THREADS;
+        hipLaunchKernelGGL(binarize_filter_kernel, dim3((unsigned)f.filters + count_blocks),
+                dim3(FILTER_THREADS), lds, s, w, bits, frag, alpha, opc, geometry(g), f);
+        return hipGetLastError();
+    }
     const size_t words = (size_t)g.ocb * g.kh * g.kw * g.xw * g.q;
     hipLaunchKernelGGL(pack_weights_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256),
             0, s, w, bits, geometry(g));
@@ -268,6 +563,7 @@ hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits
                 alpha, geometry(g), chw, FastDiv::make((uint32_t)(g.kh * g.kw)),
                 FastDiv::make((uint32_t)g.kw));
     hipLaunchKernelGGL(op_count_kernel, dim3((g.ohw + 255) / 256), dim3(256), 0, s, opc, geometry(g));
+    if (frag != nullptr) return launch_pack_weights_fp4(g, w, frag, s);
     return hipGetLastError();
 }
 
@@ -277,8 +573,13 @@ int weights_float_parts() { return PARTS; }
 hipError_t launch_weights_float(const float *from, float *to, size_t n, float *parts,
         hipStream_t s) {
     hipLaunchKernelGGL(partial_sum_kernel, dim3(PARTS), dim3(256), 0, s, from, parts, n);
-    hipLaunchKernelGGL(sign_times_mean_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256),
-            0, s, from, to, parts, n, 1.f / (float)n);
+    const dim3 grid((unsigned)((n + 1023) / 1024));
+    if ((((size_t)from | (size_t)to) & 15) == 0)
+        hipLaunchKernelGGL(sign_times_mean_kernel<true>, grid, dim3(256), 0, s, from, to, parts, n,
+                1.f / (float)n);
+    else
+        hipLaunchKernelGGL(sign_times_mean_kernel<false>, grid, dim3(256), 0, s, from, to, parts,
+                n, 1.f / (float)n);
     return hipGetLastError();
 }
 

@@ -205,8 +205,9 @@ hipError_t launch_box_filter(const Plan &g, const float *a, float *k, hipStream_
 // calibration: one pass of plain 16-byte reads over bytes / 16 * 16 bytes of device memory
 hipError_t launch_plain_read(const void *buf, size_t bytes, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
+// (frag_or_null: where the matrix-core kernel's fragments go, when it applies)
 hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits,
-        float *alpha, int32_t *opc, hipStream_t s);
+        uint32_t *frag_or_null, float *alpha, int32_t *opc, hipStream_t s);
 hipError_t launch_convolution(const Plan &g, const uint32_t *xbits,
         const uint32_t *wbits, const float *alpha, const float *k, const int32_t *opc,
         float *dst, int32_t *popc_or_null, hipStream_t s,
