@@ -171,3 +171,39 @@ def test_float_weights_at_any_length_and_alignment(oracle, gpu, n, shift):
         assert np.all(np.abs(np.abs(got[:n]) - abs(mean)) <= 1e-6 * np.mean(np.abs(w)))
     finally:
         conv.close()
+
+
+@pytest.mark.parametrize("t", [
+    (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0),        # four bytes each way
+    (1, 3, 5, 7, 7, 3, 3, 1, 1, 1, 1),        # byte counts that are no multiples of 16
+    (3, 31, 9, 47, 53, 3, 3, 1, 1, 1, 1),     # a little over a slice, one piece
+    (5, 67, 70, 61, 59, 3, 3, 1, 1, 1, 1),    # several pieces both ways, helpers
+    (2, 600, 8, 20, 20, 3, 3, 2, 2, 0, 0),    # much in, little out
+    (2, 4200, 8, 5, 5, 1, 1, 1, 1, 0, 0),     # no matrix cores: through the executors
+], ids=str)
+def test_host_tensors(oracle, t):
+    """Forward passes between host arrays, twice in a row on other inputs, with the arrays at odd
+    addresses."""
+    d, x, w = problem(t)
+    s = oracle_shape(oracle, d)
+    conv = make(d, w)
+    try:
+        for scale in (1.0, -2.0):
+            xs = x * np.float32(scale)
+            want = oracle.forward(s, xs, w)
+            held = np.full(xs.size + 1, np.float32(np.nan))[1:].reshape(xs.shape)
+            held[:] = xs
+            dst = np.full(want["dst"].size + 3, np.float32(7))
+            conv.forward(held, dst[1:-2])
+            assert same_bits(dst[1:-2], want["dst"].ravel())
+            assert dst[0] == 7 and np.all(dst[-2:] == 7)
+            assert same_bits(conv.export_floats(capi.RES_K), want["k"])
+            # ... and stage by stage
+            dst[:] = 7
+            conv.stage("binarize_data", src=held, dst=dst[1:-2])
+            conv.stage("calculate_k")
+            conv.stage("forward")
+            assert same_bits(dst[1:-2], want["dst"].ravel())
+            assert dst[0] == 7 and np.all(dst[-2:] == 7)
+    finally:
+        conv.close()

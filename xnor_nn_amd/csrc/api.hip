@@ -42,15 +42,30 @@ bool on_device(const void *p) {
     return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
 }
 
-// Device view of a user tensor the kernels read: the pointer itself, or a staged copy.
+// A staging buffer of the descriptor, allocated on first use.
+xnor_nn_status_t stage_buffer(void **slot, size_t bytes) {
+    if (*slot || hipMalloc(slot, (bytes + 15) & ~(size_t)15) == hipSuccess) return xnor_nn_success;
+    (void)hipGetLastError();
+    *slot = nullptr;
+    return xnor_nn_error_memory;
+}
+
+// Device view of a user tensor the kernels read: the pointer itself, or a staged copy.  `once`: a
+// tensor that is not staged on every pass goes through the runtime's own staging; pinned buffers
+// for it would take longer to allocate than they save.
 xnor_nn_status_t stage_in(State *st, void **slot, const void *user, size_t bytes,
-        const void **dev) {
+        const void **dev, bool once = false) {
     if (on_device(user)) { *dev = user; return xnor_nn_success; }
-    if (!*slot && hipMalloc(slot, bytes) != hipSuccess) return xnor_nn_error_memory;
-    if (hipMemcpyAsync(*slot, user, bytes, hipMemcpyHostToDevice, st->stream) != hipSuccess)
+    const xnor_nn_status_t rc = stage_buffer(slot, bytes);
+    if (rc != xnor_nn_success) return rc;
+    // (the bytes have left the user's buffer when this returns)
+    if (once) {
+        if (hipMemcpyAsync(*slot, user, bytes, hipMemcpyHostToDevice, st->stream) != hipSuccess
+                || hipStreamSynchronize(st->stream) != hipSuccess)
+            return xnor_nn_error_memory;
+    } else if (!st->io.run(st->stream, static_cast<const char *>(user), bytes,
+                static_cast<char *>(*slot), nullptr, 0, nullptr, [] { return true; }))
         return xnor_nn_error_memory;
-    // the host buffer may be pageable: the copy must have left it before we return
-    if (hipStreamSynchronize(st->stream) != hipSuccess) return xnor_nn_error_memory;
     *dev = *slot;
     return xnor_nn_success;
 }
@@ -281,7 +296,7 @@ xnor_nn_status_t exec_binarize_weights(const xnor_nn_convolution_t *c,
     withdraw_ready(res[xnor_nn_resource_a]);
     const void *w = nullptr;
     xnor_nn_status_t rc = stage_in(st, &st->stage_weights, res[xnor_nn_resource_user_weights],
-            weights_elems(st->g) * sizeof(float), &w);
+            weights_elems(st->g) * sizeof(float), &w, true);
     if (rc != xnor_nn_success) return rc;
     if (st->verbose) printf("xnor_nn exec binarize_weights: pack/alpha/op_count kernels\n");
     char *packed = static_cast<char *>(res[xnor_nn_resource_bin_weights]);
@@ -305,8 +320,8 @@ xnor_nn_status_t run_convolution(const xnor_nn_convolution_t *c, xnor_nn_resourc
     void *out = user_out;
     const bool direct = on_device(user_out);
     if (!direct) {
-        if (!st->stage_dst && hipMalloc(&st->stage_dst, bytes) != hipSuccess)
-            return xnor_nn_error_memory;
+        const xnor_nn_status_t rc = stage_buffer(&st->stage_dst, bytes);
+        if (rc != xnor_nn_success) return rc;
         out = st->stage_dst;
     }
     const uint32_t *xbits = static_cast<const uint32_t *>(res[xnor_nn_resource_bin_src]);
@@ -343,11 +358,9 @@ xnor_nn_status_t run_convolution(const xnor_nn_convolution_t *c, xnor_nn_resourc
                 dst, popc, st->stream, st->time_convolution.next());
     }
     if (err != hipSuccess) return xnor_nn_error_memory;
-    if (!direct) {
-        if (hipMemcpyAsync(user_out, out, bytes, hipMemcpyDeviceToHost, st->stream) != hipSuccess
-                || hipStreamSynchronize(st->stream) != hipSuccess)
-            return xnor_nn_error_memory;
-    }
+    if (!direct && !st->io.run(st->stream, nullptr, 0, nullptr, static_cast<char *>(user_out),
+                bytes, static_cast<const char *>(out), [] { return true; }))
+        return xnor_nn_error_memory;
     return xnor_nn_success;
 }
 
@@ -365,6 +378,21 @@ xnor_nn_status_t exec_forward(const xnor_nn_convolution_t *c, xnor_nn_resources_
     return run_convolution(c, res, res[xnor_nn_resource_user_dst], false);
 }
 
+// Withdraws what other calls have handed over through the buffers a whole forward pass is about
+// to overwrite.  Called with st->mu held.
+xnor_nn_status_t settle_before_pass(State *st, const float *a, const float *k) {
+    bool others = false; // box filters of other K planes that still have to read `a`
+    {
+        std::lock_guard<std::mutex> lock(handover_mu);
+        if (!ready_by_a.empty()) ready_by_a.erase(a);
+        if (!owed_by_k.empty()) {
+            owed_by_k.erase(k); // superseded: the plane is about to be written
+            for (const auto &e : owed_by_k) others = others || e.second.a == a;
+        }
+    }
+    return others ? settle_readers_of(st, a, k) : xnor_nn_success;
+}
+
 // A forward pass on device buffers in one call: what the three executors do one after the
 // other, without the records that hand mean|x| from one to the next (nothing can come between
 // the stages).  Two launches on the descriptor's stream.  Called with st->mu held.
@@ -372,19 +400,8 @@ xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const flo
         float *y) {
     float *a = static_cast<float *>(res[xnor_nn_resource_a]);
     float *k = static_cast<float *>(res[xnor_nn_resource_k]);
-    bool others = false; // box filters of other K planes that still have to read `a`
-    {
-        std::lock_guard<std::mutex> lock(handover_mu);
-        if (!ready_by_a.empty()) ready_by_a.erase(a);
-        if (!owed_by_k.empty()) {
-            owed_by_k.erase(k); // superseded: the plane is written below
-            for (const auto &e : owed_by_k) others = others || e.second.a == a;
-        }
-    }
-    if (others) {
-        const xnor_nn_status_t rc = settle_readers_of(st, a, k);
-        if (rc != xnor_nn_success) return rc;
-    }
+    const xnor_nn_status_t rc = settle_before_pass(st, a, k);
+    if (rc != xnor_nn_success) return rc;
     uint32_t *xbits = static_cast<uint32_t *>(res[xnor_nn_resource_bin_src]);
     if (launch_binarize_data(st->g, x, xbits, a, st->stream, st->time_binarize.next())
             != hipSuccess)
@@ -395,6 +412,26 @@ xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const flo
                    static_cast<const float *>(res[xnor_nn_resource_alpha]), k, y, nullptr, a, k,
                    st->stream, st->time_convolution.next()) == hipSuccess
         ? xnor_nn_success : xnor_nn_error_memory;
+}
+
+// A forward pass between host tensors (host_io.hpp): the input arrives piece by piece, the
+// kernels run, the output leaves piece by piece, without a synchronisation in between.  Called
+// with st->mu held.
+xnor_nn_status_t forward_on_host(State *st, xnor_nn_resources_t res, const void *src, void *dst) {
+    const Plan &g = st->g;
+    const size_t in_bytes = src_elems(g) * 4, out_bytes = dst_elems(g) * 4;
+    xnor_nn_status_t rc = stage_buffer(&st->stage_src, in_bytes);
+    if (rc == xnor_nn_success) rc = stage_buffer(&st->stage_dst, out_bytes);
+    if (rc != xnor_nn_success) return rc;
+    auto compute = [&] {
+        rc = forward_on_device(st, res, static_cast<const float *>(st->stage_src),
+                static_cast<float *>(st->stage_dst));
+        return rc == xnor_nn_success;
+    };
+    return st->io.run(st->stream, static_cast<const char *>(src), in_bytes,
+                   static_cast<char *>(st->stage_src), static_cast<char *>(dst), out_bytes,
+                   static_cast<const char *>(st->stage_dst), compute)
+        ? xnor_nn_success : rc != xnor_nn_success ? rc : xnor_nn_error_memory;
 }
 
 // The descriptor's stream, with st->mu held.
@@ -496,6 +533,7 @@ xnor_nn_status_t xnor_nn_init_convolution(xnor_nn_convolution_t *c,
 
     State *st = new (std::nothrow) State();
     if (!st) return xnor_nn_success; // executors stay "unimplemented", like a failed match
+    host_io_descriptor_created();
     Plan &g = st->g;
     g.mb = mb; g.ic = ic; g.ih = ih; g.iw = iw; g.oc = oc; g.oh = c->oh; g.ow = c->ow;
     g.kh = kh; g.kw = kw; g.sh = sh; g.sw = sw; g.ph = ph; g.pw = pw;
@@ -569,6 +607,7 @@ void xnor_nn_destroy_convolution(xnor_nn_convolution_t *c) {
     drop_timer(st->time_binarize);
     drop_timer(st->time_convolution);
     delete st;
+    host_io_descriptor_destroyed();
     c->state = nullptr;
 }
 
@@ -697,13 +736,20 @@ xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
             && is_data_format(c->dst_format);
         for (int i = xnor_nn_resource_internal; i < xnor_nn_resource_number; i++)
             complete = complete && res[i] != nullptr;
-        if (complete && st->g.use_mfma && fusion_on(st) && !st->verbose
-                && ((flags & XNOR_NN_HIP_DEVICE_POINTERS) || (on_device(src) && on_device(dst)))) {
-            const xnor_nn_status_t rc = forward_on_device(st, res, static_cast<const float *>(src),
-                    static_cast<float *>(dst));
-            if (rc == xnor_nn_success)
-                res[xnor_nn_resource_user_src] = res[xnor_nn_resource_user_dst] = nullptr;
-            return rc;
+        if (complete && st->g.use_mfma && fusion_on(st) && !st->verbose) {
+            const bool vouched = flags & XNOR_NN_HIP_DEVICE_POINTERS;
+            const bool in = vouched || on_device(src), out = vouched || on_device(dst);
+            xnor_nn_status_t rc = xnor_nn_unimplemented; // one of each: through the executors
+            if (in && out)
+                rc = forward_on_device(st, res, static_cast<const float *>(src),
+                        static_cast<float *>(dst));
+            else if (!in && !out)
+                rc = forward_on_host(st, res, src, dst);
+            if (rc != xnor_nn_unimplemented) {
+                if (rc == xnor_nn_success)
+                    res[xnor_nn_resource_user_src] = res[xnor_nn_resource_user_dst] = nullptr;
+                return rc;
+            }
         }
     }
     res[xnor_nn_resource_user_src] = const_cast<void *>(src);

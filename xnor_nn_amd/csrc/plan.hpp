@@ -15,6 +15,7 @@
 #include <mutex>
 #include <vector>
 
+#include "host_io.hpp"
 #include "xnor_nn.h"
 
 // Byte offset that the kernels give a buffer access they want the hardware to drop (a channel
@@ -177,8 +178,10 @@ struct State {
     // the order in which a call's launches and copies are enqueued belong to one call at a
     // time.
     std::mutex mu;
-    // staging buffers for host-side user tensors (allocated on first use)
+    // staging buffers for host-side user tensors (allocated on first use, a multiple of 16 bytes)
+    // and what moves the bytes
     void *stage_src = nullptr, *stage_weights = nullptr, *stage_dst = nullptr;
+    HostIo io;
     // partial sums of xnor_nn_binarize_weights_float (allocated on first use)
     float *float_parts = nullptr;
     // Stage fusion (xnor_nn_hip_set_stage_fusion): binarize_data hands mean|x| to the
