@@ -207,3 +207,21 @@ def test_host_tensors(oracle, t):
             assert dst[0] == 7 and np.all(dst[-2:] == 7)
     finally:
         conv.close()
+
+
+@pytest.mark.parametrize("separate_k", [False, True])
+@pytest.mark.parametrize("t", [
+    (1, 33, 8, 1, 1, 1, 1, 1, 1, 0, 0),        # one pixel, a word and one channel
+    (1, 128, 8, 4, 4, 1, 1, 1, 1, 0, 0),       # a set of words exactly, a tile exactly
+    (3, 129, 8, 5, 7, 3, 3, 1, 1, 1, 1),       # one channel more, tiles across images
+    (2, 1024, 8, 3, 3, 1, 1, 1, 1, 0, 0),      # one chunk, exactly
+    (2, 1025, 8, 3, 3, 1, 1, 1, 1, 0, 0),      # two chunks
+    (1, 3100, 8, 7, 7, 1, 1, 1, 1, 0, 0),      # four chunks, the last one ragged
+    (16, 40, 8, 16, 16, 3, 3, 1, 1, 1, 1),     # 64 tiles of 64 pixels: the last that are few
+    (16, 40, 8, 16, 17, 3, 3, 1, 1, 1, 1),     # 68: too many
+], ids=str)
+def test_few_input_pixels(oracle, monkeypatch, t, separate_k):
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, x, w)

@@ -202,6 +202,125 @@ void binarize_nhwc_tiled_kernel(const float *__restrict__ x, uint32_t *__restric
             tiles_per_xcd);
 }
 
+// NCHW input with few tiles of 64 pixels: tiles of T = 16 pixels, and a wave of its own for the
+// ordered sum.
+// The tiled kernel above walks the running sum from wave to wave, with a barrier at every
+// hand-over, and gives a tile's whole transfer to one compute unit: 2048 channels on 7x7,
+// minibatch 64, were 49 workgroups of 11 waves that took six rounds, 23.6 us.  Here a wave loads
+// four words (128 channels) of 16 pixels at a time, lane = (pixel, word); the loaders pack the
+// sign words and leave the magnitudes in LDS, channel by channel along a pixel's row, and the
+// last wave of the workgroup adds them, reading 32 values ahead, while the loaders fetch the next
+// chunk.  What bounds it is that chain: one addition per eight cycles and channel, 7 us for 2048
+// channels; 16.4 us in all there.
+struct SplitPlan {
+    uint32_t npix, ihw, ntiles, tiles_per_xcd;
+    int ic, xw, loaders, chunks;
+    FastDiv div_ihw;
+};
+constexpr int SPLIT_TILE = 16, SPLIT_WORDS = 64 / SPLIT_TILE, SPLIT_LOADERS = 8;
+
+template <int T, bool WRITE_BITS, bool WRITE_A>
+__global__ __launch_bounds__(64 * (SPLIT_LOADERS + 1))
+void binarize_nchw_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
+        float *__restrict__ a, const SplitPlan s, const float inv_ic) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    constexpr int G = 64 / T; // words a wave loads together
+    extern __shared__ __attribute__((aligned(16))) float split_lds[];
+    // a pixel's row in floats: 4 mod 64, so that the 16-byte accesses of both sides spread over
+    // the banks
+    const int chunk_words = s.loaders * G, row = chunk_words * 32 + 4;
+    // [one or two buffers][T pixels][row], then the packed words [T][xw]
+    uint32_t *stage = reinterpret_cast<uint32_t *>(split_lds + (s.chunks > 1 ? 2 : 1) * T * row);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = (blockIdx.x & 7) * s.tiles_per_xcd + (blockIdx.x >> 3);
+    if (tile >= s.ntiles) return;
+    const int lp = lane & (T - 1), lg = lane / T;
+    const uint32_t p = tile * T + lp;
+    auto meet = [] { // LDS is in place; loads from memory stay under way
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    if (wave < s.loaders) {
+        const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float *>(x), 0, (int)(s.npix * (uint32_t)s.ic * 4u), 0x00020000);
+        const uint32_t pc = p < s.npix ? p : s.npix - 1, img = s.div_ihw.div(pc);
+        const uint32_t plane = s.ihw * 4u;
+        const uint32_t pixel = (img * (uint32_t)s.ic * s.ihw + (pc - img * s.ihw)) * 4u;
+        float t[32];
+        auto load = [&](int k) { // this lane's word of chunk k
+            const int set = k * s.loaders + wave, j = set * G + lg, left = s.ic - 32 * j;
+            const uint32_t off = pixel + (uint32_t)(32 * j) * plane;
+            if (32 * (set + 1) * G <= s.ic) { // uniform: whole words
+#pragma unroll
+                for (int i = 0; i < 32; i++)
+                    t[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                            src, off, (uint32_t)i * plane, 0));
+            } else { // a channel past the end: an offset outside the buffer, which reads +0
+#pragma unroll
+                for (int i = 0; i < 32; i++)
+                    t[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                            src, i < left ? off + (uint32_t)i * plane : 0xFFFFFFF0u, 0, 0));
+            }
+        };
+        load(0);
+        for (int k = 0; k < s.chunks; k++) {
+            const int j = (k * s.loaders + wave) * G + lg;
+            uint32_t neg = 0; // sign bits, first channel ends up in the MSB
+            // (the sum of chunk k - 2, which used this buffer, ended ahead of the last barrier)
+            v4f *to = reinterpret_cast<v4f *>(split_lds + ((k & 1) * T + lp) * row
+                    + (wave * G + lg) * 32);
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                neg = __builtin_amdgcn_alignbit(neg, fbits(t[i]), 31);
+                t[i] = __fmul_rn(__builtin_fabsf(t[i]), inv_ic);
+            }
+            if (WRITE_A) {
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    to[i] = v4f{t[4 * i], t[4 * i + 1], t[4 * i + 2], t[4 * i + 3]};
+            }
+            if (WRITE_BITS && j < s.xw) stage[lp * s.xw + j] = (~neg) & top_bits(s.ic - 32 * j);
+            if (k + 1 < s.chunks) load(k + 1);
+            meet();
+        }
+    } else {
+        float sum = 0.f;
+        for (int k = 0; k < s.chunks; k++) {
+            meet();
+            if (!WRITE_A) continue;
+            const int words = min(chunk_words, s.xw - k * chunk_words); // uniform
+            const v4f *at = reinterpret_cast<const v4f *>(split_lds + ((k & 1) * T + lp) * row);
+            v4f u[8], v[8];
+            auto read = [&](v4f (&to)[8], int w) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) to[i] = at[8 * w + i];
+            };
+            auto add = [&](const v4f (&from)[8]) {
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) sum = __fadd_rn(sum, from[i][e]);
+            };
+            read(u, 0);
+            for (int w = 0; w < words; w += 2) {
+                if (w + 1 < words) read(v, w + 1);
+                add(u);
+                if (w + 1 < words) {
+                    if (w + 2 < words) read(u, w + 2);
+                    add(v);
+                }
+            }
+        }
+        if (WRITE_A && lane < T && p < s.npix) a[p] = sum;
+    }
+    if (!WRITE_BITS) return;
+    meet();
+    const uint32_t first = tile * (uint32_t)(T * s.xw), total = s.npix * (uint32_t)s.xw;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)(T * s.xw); i += blockDim.x)
+        if (first + i < total) bits[first + i] = stage[i];
+}
+
 // NCHW input of at most 32 channels (one packed word per pixel): a lane takes all channels of U
 // pixels 256 apart, so nothing is handed over between waves and nothing goes through LDS.  CH is
 // the channel count rounded up to a power of two (4 to 32), U = 32 / CH, so that a lane has up to
@@ -412,6 +531,35 @@ void launch_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipSt
                 dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
 }
 
+size_t split_lds_bytes(const Plan &g, int *loaders, int *chunks) {
+    const int sets = (g.xw + SPLIT_WORDS - 1) / SPLIT_WORDS; // of words that a wave loads together
+    *loaders = sets < SPLIT_LOADERS ? sets : SPLIT_LOADERS;
+    *chunks = (sets + *loaders - 1) / *loaders;
+    return sizeof(float) * ((*chunks > 1 ? 2 : 1) * SPLIT_TILE * (*loaders * SPLIT_WORDS * 32 + 4)
+            + SPLIT_TILE * (size_t)g.xw);
+}
+
+template <bool WRITE_BITS, bool WRITE_A>
+hipError_t launch_split(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
+        const KernelEvents &ev) {
+    SplitPlan p{};
+    p.npix = g.npix_in;
+    p.ihw = (uint32_t)g.ihw;
+    p.ntiles = (g.npix_in + SPLIT_TILE - 1) / SPLIT_TILE;
+    p.tiles_per_xcd = (p.ntiles + 7) / 8;
+    p.ic = g.ic;
+    p.xw = g.xw;
+    p.div_ihw = g.div_ihw;
+    const size_t lds = split_lds_bytes(g, &p.loaders, &p.chunks);
+    const auto kernel = binarize_nchw_kernel<SPLIT_TILE, WRITE_BITS, WRITE_A>;
+    static LdsGrant grant;
+    const hipError_t e = grant.ask((const void *)kernel, lds);
+    if (e != hipSuccess) return e;
+    launch_kernel(kernel, dim3(p.tiles_per_xcd * 8), dim3(64 * (p.loaders + 1)), lds, s, ev, x, bits,
+            a, p, 1.f / g.ic);
+    return hipSuccess;
+}
+
 template <int CH, bool WRITE_BITS, bool WRITE_A>
 void launch_shallow(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
         const KernelEvents &ev) {
@@ -464,6 +612,18 @@ static bool shallow_nchw(const Plan &g) {
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < (1ull << 31);
 }
 
+// Up to one tile of 64 pixels for every four compute units: AlexNet conv4 (384 channels) at
+// minibatch 1 / 8 / 32 (3 / 22 / 85 tiles) 4.2 / 4.5 / 5.9 us against 4.6 / 4.7 / 5.3 for the tiled
+// kernel, 1024 channels on 14x14 at minibatch 8 / 32 (25 / 98 tiles) 7.8 / 14.1 against 11.2 / 11.6,
+// 2048 channels on 7x7 at minibatch 1 / 64 (1 / 49 tiles) 10.4 / 16.4 against 18.0 / 23.0: with
+// more tiles the tiled kernel's whole cache lines count for more than the shorter walk.
+static bool split_nchw(const Plan &g) {
+    int loaders, chunks;
+    const uint32_t tiles = (g.npix_in + TILE - 1) / TILE;
+    return tiled_nchw(g) && tiles <= (uint32_t)g.cus / 4
+        && split_lds_bytes(g, &loaders, &chunks) <= 160 * 1024;
+}
+
 // The NHWC kernel reads 16 bytes per load at 32-bit byte offsets (and drops pieces past the
 // last channel the same way).
 static bool vector_nhwc(const Plan &g) {
@@ -497,6 +657,10 @@ hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
     if (shallow_nchw(g)) {
         if (a_or_null) launch_shallow_any<true, true>(g, x, bits, a_or_null, s, ev);
         else launch_shallow_any<true, false>(g, x, bits, nullptr, s, ev);
+    } else if (split_nchw(g)) {
+        const hipError_t e = a_or_null ? launch_split<true, true>(g, x, bits, a_or_null, s, ev)
+                                       : launch_split<true, false>(g, x, bits, nullptr, s, ev);
+        if (e != hipSuccess) return e;
     } else if (tiled_nchw(g)) {
         if (a_or_null) launch_tiled<false, true, true>(g, x, bits, a_or_null, s, ev);
         else launch_tiled<false, true, false>(g, x, bits, nullptr, s, ev);
@@ -527,6 +691,9 @@ hipError_t launch_mean_abs(const Plan &g, const float *x, float *a, hipStream_t 
     const float inv_ic = 1.f / g.ic;
     if (shallow_nchw(g)) {
         launch_shallow_any<false, true>(g, x, nullptr, a, s, KernelEvents{});
+    } else if (split_nchw(g)) {
+        const hipError_t e = launch_split<false, true>(g, x, nullptr, a, s, KernelEvents{});
+        if (e != hipSuccess) return e;
     } else if (tiled_nchw(g)) {
         launch_tiled<false, false, true>(g, x, nullptr, a, s, KernelEvents{});
     } else if (vector_nhwc(g) && !nhwc_by_lane(g)) {
