@@ -225,3 +225,37 @@ def test_few_input_pixels(oracle, monkeypatch, t, separate_k):
         monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
     d, x, w = problem(t, zeros=True)
     run_and_compare(oracle, d, x, w)
+
+
+@pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
+@pytest.mark.parametrize("t", [
+    (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0),         # one value
+    (1, 32, 33, 4, 8, 3, 3, 1, 1, 1, 1),       # a word, a tile exactly; paired taps
+    (2, 31, 70, 5, 7, 3, 3, 1, 1, 1, 1),       # ragged word, filters and tiles across images
+    (3, 32, 8, 9, 11, 1, 1, 2, 2, 0, 0),       # input pixels that no output reads
+    (2, 8, 40, 13, 12, 2, 3, 5, 4, 0, 1),      # the same, between and behind the tiles
+    (1, 33, 32, 6, 6, 3, 3, 1, 1, 2, 2),       # two words, ragged
+    (9, 64, 64, 7, 7, 3, 3, 1, 1, 1, 1),       # two words, many tiles
+    (1, 64, 96, 19, 40, 5, 3, 2, 1, 2, 0),     # a span of several rows a lane
+    (1, 24, 16, 12, 12, 7, 7, 1, 1, 3, 3),     # eight waves, paired taps
+    (1, 64, 16, 12, 12, 5, 5, 1, 1, 2, 2),     # eight waves, two words
+    (1, 20, 8, 200, 3, 3, 3, 1, 1, 0, 0),      # one pixel a row
+], ids=str)
+def test_one_launch_forward(oracle, gpu, monkeypatch, t, fmts, separate_k):
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, *in_layout(x, w, fmts), fmts, True, gpu)
+
+
+@pytest.mark.parametrize("t", [
+    (1, 160, 40, 12, 12, 5, 5, 1, 1, 2, 2),    # paired taps, 65 steps
+    (1, 96, 32, 9, 9, 5, 5, 1, 1, 2, 2),       # 39 steps
+    (1, 128, 70, 9, 9, 1, 1, 1, 1, 0, 0),      # two steps for four waves
+    (1, 384, 33, 5, 6, 1, 2, 1, 1, 0, 0),      # twelve steps for eight waves
+    (1, 384, 33, 5, 6, 1, 1, 1, 1, 0, 0),      # six steps
+    (2, 1030, 64, 7, 7, 3, 3, 1, 1, 1, 1),     # more than a ring per wave
+], ids=str)
+def test_steps_shared_by_waves(oracle, t):
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, x, w)

@@ -395,7 +395,8 @@ xnor_nn_status_t settle_before_pass(State *st, const float *a, const float *k) {
 
 // A forward pass on device buffers in one call: what the three executors do one after the
 // other, without the records that hand mean|x| from one to the next (nothing can come between
-// the stages).  Two launches on the descriptor's stream.  Called with st->mu held.
+// the stages).  One or two launches on the descriptor's
+// stream.  Called with st->mu held.
 xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const float *x,
         float *y) {
     float *a = static_cast<float *>(res[xnor_nn_resource_a]);
@@ -403,11 +404,16 @@ xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const flo
     const xnor_nn_status_t rc = settle_before_pass(st, a, k);
     if (rc != xnor_nn_success) return rc;
     uint32_t *xbits = static_cast<uint32_t *>(res[xnor_nn_resource_bin_src]);
+    const uint32_t *wfrag = reinterpret_cast<const uint32_t *>(
+            static_cast<const char *>(res[xnor_nn_resource_bin_weights]) + st->g.wfrag_offset);
+    // (kernel timing is per stage: two launches)
+    if (st->g.one_launch && st->time_binarize.ring.empty())
+        return launch_forward_small(st->g, x, xbits, a, wfrag,
+                       static_cast<const float *>(res[xnor_nn_resource_alpha]), k, y, st->stream)
+                == hipSuccess ? xnor_nn_success : xnor_nn_error_memory;
     if (launch_binarize_data(st->g, x, xbits, a, st->stream, st->time_binarize.next())
             != hipSuccess)
         return xnor_nn_error_memory;
-    const uint32_t *wfrag = reinterpret_cast<const uint32_t *>(
-            static_cast<const char *>(res[xnor_nn_resource_bin_weights]) + st->g.wfrag_offset);
     return launch_convolution_mfma(st->g, xbits, wfrag,
                    static_cast<const float *>(res[xnor_nn_resource_alpha]), k, y, nullptr, a, k,
                    st->stream, st->time_convolution.next()) == hipSuccess

@@ -1434,6 +1434,7 @@ void mfma_plan(Plan &g) {
     g.mfma_big_per_xcd = g.mfma_blocks_per_xcd = 0;
     g.mfma_small = g.mfma_small_rows = 0;
     g.mfma_small_lds = 0;
+    g.one_launch = 0;
     g.mfma_persist = g.mfma_reverse = 0;
     g.mfma_tiles_per_round = g.mfma_rounds = g.mfma_stagger = 0;
     g.mfma_parts = 1;
@@ -1454,6 +1455,7 @@ void mfma_plan(Plan &g) {
             g.mfma_small = 1;
             g.mfma_small_rows = rows;
             g.mfma_small_lds = lds;
+            g.one_launch = one_launch_applies(g) ? 1 : 0;
         }
     }
     // Two tile sizes in one launch (see the kernel): worth it when every compute unit gets

@@ -1,20 +1,31 @@
 // Stage 3 on the matrix cores for launches of few tiles (small batches): the same FP4
-// implicit GEMM as kernels_conv_mfma.hip, cut the other way.
+// implicit GEMM as kernels_conv_mfma.hip, cut the other way; and, for inputs of few channels, the
+// whole forward pass in one launch.
 // Semantics: reference src/default/bcast_convolution_default.cpp:60-105.
 //
 // The large-launch kernel gives a workgroup 32*PS pixels x 256 filters and every wave all
 // taps of its 64 filters: at minibatch 1 of AlexNet conv4 that is 6 workgroups on a chip of
 // 256 compute units, each wave walking 54 steps one behind the other with the latency of a
 // weight fetch between the groups.  Here a workgroup is one block of 32 pixels x ONE block of
-// 32 filters, and its four waves split the (tap, channel step) sequence between them: 48
-// workgroups for that problem, 13 or 14 matrix instructions per wave.  The partial sums are
-// exact integers in FP32, so the four waves' accumulators add up to the same bits in any
-// order; they meet in LDS and every wave scales and stores a quarter of the block.
+// 32 filters, and its waves split the (tap, channel step) sequence between them: 48
+// workgroups for that problem, 6 or 7 matrix instructions per wave.  The partial sums are
+// exact integers in FP32, so the waves' accumulators add up to the same bits in any order; they
+// meet in LDS and every wave scales and stores an eighth of the block.
 //
-// Nothing is hand-scheduled: a wave asks for its first weight fragments before it stages
-// the input (they arrive meanwhile), keeps a ring of eight fragments in flight and leaves
-// the waits to the compiler.
+// Nothing is hand-scheduled: a wave asks for its first eight weight fragments before it stages
+// the input (they arrive meanwhile; with eight waves they are usually all it needs), and the
+// waits are the compiler's.  What bounds it is one latency after the other: arguments, input,
+// barrier, operands, barrier, stores.
+//
+// FUSED (up to 64 channels): the workgroup starts from the float input.  A lane takes a pixel of
+// the tile's span: sign words straight to FP4 rows in LDS, mean|x| (in channel order, the
+// reference's) beside them.  Workgroups of the first filter block also store the packed words and
+// mean|x| of their share of the input, so that the pass leaves behind what the separate stages
+// leave.  Every filter block repeats the packing, which costs less than a second launch as long
+// as the launch is small: a pass is then bound by the host's 2.8 us per launch no more than by
+// the GPU.
 #include <cstdlib>
+#include <type_traits>
 
 #include "plan.hpp"
 
@@ -26,10 +37,15 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int SMALL_ROW_PAD = 16;     // spare bytes per LDS row, as in the large-launch kernel
 constexpr int SMALL_TABLE_BYTES = 1024;
 constexpr int SMALL_RING = 8;         // weight fragments in flight per wave
 constexpr uint32_t SMALL_DROP = 0xFFFFFFF0u;
+
+struct SmallPlan {
+    int max_rows, ks, nsteps, subs, row_bytes;
+    uint32_t blocks, wfrag_bytes;
+    FastDiv div_xw, div_ks, div_kw;
+};
 
 __device__ __forceinline__ v16f small_mfma_fp4(const v4i a, const v4i b, const v16f c) {
     const v8i a8 = {a.x, a.y, a.z, a.w, 0, 0, 0, 0};
@@ -38,64 +54,70 @@ __device__ __forceinline__ v16f small_mfma_fp4(const v4i a, const v4i b, const v
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a8, b8, c, 4, 4, 0, 0, 0, 0);
 }
 
-// FP4 codes of eight channels from one byte of packed sign bits (bit 7 = first channel,
-// set = sign bit clear = +1): nibble i = channel i, +1 -> 0x2, -1 -> 0xA.
+// FP4 codes of eight channels from one byte of sign bits, bit i (set = sign bit clear = +1) to
+// nibble i: +1 -> 0x2, -1 -> 0xA.
 __device__ __forceinline__ uint32_t small_fp4_of_byte(uint32_t byte) {
-    uint32_t out = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-        out |= (((byte >> (7 - i)) & 1u) ? 0x2u : 0xAu) << (4 * i);
-    return out;
+    uint32_t x = byte & 0xFFu;
+    x = (x | x << 12) & 0x000F000Fu;
+    x = (x | x << 6) & 0x03030303u;
+    x = (x | x << 3) & 0x11111111u;
+    return 0xAAAAAAAAu ^ (x << 3);
 }
 
-// LDS: [table 1 KB][rows: zero row + max_rows rows of ks*32 + 16 bytes][mean|x| of the staged
-// pixels + one slot of zero][partial sums: 4 waves x 12 registers x 64 lanes]
-__global__ __launch_bounds__(256)
+// LDS: [table 1 KB][rows: zero row + max_rows rows of row_bytes][mean|x| of the staged
+// pixels + one slot of zero][partial sums]
+// PAIR: the weight fragments of kernels_conv_mfma.hip's paired taps (an odd number KS of words
+// per pixel: two taps share KS steps, and the two halves of a wave may be at different taps).
+// WORDS: words per pixel that FUSED takes (0: from the packed input).
+template <int WAVES, int WORDS, bool PAIR>
+__global__ __launch_bounds__(64 * WAVES)
 void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag,
         const float *__restrict__ alpha, const float *__restrict__ kplane,
-        float *__restrict__ dst, const Geometry g, const int max_rows, const int ks,
-        const int subs, const uint32_t wfrag_bytes, const float *__restrict__ a_plane,
-        float *__restrict__ k_out, const float inv_khw, const FastDiv div_xw) {
-    extern __shared__ unsigned char smem[];
+        float *__restrict__ dst, const Geometry g, const SmallPlan s,
+        const float *__restrict__ a_plane, float *__restrict__ k_out, const float inv_khw,
+        const float *__restrict__ x, uint32_t *__restrict__ bits_out, float *__restrict__ a_out,
+        const float inv_ic) {
+    constexpr bool FUSED = WORDS > 0;
+    constexpr int THREADS = 64 * WAVES, KEEP = 16 / WAVES; // accumulator registers a wave finishes
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint32_t *table = reinterpret_cast<uint32_t *>(smem);
     unsigned char *rows = smem + SMALL_TABLE_BYTES;
-    const int row_bytes = ks * 32 + SMALL_ROW_PAD;
-    float *a_lds = reinterpret_cast<float *>(rows + (size_t)(1 + max_rows) * row_bytes);
-    float *parts = a_lds + ((max_rows + 1 + 3) & ~3);
+    float *a_lds = reinterpret_cast<float *>(rows + (size_t)(1 + s.max_rows) * s.row_bytes);
+    float *parts = a_lds + ((s.max_rows + 1 + 3) & ~3);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t block = blockIdx.x / (uint32_t)subs;
-    const int sub = (int)(blockIdx.x - block * (uint32_t)subs); // 32-filter block
+    const int half = lane >> 5;
+    const uint32_t block = s.subs == 1 ? blockIdx.x : blockIdx.x / (uint32_t)s.subs;
+    const int sub = (int)(blockIdx.x - block * (uint32_t)s.subs); // 32-filter block
     const uint32_t p_first = block * 32u, p_limit = g.npix_out;
-    const int taps = g.kh * g.kw, nsteps = taps * ks;
     // this wave's share of the steps
-    const int s_lo = (wave * nsteps) / 4, s_hi = ((wave + 1) * nsteps) / 4;
+    const int s_lo = (wave * s.nsteps) / WAVES, s_hi = ((wave + 1) * s.nsteps) / WAVES;
 
     // ---- weight fragments: [32-filter block][tap][step][lane]; the first ring is asked for now
     const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<v4i *>(wfrag), 0, (int)wfrag_bytes, 0x00020000);
+            const_cast<v4i *>(wfrag), 0, (int)s.wfrag_bytes, 0x00020000);
     const uint32_t wvoff = (uint32_t)lane * 16u;
-    const uint32_t wbase = (uint32_t)sub * (uint32_t)nsteps * 1024u;
-    auto fragment = [&](int s) { // a step past the wave's share reads outside the buffer: zeros
+    const uint32_t wbase = (uint32_t)sub * (uint32_t)s.nsteps * 1024u;
+    auto fragment = [&](int st) { // a step past the wave's share reads outside the buffer: zeros
         return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf,
-                s < s_hi ? wvoff : SMALL_DROP, s < s_hi ? wbase + (uint32_t)s * 1024u : 0u, 0));
+                st < s_hi ? wvoff : SMALL_DROP, st < s_hi ? wbase + (uint32_t)st * 1024u : 0u, 0));
     };
     v4i ring[SMALL_RING];
 #pragma unroll
     for (int i = 0; i < SMALL_RING; i++) ring[i] = fragment(s_lo + i);
 
-    // the alphas of the four filters this lane will scale (registers 4*wave .. +3 of the block:
-    // filters 8*wave + 4*(lane/32) + 0..3), asked for now so that the epilogue does not wait
-    const int f0 = sub * 32 + 8 * wave + 4 * (lane >> 5);
-    float al[4];
+    // the alphas of the filters this lane will scale (register i of the block is filter
+    // 8*(i/4) + 4*half + i%4), asked for now so that the epilogue does not wait
+    const int i0 = KEEP * wave, f0 = sub * 32 + 8 * (i0 >> 2) + 4 * half + (i0 & 3);
+    float al[KEEP];
 #pragma unroll
-    for (int ii = 0; ii < 4; ii++) al[ii] = f0 + ii < g.oc ? alpha[f0 + ii] : 0.f;
+    for (int ii = 0; ii < KEEP; ii++) al[ii] = f0 + ii < g.oc ? alpha[f0 + ii] : 0.f;
 
     // ---- the block's pixels, one per lane (both halves of the wave hold the same 32)
     int lo, hi;
     tile_span(g, p_first, min(p_first + 32u, p_limit), lo, hi);
-    const int nrows = min(hi - lo + 1, max_rows);
+    const int nrows = min(hi - lo + 1, s.max_rows);
     const uint32_t pix = p_first + (lane & 31);
     const bool live = pix < p_limit;
     const uint32_t pc = live ? pix : p_limit - 1;
@@ -111,64 +133,144 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     };
     const uint32_t rowmask = live ? run_of_bits(-ih0, g.ih - 1 - ih0) : 0u;
     const uint32_t colmask = run_of_bits(-iw0, g.iw - 1 - iw0);
-    // byte offsets into `rows`: the zero row, and the row of tap (0,0) of the lane's pixel
-    // (the upper half of the wave reads the second 32 channels of a step)
-    const int zero_off = (lane >> 5) * 16;
-    const int base_off = zero_off + (1 + in0) * row_bytes;
+    // byte offsets into `rows` of the row of tap (0,0) of the lane's pixel; row 0 is zero
+    const int base_off = (1 + in0) * s.row_bytes;
 
-    // ---- staging: table, zero row, mean|x|, FP4 rows
-    const bool fuse_k = a_plane != nullptr; // uniform
+    // ---- staging: zero row, mean|x|, FP4 rows
+    const bool fuse_k = FUSED || a_plane != nullptr; // uniform
     const float k_read = fuse_k ? 0.f : kplane[live ? pix : 0]; // asked for early
-    table[tid] = small_fp4_of_byte(tid);
-    for (int i = tid; i < row_bytes / 4; i += 256) reinterpret_cast<uint32_t *>(rows)[i] = 0;
-    if (fuse_k) {
-        for (int i = tid; i < nrows; i += 256) a_lds[i] = a_plane[lo + i];
-        if (tid == 0) a_lds[max_rows] = 0.f;
+    for (int i = tid; i < s.row_bytes / 4; i += THREADS) reinterpret_cast<uint32_t *>(rows)[i] = 0;
+    if (tid == 0) a_lds[s.max_rows] = 0.f;
+    if constexpr (FUSED) {
+        // The input pixels this workgroup packs: the tile's span and, in the first filter block,
+        // all from here to where the next tile's span begins (every input pixel is in exactly one
+        // such stretch).
+        const bool writes = sub == 0; // uniform
+        int from = lo, to = lo + nrows, w_from = 0, w_to = 0;
+        if (writes) {
+            int nlo, nhi;
+            w_from = block == 0 ? 0 : lo;
+            if (block + 1 < s.blocks) tile_span(g, p_first + 32u, min(p_first + 64u, p_limit), nlo, nhi);
+            else nlo = (int)g.npix_in;
+            w_to = nlo;
+            from = min(from, w_from);
+            to = max(to, w_to);
+        }
+        const bool planar = g.src_fmt == xnor_nn_data_format_nchw;
+        const uint32_t step = planar ? (uint32_t)g.ihw * 4u : 4u; // bytes from a channel to the next
+        const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float *>(x), 0, (int)(g.npix_in * (uint32_t)g.ic * 4u), 0x00020000);
+        for (int p0 = from; p0 < to; p0 += THREADS) {
+            const int p = p0 + tid;
+            const uint32_t q = p < to ? (uint32_t)p : (uint32_t)(to - 1);
+            const uint32_t im = g.div_ihw.div(q);
+            const uint32_t off = (planar ? im * (uint32_t)(g.ic * g.ihw) + (q - im * g.ihw)
+                                         : q * (uint32_t)g.ic) * 4u;
+            float v[WORDS * 32];
+#pragma unroll
+            for (int c = 0; c < WORDS * 32; c++)
+                v[c] = c < g.ic ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                        src, off, (uint32_t)c * step, 0)) : 0.f; // (uniform) |+0| adds nothing
+            float acc = 0.f;
+            uint32_t word[WORDS];
+#pragma unroll
+            for (int j = 0; j < WORDS; j++) {
+                uint32_t neg = 0; // sign bits, first channel ends up in the MSB
+#pragma unroll
+                for (int i = 0; i < 32; i++) {
+                    const float t = v[32 * j + i];
+                    neg = __builtin_amdgcn_alignbit(neg, __float_as_uint(t), 31);
+                    acc = __fadd_rn(acc, __fmul_rn(__builtin_fabsf(t), inv_ic));
+                }
+                const int left = g.ic - 32 * j;
+                word[j] = ~neg & (left >= 32 ? 0xFFFFFFFFu : ~(0xFFFFFFFFu >> left));
+            }
+            if (p >= to) continue;
+            if (p >= lo && p < lo + nrows) {
+                a_lds[p - lo] = acc;
+#pragma unroll
+                for (int j = 0; j < WORDS; j++) {
+                    const uint32_t r = __brev(word[j]);
+                    *reinterpret_cast<v4i *>(rows + (size_t)(1 + p - lo) * s.row_bytes + j * 16) =
+                        v4i{(int)small_fp4_of_byte(r), (int)small_fp4_of_byte(r >> 8),
+                            (int)small_fp4_of_byte(r >> 16), (int)small_fp4_of_byte(r >> 24)};
+                }
+            }
+            if (writes && p >= w_from && p < w_to) {
+                a_out[p] = acc;
+#pragma unroll
+                for (int j = 0; j < WORDS; j++) bits_out[(size_t)p * WORDS + j] = word[j];
+            }
+        }
+    } else {
+        if (fuse_k)
+            for (int i = tid; i < nrows; i += THREADS) a_lds[i] = a_plane[lo + i];
+        const int nitems = nrows * g.xw;
+        const uint32_t *run = xbits + (size_t)lo * g.xw;
+        uint32_t word[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            word[u] = u * THREADS + tid < nitems ? run[u * THREADS + tid] : 0u;
+        if (tid < 256) table[tid] = small_fp4_of_byte(__brev((uint32_t)tid) >> 24);
+        __syncthreads();
+        auto expand = [&](int i, uint32_t w) { // item i of the run -> 32 FP4 codes of its row
+            const int r = (int)s.div_xw.div((uint32_t)i), j = i - r * g.xw;
+            v4i q;
+            q.x = table[w >> 24];
+            q.y = table[(w >> 16) & 0xFF];
+            q.z = table[(w >> 8) & 0xFF];
+            q.w = table[w & 0xFF];
+            *reinterpret_cast<v4i *>(rows + (size_t)(1 + r) * s.row_bytes + j * 16) = q;
+        };
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (u * THREADS + tid < nitems) expand(u * THREADS + tid, word[u]);
+        for (int i = 4 * THREADS + tid; i < nitems; i += THREADS) expand(i, run[i]);
     }
-    const int nitems = nrows * g.xw;
-    const uint32_t *run = xbits + (size_t)lo * g.xw;
-    uint32_t word[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) word[u] = u * 256 + tid < nitems ? run[u * 256 + tid] : 0u;
-    __syncthreads();
-    auto expand = [&](int i, uint32_t w) { // item i of the run -> 32 FP4 codes of its row
-        const int r = (int)div_xw.div((uint32_t)i), j = i - r * g.xw;
-        v4i q;
-        q.x = table[w >> 24];
-        q.y = table[(w >> 16) & 0xFF];
-        q.z = table[(w >> 8) & 0xFF];
-        q.w = table[w & 0xFF];
-        *reinterpret_cast<v4i *>(rows + (size_t)(1 + r) * row_bytes + j * 16) = q;
-    };
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-        if (u * 256 + tid < nitems) expand(u * 256 + tid, word[u]);
-    for (int i = 1024 + tid; i < nitems; i += 256) expand(i, run[i]);
     __syncthreads();
 
-    // ---- this wave's steps: two accumulators in turn (the sums are exact, any order)
+    // ---- this wave's steps: two accumulators in turn (the sums are exact, any order).  The lane's
+    // operand of step st: word 2*(st % KS) + half of the words of its tap (PAIR: of the 2*KS words
+    // of a pair of taps).
     v16f acc0, acc1;
 #pragma unroll
     for (int i = 0; i < 16; i++) acc0[i] = acc1[i] = 0.f;
-    int tap = s_lo / ks, cs = s_lo - tap * ks; // uniform
-    auto row_of_tap = [&](int t) {
-        const int kh = t / g.kw, kw = t - kh * g.kw;
+    auto row_of_tap = [&](int t) { // a tap outside the image: the zero row
+        const int kh = (int)s.div_kw.div((uint32_t)t), kw = t - kh * g.kw;
         const uint32_t ok = (rowmask >> kh) & (colmask >> kw) & 1u;
-        return ok ? base_off + (kh * g.iw + kw) * row_bytes : zero_off;
+        return ok ? base_off + (kh * g.iw + kw) * s.row_bytes : 0;
     };
-    int rowoff = row_of_tap(tap < taps ? tap : 0);
-    for (int s = s_lo; s < s_hi; s += SMALL_RING) {
+    const int taps = g.kh * g.kw;
+    const int unit0 = (int)s.div_ks.div((uint32_t)s_lo);
+    int unit = unit0, cs = s_lo - unit0 * s.ks; // uniform
+    int first_row = 0, second_row = 0;
+    auto enter_unit = [&]() {
+        if constexpr (PAIR) {
+            first_row = 2 * unit < taps ? row_of_tap(2 * unit) : 0;
+            second_row = 2 * unit + 1 < taps ? row_of_tap(2 * unit + 1) : 0;
+        } else {
+            first_row = row_of_tap(unit < taps ? unit : 0);
+        }
+    };
+    enter_unit();
+    auto operand = [&]() {
+        const int w = 2 * cs + half;
+        const int at = PAIR ? (w < s.ks ? first_row + w * 16 : second_row + (w - s.ks) * 16)
+                            : first_row + w * 16;
+        return *reinterpret_cast<const v4i *>(rows + at);
+    };
+    for (int st = s_lo; st < s_hi; st += SMALL_RING) {
 #pragma unroll
         for (int i = 0; i < SMALL_RING; i++) {
-            if (s + i < s_hi) { // uniform
-                const v4i b = *reinterpret_cast<const v4i *>(rows + rowoff + cs * 32);
+            if (st + i < s_hi) { // uniform
+                const v4i b = operand();
                 if (i & 1) acc1 = small_mfma_fp4(ring[i], b, acc1);
                 else acc0 = small_mfma_fp4(ring[i], b, acc0);
-                ring[i] = fragment(s + i + SMALL_RING);
-                if (++cs == ks) {
+                ring[i] = fragment(st + i + SMALL_RING);
+                if (++cs == s.ks) {
                     cs = 0;
-                    tap++;
-                    rowoff = row_of_tap(tap < taps ? tap : 0);
+                    unit++;
+                    enter_unit();
                 }
             }
         }
@@ -176,47 +278,50 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
 #pragma unroll
     for (int i = 0; i < 16; i++) acc0[i] += acc1[i];
 
-    // ---- the four partial sums meet in LDS: wave w keeps registers 4w .. 4w+3 (filters
-    // 8w + 4*(lane/32) + 0..3 of the block) and gets the other waves' values for them
+    // ---- the partial sums meet in LDS: a wave keeps KEEP registers and gets the other waves'
+    // values for them
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (q == wave) continue; // uniform
-        const int slot = wave < q ? wave : wave - 1; // 0..2 among the three givers of quarter q
-#pragma unroll
-        for (int ii = 0; ii < 4; ii++)
-            parts[((q * 3 + slot) * 4 + ii) * 64 + lane] = acc0[4 * q + ii];
-    }
+    for (int i = 0; i < 16; i++)
+        if (i / KEEP != wave) parts[(wave * 16 + i) * 64 + lane] = acc0[i]; // uniform
     // ---- K of the lane's pixel, while the other waves finish their steps: the box filter's
     // own order (in-bounds taps, row-major, every product rounded, then added: reference
     // src/bcast_calculate_k.cpp:69-85), unless it came from the K plane
     float kv = k_read;
     if (fuse_k) {
         for (int kh = 0; kh < g.kh; kh++)
-            for (int kw = 0; kw < g.kw; kw++) {
-                const bool ok = (rowmask >> kh) & (colmask >> kw) & 1u;
-                // a tap outside the image reads the slot that holds zero: + 0 changes nothing
-                kv = __fadd_rn(kv, __fmul_rn(a_lds[ok ? in0 + kh * g.iw + kw : max_rows], inv_khw));
+            for (int kw0 = 0; kw0 < g.kw; kw0 += 4) { // four taps' reads under way together
+                float t[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int kw = kw0 + u;
+                    const bool ok = kw < g.kw && ((rowmask >> kh) & (colmask >> (kw & 31)) & 1u);
+                    // a tap outside the image reads the slot that holds zero: + 0 changes nothing
+                    t[u] = __fmul_rn(a_lds[ok ? in0 + kh * g.iw + kw : s.max_rows], inv_khw);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) kv = __fadd_rn(kv, t[u]);
             }
         if (sub == 0 && wave == 0 && lane < 32 && live) k_out[pix] = kv;
     }
 
     __syncthreads();
-    float sum[4];
+    float sum[KEEP];
 #pragma unroll
-    for (int ii = 0; ii < 4; ii++) {
+    for (int ii = 0; ii < KEEP; ii++) {
         float v = 0.f;
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (q == wave) v = acc0[4 * q + ii]; // uniform
+        for (int q = 0; q < WAVES; q++)
+            if (q == wave) v = acc0[KEEP * q + ii]; // uniform
 #pragma unroll
-        for (int slot = 0; slot < 3; slot++) v += parts[((wave * 3 + slot) * 4 + ii) * 64 + lane];
+        for (int q = 0; q < WAVES; q++)
+            if (q != wave) v += parts[(q * 16 + i0 + ii) * 64 + lane]; // uniform
         sum[ii] = v; // = 2*popc - n, exactly
     }
 
     // ---- epilogue: dst = fl(fl((float)(2*popc - n) * alpha) * k), every product rounded
     const bool nchw = g.dst_fmt == xnor_nn_data_format_nchw;
 #pragma unroll
-    for (int ii = 0; ii < 4; ii++) {
+    for (int ii = 0; ii < KEEP; ii++) {
         const int f = f0 + ii;
         if (f < g.oc && live) {
             const float out = __fmul_rn(__fmul_rn(sum[ii], al[ii]), kv);
@@ -227,31 +332,54 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     }
 }
 
+// Waves per workgroup: eight from twelve steps on (kernel plus binarize kernel, us with 4 / 8 waves:
+// 384 channels 3x3 (54 steps) 10.8 / 10.2, 48 channels 7x7 (49) 12.5 / 11.1, 128 channels 3x3 (18)
+// 9.5 / 8.8, 64 channels 3x3 (9) 8.1 / 8.4).
+int small_waves(const Plan &g) {
+    const int nsteps = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
+    return nsteps >= 12 ? 8 : 4;
+}
+
+int small_row_bytes(const Plan &g) {
+    // an odd number of 16-byte words per row spreads the fragment reads over the banks
+    return g.mfma_pair ? g.xw * 16 : g.mfma_steps * 32 + 16;
+}
+
+SmallPlan small_plan(const Plan &g) {
+    SmallPlan s{};
+    s.max_rows = g.mfma_small_rows;
+    s.ks = g.mfma_steps;
+    s.nsteps = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
+    s.subs = (g.oc + 31) / 32;
+    s.row_bytes = small_row_bytes(g);
+    s.blocks = (g.npix_out + 31) / 32;
+    s.wfrag_bytes = g.mfma_wbytes;
+    s.div_xw = FastDiv::make((uint32_t)g.xw);
+    s.div_ks = FastDiv::make((uint32_t)g.mfma_steps);
+    s.div_kw = FastDiv::make((uint32_t)g.kw);
+    return s;
+}
+
 } // namespace
 
-// Which problems take this kernel: one channel part, no tap pairing (the fragment layout of
-// paired taps is walked differently), and few enough (pixel block, filter block) pairs that
-// the large-launch kernel would leave most of the chip idle.  XNOR_NN_HIP_MFMA_SMALL=0|1
-// overrides the size rule (for measurements).
+// Which problems take this kernel: one channel part and few enough (pixel block, filter block)
+// pairs that the large-launch kernel would leave most of the chip idle.
+// XNOR_NN_HIP_MFMA_SMALL=0|1 overrides the size rule (for measurements).
 bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
-    if (!g.use_mfma || g.mfma_pair || g.mfma_parts > 1) return false;
+    if (!g.use_mfma || g.mfma_parts > 1) return false;
     const uint32_t blocks = (g.npix_out + 31) / 32;
     const uint32_t subs = (uint32_t)(g.oc + 31) / 32;
-    // measured on AlexNet conv4 (8 filter blocks): minibatch 1 / 2 / 4 / 8, i.e. 48 to 344
-    // pairs, 6.2 / 6.2 / 6.3 / 7.1 us against 7.4 / 7.5 / 7.6 / 7.9 us for the large-launch
-    // kernel; minibatch 16 (680 pairs) 8.4 against 8.1 us, minibatch 32 13.5 against 8.7 us
-    // With long walks (48 steps and more: conv4's 54, 72 for 512 channels) the split of the steps
-    // over four waves still pays at up to two pairs per compute unit: conv4 minibatch 12 (512
-    // pairs) 7.2 against 7.6 us, 512 -> 512 channels on 28x28 minibatch 1 (400 pairs) 8.0 against
-    // 8.6, on 14x14 minibatch 4 7.6 against 8.4, on 7x7 minibatch 20 (496 pairs) 7.5 against
-    // 8.5; with 36 steps (256 channels) the large-launch kernel is ahead there (6.9 against 7.2).
     const uint64_t pairs = (uint64_t)blocks * subs;
-    const int walk = g.kh * g.kw * g.mfma_steps;
+    const int walk = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
     bool take = pairs <= (uint64_t)g.cus + (uint64_t)g.cus / 2
         || (walk >= 48 && pairs <= 2 * (uint64_t)g.cus);
-    // a tile size, tile mix or persistent workgroups asked for by name mean the other kernel
+    // paired taps: from packed words only on long walks (160 channels 5x5, 65 steps: 11.2 us a pass
+    // against 13.5; 96 channels 3x3, 15 steps: 9.1 against 8.7 in the large kernel)
+    if (g.mfma_pair && g.xw > 1 && walk < 24) take = false;
+    // a tile size, tap pairing, tile mix or persistent workgroups asked for by name mean the
+    // other kernel
     if (getenv("XNOR_NN_HIP_MFMA_PS") || getenv("XNOR_NN_HIP_MFMA_MIX")
-            || getenv("XNOR_NN_HIP_MFMA_PERSIST"))
+            || getenv("XNOR_NN_HIP_MFMA_PERSIST") || getenv("XNOR_NN_HIP_MFMA_PAIR"))
         take = false;
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_SMALL")) take = e[0] == '1';
     if (!take) return false;
@@ -265,25 +393,72 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     };
     for (uint32_t b = 0; b < look; b++) see(b);
     see(blocks - 1);
-    const size_t row_bytes = (size_t)g.mfma_steps * 32 + SMALL_ROW_PAD;
-    const size_t lds = SMALL_TABLE_BYTES + (1 + (size_t)most) * row_bytes
-        + (((size_t)most + 1 + 3) & ~(size_t)3) * 4 + 4 * 3 * 4 * 64 * 4;
-    if (lds > 64 * 1024) return false;
+    const size_t lds = SMALL_TABLE_BYTES + (1 + (size_t)most) * small_row_bytes(g)
+        + (((size_t)most + 1 + 3) & ~(size_t)3) * 4 + small_waves(g) * (size_t)(16 * 64 * 4);
+    if (lds > 160 * 1024) return false;
     if (rows_out) *rows_out = most;
     if (lds_out) *lds_out = (uint32_t)lds;
     return true;
 }
 
+// Whether a forward pass on device buffers may run the one-launch form: up to 64 channels, 32-bit
+// offsets into the input (with room for the dropped one).  Measured per pass, device-bound: 32
+// channels 3x3 on 14x14, minibatch 1: 7.0 us against 8.2 for two launches, 64 channels on 56x56:
+// 8.1 against 8.5; called from Python through the torch module 8.5 against 11.4 (the host's part).
+bool one_launch_applies(const Plan &g) {
+    return g.mfma_small && g.xw <= 2
+        && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET;
+}
+
+#define XNOR_SMALL(WAVES_, WORDS_, PAIR_) \
+    do { \
+        static LdsGrant grant; \
+        const auto kernel = conv_mfma_fp4_small_kernel<WAVES_, WORDS_, PAIR_>; \
+        const hipError_t e = grant.ask((const void *)kernel, g.mfma_small_lds); \
+        if (e != hipSuccess) return e; \
+        launch_kernel(kernel, dim3(s.blocks * (uint32_t)s.subs), dim3(64 * WAVES_), \
+                (size_t)g.mfma_small_lds, stream, ev, xbits, wf, alpha, k, dst, geometry(g), s, \
+                a_or_null, k_out, 1.f / g.kh / g.kw, x, bits_out, a_out, 1.f / g.ic); \
+    } while (0)
+
 hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
-        const float *a_or_null, float *k_out, hipStream_t s, const KernelEvents &ev) {
-    const uint32_t blocks = (g.npix_out + 31) / 32;
-    const int subs = (g.oc + 31) / 32;
-    launch_kernel(conv_mfma_fp4_small_kernel, dim3(blocks * (uint32_t)subs), dim3(256),
-            (size_t)g.mfma_small_lds, s, ev, xbits, reinterpret_cast<const v4i *>(wfrag), alpha, k,
-            dst, geometry(g), g.mfma_small_rows, g.mfma_steps, subs, g.mfma_wbytes, a_or_null, k_out,
-            1.f / g.kh / g.kw, FastDiv::make((uint32_t)g.xw));
+        const float *a_or_null, float *k_out, hipStream_t stream, const KernelEvents &ev) {
+    const SmallPlan s = small_plan(g);
+    const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
+    const float *x = nullptr;
+    uint32_t *bits_out = nullptr;
+    float *a_out = nullptr;
+    if (small_waves(g) == 8) {
+        if (g.mfma_pair) XNOR_SMALL(8, 0, true);
+        else XNOR_SMALL(8, 0, false);
+    } else {
+        if (g.mfma_pair) XNOR_SMALL(4, 0, true);
+        else XNOR_SMALL(4, 0, false);
+    }
     return hipGetLastError();
 }
+
+// A whole forward pass (one_launch_applies): from the float input, leaving packed words, mean|x|
+// and K behind like the separate stages.
+hipError_t launch_forward_small(const Plan &g, const float *x, uint32_t *bits_out, float *a_out,
+        const uint32_t *wfrag, const float *alpha, float *k_out, float *dst, hipStream_t stream) {
+    const SmallPlan s = small_plan(g);
+    const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
+    const uint32_t *xbits = nullptr;
+    const float *k = nullptr, *a_or_null = nullptr;
+    const KernelEvents ev{};
+    if (small_waves(g) == 8) {
+        if (g.mfma_pair) XNOR_SMALL(8, 1, true);
+        else if (g.xw == 1) XNOR_SMALL(8, 1, false);
+        else XNOR_SMALL(8, 2, false);
+    } else {
+        if (g.mfma_pair) XNOR_SMALL(4, 1, true);
+        else if (g.xw == 1) XNOR_SMALL(4, 1, false);
+        else XNOR_SMALL(4, 2, false);
+    }
+    return hipGetLastError();
+}
+#undef XNOR_SMALL
 
 } // namespace xnor_hip

@@ -99,6 +99,7 @@ struct Plan : Geometry {
     int mfma_small;             // 1: few tiles: the small-problem kernel (kernels_conv_small.hip),
     int mfma_small_rows;        // the input pixels one of its blocks stages at most
     uint32_t mfma_small_lds;    // and its LDS bytes per workgroup
+    int one_launch;             // 1: a forward pass on device buffers is that kernel alone
     int mfma_shallow;           // > 0: few channels: the kernel of kernels_conv_shallow.hip with
                                 // tiles of this many output pixels,
     int mfma_shallow_rows;      // padded input rows per tile at most
@@ -241,6 +242,9 @@ hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s);
 const char *convolution_kernel_name(const Plan &g);
 // The matrix-core kernel for launches of few tiles (filled in by mfma_plan: g.mfma_small).
 bool small_kernel_applies(const Plan &g, int *rows, uint32_t *lds);
+bool one_launch_applies(const Plan &g);
+hipError_t launch_forward_small(const Plan &g, const float *x, uint32_t *bits_out, float *a_out,
+        const uint32_t *wfrag, const float *alpha, float *k_out, float *dst, hipStream_t s);
 hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
         const float *a_or_null, float *k_out, hipStream_t s,

@@ -62,23 +62,25 @@ class XnorConv2d(torch.nn.Module):
         self._weights_changed = False
 
     def forward(self, x):
-        if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 4
-                and x.shape[1] == self.in_channels):
+        shape, device = x.shape, x.device
+        if not (x.is_cuda and x.dtype is torch.float32 and len(shape) == 4
+                and shape[1] == self.in_channels):
             raise ValueError("XnorConv2d takes a float32 NCHW tensor on the GPU with %d channels"
                              % self.in_channels)
-        if self.weight.device != x.device:
+        weight = self.weight
+        if weight.device != device:
             raise ValueError("weight and input live on different devices")
         x = x.contiguous()
-        stream = _stream_handle(x.device)
+        stream = _stream_handle(device)
         # every kernel of this call, the weight stage included, goes to torch's current stream:
         # that orders it behind the writes to `weight` and `x` already enqueued there
-        if self._conv is None or self._shape != x.shape:
+        if self._conv is None or self._shape != shape:
             self._build(x)
         elif self._weights_changed:
             self._conv.set_stream(stream)
-            self._conv.change_weights(self.weight.data)
+            self._conv.change_weights(weight.data)
             self._weights_changed = False
-        y = torch.empty(self._out_shape, dtype=torch.float32, device=x.device)
+        y = x.new_empty(self._out_shape)
         self._conv.forward_on_stream(x, y, stream)
         return y
 
