@@ -317,3 +317,25 @@ def test_persistent_workgroups_are_planned_on_request_only(monkeypatch):
     # sixteen steps per tap have no four-block tile: never persistent
     assert kernel_names((8, 256, 1024, 14, 14, 3, 3, 1, 1, 1, 1))[1].startswith(
         "conv_mfma_fp4_kernel<KS=16")
+
+
+@pytest.mark.parametrize("t,small", [
+    ((2, 512, 128, 16, 16, 3, 3, 1, 1, 1, 1), True),    # one workgroup per compute unit (256)
+    ((2, 513, 128, 16, 16, 3, 3, 1, 1, 1, 1), False),   # a few more
+    ((8, 512, 256, 8, 8, 3, 3, 1, 1, 1, 1), True),      # 36 steps
+    ((8, 512, 384, 8, 8, 3, 3, 1, 1, 1, 1), True),      # 54 steps
+    ((16, 512, 384, 8, 8, 3, 3, 1, 1, 1, 1), True),     # ... two workgroups per compute unit
+    ((16, 513, 384, 8, 8, 3, 3, 1, 1, 1, 1), False),
+    ((1, 256, 384, 32, 64, 3, 3, 1, 1, 1, 1), False),   # ... a block touches 3 rows of 64
+    ((3, 512, 64, 16, 16, 3, 3, 1, 1, 1, 1), True),     # one launch a pass: 1.5
+    ((3, 513, 64, 16, 16, 3, 3, 1, 1, 1, 1), False),
+    ((3, 512, 64, 16, 16, 5, 5, 1, 1, 2, 2), False),    # ... not with 25 steps
+    ((1, 64, 256, 16, 16, 1, 1, 1, 1, 0, 0), False),    # four steps
+    ((1, 64, 384, 16, 16, 1, 1, 1, 1, 0, 0), True),     # six
+], ids=str)
+def test_where_the_kernel_for_few_tiles_begins(monkeypatch, t, small):
+    """Its size rule, on either side of each line (256 compute units)."""
+    for key in ("XNOR_NN_HIP_CONV", "XNOR_NN_HIP_MFMA_PS", "XNOR_NN_HIP_MFMA_MIX",
+                "XNOR_NN_HIP_MFMA_PAIR", "XNOR_NN_HIP_MFMA_PERSIST", "XNOR_NN_HIP_MFMA_SMALL"):
+        monkeypatch.delenv(key, raising=False)
+    assert kernel_names(t)[1].startswith("conv_mfma_fp4_small_kernel") == small

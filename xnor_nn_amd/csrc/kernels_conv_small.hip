@@ -362,27 +362,29 @@ SmallPlan small_plan(const Plan &g) {
 
 } // namespace
 
-// Which problems take this kernel: one channel part and few enough (pixel block, filter block)
-// pairs that the large-launch kernel would leave most of the chip idle.
+// Which problems take this kernel: one channel part and so few (pixel block, filter block) pairs,
+// a workgroup each, that the large-launch kernel would leave most of the chip idle.  Both were
+// timed on 150 problems (0.2 to 3 pairs per compute unit, 1x1 to 5x5, 17 to 1024 channels, 16 to
+// 768 filters; us a pass, large-launch / this):
+//   up to one pair per compute unit this kernel is ahead, by 1.06 to 1.55 (544 channels 3x3
+//   24.1 / 15.5), beyond it a second workgroup waits for the first and the large tiles are ahead
+//   (64 channels 5x5 on 12x12, 1.4 pairs: 10.8 / 12.6; 128 channels 3x3 on 22x22, 1.2: 9.4 / 10.4);
+//   with 48 steps or more in a walk, where the large-launch kernel is one long chain, two per
+//   compute unit while a block stages 112 input pixels at most (1000 channels 3x3 on 17x17, 2.0
+//   pairs: 17.7 / 15.5; conv4 of AlexNet, minibatch 12: 7.6 / 7.2 in the kernel; with more to stage
+//   2.0 pairs of 602 channels on 26x26: 19.7 / 20.6, 1.75 of 660 on 45x45: 27.3 / 30.8);
+//   with up to 64 channels and a short walk the pass is one launch here, which saves the host
+//   more than the kernel loses (1.1 pairs: 8.6 / 9.4 on the device, 11.4 / 8.5 through the torch
+//   module): 1.5 pairs;
+//   walks of up to four steps are not worth splitting (104 channels 1x1, 0.7 pairs: 7.8 / 8.3).
 // XNOR_NN_HIP_MFMA_SMALL=0|1 overrides the size rule (for measurements).
 bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     if (!g.use_mfma || g.mfma_parts > 1) return false;
     const uint32_t blocks = (g.npix_out + 31) / 32;
     const uint32_t subs = (uint32_t)(g.oc + 31) / 32;
-    const uint64_t pairs = (uint64_t)blocks * subs;
+    const uint64_t pairs = (uint64_t)blocks * subs, cus = (uint64_t)g.cus;
     const int walk = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
-    bool take = pairs <= (uint64_t)g.cus + (uint64_t)g.cus / 2
-        || (walk >= 48 && pairs <= 2 * (uint64_t)g.cus);
-    // paired taps: from packed words only on long walks (160 channels 5x5, 65 steps: 11.2 us a pass
-    // against 13.5; 96 channels 3x3, 15 steps: 9.1 against 8.7 in the large kernel)
-    if (g.mfma_pair && g.xw > 1 && walk < 24) take = false;
-    // a tile size, tap pairing, tile mix or persistent workgroups asked for by name mean the
-    // other kernel
-    if (getenv("XNOR_NN_HIP_MFMA_PS") || getenv("XNOR_NN_HIP_MFMA_MIX")
-            || getenv("XNOR_NN_HIP_MFMA_PERSIST") || getenv("XNOR_NN_HIP_MFMA_PAIR"))
-        take = false;
-    if (const char *e = getenv("XNOR_NN_HIP_MFMA_SMALL")) take = e[0] == '1';
-    if (!take) return false;
+    const bool one_launch = g.xw <= 2 && walk < 16;
     // input pixels a block of 32 output pixels touches at most (blocks start at multiples of 32)
     int most = 1;
     const uint32_t look = blocks < (uint32_t)g.ohw + 1 ? blocks : (uint32_t)g.ohw + 1;
@@ -393,6 +395,18 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     };
     for (uint32_t b = 0; b < look; b++) see(b);
     see(blocks - 1);
+    bool take = one_launch ? 2 * pairs <= 3 * cus
+        : walk >= 48 && most <= 112 ? pairs <= 2 * cus : walk > 4 && pairs <= cus;
+    // paired taps: from packed words only on long walks (160 channels 5x5, 65 steps: 11.2 us a pass
+    // against 13.5; 96 channels 3x3, 15 steps: 9.1 against 8.7 in the large kernel)
+    if (g.mfma_pair && g.xw > 1 && walk < 24) take = false;
+    // a tile size, tap pairing, tile mix or persistent workgroups asked for by name mean the
+    // other kernel
+    if (getenv("XNOR_NN_HIP_MFMA_PS") || getenv("XNOR_NN_HIP_MFMA_MIX")
+            || getenv("XNOR_NN_HIP_MFMA_PERSIST") || getenv("XNOR_NN_HIP_MFMA_PAIR"))
+        take = false;
+    if (const char *e = getenv("XNOR_NN_HIP_MFMA_SMALL")) take = e[0] == '1';
+    if (!take) return false;
     const size_t lds = SMALL_TABLE_BYTES + (1 + (size_t)most) * small_row_bytes(g)
         + (((size_t)most + 1 + 3) & ~(size_t)3) * 4 + small_waves(g) * (size_t)(16 * 64 * 4);
     if (lds > 160 * 1024) return false;
