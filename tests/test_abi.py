@@ -339,3 +339,25 @@ def test_where_the_kernel_for_few_tiles_begins(monkeypatch, t, small):
                 "XNOR_NN_HIP_MFMA_PAIR", "XNOR_NN_HIP_MFMA_PERSIST", "XNOR_NN_HIP_MFMA_SMALL"):
         monkeypatch.delenv(key, raising=False)
     assert kernel_names(t)[1].startswith("conv_mfma_fp4_small_kernel") == small
+
+
+@pytest.mark.parametrize("t,shallow", [
+    ((5, 64, 12, 32, 32, 5, 5, 1, 1, 2, 2), True),      # five steps, thirteen pairs of taps
+    ((5, 64, 13, 32, 32, 5, 5, 1, 1, 2, 2), False),     # six
+    ((4, 600, 11, 150, 150, 11, 11, 4, 4, 0, 0), True), # 22 of 61
+    ((4, 600, 12, 150, 150, 11, 11, 4, 4, 0, 0), False),
+    ((33, 32, 3, 32, 32, 3, 3, 1, 1, 1, 1), True),      # 264 tiles of 128 pixels
+    ((32, 32, 3, 32, 32, 3, 3, 1, 1, 1, 1), False),
+    ((132, 32, 3, 32, 32, 3, 3, 2, 2, 1, 1), False),
+    ((8, 32, 6, 32, 32, 7, 7, 1, 1, 3, 3), True),       # few tiles: six steps of 25, one launch
+    ((8, 32, 7, 32, 32, 7, 7, 1, 1, 3, 3), False),      # seven
+    ((9, 32, 7, 32, 32, 7, 7, 1, 1, 3, 3), True),       # ... not few
+    ((49, 97, 5, 8, 8, 7, 7, 2, 2, 3, 3), False),       # many padded rows to 64 pixels
+], ids=str)
+def test_where_the_kernel_for_few_channels_is_taken(monkeypatch, t, shallow):
+    """Its rule, on either side of each line (256 compute units)."""
+    for key in ("XNOR_NN_HIP_CONV", "XNOR_NN_HIP_MFMA_PS", "XNOR_NN_HIP_MFMA_MIX",
+                "XNOR_NN_HIP_MFMA_PAIR", "XNOR_NN_HIP_MFMA_PERSIST", "XNOR_NN_HIP_MFMA_SMALL",
+                "XNOR_NN_HIP_MFMA_GROUPS"):
+        monkeypatch.delenv(key, raising=False)
+    assert kernel_names(t)[1].startswith("conv_mfma_fp4_shallow_kernel") == shallow

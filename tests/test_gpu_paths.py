@@ -108,6 +108,21 @@ def test_few_channels(oracle, monkeypatch, t, fmts, separate_k):
 
 
 @pytest.mark.parametrize("t", [
+    (22, 3, 70, 227, 227, 11, 11, 4, 4, 0, 0),  # mean|x| in the operands' place, eight waves
+    (4, 3, 40, 33, 31, 5, 5, 1, 1, 2, 2),       # two bytes of codes per kernel row, rows left over
+    (3, 3, 70, 60, 58, 7, 7, 2, 2, 3, 3),       # three
+    (2, 4, 9, 40, 37, 7, 7, 1, 1, 3, 3),        # four
+    (2, 8, 130, 64, 64, 7, 7, 1, 1, 3, 3),      # seven: stored one by one
+    (2, 1, 8, 90, 90, 9, 9, 2, 2, 4, 4),        # a kernel width the sums of K are not unrolled for
+    (40, 2, 20, 30, 30, 3, 3, 1, 1, 1, 1),      # 17 pixels reach into a dword of the string
+], ids=str)
+def test_few_channels_gathering(oracle, t):
+    d, x, w = problem(t, zeros=True)
+    assert make(d, w).kernel_name(0).startswith("conv_mfma_fp4_shallow_kernel")
+    run_and_compare(oracle, d, x, w)
+
+
+@pytest.mark.parametrize("t", [
     (1, 1, 1, 3, 3, 1, 1, 1, 1, 0, 0),        # one value
     (1, 7, 5, 4, 4, 3, 3, 1, 1, 1, 1),        # 63 values: one short of a row of the sum
     (1, 257, 33, 4, 4, 1, 1, 1, 1, 0, 0),     # 257: one more than it holds; channels past a word

@@ -7,10 +7,12 @@
 // with three channels 29 of every 32 products are zeros, and AlexNet's first layer (3 channels,
 // 11x11) is 61 steps of 64 where its 363 products fill six.  Here the products of one kernel row
 // are packed back to back (33 bits there, rounded up to bytes): seven steps.  What bounds the
-// kernel then is its output and the instructions that gather the operands, so both are kept
-// few: a first version that collected a pixel's operand tap by tap issued 2000 scalar and 1200
-// vector instructions per wave and took 84 us on that layer (minibatch 64); this one takes
-// 34 us, the large-launch kernel 160 us.
+// kernel then is its output and the instructions and cache lines it takes to gather the operands,
+// so these are kept few: a first version that collected a pixel's operand tap by tap issued 2000
+// scalar and 1200 vector instructions per wave and took 84 us on that layer (minibatch 64), the
+// large-launch kernel 160 us; with rows as strings 34 us; with four pixels to a load of the
+// strings, two instructions to a pixel of them, 16-byte stores of the gathered codes and mean|x|
+// laid out by the stride (LDS bank conflicts 4.3 -> 1.2 million cycles) 31 us (the pass 53.4 -> 50.3).
 //
 // Workgroup = P consecutive output pixels (flattened mb, oh, ow) x a run of 32-filter blocks:
 //   1. rows: every input row the tile touches goes to LDS as one string of sign bits (IC bits per
@@ -61,11 +63,13 @@ struct ShallowPlan {
     int row_pixels;              // pixels that share one of them at most
     int row_bytes;               // of a pixel's FP4 row: steps * 32 + 16
     int blocks, blocks_per_wg;   // 32-filter blocks: all, and of one workgroup
-    int gathers;                 // waves that share the kernel rows of 64 pixels
+    int a_cols;                  // cells of a padded row's mean|x| with the same column mod stride
+    int a_shares_rows;           // 1: its LDS is that of the operands, which are gathered after it
+    int gathers;                 // waves that share the kernel rows of 64 pixels, four rows each
     uint32_t tiles, units, units_per_xcd;
     uint32_t wfrag_bytes;
     int nchw, stream;
-    FastDiv div_ohw, div_ow, div_prows, div_words, div_ic;
+    FastDiv div_ohw, div_ow, div_prows, div_words, div_ic, div_acols;
 };
 
 // First and last padded row (image * prows + row) that the output pixels [p0, p1) reach.
@@ -77,8 +81,14 @@ __host__ __device__ inline void padded_rows(const ShallowPlan &s, uint32_t p0, u
     r1 = i1 * s.prows + y1 * s.sh + s.kh - 1;
 }
 
+// LDS of the gathered operands and of mean|x|, in one place or one after the other.
+__host__ __device__ inline int operand_bytes(const ShallowPlan &s, int pixels, int rows) {
+    const int operands = pixels * s.row_bytes, cells = (rows * s.a_cols * s.sw * 4 + 15) & ~15;
+    return !s.a_shares_rows ? operands + cells : operands > cells ? operands : cells;
+}
+
 template <int P, int WAVES, bool RAW>
-__global__ __launch_bounds__(64 * WAVES)
+__global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 6 : 1) // three workgroups of eight waves
 void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
         const v4i *__restrict__ wfrag, const float *__restrict__ alpha,
         const float *__restrict__ kplane, float *__restrict__ dst, int32_t *__restrict__ popc,
@@ -91,8 +101,10 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
     float *k_lds = reinterpret_cast<float *>(smem + SHALLOW_TABLES);
     float *alpha_lds = k_lds + P;
     unsigned char *rows = reinterpret_cast<unsigned char *>(alpha_lds + s.blocks_per_wg * 32);
-    uint32_t *strings = reinterpret_cast<uint32_t *>(rows + P * s.row_bytes);
-    float *a_cells = reinterpret_cast<float *>(strings + s.max_rows * s.row_words);
+    const int a_pitch = s.a_cols * s.sw; // floats of mean|x| per padded row
+    float *a_cells = reinterpret_cast<float *>(s.a_shares_rows ? rows : rows + P * s.row_bytes);
+    uint32_t *strings = reinterpret_cast<uint32_t *>(rows
+            + operand_bytes(s, P, s.max_rows));
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -116,18 +128,21 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
     const __amdgpu_buffer_rsrc_t abuf = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float *>(a_plane), 0, fuse_k ? (int)in_bytes : 0, 0x00020000);
     // mean|x|: copied straight to LDS (nothing waits here and no register is held), a wave takes
-    // a row at a time, 64 pixels per instruction; outside the image the copy reads zero
+    // a row at a time, 64 pixels per instruction; outside the image the copy reads zero.  Columns
+    // that differ by the stride lie side by side: neighbouring output pixels then read
+    // neighbouring banks (with stride 4 a plain row had four lanes on every bank in use).
     if (fuse_k) {
         for (int r = wave; r < nrows; r += WAVES) {
             const uint32_t R = r0 + r, img = s.div_prows.div(R); // uniform
             const int y = (int)(R - img * s.prows) - s.ph;
             const bool row_ok = (unsigned)y < (unsigned)s.ih;
             const uint32_t at = ((img * s.ih + y) * s.iw - s.pw) * 4u;
-            for (int c0 = 0; c0 < s.pcols; c0 += 64) {
-                const int c = c0 + lane;
-                if (c < s.pcols)
+            for (int c0 = 0; c0 < a_pitch; c0 += 64) {
+                const int phase = (int)s.div_acols.div((uint32_t)(c0 + lane));
+                const int c = (c0 + lane - phase * s.a_cols) * s.sw + phase;
+                if (c0 + lane < a_pitch)
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(abuf,
-                            (lds_word *)(a_cells + r * s.pcols + c0), 4,
+                            (lds_word *)(a_cells + r * a_pitch + c0), 4,
                             row_ok && (unsigned)(c - s.pw) < (unsigned)s.iw ? at + 4u * c
                                                                             : SHALLOW_DROP,
                             0, 0, 0);
@@ -149,44 +164,58 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
             const int f = chunk * s.blocks_per_wg * 32 + i;
             alpha_lds[i] = f < s.oc ? alpha[f] : 0.f;
         }
-    // bit strings: a lane is a dword of one; it reads the pixels that reach into it
+    // bit strings: a lane is a dword of one; it reads the pixels that reach into it, last one
+    // first, and shifts the string along by a pixel's bits for each (two vector instructions a
+    // pixel).  Pixels outside the image are masked at the end: what was read for them is another
+    // pixel of the input, or zero outside the buffer.
     for (int i = tid; i < nrows * s.row_words; i += THREADS) {
         const int r = (int)s.div_words.div((uint32_t)i), d = i - r * s.row_words;
         const uint32_t R = r0 + r, img = s.div_prows.div(R);
         const int y = (int)(R - img * s.prows) - s.ph;
-        const bool row_ok = (unsigned)y < (unsigned)s.ih;
-        int x = (int)s.div_ic.div(32u * d) - s.pw;   // first pixel, may begin in the dword before
-        int pos = (x + s.pw) * s.ic - 32 * d;        // bit its first channel would have: <= 0
-        const uint32_t at = (img * s.ih + y) * s.iw * 4u;
+        const int first = (int)s.div_ic.div(32u * d), x = first - s.pw; // may begin in the dword before
+        const int pos = first * s.ic - 32 * d;  // bit its first channel would have: -IC < pos <= 0
+        const uint32_t at = ((img * s.ih + y) * s.iw + x) * 4u;
         uint32_t out = 0;
         auto collect = [&](auto batch) { // all loads of a batch are under way together
             constexpr int N = decltype(batch)::value;
-            for (int k0 = 0; k0 < s.row_pixels; k0 += N) { // uniform
+            // Four pixels a load: a wave's lanes are a dword of string apart and every load
+            // touches as many cache lines as four would, which is what these loads cost.  Only
+            // where all of them lie in the buffer: one that begins outside may be dropped whole.
+            const uint32_t reach = (uint32_t)((s.row_pixels + N - 1) / N * N) * 4u;
+            const bool wide = __all(reach <= in_bytes && at <= in_bytes - reach);
+            for (int k0 = (s.row_pixels - 1) / N * N; k0 >= 0; k0 -= N) { // uniform
                 uint32_t w[N];
+                if (wide) {
 #pragma unroll
-                for (int k = 0; k < N; k++) { // a pixel outside the image reads zero
-                    const bool ok = row_ok && (unsigned)(x + k0 + k) < (unsigned)s.iw;
-                    w[k] = __builtin_amdgcn_raw_buffer_load_b32(xbuf,
-                            ok ? at + 4u * (x + k0 + k) : SHALLOW_DROP, 0, 0);
+                    for (int k = 0; k < N; k += 4) {
+                        const v4i v = __builtin_bit_cast(v4i,
+                                __builtin_amdgcn_raw_buffer_load_b128(xbuf, at + 4u * (k0 + k), 0, 0));
+#pragma unroll
+                        for (int n = 0; n < 4; n++) w[k + n] = (uint32_t)v[n];
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+                        w[k] = __builtin_amdgcn_raw_buffer_load_b32(xbuf, at + 4u * (k0 + k), 0, 0);
                 }
 #pragma unroll
-                for (int k = 0; k < N; k++) {
-                    const uint32_t v = __brev(w[k]); // first channel lowest
-                    const int to = pos + (k0 + k) * s.ic;
-                    // (only the first pixel may begin in the dword before)
-                    if (k == 0) out |= to < 0 ? v >> -to : to < 32 ? v << to : 0u;
-                    else out |= to < 32 ? v << to : 0u;
-                }
+                for (int k = N - 1; k > 0; k--) // first channel lowest
+                    out = out << s.ic | __brev(w[k]);
+                if (k0 > 0) out = out << s.ic | __brev(w[0]);
+                else out = out << (s.ic + pos) | __brev(w[0]) >> -pos;
             }
         };
         if (s.row_pixels <= 4) collect(std::integral_constant<int, 4>{});
         else collect(std::integral_constant<int, 12>{});
-        strings[i] = out;
+        // bits of pixels inside the image: [lo, hi) of the dword
+        const int lo = max(max(-x, 0) * s.ic + pos, 0), hi = min((s.iw - x) * s.ic + pos, 32);
+        const bool some = (unsigned)y < (unsigned)s.ih && lo < hi;
+        strings[i] = some ? out & 0xFFFFFFFFu << lo & 0xFFFFFFFFu >> (32 - hi) : 0u;
     }
     __syncthreads();
 
-    // ---- gather: jobs of one wave over 64 pixels; part 0 sums K, parts 1.. take kernel rows -----
-    for (int job = wave; job < PB * (1 + s.gathers); job += WAVES) {
+    // ---- gather ----------------------------------------------------------------------------
+    auto gather_job = [&](const int job) {
         const int pb = job % PB, part = job / PB; // uniform
         const uint32_t p = p_first + pb * 64 + lane;
         const bool live = p < s.npix_out;
@@ -199,15 +228,30 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
             float sum = 0.f;
             if (fuse_k) { // in-bounds taps in row-major order, each product rounded, then added;
                           // a cell outside the image holds +0, which changes no sum
-                const float *row = a_cells + row0 * s.pcols + col0;
-                auto add_rows = [&](auto width) {
+                const float *row = a_cells + row0 * a_pitch + ox;
+                auto add_rows = [&](auto width) { // a row is asked for while the last one is added
                     constexpr int KW = decltype(width)::value;
-                    for (int y = 0; y < s.kh; y++, row += s.pcols) {
-                        float t[KW];
+                    int at[KW]; // uniform
 #pragma unroll
-                        for (int x = 0; x < KW; x++) t[x] = __fmul_rn(row[x], inv_khw);
+                    for (int x = 0, phase = 0, q = 0; x < KW; x++) {
+                        at[x] = phase * s.a_cols + q;
+                        if (++phase == s.sw) phase = 0, q++;
+                    }
+                    float t[KW];
 #pragma unroll
-                        for (int x = 0; x < KW; x++) sum = __fadd_rn(sum, t[x]);
+                    for (int x = 0; x < KW; x++) t[x] = row[at[x]];
+                    for (int y = 1; y <= s.kh; y++) {
+                        float next[KW];
+                        row += y < s.kh ? a_pitch : 0;
+#pragma unroll
+                        for (int x = 0; x < KW; x++) next[x] = row[at[x]];
+#pragma unroll
+                        for (int x = 0; x < KW; x++) t[x] = __fmul_rn(t[x], inv_khw);
+#pragma unroll
+                        for (int x = 0; x < KW; x++) {
+                            sum = __fadd_rn(sum, t[x]);
+                            t[x] = next[x];
+                        }
                     }
                 };
                 switch (s.kw) { // uniform
@@ -216,8 +260,14 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
                 case 7: add_rows(std::integral_constant<int, 7>{}); break;
                 case 11: add_rows(std::integral_constant<int, 11>{}); break;
                 default:
-                    for (int y = 0; y < s.kh; y++, row += s.pcols)
-                        for (int x = 0; x < s.kw; x++) sum = __fadd_rn(sum, __fmul_rn(row[x], inv_khw));
+                    for (int y = 0; y < s.kh; y++, row += a_pitch)
+                        if (s.sw == 1)
+                            for (int x = 0; x < s.kw; x++) sum = __fadd_rn(sum, __fmul_rn(row[x], inv_khw));
+                        else
+                            for (int x = 0, phase = 0, q = 0; x < s.kw; x++) {
+                                sum = __fadd_rn(sum, __fmul_rn(row[phase * s.a_cols + q], inv_khw));
+                                if (++phase == s.sw) phase = 0, q++;
+                            }
                 }
                 if (chunk == 0 && live) k_out[p] = sum;
             } else if (!RAW) {
@@ -228,9 +278,9 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
                 sum = (float)(ny > 0 && nx > 0 ? ny * nx * s.ic : 0);
             }
             k_lds[pb * 64 + lane] = sum;
-            continue;
+            return;
         }
-        const int ya = (part - 1) * s.kh / s.gathers, yb = part * s.kh / s.gathers;
+        const int ya = (part - 1) * 4, yb = min(ya + 4, s.kh); // gathers * 4 >= kh
         const uint32_t bit0 = col0 * s.ic; // where the pixel's products begin in a row's string
         const uint32_t shift = bit0 & 31u;
         const uint32_t *string = strings + row0 * s.row_words + (bit0 >> 5);
@@ -238,55 +288,93 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
         const int iy = (int)oy * s.sh - s.ph, ix = (int)ox * s.sw - s.pw;
         // products outside the image in this pixel's kernel rows: all but [in_a, in_b)
         const int in_a = max(0, -ix) * s.ic, in_b = min(s.kw, s.iw - ix) * s.ic;
-        auto gather = [&](auto edges) { // edges: some lane has taps outside its image
+        // The codes of the four rows are 4 * row_codes consecutive dwords of the pixel's operand, a
+        // whole number of 16-byte units: with the number known to the compiler they are stored as
+        // such (16-byte stores an odd number of units apart touch every bank, 4-byte stores a
+        // quarter of them).  What the units hold past the last kernel row meets weights of zero.
+        auto gather = [&](auto edges, auto width) { // edges: some lane has taps outside its image
             constexpr bool EDGES = decltype(edges)::value;
-            for (int y = ya; y < yb; y += 4) { // four kernel rows at a time (uniform)
-                const uint32_t *at[4];
-                uint32_t lo[4], *to[4];
-                bool row_in[4];
+            constexpr int RC = decltype(width)::value; // row_codes, 0: any
+            const int row_codes = RC ? RC : s.row_codes;
+            const uint32_t *at[4];
+            uint32_t lo[4];
+            bool row_in[4];
+            [[maybe_unused]] uint32_t unit[RC ? 4 * RC : 1];
 #pragma unroll
-                for (int k = 0; k < 4; k++) { // past the last: the last one again
-                    const int yk = min(y + k, yb - 1);
-                    at[k] = string + yk * s.row_words;
-                    to[k] = out + yk * s.row_codes;
-                    row_in[k] = (unsigned)(iy + yk) < (unsigned)s.ih;
-                    lo[k] = at[k][0];
+            for (int k = 0; k < 4; k++) { // past the last: the last one again
+                const int yk = min(ya + k, yb - 1);
+                at[k] = string + yk * s.row_words;
+                row_in[k] = (unsigned)(iy + yk) < (unsigned)s.ih;
+                lo[k] = at[k][0];
+            }
+            auto word = [&](const int c) { // codes c to c + 3
+                uint32_t bits[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const uint32_t hi = at[k][c / 4 + 1];
+                    bits[k] = __builtin_amdgcn_alignbit(hi, lo[k], shift);
+                    lo[k] = hi;
                 }
-                for (int c = 0; c < s.row_codes; c += 4) { // uniform
-                    uint32_t bits[4];
+                uint32_t columns = 0;
+                if constexpr (EDGES) {
+                    const int va = max(in_a - 8 * c, 0), vb = min(in_b - 8 * c, 32);
+                    if (va < vb) columns = (0xFFFFFFFFu << va) & (0xFFFFFFFFu >> (32 - vb));
+                }
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const uint32_t hi = at[k][c / 4 + 1];
-                        bits[k] = __builtin_amdgcn_alignbit(hi, lo[k], shift);
-                        lo[k] = hi;
-                    }
-                    uint32_t columns = 0;
-                    if constexpr (EDGES) {
-                        const int va = max(in_a - 8 * c, 0), vb = min(in_b - 8 * c, 32);
-                        if (va < vb) columns = (0xFFFFFFFFu << va) & (0xFFFFFFFFu >> (32 - vb));
-                    }
+                for (int i = 0; i < 4; i++)
+                    if (c + i < row_codes) { // uniform
+                        uint32_t q[4];
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (c + i < s.row_codes) { // uniform
-                            uint32_t q[4];
+                        for (int k = 0; k < 4; k++) q[k] = codes[(bits[k] >> (8 * i)) & 0xFF];
+                        if constexpr (EDGES) {
+                            const uint32_t in = masks[(columns >> (8 * i)) & 0xFF];
 #pragma unroll
-                            for (int k = 0; k < 4; k++) q[k] = codes[(bits[k] >> (8 * i)) & 0xFF];
-                            if constexpr (EDGES) {
-                                const uint32_t in = masks[(columns >> (8 * i)) & 0xFF];
-#pragma unroll
-                                for (int k = 0; k < 4; k++) q[k] = row_in[k] ? q[k] & in : 0u;
-                            }
-#pragma unroll
-                            for (int k = 0; k < 4; k++)
-                                if (y + k < yb) to[k][c + i] = q[k]; // uniform
+                            for (int k = 0; k < 4; k++) q[k] = row_in[k] ? q[k] & in : 0u;
                         }
-                }
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            if constexpr (RC > 0) unit[k * RC + c + i] = q[k];
+                            else if (ya + k < yb) out[(ya + k) * row_codes + c + i] = q[k]; // uniform
+                        }
+                    }
+            };
+            if constexpr (RC > 0) {
+#pragma unroll
+                for (int c = 0; c < RC; c += 4) word(c);
+            } else {
+                for (int c = 0; c < row_codes; c += 4) word(c); // uniform
+            }
+            if constexpr (RC > 0) {
+                v4i *to = reinterpret_cast<v4i *>(out + ya * RC);
+#pragma unroll
+                for (int u = 0; u < RC; u++)
+                    if (ya * RC + 4 * u < s.kh * RC) // uniform
+                        to[u] = v4i{(int)unit[4 * u], (int)unit[4 * u + 1], (int)unit[4 * u + 2],
+                                (int)unit[4 * u + 3]};
+            }
+        };
+        auto gather_rows = [&](auto edges) {
+            switch (s.row_codes) { // uniform
+            case 2: gather(edges, std::integral_constant<int, 2>{}); break;
+            case 3: gather(edges, std::integral_constant<int, 3>{}); break;
+            case 4: gather(edges, std::integral_constant<int, 4>{}); break;
+            case 5: gather(edges, std::integral_constant<int, 5>{}); break;
+            default: gather(edges, std::integral_constant<int, 0>{});
             }
         };
         const bool inside = !live || (iy >= 0 && iy + s.kh <= s.ih && ix >= 0
                 && ix + s.kw <= s.iw);
-        if (__all(inside)) gather(std::false_type{});
-        else gather(std::true_type{});
+        if (__all(inside)) gather_rows(std::false_type{});
+        else gather_rows(std::true_type{});
+    };
+    // jobs of one wave over 64 pixels; part 0 sums K, parts 1.. take kernel rows, after all of part
+    // 0 where mean|x| lies in the operands' place
+    for (int job = 0, end = s.a_shares_rows ? PB : PB * (1 + s.gathers);;) {
+        for (job += wave; job < end; job += WAVES) gather_job(job);
+        if (end > PB) break;
+        __syncthreads();
+        job = PB;
+        end = PB * (1 + s.gathers);
     }
     __syncthreads();
 
@@ -309,10 +397,9 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
         v16f acc[2];
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[0][i] = acc[1][i] = 0.f;
-        auto fragment = [&](int st) { // a step past the last reads outside the buffer: zeros
+        auto fragment = [&](int st) { // past the last step: the last one again, not used
             return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf,
-                    st < s.steps ? (uint32_t)lane * 16u : SHALLOW_DROP,
-                    st < s.steps ? wbase + (uint32_t)st * 1024u : 0u, 0));
+                    (uint32_t)lane * 16u, wbase + (uint32_t)min(st, s.steps - 1) * 1024u, 0));
         };
         v4i w[SHALLOW_AHEAD];
 #pragma unroll
@@ -339,8 +426,9 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
             // dst = fl(fl((float)(2*popc - n) * alpha) * k), rounded per product
             else return __float_as_uint(__fmul_rn(__fmul_rn(d, al), kv[q]));
         };
-        auto store_planes = [&](auto policy) { // NCHW: 64 consecutive pixels of a filter
+        auto store_planes = [&](auto policy, auto whole) { // NCHW: 64 consecutive pixels of a filter
             constexpr int AUX = decltype(policy)::value;
+            constexpr bool ALL = decltype(whole)::value; // no filter past the last
             const uint32_t p = p64 + lane, pc = p < s.npix_out ? p : s.npix_out - 1;
             const uint32_t im = s.div_ohw.div(pc);
             const uint32_t off = p < s.npix_out
@@ -355,18 +443,22 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
                     const auto r = __builtin_amdgcn_permlane32_swap(value(0, 4 * i4 + ii, al[ii]),
                             value(1, 4 * i4 + ii, al[ii]), false, false);
                     // r[0]: filter f, pixels lane; r[1]: filter f + 4
-                    if (all || f < s.oc)
+                    if (ALL || f < s.oc)
                         __builtin_amdgcn_raw_buffer_store_b32(r[0], outbuf, off,
                                 (uint32_t)f * fstep, AUX);
-                    if (all || f + 4 < s.oc)
+                    if (ALL || f + 4 < s.oc)
                         __builtin_amdgcn_raw_buffer_store_b32(r[1], outbuf, off,
                                 (uint32_t)(f + 4) * fstep, AUX);
                 }
             }
         };
         if (nchw) {
-            if (s.stream) store_planes(std::integral_constant<int, 2>{}); // nt
-            else store_planes(std::integral_constant<int, 0>{});
+            auto store = [&](auto policy) {
+                if (all) store_planes(policy, std::true_type{});
+                else store_planes(policy, std::false_type{});
+            };
+            if (s.stream) store(std::integral_constant<int, 2>{}); // nt
+            else store(std::integral_constant<int, 0>{});
         } else { // a lane holds four consecutive filters of a pixel
 #pragma unroll
             for (int q = 0; q < 2; q++) {
@@ -436,6 +528,9 @@ ShallowPlan make_plan(const Plan &g) {
     // (the last pixel's kernel row begins in the string and reads one dword past its last one)
     s.row_words = (s.pcols * g.ic + 31) / 32 + 2;
     s.row_pixels = 31 / g.ic + 2;
+    s.a_cols = (s.pcols + s.sw - 1) / s.sw;
+    s.gathers = (s.kh + 3) / 4;
+    s.div_acols = FastDiv::make((uint32_t)s.a_cols);
     s.row_bytes = s.steps * 32 + 16; // 4 mod 8 dwords: fragment reads spread over the banks
     s.blocks = (g.oc + 31) / 32;
     s.nchw = g.dst_fmt == xnor_nn_data_format_nchw ? 1 : 0;
@@ -467,21 +562,27 @@ int most_rows(const ShallowPlan &s, int pixels) {
 
 // The rest of the plan for tiles of `pixels` with `rows` padded rows at most and `per_wg` filter
 // blocks per workgroup; returns the LDS bytes.
-size_t set_tile(ShallowPlan &s, int pixels, int per_wg, int rows) {
+size_t set_tile(ShallowPlan &s, int pixels, int per_wg, int rows, int cus) {
     s.tiles = (s.npix_out + pixels - 1) / pixels;
     s.blocks_per_wg = per_wg;
     const uint32_t chunks = (uint32_t)(s.blocks + per_wg - 1) / per_wg;
     s.units = s.tiles * chunks;
     s.units_per_xcd = (s.units + 7) / 8;
-    s.gathers = 3; // with the wave that sums K: every wave has one job, or two
     s.max_rows = rows;
-    return SHALLOW_TABLES + ((size_t)pixels + 32 * per_wg) * 4 + (size_t)pixels * s.row_bytes
-        + (size_t)rows * (s.row_words + s.pcols) * 4;
+    auto lds = [&](int shares) {
+        s.a_shares_rows = shares;
+        return SHALLOW_TABLES + ((size_t)pixels + 32 * per_wg) * 4
+            + (size_t)operand_bytes(s, pixels, rows) + (size_t)rows * s.row_words * 4;
+    };
+    // A place of its own for mean|x| lets K be summed beside the gathering; sharing one lets more
+    // workgroups fit a compute unit, which is worth more where there are more of them (8 images of
+    // 227x227, 3 channels, 11x11, 379 tiles: 15.1 us a pass with its own, 17.9 shared).
+    const size_t own = lds(0), shared = lds(1), fit = SHALLOW_LDS / own;
+    return SHALLOW_LDS / shared > fit && fit < 4 && s.units > fit * (uint32_t)cus ? shared : lds(0);
 }
 
 // Output pixels per tile and filter blocks per workgroup.
 size_t choose_tile(const Plan &g, ShallowPlan &s, int *pixels) {
-    
     for (int p : {128, 64}) {
         // below two tiles of 128 per compute unit the smaller ones fill the chip better (100 images
         // of 32x32, 3 channels, 5x5: 12.2 us with 800 tiles of 128, 14.0 with 1600 of 64; 82 images
@@ -492,7 +593,7 @@ size_t choose_tile(const Plan &g, ShallowPlan &s, int *pixels) {
         uint32_t chunks = (2u * (uint32_t)g.cus + tiles - 1) / tiles;
         if (chunks > (uint32_t)s.blocks) chunks = (uint32_t)s.blocks;
         const int per_wg = (s.blocks + (int)chunks - 1) / (int)chunks;
-        const size_t lds = set_tile(s, p, per_wg, most_rows(s, p));
+        const size_t lds = set_tile(s, p, per_wg, most_rows(s, p), g.cus);
         if (lds <= (p == 128 ? SHALLOW_LDS / 2 : SHALLOW_LDS)) { *pixels = p; return lds; }
     }
     return 0;
@@ -500,11 +601,18 @@ size_t choose_tile(const Plan &g, ShallowPlan &s, int *pixels) {
 
 } // namespace
 
-// Up to 16 input channels and 20 taps or more (5x5 and up), where the large-launch kernel's pairs
-// of taps are mostly padding: 5x5, 30 to 100 images of 32x32, 3 to 16 channels: 6.4 to 15.1 us
-// against 8.3 to 14.9; 11x11 with stride 4: two to four times as fast.  With 3x3 kernels (five
-// pairs) the gathering costs more than it saves (64 images of 56x56, 16 channels, 64 filters: 19.1
-// against 16.7 us) unless the steps are a quarter (1 to 3 channels: equal or a little ahead).
+// Up to 16 input channels, where the large-launch kernel's pairs of taps are mostly padding.  Timed
+// beside it and beside the kernel for few tiles on 110 problems (us a pass, other / this):
+//   20 taps or more (5x5 and up) and at most 5/13 as many steps as pairs: ahead throughout, 5x5 of
+//   3 channels on 27x27 22.5 / 19.6, 7x7 of 5 channels on 46x46 34.2 / 19.2, 11x11 stride 4 of 3
+//   channels 28.3 / 13.1; with more steps the operands fill the LDS and the gathering costs what
+//   the shorter walk saves (16 channels 5x5 stride 2 on 24x24 10.4 / 13.2, on 94x94 17.9 / 14.9; 12
+//   channels 11x11 33.8 / 38.1);
+//   fewer taps: a quarter of the steps, stride 1 and a tile of 128 pixels per compute unit (3x3 of 3
+//   channels on 47x47 12.4 / 9.4; smaller or strided 6.5 / 7.5, 7.6 / 9.6);
+//   where the kernel for few tiles makes the pass one launch it stays ahead if the steps are more
+//   than a quarter, or a tile of 64 pixels reaches over many padded rows (7x7 of 7 channels on
+//   12x12 9.1 / 9.7, stride 2 on 7x7 8.9 / 12.9; 11x11 of 5 channels on 128x128 15.9 / 11.9).
 // Only where a tile's padded input rows fit the LDS; a tile shape or variant of another kernel
 // asked for by name means that kernel.
 bool shallow_plan(Plan &g) {
@@ -520,11 +628,17 @@ bool shallow_plan(Plan &g) {
         return false;
     ShallowPlan s = make_plan(g);
     const int taps = g.kh * g.kw, pairs = (taps + 1) / 2;
-    if (taps < 20 && 4 * s.steps > pairs) return false;
+    if (taps < 20 ? 4 * s.steps > pairs || g.sh > 1 || g.sw > 1
+                || g.npix_out <= 128u * (uint32_t)g.cus
+                  : 13 * s.steps > 5 * pairs)
+        return false;
     if ((uint64_t)s.blocks * s.steps * 1024u >= XNOR_HIP_DROPPED_OFFSET) return false;
     int pixels = 0;
     const size_t lds = choose_tile(g, s, &pixels);
     if (lds == 0) return false;
+    if ((uint64_t)((g.npix_out + 31) / 32) * (uint64_t)s.blocks <= (uint64_t)g.cus
+            && (4 * s.steps > pairs || s.max_rows > 40))
+        return false;
     g.mfma_shallow = pixels;
     g.mfma_shallow_rows = s.max_rows;
     g.mfma_shallow_blocks = s.blocks_per_wg;
@@ -538,7 +652,7 @@ hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t stream, const KernelEvents &ev) {
     ShallowPlan s = make_plan(g);
-    set_tile(s, g.mfma_shallow, g.mfma_shallow_blocks, g.mfma_shallow_rows);
+    set_tile(s, g.mfma_shallow, g.mfma_shallow_blocks, g.mfma_shallow_rows, g.cus);
     const dim3 grid(s.units_per_xcd * 8);
     const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
     const float inv_khw = 1.f / g.kh / g.kw;
@@ -551,9 +665,10 @@ hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         launch_kernel(kernel, grid, dim3(64 * W_), g.mfma_lds, stream, ev, xbits, wf, alpha, k, \
                 dst, popc, a_or_null, k_out, inv_khw, s); \
     } while (0)
-    if (g.mfma_shallow == 128 && g.mfma_lds > SHALLOW_LDS / 4) {
-        // few workgroups fit a compute unit: eight waves each (AlexNet's first layer, minibatch
-        // 64: 34 us against 44 with four; where four or more fit, four waves are as fast or faster)
+    if (g.mfma_shallow == 128 && g.mfma_shallow_blocks > 2 && g.mfma_lds > SHALLOW_LDS / 8) {
+        // with three filter blocks or more there are jobs for eight waves (us a pass with four and
+        // eight: AlexNet's first layer, minibatch 64, 48.9 / 43.0; 100 filters 16.6 / 15.1; with 64
+        // filters, 8 channels 7x7 on 112x112, 19.6 / 22.6), unless many workgroups fit
         if (popc) XNOR_SHALLOW(128, 8, true);
         else XNOR_SHALLOW(128, 8, false);
     } else if (g.mfma_shallow == 128) {
