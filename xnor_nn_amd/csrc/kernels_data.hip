@@ -285,6 +285,9 @@ void binarize_nchw_kernel(const float *__restrict__ x, uint32_t *__restrict__ bi
             meet();
         }
     } else {
+        // the chain is what the workgroup waits for: ahead of the loaders' packing on its SIMD (2048
+        // channels on 7x7, a pass at minibatch 1 / 64: 17.7 / 24.5 -> 17.0 / 23.7 us)
+        __builtin_amdgcn_s_setprio(3);
         float sum = 0.f;
         for (int k = 0; k < s.chunks; k++) {
             meet();
