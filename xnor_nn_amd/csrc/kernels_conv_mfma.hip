@@ -1403,18 +1403,23 @@ size_t mfma_weight_bytes(const Plan &g) {
     return (size_t)oc_subblocks(g) * units * steps_per_tap(g) * 1024;
 }
 
-// Output stores stream past the caches when the input of the next forward pass and this
-// output cannot both stay in the 256 MB Infinity Cache, and the runs of one filter start
-// on 64-byte boundaries: with ragged planes (13 x 13, 27 x 27) streaming stores leave
-// partial lines behind and cost the kernel 15 to 25 %, more than the next pass gains.
+// Output stores stream past the caches (nt) when the runs of one filter (NCHW) or of one pixel's
+// filters (NHWC) start on 64-byte boundaries and the output has more than 4 MB.  Written back, the
+// output pushes the input out of the 256 MB Infinity Cache and is still on its way to memory while
+// the next kernel reads.  us a pass written back / streamed, on changing buffers, and with a kernel
+// after it that reads the output: NHWC 100x32x32, 128 to 256 channels 48.3 / 39.1, 78.7 / 72.8;
+// NCHW 56x56 of 256 channels, minibatch 16, 39.3 / 31.8, 52.9 / 49.2; 64 channels, minibatch 64,
+// 33.1 / 27.4, 47.2 / 45.2; 32 to 64 channels 5x5 on 32x32 21.0 / 16.5, 29.5 / 28.2; on the same
+// buffers again 0.96 to 1.16 times as fast.  Below 4 MB nothing is gained (3 MB: 9.2 / 9.1, read
+// afterwards 11.7 / 11.8), and ragged planes leave partial lines behind: 13x13 44.5 / 46.7, on the
+// same buffers 36.6 / 43.1; 7x7 18.5 / 22.7; 14x14 22.1 / 21.0, read afterwards 30.8 / 32.4.
 // XNOR_NN_HIP_STREAM_DST=0|1 overrides, for measurements.
 static int stream_output(const Plan &g) {
     if (const char *e = getenv("XNOR_NN_HIP_STREAM_DST")) return e[0] == '1' ? 1 : 0;
-    const uint64_t in_bytes = (uint64_t)g.npix_in * g.ic * 4u;
     const uint64_t out_bytes = (uint64_t)g.npix_out * g.oc * 4u;
     const uint32_t run_bytes = g.dst_fmt == xnor_nn_data_format_nchw ? (uint32_t)g.ohw * 4u
                                                                      : (uint32_t)g.oc * 4u;
-    return in_bytes + out_bytes > (200ull << 20) && run_bytes % 64 == 0 ? 1 : 0;
+    return out_bytes > (4u << 20) && run_bytes % 64 == 0 ? 1 : 0;
 }
 
 void mfma_plan(Plan &g) {
