@@ -270,7 +270,7 @@ def test_kernel_variants_planned_for_known_shapes(monkeypatch):
         == "conv_mfma_fp4_kernel<KS=1,PS=2,GROUPS=4>"
     assert kernel_names((64, 128, 128, 56, 56, 3, 3, 1, 1, 1, 1))[1] \
         == "conv_mfma_fp4_kernel<KS=2,PS=2,GROUPS=2>"
-    # their one-block tiles are cheaper than the weight stream makes others, up to 63 steps
+    # their one-block tiles are cheaper than the weight stream makes others, up to 47 steps
     assert kernel_names((39, 96, 64, 30, 30, 3, 3, 1, 1, 1, 1))[1] \
         == "conv_mfma_fp4_kernel<KS=1,PS=1,GROUPS=2>"
     assert kernel_names((30, 96, 192, 24, 24, 5, 5, 1, 1, 2, 2))[1] \

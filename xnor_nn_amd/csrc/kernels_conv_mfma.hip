@@ -1181,7 +1181,8 @@ size_t lds_bytes(const Plan &g, int ps) {
 //               fewer) two or four waves of a workgroup read the same fragments and it costs
 //               1.3, unless the walk is long (64 to 96 channels 3x3 on 30x30, minibatch 39,
 //               a pass with one / three blocks 12.5 / 14.2 us; 76 to 40 on 59x59 one / two
-//               12.9 / 14.0; but 192 to 96 channels 5x5, 75 steps, 19.6 / 17.6: on 60 layers of
+//               12.9 / 14.0; but 384 to 64 channels 3x3 on 73x73, 54 steps, one / three 41.8 /
+//               39.7, 192 to 96 channels 5x5, 75 steps, one / two 19.6 / 17.6: on 60 layers of
 //               16 to 128 filters the mean distance from the fastest tile is 2.1 -> 1.0 %);
 //               Tiles of two pixel blocks pay 10 % more per step: their weight stream is
 //               as wide as the vector-memory return path of the CU;
@@ -1247,7 +1248,7 @@ int pick_ps(const Plan &g) {
         const double busiest = per_simd <= 1 ? 1.0
             : per_simd <= 4 ? (double)(long)(per_simd + 0.999999) : per_simd + 0.5;
         const double words = (double)max_tile_rows(g, mt) * g.xw;
-        const double one_block = g.mfma_groups > 1 && steps_total < 64 ? 1.3 : 2.0;
+        const double one_block = g.mfma_groups > 1 && steps_total < 48 ? 1.3 : 2.0;
         const double stream_bound = ps < 2 && per_simd > 1 ? one_block : (double)ps;
         const double wave = 3700.0 + 264.0 * words / 256.0 + 1700.0 * ps
             + (ps == 2 ? 70.4 : 64.0) * steps_total * stream_bound;

@@ -21,7 +21,8 @@
 //      row's string: one funnel shift per 32 of them, whatever the stride and channel count.
 //      They are expanded to FP4 through a 256-entry table (a second table clears the codes of
 //      taps outside the image) and stored as one LDS row per pixel.  One wave per 64 pixels sums
-//      K meanwhile (box filter of mean|x|, the reference's order).
+//      K meanwhile (box filter of mean|x|, the reference's order), or ahead of it where mean|x|
+//      shares the operands' LDS.
 //   3. multiply and store: a wave takes 32 filters x 64 pixels at a time; a pixel's row is read
 //      from front to back, there are no taps left.
 #include <cstdlib>
