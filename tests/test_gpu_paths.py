@@ -165,6 +165,36 @@ def test_scale_of_weights_the_sum_rounds_oddly(oracle, kind):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("kind", ["infinite", "late", "nan", "both", "outgrows"])
+def test_scale_of_weights_that_is_not_finite(oracle, kind):
+    """An infinite or NaN weight among the largest finite ones: the running sum stays what it has
+    become, bit for bit where it is a number."""
+    outgrows = kind == "outgrows" # 160 times the largest number, scaled by 1 / 160 and rounded
+    d, _, w = problem((1, 160, 16, 3, 3, 1, 1, 1, 1, 0, 0) if outgrows
+                      else (1, 64, 16, 3, 3, 4, 4, 1, 1, 1, 1))
+    flat = w.reshape(16, -1)
+    big = np.float32(2.0) ** np.arange(112, 128, dtype=np.float32) # scaled: 2^102 and up
+    flat[:] = np.sign(flat) * big[:, None]
+    rows = np.arange(16)
+    if kind in ("infinite", "both"):
+        flat[rows, rows] = np.float32(np.inf)
+    if kind == "late":
+        flat[rows, 900 + rows] = np.float32(-np.inf)
+    if kind in ("nan", "both"):
+        flat[rows[::2], 500 + rows[::2]] = np.float32(np.nan)
+    if outgrows:
+        flat[:] = np.finfo(np.float32).max
+    _, want, _ = oracle.binarize_weights(oracle_shape(oracle, d), w)
+    conv = make(d, w)
+    try:
+        got = conv.export_floats(capi.RES_ALPHA)
+    finally:
+        conv.close()
+    assert not np.all(np.isfinite(want))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert same_bits(got[~np.isnan(want)], want[~np.isnan(want)])
+
+
 @pytest.mark.parametrize("n,shift", [(1, 0), (255, 0), (1025, 1), (4096, 0), (600001, 0),
                                      (600001, 3)])
 def test_float_weights_at_any_length_and_alignment(oracle, gpu, n, shift):

@@ -54,7 +54,8 @@ struct FilterPlan {
 // except when x / u lies halfway between two integers, where the sum's own last bit decides.
 // The moves are integers, so those of 64 values can be added in any order.  A row of 64 values
 // that has such a tie, or that carries the sum into the next binade (each binade once), is added
-// one by one.
+// one by one; so is what meets an infinite or NaN sum (exponent 255), which has no units, and a
+// sum below 2^-103 (exponent under 24), whose unit may have no float for its reciprocal.
 __device__ __forceinline__ float ordered_sum(const float *v, const int n, const int lane) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     uint32_t sum = 0; // bits of the running sum; adding m to them moves it by m units
@@ -75,7 +76,7 @@ __device__ __forceinline__ float ordered_sum(const float *v, const int n, const 
                 v + (base + FILTER_CHUNK < n ? base + FILTER_CHUNK : 0))[lane];
         for (int row = 0; row < 4;) { // uniform
             const uint32_t exponent = sum >> 23;
-            if (exponent >= 24) {
+            if (exponent >= 24 && exponent < 255) {
                 const float per_unit = __uint_as_float((277u - exponent) << 23); // 1 / u
                 uint32_t moves = 0;
                 bool tie = false;
