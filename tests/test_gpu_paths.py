@@ -254,6 +254,37 @@ def test_host_tensors(oracle, t):
         conv.close()
 
 
+@pytest.mark.parametrize("which", ["src", "dst", "both"])
+@pytest.mark.parametrize("t", [
+    (1, 128, 40, 23, 21, 3, 3, 1, 1, 1, 1),   # small: through the library's buffers
+    (5, 67, 70, 61, 59, 3, 3, 1, 1, 1, 1),    # in place, byte counts that are no multiples of 16
+], ids=str)
+def test_pinned_host_tensors(oracle, gpu, t, which):
+    """Host tensors that the user has pinned, one or both, at odd addresses."""
+    import torch
+    d, x, w = problem(t)
+    want = oracle.forward(oracle_shape(oracle, d), x, w)["dst"]
+    pin = {n: which in (n, "both") for n in ("src", "dst")}
+    src = torch.full((x.size + 1,), float("nan"), pin_memory=pin["src"])
+    dst = torch.full((want.size + 3,), 7.0, pin_memory=pin["dst"])
+    src[1:] = torch.from_numpy(x.ravel())
+    conv = make(d, w)
+    try:
+        for stages in (False, True):
+            dst.fill_(7)
+            if stages:
+                conv.stage("binarize_data", src=src[1:].numpy(), dst=dst[1:-2].numpy())
+                conv.stage("calculate_k")
+                conv.stage("forward")
+            else:
+                conv.forward(src[1:].numpy(), dst[1:-2].numpy())
+            got = dst.numpy()
+            assert same_bits(got[1:-2], want.ravel())
+            assert got[0] == 7 and np.all(got[-2:] == 7)
+    finally:
+        conv.close()
+
+
 @pytest.mark.parametrize("separate_k", [False, True])
 @pytest.mark.parametrize("t", [
     (1, 33, 8, 1, 1, 1, 1, 1, 1, 0, 0),        # one pixel, a word and one channel

@@ -3,9 +3,10 @@
 // A pageable buffer handed to hipMemcpyAsync goes through the runtime's own staging at 32 (in)
 // and 18 GB/s (out).  Here the bytes go through pinned buffers of this library: the calling
 // thread and up to three helpers copy slices between the user's memory and the pinned buffers while a small
-// kernel moves the pieces that are ready over the link (a kernel reaches 53 GB/s on pinned
+// kernel moves the pieces that are ready over the link (a kernel reaches 51 GB/s on pinned
 // memory and costs a launch, where a copy engine costs 9 us per transfer), and flags in pinned
-// memory tell the host what has come back (no stream or event to wait for).  What bounds it is
+// memory tell the host what has come back (no stream or event to wait for).  A tensor that the
+// user has pinned is moved by a copy engine, in place.  What bounds it is
 // the link, in and then out.  Sending results back while input still arrives was built with a
 // second stream and is not used: two kernels together move 76 GB/s, but what ties the streams
 // together (events, or the host) cost more than that gained.
