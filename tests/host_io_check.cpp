@@ -70,7 +70,7 @@ std::map<const char *, size_t> host_blocks; // pinned, the library's and the use
 size_t host_bytes = 0, host_bytes_most = 0;
 std::atomic<long> host_allocations_left{1 << 30};
 std::atomic<int> launches{0}, engine_copies{0};
-std::atomic<bool> fail_queries{false};
+std::atomic<bool> fail_queries{false}, capturing{false};
 
 bool in_pinned(const char *p) {
     std::lock_guard<std::mutex> l(mem_mu);
@@ -98,16 +98,17 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
     *g = config.grid, *b = config.block, *lds = config.lds, *s = config.stream;
     return hipSuccess;
 }
-// link_copy_kernel(from, to, n, waiting, flag)
+// link_copy_kernel(from, to, n, waiting, flag, arrived)
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s) {
     launches++;
     const char *from = *static_cast<const char **>(args[0]);
     char *to = *static_cast<char **>(args[1]);
     const size_t n = *static_cast<size_t *>(args[2]);
     uint32_t *flag = *static_cast<uint32_t **>(args[4]);
+    const uint32_t arrived = *static_cast<uint32_t *>(args[5]);
     stream_of(s)->put([=] {
         memcpy(to, from, 16 * n);
-        if (flag) __atomic_store_n(flag, 1u, __ATOMIC_RELEASE);
+        if (flag) __atomic_store_n(flag, arrived, __ATOMIC_RELEASE);
     });
     return hipSuccess;
 }
@@ -133,7 +134,14 @@ hipError_t hipHostFree(void *p) {
 }
 hipError_t hipMalloc(void **p, size_t bytes) { return (*p = malloc(bytes)) ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipFree(void *p) { free(p); return hipSuccess; }
-hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) {
+    stream_of(s)->put([=] { memset(p, v, n); });
+    return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c) {
+    *c = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t s) {
     return fail_queries ? hipErrorUnknown : stream_of(s)->done() ? hipSuccess : hipErrorNotReady;
@@ -232,10 +240,83 @@ void pinned_tensors() {
             pass(io, stream, n, 2 * MB - 8, 4 + which, which & 1, which & 2, 12);
 }
 
+void sizes() {
+    Stream stream;
+    xnor_hip::HostIo io;
+    const size_t some[] = {0, 1, 4, 15, 16, MB / 4 - 1, MB / 4, MB / 4 + 1, MB / 2, 2 * MB - 4, 2 * MB,
+                           2 * MB + 4, 5 * MB + 12, 16 * MB, 16 * MB + 4, 41 * MB + 8};
+    unsigned seed = 0;
+    for (size_t in : some)
+        for (size_t out : some)
+            if (in + out > 0 && in + out < 60 * MB) {
+                seed++;
+                pass(io, stream, in, out, seed, false, false, seed % 16);
+            }
+}
+
+// The memory held is that of a pass's blocks, whatever the size of the tensors, and goes from pass to
+// pass and from descriptor to descriptor.
+void bounded() {
+    Stream stream;
+    for (int i = 0; i < 3; i++) {
+        xnor_hip::HostIo io;
+        pass(io, stream, 100 * MB, 60 * MB, i);
+        pass(io, stream, 60 * MB, 0, i);
+        pass(io, stream, 0, 70 * MB, i);
+    }
+    check(host_bytes_most <= 33 * MB, "pinned bytes at most", host_bytes_most);
+}
+
+// Without memory to pin the runtime copies; with some the blocks there are have to do.
+void no_pinned_memory() {
+    Stream stream;
+    for (long left = 0; left < 6; left++) {
+        xnor_hip::HostIo io;
+        host_allocations_left = left;
+        for (int i = 0; i < 3; i++) pass(io, stream, 9 * MB + 4, 7 * MB + 8, left + i);
+        check(left >= 2 || engine_copies == 6 * (left + 1), "passes by the runtime", left, engine_copies);
+        host_allocations_left = 1 << 30;
+        xnor_hip::host_io_descriptor_destroyed(); // the blocks go back to the system
+        xnor_hip::host_io_descriptor_created();
+    }
+}
+
+void threads() {
+    std::vector<std::thread> all;
+    for (unsigned t = 0; t < 4; t++)
+        all.emplace_back([t] {
+            Stream stream;
+            for (int i = 0; i < 6; i++) {
+                xnor_hip::HostIo io;
+                for (int j = 0; j < 3; j++) pass(io, stream, (3 + 5 * t + i) * MB + 4, 6 * MB - 4 * t, t + j);
+            }
+        });
+    for (std::thread &t : all) t.join();
+}
+
+// A stream that has failed, and one that is being captured, end the call.
+void refused() {
+    Stream stream;
+    xnor_hip::HostIo io;
+    pass(io, stream, 3 * MB, MB, 1);
+    capturing = true;
+    const int before = launches;
+    pass(io, stream, 3 * MB, MB, 2, false, false, 0, false);
+    check(launches == before, "launches under capture", launches - before);
+    capturing = false;
+    fail_queries = true;
+    stream.put([] { std::this_thread::sleep_for(std::chrono::milliseconds(300)); });
+    pass(io, stream, 3 * MB, MB, 3, false, false, 0, false);
+    fail_queries = false;
+    pass(io, stream, 3 * MB, MB, 4);
+}
+
 } // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, void (*)()> cases = {{"pinned tensors", pinned_tensors}};
+    const std::map<std::string, void (*)()> cases = {
+        {"pinned tensors", pinned_tensors}, {"sizes", sizes}, {"bounded", bounded},
+        {"no pinned memory", no_pinned_memory}, {"threads", threads}, {"refused", refused}};
     auto it = cases.find(argc > 1 ? argv[1] : "");
     if (it == cases.end()) {
         for (auto &c : cases) printf("%s\n", c.first.c_str());

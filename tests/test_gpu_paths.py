@@ -9,6 +9,7 @@ from test_gpu_boundary import make, same_bits, second_table
 from test_gpu_parity import run_and_compare
 from util import oracle_shape
 from xnor_nn_amd import capi, synth
+from xnor_nn_amd.convolution import XnorNNError
 
 pytestmark = pytest.mark.gpu
 
@@ -225,6 +226,7 @@ def test_float_weights_at_any_length_and_alignment(oracle, gpu, n, shift):
     (5, 67, 70, 61, 59, 3, 3, 1, 1, 1, 1),    # several pieces both ways, helpers
     (2, 600, 8, 20, 20, 3, 3, 2, 2, 0, 0),    # much in, little out
     (2, 4200, 8, 5, 5, 1, 1, 1, 1, 0, 0),     # no matrix cores: through the executors
+    (3, 67, 130, 191, 187, 3, 3, 1, 1, 1, 1), # more than the pinned blocks of a pass, both ways
 ], ids=str)
 def test_host_tensors(oracle, t):
     """Forward passes between host arrays, twice in a row on other inputs, with the arrays at odd
@@ -250,6 +252,29 @@ def test_host_tensors(oracle, t):
             conv.stage("forward")
             assert same_bits(dst[1:-2], want["dst"].ravel())
             assert dst[0] == 7 and np.all(dst[-2:] == 7)
+    finally:
+        conv.close()
+
+
+def test_host_tensors_under_capture(oracle, gpu):
+    """Nothing would arrive before the graph runs: refused, and the stream stays usable."""
+    import torch
+    d, x, w = problem((5, 67, 70, 61, 59, 3, 3, 1, 1, 1, 1))
+    want = oracle.forward(oracle_shape(oracle, d), x, w)["dst"]
+    conv = make(d, w)
+    try:
+        side = torch.cuda.Stream()
+        conv.set_stream(side)
+        dst = np.full(want.shape, np.nan, np.float32)
+        conv.forward(x, dst)
+        assert same_bits(dst, want)
+        dst.fill(7)
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
+            with pytest.raises(XnorNNError):
+                conv.forward(x, dst)
+        assert np.all(dst == 7)
+        conv.forward(x, dst)
+        assert same_bits(dst, want)
     finally:
         conv.close()
 
