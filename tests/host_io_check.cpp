@@ -1,7 +1,6 @@
 // HostIo (xnor_nn_amd/csrc/host_io.hip) on the CPU: its host code as it is, linked with these
 // stand-ins for the HIP runtime.  A stream is a thread that works through a queue; the transfer
 // kernel is replaced by what it does.  Usage: host_io_check CASE; prints what is wrong, if anything.
-#include <sys/resource.h>
 #include <time.h>
 
 #include <atomic>
@@ -161,7 +160,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
 
 namespace {
 
-int wrong = 0;
+std::atomic<int> wrong{0};
 void check(bool ok, const char *what, size_t a = 0, size_t b = 0) {
     if (ok) return;
     printf("wrong: %s (%zu, %zu)\n", what, a, b);
@@ -189,6 +188,13 @@ struct Tensor {
 
 unsigned char pattern(size_t i, unsigned seed) { return (unsigned char)((i * 2654435761u + seed) >> 13); }
 
+double processor_seconds() { // of all threads
+    timespec t;
+    clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t);
+    return t.tv_sec + 1e-9 * t.tv_nsec;
+}
+thread_local double run_seconds = 0; // of the last pass's call
+
 // One pass: in_bytes in, every output byte an input byte (inverted) or a pattern, out_bytes out.
 // expect: what run() has to return.
 void pass(xnor_hip::HostIo &io, Stream &stream, size_t in_bytes, size_t out_bytes, unsigned seed,
@@ -198,6 +204,7 @@ void pass(xnor_hip::HostIo &io, Stream &stream, size_t in_bytes, size_t out_byte
     for (size_t i = 0; i < in_bytes; i++) in.at[i] = (char)pattern(i, seed);
     memset(out.at, 0x5A, out_bytes + 8);
     bool computed = false;
+    const double before = processor_seconds();
     const bool ok = io.run(reinterpret_cast<hipStream_t>(&stream), in.at, in_bytes, dev_in.data(),
             out.at, out_bytes, dev_out.data(), [&] {
         computed = true;
@@ -208,6 +215,7 @@ void pass(xnor_hip::HostIo &io, Stream &stream, size_t in_bytes, size_t out_byte
         });
         return true;
     });
+    run_seconds = processor_seconds() - before;
     check(ok == expect, "result of run", in_bytes, out_bytes);
     check(expect == false || computed, "compute was not called", in_bytes, out_bytes);
     if (!ok) return;
@@ -294,6 +302,22 @@ void threads() {
     for (std::thread &t : all) t.join();
 }
 
+// A pass behind other work on the stream does not spend that time spinning.
+void busy_stream() {
+    Stream stream;
+    xnor_hip::HostIo io;
+    for (size_t in : {0 * MB, 9 * MB, 30 * MB})
+        for (size_t out : {0 * MB, 9 * MB, 30 * MB}) {
+            if (in + out == 0) continue;
+            pass(io, stream, in, out, 1);
+            const double alone = run_seconds;
+            stream.put([] { std::this_thread::sleep_for(std::chrono::milliseconds(400)); });
+            pass(io, stream, in, out, 2);
+            check(run_seconds < alone + 0.1, "processor milliseconds behind 400 of other work",
+                    (size_t)(1e3 * run_seconds), (size_t)(1e3 * alone));
+        }
+}
+
 // A stream that has failed, and one that is being captured, end the call.
 void refused() {
     Stream stream;
@@ -316,7 +340,8 @@ void refused() {
 int main(int argc, char **argv) {
     const std::map<std::string, void (*)()> cases = {
         {"pinned tensors", pinned_tensors}, {"sizes", sizes}, {"bounded", bounded},
-        {"no pinned memory", no_pinned_memory}, {"threads", threads}, {"refused", refused}};
+        {"no pinned memory", no_pinned_memory}, {"threads", threads}, {"refused", refused},
+        {"busy stream", busy_stream}};
     auto it = cases.find(argc > 1 ? argv[1] : "");
     if (it == cases.end()) {
         for (auto &c : cases) printf("%s\n", c.first.c_str());

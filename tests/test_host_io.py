@@ -33,7 +33,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["pinned tensors", "sizes", "bounded", "no pinned memory",
-                                  "threads", "refused"])
+                                  "threads", "refused", "busy stream"])
 def test_host_io(program, case):
     out = subprocess.run([program, case], capture_output=True, text=True, timeout=100)
     assert out.returncode == 0 and out.stdout == "ok\n", (out.returncode, out.stdout, out.stderr)

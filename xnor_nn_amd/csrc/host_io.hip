@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <exception>
 #include <mutex>
@@ -141,6 +142,33 @@ inline void relax() {}
 void copy_streaming(char *, const char *, size_t) {}
 #endif
 
+// One wait for something that arrives by itself, in turns: each call of turn() is one look later.
+// Looks without a pause for as long as `spin` (what an ordinary pass waits is shorter than that, and a
+// sleeping thread is woken 60 us late), then sleeps a sixteenth of the time waited so far between
+// looks: behind 53 ms of other work on the stream a pass took its four threads 213 ms of processor time.
+class Wait {
+public:
+    explicit Wait(std::chrono::microseconds spin) : spin_(spin) {}
+    void over() { turns_ = 0; }
+    bool turn() { // true after a sleep
+        if (turns_++ == 0) since_ = std::chrono::steady_clock::now();
+        relax();
+        if (turns_ % 16 != 0) return false;
+        const auto waited = std::chrono::steady_clock::now() - since_;
+        if (waited < spin_) return false;
+        std::this_thread::sleep_for(std::min<std::chrono::steady_clock::duration>(
+                waited / 16, std::chrono::microseconds(500)));
+        turns_ = 15; // (the next turn sleeps again)
+        return true;
+    }
+
+private:
+    const std::chrono::steady_clock::duration spin_;
+    std::chrono::steady_clock::time_point since_;
+    unsigned turns_ = 0;
+};
+constexpr std::chrono::microseconds SPIN_CALLER(2000), SPIN_HELPER(300);
+
 // What the copying threads share.  All counts are slices from the front of a tensor.
 struct Work {
     Ring in, out;
@@ -176,12 +204,16 @@ struct Work {
         return true;
     }
     void help() { // until every slice has been handed out
+        Wait wait(SPIN_HELPER);
         while (!stop.load(std::memory_order_relaxed)) {
-            if (copy_in_slice() || copy_out_slice()) continue;
+            if (copy_in_slice() || copy_out_slice()) {
+                wait.over();
+                continue;
+            }
             if (next_in.load(std::memory_order_relaxed) >= in_slices
                     && next_out.load(std::memory_order_relaxed) >= out_slices)
                 return;
-            relax();
+            wait.turn();
         }
     }
 };
@@ -268,7 +300,7 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
     size_t in_there = 0, in_sent = 0; // input slices in the ring; on their way
     size_t out_sent = 0, out_done = 0; // output slices on their way; in the user's memory
     bool computed = false;
-    size_t idle = 0;
+    Wait wait(SPIN_CALLER);
     while (ok) {
         while (in_there < w.in_slices && w.in_copied[in_there % w.in.slices()].load(
                         std::memory_order_acquire) == in_there + 1)
@@ -326,16 +358,15 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
             }
         }
         if (w.copy_in_slice() || w.copy_out_slice()) {
-            idle = 0;
+            wait.over();
             continue;
         }
         if (computed && out_done == w.out_slices
                 && (w.in_slices == 0 || out_bytes > 0
                     || __atomic_load_n(in_flag, __ATOMIC_ACQUIRE) == w.in_slices))
             break;
-        relax();
         // nothing to do but wait for a flag: a kernel that failed raises none
-        if (++idle % (1 << 16) == 0) {
+        if (wait.turn()) {
             const hipError_t e = hipStreamQuery(stream);
             ok = e == hipSuccess || e == hipErrorNotReady;
         }
