@@ -279,7 +279,8 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
     w.out_bytes = direct_out ? 0 : out_bytes;
     w.in_slices = (w.in_bytes + SLICE - 1) / SLICE;
     w.out_slices = (w.out_bytes + SLICE - 1) / SLICE;
-    w.in_room = std::min(w.in_slices, w.in.slices());
+    size_t in_room = std::min(w.in_slices, w.in.slices());
+    w.in_room = in_room;
     const size_t half_ring = std::max<size_t>(w.in.blocks / 2, 1) * BLOCK_SLICES;
     uint32_t *const in_flag = flags_, *const out_flag = flags_ + FLAG_BYTES / 8; // slices arrived
     bool ok = !direct_in
@@ -298,7 +299,8 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
     const size_t total = w.in_bytes + w.out_bytes;
     int helpers_wanted = total >= (8u << 20) ? 3 : total >= (4u << 20) ? 2 : total >= (2u << 20) ? 1 : 0;
     size_t in_there = 0, in_sent = 0; // input slices in the ring; on their way
-    size_t out_sent = 0, out_done = 0; // output slices on their way; in the user's memory
+    // output slices on their way; in the ring; in the user's memory
+    size_t out_sent = 0, out_there = 0, out_done = 0;
     bool computed = false;
     Wait wait(SPIN_CALLER);
     while (ok) {
@@ -320,10 +322,12 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
             in_sent = end;
             continue;
         }
-        if (in_sent < w.in_slices && w.in_slices > w.in.slices())
-            w.in_room.store(std::min<size_t>(w.in_slices, w.in.slices()
-                            + __atomic_load_n(in_flag, __ATOMIC_ACQUIRE)),
-                    std::memory_order_release);
+        if (in_room < w.in_slices) {
+            const size_t room = std::min<size_t>(w.in_slices,
+                    w.in.slices() + __atomic_load_n(in_flag, __ATOMIC_ACQUIRE));
+            // (told when it changes: the helpers read it)
+            if (room != in_room) w.in_room.store(in_room = room, std::memory_order_release);
+        }
         if (!computed && in_sent == w.in_slices) {
             ok = compute(context);
             computed = true;
@@ -336,8 +340,9 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
                         std::memory_order_acquire) == out_done + 1)
             out_done++;
         if (computed && out_sent < w.out_slices) { // the last pieces get smaller
-            const size_t n = std::min(BLOCK_SLICES - out_sent % BLOCK_SLICES,
-                    std::max<size_t>((w.out_slices - out_sent) / 2, 1));
+            const size_t room = BLOCK_SLICES - out_sent % BLOCK_SLICES; // to the end of the block
+            size_t n = std::min(room, std::max<size_t>((w.out_slices - out_sent) / 2, 1));
+            if (n > 1 && n + 1 == room) n = room; // (no piece for a slice left in the block)
             if (out_sent + n <= out_done + w.out.slices()) {
                 const size_t at = out_sent * SLICE;
                 send(dev_out + at, w.out.slice(out_sent), std::min(n * SLICE, w.out_bytes - at),
@@ -346,9 +351,11 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
                 continue;
             }
         }
-        if (out_sent > 0)
-            w.out_there.store(__atomic_load_n(out_flag, __ATOMIC_ACQUIRE),
-                    std::memory_order_release);
+        if (out_there < out_sent) {
+            const size_t there = __atomic_load_n(out_flag, __ATOMIC_ACQUIRE);
+            if (there != out_there)
+                w.out_there.store(out_there = there, std::memory_order_release);
+        }
         for (; helpers_wanted > 0 && (in_sent > 0 || computed); helpers_wanted--) { // (the link is busy)
             try {
                 helpers[started] = std::thread([&w] { w.help(); });
