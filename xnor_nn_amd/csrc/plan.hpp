@@ -146,14 +146,18 @@ inline void launch_kernel(K kernel, dim3 grid, dim3 block, size_t lds, hipStream
 }
 
 // More than 64 KB of dynamic LDS has to be asked for: once per kernel, device and size.  One
-// static object per kernel remembers what has been granted.
+// static object per kernel remembers what has been granted; the attribute and the record of it
+// change together, under the lock, and only grow.
 struct LdsGrant {
     std::atomic<size_t> have[64];
+    std::mutex mu;
     hipError_t ask(const void *kernel, size_t lds) {
         if (lds <= 64 * 1024) return hipSuccess;
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return hipErrorInvalidDevice;
         if (lds <= have[dev].load(std::memory_order_acquire)) return hipSuccess;
+        std::lock_guard<std::mutex> lock(mu);
+        if (lds <= have[dev].load(std::memory_order_relaxed)) return hipSuccess;
         const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                 (int)lds);
         if (e == hipSuccess) have[dev].store(lds, std::memory_order_release);
