@@ -1444,7 +1444,7 @@ void mfma_plan(Plan &g) {
     g.mfma_steps = g.mfma_pair = g.mfma_rows = 0;
     g.mfma_ps_small = 0;
     g.mfma_big_per_xcd = g.mfma_blocks_per_xcd = 0;
-    g.mfma_small = g.mfma_small_rows = 0;
+    g.mfma_small = 0;
     g.mfma_small_lds = 0;
     g.one_launch = 0;
     g.mfma_persist = g.mfma_reverse = 0;
@@ -1465,7 +1465,7 @@ void mfma_plan(Plan &g) {
         uint32_t lds = 0;
         if (small_kernel_applies(g, &rows, &lds)) {
             g.mfma_small = 1;
-            g.mfma_small_rows = rows;
+            g.small = small_plan(g, rows);
             g.mfma_small_lds = lds;
             g.one_launch = one_launch_applies(g) ? 1 : 0;
         }

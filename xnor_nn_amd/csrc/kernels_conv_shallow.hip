@@ -53,26 +53,6 @@ __device__ __forceinline__ v16f shallow_mfma_fp4(const v4i a, const v4i b, const
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a8, b8, c, 4, 4, 0, 0, 0, 0);
 }
 
-// What the kernel needs of the launch plan (a fraction of Geometry: less to copy per launch).
-struct ShallowPlan {
-    uint32_t npix_out, npix_in;
-    int ic, ih, iw, oc, oh, ow, ohw, kh, kw, sh, sw, ph, pw;
-    int prows, pcols;            // rows and columns of an image with the padding its taps reach
-    int row_codes, steps;        // bytes of sign bits per kernel row; 64-product steps in all
-    int max_rows;                // padded rows a tile stages at most
-    int row_words;               // dwords of a padded row's bit string (two spare ones included)
-    int row_pixels;              // pixels that share one of them at most
-    int row_bytes;               // of a pixel's FP4 row: steps * 32 + 16
-    int blocks, blocks_per_wg;   // 32-filter blocks: all, and of one workgroup
-    int a_cols;                  // cells of a padded row's mean|x| with the same column mod stride
-    int a_shares_rows;           // 1: its LDS is that of the operands, which are gathered after it
-    int gathers;                 // waves that share the kernel rows of 64 pixels, four rows each
-    uint32_t tiles, units, units_per_xcd;
-    uint32_t wfrag_bytes;
-    int nchw, stream;
-    FastDiv div_ohw, div_ow, div_prows, div_words, div_ic, div_acols;
-};
-
 // First and last padded row (image * prows + row) that the output pixels [p0, p1) reach.
 __host__ __device__ inline void padded_rows(const ShallowPlan &s, uint32_t p0, uint32_t p1,
         uint32_t &r0, uint32_t &r1) {
@@ -641,8 +621,7 @@ bool shallow_plan(Plan &g) {
             && (4 * s.steps > pairs || s.max_rows > 40))
         return false;
     g.mfma_shallow = pixels;
-    g.mfma_shallow_rows = s.max_rows;
-    g.mfma_shallow_blocks = s.blocks_per_wg;
+    g.shallow = s;
     g.mfma_lds = (uint32_t)lds;
     g.mfma_steps = s.steps;
     g.mfma_wbytes = s.wfrag_bytes;
@@ -652,8 +631,7 @@ bool shallow_plan(Plan &g) {
 hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst, int32_t *popc,
         const float *a_or_null, float *k_out, hipStream_t stream, const KernelEvents &ev) {
-    ShallowPlan s = make_plan(g);
-    set_tile(s, g.mfma_shallow, g.mfma_shallow_blocks, g.mfma_shallow_rows, g.cus);
+    const ShallowPlan &s = g.shallow;
     const dim3 grid(s.units_per_xcd * 8);
     const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
     const float inv_khw = 1.f / g.kh / g.kw;
@@ -666,7 +644,7 @@ hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         launch_kernel(kernel, grid, dim3(64 * W_), g.mfma_lds, stream, ev, xbits, wf, alpha, k, \
                 dst, popc, a_or_null, k_out, inv_khw, s); \
     } while (0)
-    if (g.mfma_shallow == 128 && g.mfma_shallow_blocks > 2 && g.mfma_lds > SHALLOW_LDS / 8) {
+    if (g.mfma_shallow == 128 && s.blocks_per_wg > 2 && g.mfma_lds > SHALLOW_LDS / 8) {
         // with three filter blocks or more there are jobs for eight waves (us a pass with four and
         // eight: AlexNet's first layer, minibatch 64, 48.9 / 43.0; 100 filters 16.6 / 15.1; with 64
         // filters, 8 channels 7x7 on 112x112, 19.6 / 22.6), unless many workgroups fit

@@ -41,12 +41,6 @@ constexpr int SMALL_TABLE_BYTES = 1024;
 constexpr int SMALL_RING = 8;         // weight fragments in flight per wave
 constexpr uint32_t SMALL_DROP = 0xFFFFFFF0u;
 
-struct SmallPlan {
-    int max_rows, ks, nsteps, subs, row_bytes;
-    uint32_t blocks, wfrag_bytes;
-    FastDiv div_xw, div_ks, div_kw;
-};
-
 __device__ __forceinline__ v16f small_mfma_fp4(const v4i a, const v4i b, const v16f c) {
     const v8i a8 = {a.x, a.y, a.z, a.w, 0, 0, 0, 0};
     const v8i b8 = {b.x, b.y, b.z, b.w, 0, 0, 0, 0};
@@ -345,9 +339,12 @@ int small_row_bytes(const Plan &g) {
     return g.mfma_pair ? g.xw * 16 : g.mfma_steps * 32 + 16;
 }
 
-SmallPlan small_plan(const Plan &g) {
+} // namespace
+
+// (once the rest of the plan is made)
+SmallPlan small_plan(const Plan &g, int rows) {
     SmallPlan s{};
-    s.max_rows = g.mfma_small_rows;
+    s.max_rows = rows;
     s.ks = g.mfma_steps;
     s.nsteps = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
     s.subs = (g.oc + 31) / 32;
@@ -359,8 +356,6 @@ SmallPlan small_plan(const Plan &g) {
     s.div_kw = FastDiv::make((uint32_t)g.kw);
     return s;
 }
-
-} // namespace
 
 // Which problems take this kernel: one channel part and so few (pixel block, filter block) pairs,
 // a workgroup each, that the large-launch kernel would leave most of the chip idle.  Both were
@@ -438,7 +433,7 @@ bool one_launch_applies(const Plan &g) {
 hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const uint32_t *wfrag, const float *alpha, const float *k, float *dst,
         const float *a_or_null, float *k_out, hipStream_t stream, const KernelEvents &ev) {
-    const SmallPlan s = small_plan(g);
+    const SmallPlan &s = g.small;
     const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
     const float *x = nullptr;
     uint32_t *bits_out = nullptr;
@@ -457,7 +452,7 @@ hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
 // and K behind like the separate stages.
 hipError_t launch_forward_small(const Plan &g, const float *x, uint32_t *bits_out, float *a_out,
         const uint32_t *wfrag, const float *alpha, float *k_out, float *dst, hipStream_t stream) {
-    const SmallPlan s = small_plan(g);
+    const SmallPlan &s = g.small;
     const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
     const uint32_t *xbits = nullptr;
     const float *k = nullptr, *a_or_null = nullptr;

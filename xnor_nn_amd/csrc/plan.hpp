@@ -73,9 +73,40 @@ struct Geometry {
     FastDiv div_ihw, div_iw, div_ohw, div_ow;
 };
 
+// What the kernel for few tiles needs beside it (kernels_conv_small.hip).
+struct SmallPlan {
+    int max_rows;     // input pixels a block stages at most
+    int ks, nsteps;   // steps per tap (or pair of taps), and in all
+    int subs;         // 32-filter blocks
+    int row_bytes;    // of an input pixel's FP4 row in LDS
+    uint32_t blocks, wfrag_bytes; // 32-pixel blocks
+    FastDiv div_xw, div_ks, div_kw;
+};
+
+// What the kernel for few input channels needs (kernels_conv_shallow.hip), in place of Geometry: less
+// to copy per launch.
+struct ShallowPlan {
+    uint32_t npix_out, npix_in;
+    int ic, ih, iw, oc, oh, ow, ohw, kh, kw, sh, sw, ph, pw;
+    int prows, pcols;            // rows and columns of an image with the padding its taps reach
+    int row_codes, steps;        // bytes of sign bits per kernel row; 64-product steps in all
+    int max_rows;                // padded rows a tile stages at most
+    int row_words;               // dwords of a padded row's bit string (two spare ones included)
+    int row_pixels;              // pixels that share one of them at most
+    int row_bytes;               // of a pixel's FP4 row: steps * 32 + 16
+    int blocks, blocks_per_wg;   // 32-filter blocks: all, and of one workgroup
+    int a_cols;                  // cells of a padded row's mean|x| with the same column mod stride
+    int a_shares_rows;           // 1: its LDS is that of the operands, which are gathered after it
+    int gathers;                 // waves that share the kernel rows of 64 pixels, four rows each
+    uint32_t tiles, units, units_per_xcd;
+    uint32_t wfrag_bytes;
+    int nchw, stream;
+    FastDiv div_ohw, div_ow, div_prows, div_words, div_ic, div_acols;
+};
+
 // What the host adds to it when a descriptor is initialised: which kernels run and with what
-// tiles.  Kernels get the Geometry part only (geometry() below): the argument block is copied on
-// every launch and read by every workgroup.
+// tiles.  Kernels get the Geometry part (geometry() below) and their own: the argument block is
+// copied on every launch and read by every workgroup.
 struct Plan : Geometry {
     int bin_waves;              // waves per workgroup of the binarize kernel at most
     int bin_nhwc_lane;          // 1: NHWC input by the one-lane-per-pixel kernel
@@ -97,13 +128,12 @@ struct Plan : Geometry {
     // bytes per workgroup, bytes of the weight fragments
     int mfma_steps, mfma_pair, mfma_parts, mfma_rows;
     int mfma_small;             // 1: few tiles: the small-problem kernel (kernels_conv_small.hip),
-    int mfma_small_rows;        // the input pixels one of its blocks stages at most
+    SmallPlan small;            // its part of the plan
     uint32_t mfma_small_lds;    // and its LDS bytes per workgroup
     int one_launch;             // 1: a forward pass on device buffers is that kernel alone
     int mfma_shallow;           // > 0: few channels: the kernel of kernels_conv_shallow.hip with
                                 // tiles of this many output pixels,
-    int mfma_shallow_rows;      // padded input rows per tile at most
-    int mfma_shallow_blocks;    // and 32-filter blocks per workgroup
+    ShallowPlan shallow;        // and its part of the plan
     uint32_t mfma_lds, mfma_wbytes;
 };
 inline const Geometry &geometry(const Plan &p) { return p; }
@@ -228,7 +258,8 @@ hipError_t launch_weights_float(const float *from, float *to, size_t n, float *p
 // memory: nothing is allocated)
 hipError_t weights_float_scratch(float **out);
 // Decides whether the matrix-core kernel takes the problem and fills use_mfma, mfma_ps and
-// the mfma_* fields (everything the launch needs, so that a forward call computes nothing).
+// the mfma_* fields and the kernels' own plans (everything the launch needs: a forward call takes
+// its arguments from here).
 void mfma_plan(Plan &g);
 const char *mfma_kernel_name(const Plan &g);
 size_t mfma_weight_bytes(const Plan &g);
@@ -246,6 +277,7 @@ hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s);
 const char *convolution_kernel_name(const Plan &g);
 // The matrix-core kernel for launches of few tiles (filled in by mfma_plan: g.mfma_small).
 bool small_kernel_applies(const Plan &g, int *rows, uint32_t *lds);
+SmallPlan small_plan(const Plan &g, int rows);
 bool one_launch_applies(const Plan &g);
 hipError_t launch_forward_small(const Plan &g, const float *x, uint32_t *bits_out, float *a_out,
         const uint32_t *wfrag, const float *alpha, float *k_out, float *dst, hipStream_t s);
@@ -254,7 +286,7 @@ hipError_t launch_convolution_small(const Plan &g, const uint32_t *xbits,
         const float *a_or_null, float *k_out, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
 // The matrix-core kernel for few input channels (chosen by mfma_plan: g.mfma_shallow).
-bool shallow_plan(Plan &g);
+bool shallow_plan(Plan &g); // mfma_shallow, shallow and the sizes that depend on them
 hipError_t launch_pack_weights_shallow(const Plan &g, const float *w, uint32_t *frag,
         hipStream_t s);
 hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
