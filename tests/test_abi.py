@@ -221,16 +221,17 @@ def test_stage_fusion_switch_and_table_bookkeeping_without_a_gpu():
     lib.xnor_nn_destroy_convolution(C.byref(c))
 
 
-def kernel_names(shape, fmts=(capi.FMT_NCHW, capi.FMT_OIHW, capi.FMT_NCHW)):
-    """(binarize kernel, convolution kernel) the library plans for a shape
-    (mb, oc, ic, ih, iw, kh, kw, sh, sw, ph, pw); planning needs no GPU (256 CUs assumed)."""
+def kernel_names(shape, fmts=(capi.FMT_NCHW, capi.FMT_OIHW, capi.FMT_NCHW),
+                 stages=(capi.OP_BINARIZE_DATA, capi.OP_CONVOLUTION_FORWARD)):
+    """(binarize kernel, convolution kernel) or those of other stages that the library plans for a
+    shape (mb, oc, ic, ih, iw, kh, kw, sh, sw, ph, pw); planning needs no GPU (256 CUs assumed)."""
     lib = capi.load()
     c = capi.ConvolutionDesc()
     assert lib.xnor_nn_init_convolution(C.byref(c), capi.ALGORITHM_BCAST, *fmts, *shape) \
         == capi.SUCCESS
     buf = C.create_string_buffer(96)
     out = []
-    for stage in (capi.OP_BINARIZE_DATA, capi.OP_CONVOLUTION_FORWARD):
+    for stage in stages:
         lib.xnor_nn_hip_kernel_name(C.byref(c), stage, buf, len(buf))
         out.append(buf.value.decode())
     lib.xnor_nn_destroy_convolution(C.byref(c))
@@ -248,7 +249,8 @@ def test_kernel_variants_planned_for_known_shapes(monkeypatch):
         monkeypatch.delenv(key, raising=False)
     conv4 = (256, 384, 13, 13, 3, 3, 1, 1, 1, 1)
     # 6 pixel blocks x 8 filter blocks: fewer (block, block) pairs than compute units
-    assert kernel_names((1,) + conv4) == ("binarize_nchw_kernel", "conv_mfma_fp4_small_kernel<KS=6>")
+    assert kernel_names((1,) + conv4) == ("binarize_nchw_split_kernel",
+                                          "conv_mfma_fp4_small_kernel<KS=6>")
     assert kernel_names((8,) + conv4)[1] == "conv_mfma_fp4_small_kernel<KS=6>"
     # up to two pairs per compute unit when a wave would walk 48 steps or more (here 54)
     assert kernel_names((12,) + conv4)[1] == "conv_mfma_fp4_small_kernel<KS=6>"
@@ -366,3 +368,25 @@ def test_where_the_kernel_for_few_channels_is_taken(monkeypatch, t, shallow):
                 "XNOR_NN_HIP_MFMA_GROUPS"):
         monkeypatch.delenv(key, raising=False)
     assert kernel_names(t)[1].startswith("conv_mfma_fp4_shallow_kernel") == shallow
+
+
+@pytest.mark.parametrize("t,name", [
+    ((16, 8, 40, 16, 16, 3, 3, 1, 1, 1, 1), "binarize_nchw_split_kernel"), # 64 tiles of 64 pixels
+    ((16, 8, 40, 16, 17, 3, 3, 1, 1, 1, 1), "binarize_nchw_kernel"),       # 68
+    ((1, 8, 33, 1, 1, 1, 1, 1, 1, 0, 0), "binarize_nchw_split_kernel"),
+    ((1, 8, 32, 1, 1, 1, 1, 1, 1, 0, 0), "binarize_nchw_shallow_kernel"),
+    ((1, 8, 8160, 7, 7, 1, 1, 1, 1, 0, 0), "binarize_nchw_split_kernel"),  # as deep as tiles go
+    ((1, 8, 8161, 7, 7, 1, 1, 1, 1, 0, 0), "binarize_generic_kernel"),
+], ids=str)
+def test_where_the_binarize_kernel_for_few_pixels_is_taken(t, name):
+    """Its rule, on either side of each line (256 compute units)."""
+    assert kernel_names(t)[0] == name
+
+
+def test_weight_stage_kernel_names():
+    """The whole stage in one launch for OIHW filters that fit, four kernels otherwise."""
+    name = lambda t, w=capi.FMT_OIHW: kernel_names(
+        t, (capi.FMT_NCHW, w, capi.FMT_NCHW), (capi.OP_BINARIZE_WEIGHTS,))[0]
+    assert name((1, 8, 1612, 4, 4, 2, 5, 1, 1, 2, 2)) == "binarize_filter_kernel"  # 16120 values
+    assert name((1, 8, 1613, 4, 4, 2, 5, 1, 1, 2, 2)) == "pack_weights_kernel"
+    assert name((1, 8, 64, 4, 4, 3, 3, 1, 1, 1, 1), capi.FMT_HWIO) == "pack_weights_kernel"

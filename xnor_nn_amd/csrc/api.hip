@@ -298,7 +298,7 @@ xnor_nn_status_t exec_binarize_weights(const xnor_nn_convolution_t *c,
     xnor_nn_status_t rc = stage_in(st, &st->stage_weights, res[xnor_nn_resource_user_weights],
             weights_elems(st->g) * sizeof(float), &w, true);
     if (rc != xnor_nn_success) return rc;
-    if (st->verbose) printf("xnor_nn exec binarize_weights: pack/alpha/op_count kernels\n");
+    if (st->verbose) printf("xnor_nn exec binarize_weights: %s\n", weights_kernel_name(st->g));
     char *packed = static_cast<char *>(res[xnor_nn_resource_bin_weights]);
     if (launch_binarize_weights(st->g, static_cast<const float *>(w),
                 reinterpret_cast<uint32_t *>(packed),
@@ -948,7 +948,7 @@ int xnor_nn_hip_kernel_name(const xnor_nn_convolution_t *c, int stage, char *buf
     case xnor_nn_operation_convolution_forward: name = convolution_kernel_name(g); break;
     case xnor_nn_operation_binarize_data: name = binarize_kernel_name(g); break;
     case xnor_nn_operation_calculate_k: name = "box_filter_kernel"; break;
-    case xnor_nn_operation_binarize_weights: name = "pack_weights_kernel"; break;
+    case xnor_nn_operation_binarize_weights: name = weights_kernel_name(g); break;
     }
     snprintf(buf, buf_bytes, "%s", name);
     return (int)strlen(buf);

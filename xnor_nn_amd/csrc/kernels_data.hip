@@ -221,7 +221,7 @@ constexpr int SPLIT_TILE = 16, SPLIT_WORDS = 64 / SPLIT_TILE, SPLIT_LOADERS = 8;
 
 template <int T, bool WRITE_BITS, bool WRITE_A>
 __global__ __launch_bounds__(64 * (SPLIT_LOADERS + 1))
-void binarize_nchw_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
+void binarize_nchw_split_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const SplitPlan s, const float inv_ic) {
     typedef float v4f __attribute__((ext_vector_type(4)));
     constexpr int G = 64 / T; // words a wave loads together
@@ -554,7 +554,7 @@ hipError_t launch_split(const Plan &g, const float *x, uint32_t *bits, float *a,
     p.xw = g.xw;
     p.div_ihw = g.div_ihw;
     const size_t lds = split_lds_bytes(g, &p.loaders, &p.chunks);
-    const auto kernel = binarize_nchw_kernel<SPLIT_TILE, WRITE_BITS, WRITE_A>;
+    const auto kernel = binarize_nchw_split_kernel<SPLIT_TILE, WRITE_BITS, WRITE_A>;
     static LdsGrant grant;
     const hipError_t e = grant.ask((const void *)kernel, lds);
     if (e != hipSuccess) return e;
@@ -649,6 +649,7 @@ void binarize_plan(Plan &g) {
 
 const char *binarize_kernel_name(const Plan &g) {
     return shallow_nchw(g) ? "binarize_nchw_shallow_kernel"
+        : split_nchw(g) ? "binarize_nchw_split_kernel"
         : tiled_nchw(g) ? "binarize_nchw_kernel"
         : !vector_nhwc(g) ? "binarize_generic_kernel"
         : nhwc_by_lane(g) ? "binarize_nhwc_kernel" : "binarize_nhwc_tiled_kernel";

@@ -524,12 +524,22 @@ void sign_times_mean_kernel(const float *__restrict__ from, float *__restrict__ 
 
 } // namespace
 
+// One launch for the whole stage: OIHW weights whose filters fit the LDS.
+static bool filter_kernel_applies(const Plan &g) {
+    const uint64_t n = (uint64_t)g.ic * g.kh * g.kw;
+    return g.w_fmt == xnor_nn_weights_format_oihw
+        && (n + FILTER_CHUNK) * sizeof(float) <= FILTER_LDS;
+}
+
+const char *weights_kernel_name(const Plan &g) {
+    return filter_kernel_applies(g) ? "binarize_filter_kernel" : "pack_weights_kernel";
+}
+
 hipError_t launch_binarize_weights(const Plan &g, const float *w, uint32_t *bits,
         uint32_t *frag, float *alpha, int32_t *opc, hipStream_t s) {
     const int taps = g.kh * g.kw;
     const uint64_t n = (uint64_t)g.ic * taps;
-    if (g.w_fmt == xnor_nn_weights_format_oihw
-            && (n + FILTER_CHUNK) * sizeof(float) <= FILTER_LDS) {
+    if (filter_kernel_applies(g)) {
         FilterPlan f{};
         f.n = (int)n;
         f.taps = taps;

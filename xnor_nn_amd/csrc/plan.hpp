@@ -294,6 +294,7 @@ hipError_t launch_convolution_shallow(const Plan &g, const uint32_t *xbits,
         const float *a_or_null, float *k_out, hipStream_t s,
         const KernelEvents &ev = KernelEvents{});
 const char *binarize_kernel_name(const Plan &g);
+const char *weights_kernel_name(const Plan &g); // the first of four, or the only one
 
 int pick_q(int oc, int xw);
 
