@@ -349,6 +349,36 @@ def test_one_launch_forward(oracle, gpu, monkeypatch, t, fmts, separate_k):
     run_and_compare(oracle, d, *in_layout(x, w, fmts), fmts, True, gpu)
 
 
+@pytest.mark.parametrize("t,launches", [
+    ((1, 32, 33, 4, 8, 3, 3, 1, 1, 1, 1), 1),
+    ((3, 64, 512, 16, 16, 3, 3, 1, 1, 1, 1), 1),   # 64 channels, 1.5 workgroups per compute unit
+    ((1, 65, 33, 4, 8, 3, 3, 1, 1, 1, 1), 2),      # a third word
+    ((3, 64, 513, 16, 16, 3, 3, 1, 1, 1, 1), 2),   # more workgroups
+    ((64, 3, 96, 227, 227, 11, 11, 4, 4, 0, 0), 2),
+], ids=str)
+def test_launches_of_a_forward_pass(gpu, t, launches):
+    """Counted as the nodes of a captured pass."""
+    import torch
+    d, x, w = problem(t)
+    conv = make(d, torch.from_numpy(w).to(gpu))
+    try:
+        xt = torch.from_numpy(x).to(gpu)
+        yt = torch.empty(d["mb"], d["oc"], conv.desc.oh, conv.desc.ow, device=gpu)
+        side = torch.cuda.Stream()
+        conv.set_stream(side)
+        conv.forward(xt, yt)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=side):
+            conv.forward(xt, yt)
+        nodes = C.c_size_t()
+        assert conv.lib.hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None,
+                                         C.byref(nodes)) == 0
+        assert nodes.value == launches
+    finally:
+        conv.close()
+
+
 @pytest.mark.parametrize("t", [
     (1, 160, 40, 12, 12, 5, 5, 1, 1, 2, 2),    # paired taps, 65 steps
     (1, 96, 32, 9, 9, 5, 5, 1, 1, 2, 2),       # 39 steps
