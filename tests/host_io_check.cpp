@@ -205,8 +205,9 @@ void pass(xnor_hip::HostIo &io, Stream &stream, size_t in_bytes, size_t out_byte
     memset(out.at, 0x5A, out_bytes + 8);
     bool computed = false;
     const double before = processor_seconds();
-    const bool ok = io.run(reinterpret_cast<hipStream_t>(&stream), in.at, in_bytes, dev_in.data(),
-            out.at, out_bytes, dev_out.data(), [&] {
+    const bool ok = io.run(reinterpret_cast<hipStream_t>(&stream), in.at,
+            xnor_hip::memory_of(in.at), in_bytes, dev_in.data(), out.at,
+            xnor_hip::memory_of(out.at), out_bytes, dev_out.data(), [&] {
         computed = true;
         char *from = dev_in.data(), *to = dev_out.data();
         stream.put([=] {

@@ -33,14 +33,7 @@ size_t weights_elems(const Plan &g) { return (size_t)g.oc * g.ic * g.kh * g.kw; 
 size_t dst_elems(const Plan &g) { return (size_t)g.mb * g.oc * g.oh * g.ow; }
 
 // True when a kernel can dereference p (device or managed allocation).
-bool on_device(const void *p) {
-    hipPointerAttribute_t attr;
-    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
-        (void)hipGetLastError(); // plain host memory: clear the sticky error
-        return false;
-    }
-    return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
-}
+bool on_device(const void *p) { return memory_of(p) == Memory::device; }
 
 // A staging buffer of the descriptor, allocated on first use.
 xnor_nn_status_t stage_buffer(void **slot, size_t bytes) {
@@ -55,7 +48,8 @@ xnor_nn_status_t stage_buffer(void **slot, size_t bytes) {
 // for it would take longer to allocate than they save.
 xnor_nn_status_t stage_in(State *st, void **slot, const void *user, size_t bytes,
         const void **dev, bool once = false) {
-    if (on_device(user)) { *dev = user; return xnor_nn_success; }
+    const Memory memory = memory_of(user);
+    if (memory == Memory::device) { *dev = user; return xnor_nn_success; }
     const xnor_nn_status_t rc = stage_buffer(slot, bytes);
     if (rc != xnor_nn_success) return rc;
     // (the bytes have left the user's buffer when this returns)
@@ -63,8 +57,9 @@ xnor_nn_status_t stage_in(State *st, void **slot, const void *user, size_t bytes
         if (hipMemcpyAsync(*slot, user, bytes, hipMemcpyHostToDevice, st->stream) != hipSuccess
                 || hipStreamSynchronize(st->stream) != hipSuccess)
             return xnor_nn_error_memory;
-    } else if (!st->io.run(st->stream, static_cast<const char *>(user), bytes,
-                static_cast<char *>(*slot), nullptr, 0, nullptr, [] { return true; }))
+    } else if (!st->io.run(st->stream, static_cast<const char *>(user), memory, bytes,
+                static_cast<char *>(*slot), nullptr, Memory::pageable, 0, nullptr,
+                [] { return true; }))
         return xnor_nn_error_memory;
     *dev = *slot;
     return xnor_nn_success;
@@ -318,7 +313,8 @@ xnor_nn_status_t run_convolution(const xnor_nn_convolution_t *c, xnor_nn_resourc
     withdraw_ready(res[xnor_nn_resource_a]);
     const size_t bytes = dst_elems(st->g) * 4;
     void *out = user_out;
-    const bool direct = on_device(user_out);
+    const Memory memory = memory_of(user_out);
+    const bool direct = memory == Memory::device;
     if (!direct) {
         const xnor_nn_status_t rc = stage_buffer(&st->stage_dst, bytes);
         if (rc != xnor_nn_success) return rc;
@@ -358,8 +354,9 @@ xnor_nn_status_t run_convolution(const xnor_nn_convolution_t *c, xnor_nn_resourc
                 dst, popc, st->stream, st->time_convolution.next());
     }
     if (err != hipSuccess) return xnor_nn_error_memory;
-    if (!direct && !st->io.run(st->stream, nullptr, 0, nullptr, static_cast<char *>(user_out),
-                bytes, static_cast<const char *>(out), [] { return true; }))
+    if (!direct && !st->io.run(st->stream, nullptr, Memory::pageable, 0, nullptr,
+                static_cast<char *>(user_out), memory, bytes, static_cast<const char *>(out),
+                [] { return true; }))
         return xnor_nn_error_memory;
     return xnor_nn_success;
 }
@@ -423,7 +420,8 @@ xnor_nn_status_t forward_on_device(State *st, xnor_nn_resources_t res, const flo
 // A forward pass between host tensors (host_io.hpp): the input arrives piece by piece, the
 // kernels run, the output leaves piece by piece, without a synchronisation in between.  Called
 // with st->mu held.
-xnor_nn_status_t forward_on_host(State *st, xnor_nn_resources_t res, const void *src, void *dst) {
+xnor_nn_status_t forward_on_host(State *st, xnor_nn_resources_t res, const void *src,
+        Memory src_memory, void *dst, Memory dst_memory) {
     const Plan &g = st->g;
     const size_t in_bytes = src_elems(g) * 4, out_bytes = dst_elems(g) * 4;
     xnor_nn_status_t rc = stage_buffer(&st->stage_src, in_bytes);
@@ -434,9 +432,9 @@ xnor_nn_status_t forward_on_host(State *st, xnor_nn_resources_t res, const void 
                 static_cast<float *>(st->stage_dst));
         return rc == xnor_nn_success;
     };
-    return st->io.run(st->stream, static_cast<const char *>(src), in_bytes,
-                   static_cast<char *>(st->stage_src), static_cast<char *>(dst), out_bytes,
-                   static_cast<const char *>(st->stage_dst), compute)
+    return st->io.run(st->stream, static_cast<const char *>(src), src_memory, in_bytes,
+                   static_cast<char *>(st->stage_src), static_cast<char *>(dst), dst_memory,
+                   out_bytes, static_cast<const char *>(st->stage_dst), compute)
         ? xnor_nn_success : rc != xnor_nn_success ? rc : xnor_nn_error_memory;
 }
 
@@ -744,13 +742,14 @@ xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
             complete = complete && res[i] != nullptr;
         if (complete && st->g.use_mfma && fusion_on(st) && !st->verbose) {
             const bool vouched = flags & XNOR_NN_HIP_DEVICE_POINTERS;
-            const bool in = vouched || on_device(src), out = vouched || on_device(dst);
+            const Memory in = vouched ? Memory::device : memory_of(src);
+            const Memory out = vouched ? Memory::device : memory_of(dst);
             xnor_nn_status_t rc = xnor_nn_unimplemented; // one of each: through the executors
-            if (in && out)
+            if (in == Memory::device && out == Memory::device)
                 rc = forward_on_device(st, res, static_cast<const float *>(src),
                         static_cast<float *>(dst));
-            else if (!in && !out)
-                rc = forward_on_host(st, res, src, dst);
+            else if (in != Memory::device && out != Memory::device)
+                rc = forward_on_host(st, res, src, in, dst, out);
             if (rc != xnor_nn_unimplemented) {
                 if (rc == xnor_nn_success)
                     res[xnor_nn_resource_user_src] = res[xnor_nn_resource_user_dst] = nullptr;

@@ -24,6 +24,7 @@ constexpr size_t BLOCK_SLICES = 8, BLOCK = BLOCK_SLICES * SLICE;
 // later passes.
 constexpr size_t RING_BLOCKS = 8, RING_SLICES = RING_BLOCKS * BLOCK_SLICES;
 constexpr size_t POOL_BLOCKS = 128;
+constexpr size_t FLAG_BYTES = 256; // of a pass's flags
 // Tensors in pinned memory go straight to a copy engine from this size on, smaller ones through the
 // pinned buffers like any other (us a pass, in place / through the buffers, both tensors pinned:
 // 0.26 + 0.17 MB 46 / 46, 0.5 + 0.35 MB 56 / 63, 8.3 + 5.5 MB 286 / 360, 66 + 44 MB 2004 / 2326;
@@ -64,9 +65,41 @@ void link_copy_kernel(const v4u *__restrict__ from, v4u *__restrict__ to, const 
 
 // ---- pinned memory --------------------------------------------------------------------------
 std::mutex pool_mu;
-char *pool[POOL_BLOCKS]; // free blocks
-size_t pool_blocks = 0;
 int descriptors = 0;
+
+// Pinned pieces of one size that nobody uses.
+template <size_t BYTES, size_t MOST>
+struct Pool {
+    char *piece[MOST];
+    size_t pieces = 0;
+
+    char *take() {
+        {
+            std::lock_guard<std::mutex> lock(pool_mu);
+            if (pieces > 0) return piece[--pieces];
+        }
+        void *p = nullptr;
+        if (hipHostMalloc(&p, BYTES, hipHostMallocPortable) == hipSuccess)
+            return static_cast<char *>(p);
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void give(char *p) {
+        {
+            std::lock_guard<std::mutex> lock(pool_mu);
+            if (descriptors > 0 && pieces < MOST) {
+                piece[pieces++] = p;
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    void clear() { // under the lock
+        while (pieces > 0) (void)hipHostFree(piece[--pieces]);
+    }
+};
+Pool<BLOCK, POOL_BLOCKS> block_pool;
+Pool<FLAG_BYTES, POOL_BLOCKS> flag_pool;
 
 // The blocks of one direction of a pass, used in turn.  Slice i of the tensor lies in place
 // i % slices().
@@ -77,29 +110,12 @@ struct Ring {
     Ring() = default;
     Ring(const Ring &) = delete;
     ~Ring() {
-        for (; blocks > 0; blocks--) {
-            {
-                std::lock_guard<std::mutex> lock(pool_mu);
-                if (descriptors > 0 && pool_blocks < POOL_BLOCKS) {
-                    pool[pool_blocks++] = block[blocks - 1];
-                    continue;
-                }
-            }
-            (void)hipHostFree(block[blocks - 1]);
-        }
+        while (blocks > 0) block_pool.give(block[--blocks]);
     }
     // As many blocks as the bytes fill, or as many as there are to be had; false without any.
     bool take(size_t bytes) {
         const size_t want = std::min((bytes + BLOCK - 1) / BLOCK, RING_BLOCKS);
-        {
-            std::lock_guard<std::mutex> lock(pool_mu);
-            while (blocks < want && pool_blocks > 0) block[blocks++] = pool[--pool_blocks];
-        }
-        for (void *p = nullptr; blocks < want; block[blocks++] = static_cast<char *>(p))
-            if (hipHostMalloc(&p, BLOCK, hipHostMallocPortable) != hipSuccess) {
-                (void)hipGetLastError();
-                break;
-            }
+        while (blocks < want && (block[blocks] = block_pool.take()) != nullptr) blocks++;
         return blocks > 0;
     }
     size_t slices() const { return blocks * BLOCK_SLICES; }
@@ -107,14 +123,6 @@ struct Ring {
         return block[i / BLOCK_SLICES % blocks] + i % BLOCK_SLICES * SLICE;
     }
 };
-
-// True for memory that the copy engines read and write in place (the user pinned it).
-bool pinned(const void *p) {
-    hipPointerAttribute_t attr;
-    if (hipPointerGetAttributes(&attr, p) == hipSuccess) return attr.type == hipMemoryTypeHost;
-    (void)hipGetLastError(); // plain host memory: clear the sticky error
-    return false;
-}
 
 #if !defined(__HIP_DEVICE_COMPILE__)
 inline void relax() { _mm_pause(); }
@@ -172,6 +180,7 @@ constexpr std::chrono::microseconds SPIN_CALLER(2000), SPIN_HELPER(300);
 // What the copying threads share.  All counts are slices from the front of a tensor.
 struct Work {
     Ring in, out;
+    uint32_t *flags = nullptr; // pinned, raised by the transfer kernels
     const char *src = nullptr;
     char *dst = nullptr;
     size_t in_bytes = 0, out_bytes = 0, in_slices = 0, out_slices = 0;
@@ -184,6 +193,9 @@ struct Work {
 
     Work() {
         for (size_t i = 0; i < RING_SLICES; i++) in_copied[i] = out_copied[i] = 0;
+    }
+    ~Work() {
+        if (flags != nullptr) flag_pool.give(reinterpret_cast<char *>(flags));
     }
     bool copy_in_slice() {
         size_t i = next_in.load(std::memory_order_relaxed);
@@ -220,6 +232,16 @@ struct Work {
 
 } // namespace
 
+Memory memory_of(const void *p) {
+    hipPointerAttribute_t attr;
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError(); // plain host memory: clear the sticky error
+        return Memory::pageable;
+    }
+    return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged ? Memory::device
+        : attr.type == hipMemoryTypeHost ? Memory::pinned : Memory::pageable;
+}
+
 void host_io_descriptor_created() {
     std::lock_guard<std::mutex> lock(pool_mu);
     descriptors++;
@@ -228,37 +250,30 @@ void host_io_descriptor_created() {
 void host_io_descriptor_destroyed() {
     std::lock_guard<std::mutex> lock(pool_mu);
     if (--descriptors > 0) return;
-    while (pool_blocks > 0) (void)hipHostFree(pool[--pool_blocks]);
+    block_pool.clear();
+    flag_pool.clear();
 }
 
 HostIo::~HostIo() {
-    if (flags_ != nullptr) (void)hipHostFree(flags_);
     if (waiting_ != nullptr) (void)hipFree(waiting_);
 }
 
-// What the transfer kernels need beside the blocks.
+// Device memory that the transfer kernels need.
 bool HostIo::prepare(hipStream_t stream) {
-    if (flags_ == nullptr
-            && hipHostMalloc((void **)&flags_, FLAG_BYTES, hipHostMallocPortable) != hipSuccess)
-        flags_ = nullptr;
-    if (flags_ != nullptr && waiting_ == nullptr) {
-        // (cleared on the stream of the kernels that count in it)
-        if (hipMalloc((void **)&waiting_, sizeof(uint32_t)) != hipSuccess
-                || hipMemsetAsync(waiting_, 0, sizeof(uint32_t), stream) != hipSuccess) {
-            if (waiting_ != nullptr) (void)hipFree(waiting_);
-            waiting_ = nullptr;
-        }
-    }
-    if (waiting_ == nullptr) {
-        (void)hipGetLastError();
-        return false;
-    }
-    memset(flags_, 0, FLAG_BYTES);
-    return true;
+    if (waiting_ != nullptr) return true;
+    // (cleared on the stream of the kernels that count in it)
+    if (hipMalloc((void **)&waiting_, sizeof(uint32_t)) == hipSuccess
+            && hipMemsetAsync(waiting_, 0, sizeof(uint32_t), stream) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    if (waiting_ != nullptr) (void)hipFree(waiting_);
+    waiting_ = nullptr;
+    return false;
 }
 
-bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *dev_in, char *dst,
-        size_t out_bytes, const char *dev_out, bool (*compute)(void *), void *context) {
+bool HostIo::move(hipStream_t stream, const char *src, Memory src_memory, size_t in_bytes,
+        char *dev_in, char *dst, Memory dst_memory, size_t out_bytes, const char *dev_out,
+        bool (*compute)(void *), void *context) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) == hipSuccess
             && capture != hipStreamCaptureStatusNone)
@@ -266,10 +281,12 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
     // Directions that the runtime copies by itself: what the user has pinned needs no copy on this
     // side, and without pinned memory of our own the runtime's staging has to do.
     Work w;
-    bool direct_in = in_bytes >= PINNED_DIRECT && pinned(src);
-    bool direct_out = out_bytes >= PINNED_DIRECT && pinned(dst);
+    bool direct_in = in_bytes >= PINNED_DIRECT && src_memory == Memory::pinned;
+    bool direct_out = out_bytes >= PINNED_DIRECT && dst_memory == Memory::pinned;
     if ((in_bytes > 0 && !direct_in) || (out_bytes > 0 && !direct_out)) {
-        const bool ready = prepare(stream);
+        if (prepare(stream)) w.flags = reinterpret_cast<uint32_t *>(flag_pool.take());
+        const bool ready = w.flags != nullptr;
+        if (ready) memset(w.flags, 0, FLAG_BYTES);
         if (in_bytes > 0 && !direct_in) direct_in = !(ready && w.in.take(in_bytes));
         if (out_bytes > 0 && !direct_out) direct_out = !(ready && w.out.take(out_bytes));
     }
@@ -282,7 +299,8 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
     size_t in_room = std::min(w.in_slices, w.in.slices());
     w.in_room = in_room;
     const size_t half_ring = std::max<size_t>(w.in.blocks / 2, 1) * BLOCK_SLICES;
-    uint32_t *const in_flag = flags_, *const out_flag = flags_ + FLAG_BYTES / 8; // slices arrived
+    // slices of the input and of the output that have arrived
+    uint32_t *const in_flag = w.flags, *const out_flag = w.flags + FLAG_BYTES / 8;
     bool ok = !direct_in
         || hipMemcpyAsync(dev_in, src, in_bytes, hipMemcpyHostToDevice, stream) == hipSuccess;
     auto send = [&](const void *from, void *to, size_t bytes, uint32_t *flag, size_t arrived) {
@@ -386,6 +404,7 @@ bool HostIo::move(hipStream_t stream, const char *src, size_t in_bytes, char *de
         if (hipStreamSynchronize(stream) != hipSuccess) {
             ok = false;
             w.in.blocks = w.out.blocks = 0;
+            w.flags = nullptr;
         }
         if (!ok) (void)hipGetLastError();
     }

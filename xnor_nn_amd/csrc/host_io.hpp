@@ -21,6 +21,11 @@
 
 namespace xnor_hip {
 
+// Where a user's tensor lies: a kernel can use it in place (device or managed memory), the copy
+// engines can, or neither.
+enum class Memory { device, pinned, pageable };
+Memory memory_of(const void *p); // asks the driver: 0.4 us
+
 class HostIo {
 public:
     HostIo() = default;
@@ -29,24 +34,23 @@ public:
     HostIo &operator=(const HostIo &) = delete;
 
     // Copies in_bytes from src to dev_in, has compute() enqueue the kernels on the stream, and
-    // copies out_bytes from dev_out to dst (either tensor may be null with 0 bytes).  The device
-    // buffers hold a multiple of 16 bytes.  Returns when dst is written, or without a dst when
+    // copies out_bytes from dev_out to dst (either tensor may be null with 0 bytes; neither lies on
+    // the device).  The device buffers hold a multiple of 16 bytes.  Returns when dst is written, or without a dst when
     // the input has arrived; false on a HIP failure.
     template <class F>
-    bool run(hipStream_t stream, const char *src, size_t in_bytes, char *dev_in, char *dst,
-            size_t out_bytes, const char *dev_out, F &&compute) {
-        return move(stream, src, in_bytes, dev_in, dst, out_bytes, dev_out,
+    bool run(hipStream_t stream, const char *src, Memory src_memory, size_t in_bytes, char *dev_in,
+            char *dst, Memory dst_memory, size_t out_bytes, const char *dev_out, F &&compute) {
+        return move(stream, src, src_memory, in_bytes, dev_in, dst, dst_memory, out_bytes, dev_out,
                 [](void *f) { return (bool)(*static_cast<std::remove_reference_t<F> *>(f))(); },
                 &compute);
     }
 
 private:
-    static constexpr size_t FLAG_BYTES = 256;
-    uint32_t *flags_ = nullptr;   // pinned: slices of the input and of the output that have arrived
     uint32_t *waiting_ = nullptr; // device: workgroups of the transfer under way
     bool prepare(hipStream_t stream);
-    bool move(hipStream_t stream, const char *src, size_t in_bytes, char *dev_in, char *dst,
-            size_t out_bytes, const char *dev_out, bool (*compute)(void *), void *context);
+    bool move(hipStream_t stream, const char *src, Memory src_memory, size_t in_bytes,
+            char *dev_in, char *dst, Memory dst_memory, size_t out_bytes, const char *dev_out,
+            bool (*compute)(void *), void *context);
 };
 
 // A pass borrows its pinned blocks of 2 MB, at most eight for each direction, and gives them back
