@@ -123,6 +123,22 @@ def test_few_channels_gathering(oracle, t):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
+@pytest.mark.parametrize("t", [
+    (4, 12, 40, 40, 40, 5, 5, 1, 1, 2, 2),      # as many channels as the kernel is given
+    (2, 5, 130, 20, 20, 7, 7, 1, 1, 3, 3),      # filters over several workgroups
+    (3, 11, 32, 150, 150, 9, 9, 1, 1, 4, 4),    # more than 64 KB of LDS
+    (9, 8, 40, 24, 22, 5, 5, 1, 1, 2, 2),       # pixels that start on bytes
+], ids=str)
+def test_few_channels_in_their_kernel(oracle, monkeypatch, t, fmts, separate_k):
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    x, w = in_layout(x, w, fmts)
+    assert make(d, w, fmts).kernel_name(0).startswith("conv_mfma_fp4_shallow_kernel")
+    run_and_compare(oracle, d, x, w, fmts)
+
+
 @pytest.mark.parametrize("t", [
     (1, 1, 1, 3, 3, 1, 1, 1, 1, 0, 0),        # one value
     (1, 7, 5, 4, 4, 3, 3, 1, 1, 1, 1),        # 63 values: one short of a row of the sum
@@ -389,4 +405,18 @@ def test_launches_of_a_forward_pass(gpu, t, launches):
 ], ids=str)
 def test_steps_shared_by_waves(oracle, t):
     d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, x, w)
+
+
+@pytest.mark.parametrize("separate_k", [False, True])
+@pytest.mark.parametrize("t", [
+    (1, 64, 70, 9, 9, 1, 1, 1, 1, 0, 0),       # one step for four waves
+    (1, 64, 70, 9, 9, 1, 2, 1, 1, 0, 0),       # two
+    (2, 1000, 64, 7, 7, 3, 3, 1, 1, 1, 1),     # 144 for eight: more than a ring each
+], ids=str)
+def test_few_tiles_in_their_kernel(oracle, monkeypatch, t, separate_k):
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    assert make(d, w).kernel_name(0).startswith("conv_mfma_fp4_small_kernel")
     run_and_compare(oracle, d, x, w)

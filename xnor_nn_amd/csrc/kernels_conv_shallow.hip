@@ -40,7 +40,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_word;
 
-constexpr int SHALLOW_CHANNELS = 16;          // half a packed word per pixel
+constexpr int SHALLOW_CHANNELS = 12;          // (13 and up never meet the rule of shallow_plan)
 constexpr int SHALLOW_TABLES = 2 * 256 * 4;   // codes and validity masks
 constexpr uint32_t SHALLOW_DROP = 0xFFFFFFF0u;
 constexpr size_t SHALLOW_LDS = 160 * 1024;     // of a compute unit
@@ -155,7 +155,7 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
         const int y = (int)(R - img * s.prows) - s.ph;
         const int first = (int)s.div_ic.div(32u * d), x = first - s.pw; // may begin in the dword before
         const int pos = first * s.ic - 32 * d;  // bit its first channel would have: -IC < pos <= 0
-        const uint32_t at = ((img * s.ih + y) * s.iw + x) * 4u;
+        const uint32_t pixel = (img * s.ih + y) * s.iw + x, at = pixel * 4u;
         uint32_t out = 0;
         auto collect = [&](auto batch) { // all loads of a batch are under way together
             constexpr int N = decltype(batch)::value;
@@ -175,9 +175,15 @@ void conv_mfma_fp4_shallow_kernel(const uint32_t *__restrict__ xbits,
                         for (int n = 0; n < 4; n++) w[k + n] = (uint32_t)v[n];
                     }
                 } else {
+                    // One by one, each inside the buffer or dropped: loads at neighbouring offsets
+                    // are merged into a wide one by the compiler, and one that begins ahead of the
+                    // first pixel then loses the pixels behind it as well.
 #pragma unroll
-                    for (int k = 0; k < N; k++)
-                        w[k] = __builtin_amdgcn_raw_buffer_load_b32(xbuf, at + 4u * (k0 + k), 0, 0);
+                    for (int k = 0; k < N; k++) {
+                        const uint32_t q = pixel + (uint32_t)(k0 + k);
+                        w[k] = __builtin_amdgcn_raw_buffer_load_b32(xbuf,
+                                q < s.npix_in ? q * 4u : SHALLOW_DROP, 0, 0);
+                    }
                 }
 #pragma unroll
                 for (int k = N - 1; k > 0; k--) // first channel lowest
@@ -582,7 +588,7 @@ size_t choose_tile(const Plan &g, ShallowPlan &s, int *pixels) {
 
 } // namespace
 
-// Up to 16 input channels, where the large-launch kernel's pairs of taps are mostly padding.  Timed
+// Up to 12 input channels, where the large-launch kernel's pairs of taps are mostly padding.  Timed
 // beside it and beside the kernel for few tiles on 110 problems (us a pass, other / this):
 //   20 taps or more (5x5 and up) and at most 5/13 as many steps as pairs: ahead throughout, 5x5 of
 //   3 channels on 27x27 22.5 / 19.6, 7x7 of 5 channels on 46x46 34.2 / 19.2, 11x11 stride 4 of 3
