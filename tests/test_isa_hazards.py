@@ -211,6 +211,28 @@ def m0_outside_asm(body):
     return out
 
 
+def overwritten_stores(body):
+    """Stores of more than 64 bits whose data a vector instruction overwrites less than two wait
+    states later: such a store still reads its data then.  The compiler keeps the distance except
+    for buffer stores with a scalar offset."""
+    found = []
+    lines = [l.split(";")[0].strip() for l in body]
+    lines = [l for l in lines if l and not l.endswith(":") and not l.startswith(("#", "."))]
+    for i, line in enumerate(lines):
+        m = re.match(r"(buffer|global|flat)_store_dwordx[34]\s+(.*)", line)
+        if not m:
+            continue
+        data = vgprs(m.group(2).split(",")[0 if m.group(1) == "buffer" else 1])
+        waited = 0
+        for after in lines[i + 1:i + 3]:
+            nop = re.match(r"s_nop\s+(\w+)", after)
+            if waited < 2 and after.startswith("v_") \
+                    and vgprs(after.split(None, 1)[1].split(",")[0]) & data:
+                found.append((line, after))
+            waited += int(nop.group(1), 0) + 1 if nop else 1
+    return found
+
+
 def by_hand(*lines):
     """The lines as the compiler prints an inline-asm statement."""
     return [ASM_BEGIN] + list(lines) + [ASM_END]
@@ -242,6 +264,28 @@ def test_no_register_is_touched_while_its_load_is_in_flight(conv_isa):
             name[:90], m0_outside_asm(body)[0])
         checked += 1
     assert checked >= EXPECTED_VARIANTS, checked
+
+
+def test_no_wide_store_loses_its_data(conv_isa):
+    wide = 0
+    for name, body in kernels_of(conv_isa, r"^_ZN\S*conv_mfma_fp4\S*kernel\S*:"):
+        body = list(body)
+        wide += sum("store_dwordx4" in l for l in body)
+        bad = overwritten_stores(body)
+        assert not bad, "%s: %d stores, first: %s" % (name[:90], len(bad), bad[0])
+    assert wide > 1000  # channels-last output
+
+
+def test_the_check_of_wide_stores_sees_a_planted_one():
+    store = "buffer_store_dwordx4 v[4:7], v1, s[0:3], s9 offen nt"
+    over, other = "v_mov_b32_e32 v6, 0", "v_mov_b32_e32 v8, 0"
+    assert overwritten_stores([store, over]) == [(store, over)]
+    assert overwritten_stores([store, other, "; comment", over]) == [(store, over)]
+    assert overwritten_stores([store, other, other, over]) == []
+    assert overwritten_stores([store, "s_nop 1", over]) == []
+    assert overwritten_stores([store, "s_nop 0", over]) == [(store, over)]
+    assert overwritten_stores([store.replace("x4 v[4:7]", " v6"), over]) == []
+    assert overwritten_stores(["global_store_dwordx4 v[0:1], v[4:7], off", over]) != []
 
 
 def test_the_walker_sees_a_planted_hazard():

@@ -780,6 +780,11 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     // 128 contiguous bytes of 8 pixels instead of 32 bytes of 32 pixels.  Rows of 144 bytes
     // keep both sides free of bank conflicts.  A piece past OC (OC is a multiple of 4 here)
     // or a pixel past the end gets an offset outside the buffer.
+    // No scalar offset in these stores: a 16-byte store still reads its data after it has been
+    // issued, and what follows it must not overwrite the data at once.  The compiler keeps that
+    // distance unless the store has a scalar offset, which is said to make it unnecessary; here
+    // the first dword of sixteen lanes was then stored as the next instruction had left it, in
+    // one pass out of many thousands.
     auto store_lines_nhwc = [&](auto policy) {
         constexpr int STORE_AUX = decltype(policy)::value;
         float *mine = turn_lds + wave * (32 * TURN_ROW);
@@ -788,8 +793,8 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
 #pragma unroll
         for (int os = 0; os < 2; os++) {
             const uint32_t fpiece = (uint32_t)(chunk * NT + (fw * 2 + os) * 32 + 4 * piece);
-            const uint32_t base = fpiece < (uint32_t)g.oc
-                ? ((p_wave + (uint32_t)prow) * (uint32_t)g.oc + fpiece) * 4u : DROP;
+            const uint32_t base = ((p_wave + (uint32_t)prow) * (uint32_t)g.oc + fpiece) * 4u;
+            const uint32_t left_here = fpiece < (uint32_t)g.oc ? left : 0u;
 #pragma unroll
             for (int ps = 0; ps < PS; ps++) {
 #pragma unroll
@@ -809,9 +814,9 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
                     const v4i r = *reinterpret_cast<const v4i *>(
                             mine + (8 * j + prow) * TURN_ROW + 4 * piece);
                     const uint32_t in_tile = (uint32_t)(ps * 32 + 8 * j); // + prow
-                    const uint32_t voff = in_tile + (uint32_t)prow < left ? base : DROP;
-                    __builtin_amdgcn_raw_buffer_store_b128(r, outbuf, voff,
-                            in_tile * (uint32_t)g.oc * 4u, STORE_AUX);
+                    const uint32_t voff = in_tile + (uint32_t)prow < left_here
+                        ? base + in_tile * (uint32_t)g.oc * 4u : DROP;
+                    __builtin_amdgcn_raw_buffer_store_b128(r, outbuf, voff, 0, STORE_AUX);
                 }
             }
         }
