@@ -784,7 +784,7 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     // issued, and what follows it must not overwrite the data at once.  The compiler keeps that
     // distance unless the store has a scalar offset, which is said to make it unnecessary; here
     // the first dword of sixteen lanes was then stored as the next instruction had left it, in
-    // one pass out of many thousands.
+    // the first pass of most processes and hardly ever later.
     auto store_lines_nhwc = [&](auto policy) {
         constexpr int STORE_AUX = decltype(policy)::value;
         float *mine = turn_lds + wave * (32 * TURN_ROW);
