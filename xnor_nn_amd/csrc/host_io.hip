@@ -275,8 +275,9 @@ bool HostIo::move(hipStream_t stream, const char *src, Memory src_memory, size_t
         char *dev_in, char *dst, Memory dst_memory, size_t out_bytes, const char *dev_out,
         bool (*compute)(void *), void *context) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) == hipSuccess
-            && capture != hipStreamCaptureStatusNone)
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess)
+        (void)hipGetLastError(); // (no later call should report it)
+    else if (capture != hipStreamCaptureStatusNone)
         return false; // nothing would arrive before the graph runs
     // Directions that the runtime copies by itself: what the user has pinned needs no copy on this
     // side, and without pinned memory of our own the runtime's staging has to do.
