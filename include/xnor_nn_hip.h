@@ -36,7 +36,9 @@ xnor_nn_status_t xnor_nn_hip_set_stream(const xnor_nn_convolution_t *c, void *st
  *   XNOR_NN_HIP_DEVICE_POINTERS  src and dst are device pointers (the caller knows; otherwise
  *                                the driver is asked);
  *   XNOR_NN_HIP_ON_STREAM        xnor_nn_hip_set_stream(c, stream) first; without it `stream`
- *                                is not looked at. */
+ *                                is not looked at.
+ * One call to other threads as well, whichever kernels it takes: everything it enqueues goes to the
+ * stream that the descriptor has when it begins. */
 #define XNOR_NN_HIP_DEVICE_POINTERS 1
 #define XNOR_NN_HIP_ON_STREAM 2
 /* binarize_weights on slot user_weights first (with XNOR_NN_HIP_DEVICE_POINTERS a device pointer as

@@ -1,6 +1,7 @@
 """Host code of the library on the CPU, as it is compiled for it, linked with stand-ins for the runtime
-calls it makes: what moves host tensors (csrc/host_io.hip, host_io_check.cpp) and what asks for LDS
-(LdsGrant in csrc/plan.hpp, lds_grant_check.cpp)."""
+calls it makes: what moves host tensors (csrc/host_io.hip, host_io_check.cpp), what asks for LDS
+(LdsGrant in csrc/plan.hpp, lds_grant_check.cpp) and a forward pass in one call (csrc/api.hip,
+pass_stream_check.cpp)."""
 import os
 import subprocess
 
@@ -53,3 +54,9 @@ def test_host_io(program, case):
 def test_lds_is_granted_to_two_threads(program):
     """Two threads that ask for different sizes: the larger one stays granted."""
     run(program(os.path.join(HERE, "lds_grant_check.cpp")))
+
+
+@pytest.mark.parametrize("case", ["one pass", "stage fusion off", "popcount kernel", "old weights"])
+def test_a_pass_keeps_its_stream(program, case):
+    """Two threads with a stream each on one descriptor: all of a pass goes to its own."""
+    run(program(os.path.join(build.SRC, "api.hip"), os.path.join(HERE, "pass_stream_check.cpp")), case)

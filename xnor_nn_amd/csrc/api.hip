@@ -201,7 +201,7 @@ xnor_nn_status_t exec_binarize_data(const xnor_nn_convolution_t *c, xnor_nn_reso
         return xnor_nn_error_invalid_input;
     if (!is_data_format(c->src_format)) return xnor_nn_unimplemented;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     const void *x = nullptr;
     xnor_nn_status_t rc = stage_in(st, &st->stage_src, res[xnor_nn_resource_user_src],
             src_elems(st->g) * sizeof(float), &x);
@@ -235,7 +235,7 @@ xnor_nn_status_t exec_calculate_k(const xnor_nn_convolution_t *c, xnor_nn_resour
         return xnor_nn_error_invalid_input;
     if (!is_data_format(c->src_format)) return xnor_nn_unimplemented;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     float *a = static_cast<float *>(res[xnor_nn_resource_a]);
     float *k = static_cast<float *>(res[xnor_nn_resource_k]);
     const bool fuse = fusion_on(st);
@@ -293,7 +293,7 @@ xnor_nn_status_t exec_binarize_weights(const xnor_nn_convolution_t *c,
         return xnor_nn_error_invalid_input;
     if (!is_weights_format(c->weights_format)) return xnor_nn_unimplemented;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     withdraw_ready(res[xnor_nn_resource_a]);
     const void *w = nullptr;
     xnor_nn_status_t rc = stage_in(st, &st->stage_weights, res[xnor_nn_resource_user_weights],
@@ -315,7 +315,7 @@ xnor_nn_status_t exec_binarize_weights(const xnor_nn_convolution_t *c,
 xnor_nn_status_t run_convolution(const xnor_nn_convolution_t *c, xnor_nn_resources_t res,
         void *user_out, bool raw) {
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     withdraw_ready(res[xnor_nn_resource_a]);
     const size_t bytes = dst_elems(st->g) * 4;
     void *out = user_out;
@@ -677,9 +677,9 @@ void xnor_nn_binarize_weights_float(const xnor_nn_convolution_t *c,
     const bool from_dev = on_device(from), to_dev = on_device(to);
     float *dfrom = nullptr, *dto = nullptr, *own_parts = nullptr, *parts = nullptr;
     bool ok = true;
-    std::unique_lock<std::mutex> call;
+    std::unique_lock<std::recursive_mutex> call;
     if (st) { // the partial sums live with the descriptor
-        call = std::unique_lock<std::mutex>(st->mu);
+        call = std::unique_lock<std::recursive_mutex>(st->mu);
         if (!st->float_parts)
             ok = hipMalloc((void **)&st->float_parts, weights_float_parts() * sizeof(float))
                 == hipSuccess;
@@ -742,7 +742,7 @@ xnor_nn_status_t xnor_nn_hip_binarize_weights_float_noalloc(const xnor_nn_convol
 xnor_nn_status_t xnor_nn_hip_set_stream(const xnor_nn_convolution_t *c, void *stream) {
     if (!bcast_descriptor(c)) return xnor_nn_error_invalid_input;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     return change_stream(st, static_cast<hipStream_t>(stream));
 }
 
@@ -750,14 +750,16 @@ xnor_nn_status_t xnor_nn_hip_set_stream(const xnor_nn_convolution_t *c, void *st
 // buffers and the matrix-core convolution the pass is two launches and nothing else on the
 // host: one lock, no pointer query where the caller vouches for the buffers (a query is
 // 0.4 us, an executor call through ctypes as much again), no hand-over records.  Everything
-// else goes through the executors.
+// else goes through the executors, under the same hold of the lock: a stream that another thread sets
+// on the descriptor meanwhile counts from its next call on, not from the next stage of this one.
 xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
         xnor_nn_resources_t res, const void *src, void *dst, void *stream, int flags) {
     if (c == nullptr || res == nullptr) return xnor_nn_error_invalid_input;
     const bool weights_due = flags & XNOR_NN_HIP_NEW_WEIGHTS;
+    std::unique_lock<std::recursive_mutex> call;
     if (bcast_descriptor(c)) {
         State *st = state_of(c);
-        std::lock_guard<std::mutex> call(st->mu);
+        call = std::unique_lock<std::recursive_mutex>(st->mu);
         if (flags & XNOR_NN_HIP_ON_STREAM) {
             const xnor_nn_status_t rc = change_stream(st, static_cast<hipStream_t>(stream));
             if (rc != xnor_nn_success) return rc;
@@ -807,7 +809,7 @@ xnor_nn_status_t xnor_nn_hip_forward_pass(const xnor_nn_convolution_t *c,
 xnor_nn_status_t xnor_nn_hip_set_stage_fusion(const xnor_nn_convolution_t *c, int on) {
     if (!bcast_descriptor(c)) return xnor_nn_error_invalid_input;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     st->fuse_stages = on != 0;
     return xnor_nn_success;
 }
@@ -816,7 +818,7 @@ xnor_nn_status_t xnor_nn_hip_time_kernels(const xnor_nn_convolution_t *c, int ca
     if (!bcast_descriptor(c) || capacity < 0 || capacity > 65536)
         return xnor_nn_error_invalid_input;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     if (hipStreamSynchronize(st->stream) != hipSuccess) return xnor_nn_error_memory;
     if (!make_timer(st->time_binarize, capacity) || !make_timer(st->time_convolution, capacity)) {
         drop_timer(st->time_binarize); // never one stage timed and the other not
@@ -829,7 +831,7 @@ xnor_nn_status_t xnor_nn_hip_time_kernels(const xnor_nn_convolution_t *c, int ca
 int xnor_nn_hip_kernel_times(const xnor_nn_convolution_t *c, int stage, float *ms, int max) {
     if (!bcast_descriptor(c) || ms == nullptr || max < 0) return -1;
     State *st = state_of(c);
-    std::lock_guard<std::mutex> call(st->mu);
+    std::lock_guard<std::recursive_mutex> call(st->mu);
     KernelTimer *t = stage == xnor_nn_operation_binarize_data ? &st->time_binarize
         : stage == xnor_nn_operation_convolution_forward ? &st->time_convolution : nullptr;
     if (t == nullptr) return -1;
@@ -923,7 +925,7 @@ xnor_nn_status_t xnor_nn_hip_export_floats(const xnor_nn_convolution_t *c,
     if (!res[slot] || dst_bytes != c->resource_size[slot]) return xnor_nn_error_invalid_input;
     if (slot == xnor_nn_resource_k) { // a deferred box filter has to run before K is read
         State *st = state_of(c);
-        std::lock_guard<std::mutex> call(st->mu);
+        std::lock_guard<std::recursive_mutex> call(st->mu);
         xnor_nn_status_t rc = settle_k(st, static_cast<float *>(res[slot]));
         if (rc != xnor_nn_success) return rc;
     }

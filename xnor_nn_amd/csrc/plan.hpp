@@ -248,8 +248,8 @@ struct State {
     // Held for the length of every executor call: two host threads may share one descriptor
     // (each with a resource table of its own), and the staging buffers below, the stream and
     // the order in which a call's launches and copies are enqueued belong to one call at a
-    // time.
-    std::mutex mu;
+    // time.  Recursive: xnor_nn_hip_forward_pass holds it over the executors it calls.
+    std::recursive_mutex mu;
     // staging buffers for host-side user tensors (allocated on first use, a multiple of 16 bytes)
     // and what moves the bytes
     void *stage_src = nullptr, *stage_weights = nullptr, *stage_dst = nullptr;
