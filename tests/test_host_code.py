@@ -1,7 +1,8 @@
 """Host code of the library on the CPU, as it is compiled for it, linked with stand-ins for the runtime
 calls it makes: what moves host tensors (csrc/host_io.hip, host_io_check.cpp), what asks for LDS
 (LdsGrant in csrc/plan.hpp, lds_grant_check.cpp) and a forward pass in one call (csrc/api.hip,
-pass_stream_check.cpp)."""
+pass_stream_check.cpp); and the rows that the matrix-core kernels read (csrc/tap_walk.hpp,
+tap_walk_check.cpp)."""
 import os
 import subprocess
 
@@ -60,3 +61,8 @@ def test_lds_is_granted_to_two_threads(program):
 def test_a_pass_keeps_its_stream(program, case):
     """Two threads with a stream each on one descriptor: all of a pass goes to its own."""
     run(program(os.path.join(build.SRC, "api.hip"), os.path.join(HERE, "pass_stream_check.cpp")), case)
+
+
+def test_kernel_taps_read_staged_rows(program):
+    """Nothing is read past what a tile has staged, not behind the last tap either."""
+    run(program(os.path.join(HERE, "tap_walk_check.cpp")))

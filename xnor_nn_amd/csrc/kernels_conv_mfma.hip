@@ -34,6 +34,7 @@
 
 #include "box_sum.hpp"
 #include "plan.hpp"
+#include "tap_walk.hpp"
 
 namespace xnor_hip {
 
@@ -332,15 +333,8 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
         in0[ps] = (int)(img[ps] * g.ihw) + ih0 * g.iw + iw0 - lo;
         taprow[ps] = (uint32_t)(size_t)rows + (uint32_t)((1 + in0[ps]) * ROW_BYTES)
             + (lane >> 5) * 16;
-        // kernel rows kh with 0 <= ih0 + kh < ih, as a run of bits (kh < 32)
-        auto run_of_bits = [](int first, int last) -> uint32_t { // bits first..last, clipped
-            if (first < 0) first = 0;
-            if (last > 31) last = 31;
-            if (last < first) return 0u;
-            return (0xFFFFFFFFu >> (31 - last)) & (0xFFFFFFFFu << first);
-        };
-        rowmask[ps] = live[ps] ? run_of_bits(-ih0, g.ih - 1 - ih0) : 0u;
-        colmask[ps] = run_of_bits(-iw0, g.iw - 1 - iw0);
+        rowmask[ps] = live[ps] ? taps_inside(ih0, g.ih, g.kh) : 0u;
+        colmask[ps] = taps_inside(iw0, g.iw, g.kw);
     }
     const uint32_t zero_addr = (uint32_t)(size_t)rows + (lane >> 5) * 16;
 
@@ -466,36 +460,14 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
             load_frag_async<(hs & 3) * 1024>(w[hs][os], wdesc, wvoff,
                     wbase[os] + (uint32_t)(group * HS + (hs & ~3)) * 1024u);
     };
-    // LDS address of each pixel's row for the next tap of the walk: the row `taprow` of the tap, or
-    // the zero row when the tap falls outside the image.  Every in-bounds tap of a tile lies inside
-    // the span of rows the tile has staged (tile_span).  The masks are kept reversed, so that a tap is
-    // valid if the top bit of both, shifted to it, is set, and the address moves along: six
-    // instructions per tap and block (an address computed from (kh, kw) took fifteen, most of the
-    // loop where a tap is one step).  Behind the last tap the row mask is empty: the zero row.
-    uint32_t colbits[PS], rowbits[PS];
+    // LDS address of each pixel's row for the next tap of the walk (tap_walk.hpp).  Every in-bounds tap
+    // of a tile lies inside the span of rows the tile has staged (tile_span).
+    TapWalk<PS, DEEP> walk;
 #pragma unroll
-    for (int ps = 0; ps < PS; ps++) {
-        colbits[ps] = __brev(colmask[ps]);
-        rowbits[ps] = __brev(rowmask[ps]);
-    }
+    for (int ps = 0; ps < PS; ps++) walk.begin(ps, taprow[ps], rowmask[ps], colmask[ps]);
     const uint32_t row_step = (uint32_t)((g.iw - g.kw + 1) * ROW_BYTES); // last column to next row
-    int nkw = 0, npart = 0; // column, and DEEP: channel part, of the next tap
     auto tap_rows = [&](uint32_t (&out)[PS]) {
-#pragma unroll
-        for (int ps = 0; ps < PS; ps++)
-            out[ps] = (int)(rowbits[ps] & (colbits[ps] << nkw)) < 0
-                ? taprow[ps] + (DEEP ? (uint32_t)(npart * KS * 32) : 0u) : zero_addr;
-        if constexpr (DEEP) {
-            if (++npart < ic_parts) return;
-            npart = 0;
-        }
-        const bool next_row = ++nkw == g.kw; // uniform
-        nkw = next_row ? 0 : nkw;
-#pragma unroll
-        for (int ps = 0; ps < PS; ps++) {
-            rowbits[ps] <<= next_row ? 1 : 0;
-            taprow[ps] += next_row ? row_step : (uint32_t)ROW_BYTES;
-        }
+        walk.next(out, zero_addr, (uint32_t)ROW_BYTES, row_step, g.kw, ic_parts, KS * 32);
     };
     // PAIR: rows of the two taps of a pair (index 0 and 1).  A missing second tap (odd number of
     // taps, or a pair behind the last) reads the zero row.
@@ -699,13 +671,12 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     const bool nchw = RAW || g.dst_fmt == xnor_nn_data_format_nchw;
     const uint32_t fstep = nchw ? (uint32_t)g.ohw * 4u : 4u; // bytes from a filter to the next
     int n[PS];
-    const uint32_t kh_bits = 0xFFFFFFFFu >> (32 - g.kh), kw_bits = 0xFFFFFFFFu >> (32 - g.kw);
     uint32_t off1[PS]; // one block: lanes 0..31 filter f, lanes 32..63 filter f + 4
 #pragma unroll
     for (int ps = 0; ps < PS; ps++) {
         // operation count of the pixel (reference src/bcast_binarize_weights.cpp:126-142):
         // channels times the taps inside the image, from the same masks the main loop used
-        n[ps] = RAW ? g.ic * __popc(rowmask[ps] & kh_bits) * __popc(colmask[ps] & kw_bits) : 0;
+        n[ps] = RAW ? g.ic * __popc(rowmask[ps]) * __popc(colmask[ps]) : 0;
         const uint32_t at = nchw ? (img[ps] * (uint32_t)g.oc * (uint32_t)g.ohw + rem[ps]) * 4u
                                  : pix[ps] * (uint32_t)g.oc * 4u;
         off1[ps] = live[ps] ? at + (uint32_t)lane_hi * 4u * fstep : DROP;

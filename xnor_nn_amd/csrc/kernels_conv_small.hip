@@ -32,6 +32,7 @@
 
 #include "box_sum.hpp"
 #include "plan.hpp"
+#include "tap_walk.hpp"
 
 namespace xnor_hip {
 
@@ -136,14 +137,8 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     const int oh = (int)g.div_ow.div(rem), ow = (int)rem - oh * g.ow;
     const int ih0 = oh * g.sh - g.ph, iw0 = ow * g.sw - g.pw; // input pixel of tap (0,0)
     const int in0 = (int)(img * g.ihw) + ih0 * g.iw + iw0 - lo;
-    auto run_of_bits = [](int first, int last) -> uint32_t { // bits first..last, clipped
-        if (first < 0) first = 0;
-        if (last > 31) last = 31;
-        if (last < first) return 0u;
-        return (0xFFFFFFFFu >> (31 - last)) & (0xFFFFFFFFu << first);
-    };
-    const uint32_t rowmask = live ? run_of_bits(-ih0, g.ih - 1 - ih0) : 0u;
-    const uint32_t colmask = run_of_bits(-iw0, g.iw - 1 - iw0);
+    const uint32_t rowmask = live ? taps_inside(ih0, g.ih, g.kh) : 0u;
+    const uint32_t colmask = taps_inside(iw0, g.iw, g.kw);
     // byte offsets into `rows` of the row of tap (0,0) of the lane's pixel; row 0 is zero
     const int base_off = (1 + in0) * s.row_bytes;
 
