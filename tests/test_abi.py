@@ -313,6 +313,18 @@ def test_inputs_that_reach_the_dropped_offset_take_the_generic_kernel():
         == "binarize_nhwc_tiled_kernel"
 
 
+def test_channels_last_input_is_streamed_by_size():
+    """Not where the L2s may hold it, nor where it is large."""
+    nhwc = (capi.FMT_NHWC, capi.FMT_OIHW, capi.FMT_NHWC)
+    for t, streams in (((2, 8, 1024, 64, 64, 1, 1, 1, 1, 0, 0), False),      # 32 MB
+                       ((13, 8, 100, 81, 80, 3, 3, 1, 1, 1, 1), True),       # a little more
+                       ((100, 256, 128, 32, 32, 3, 3, 1, 1, 1, 1), True),
+                       ((1, 8, 1040, 161, 160, 1, 1, 1, 1, 0, 0), True),     # 102 MB
+                       ((1, 8, 1040, 162, 162, 1, 1, 1, 1, 0, 0), False)):   # 104 MB and a little
+        assert kernel_names(t, nhwc)[0] \
+            == "binarize_nhwc_tiled_kernel" + ("<STREAM>" if streams else ""), t
+
+
 def test_persistent_workgroups_are_planned_on_request_only(monkeypatch):
     """XNOR_NN_HIP_MFMA_PERSIST=N: N workgroups per XCD that walk over the tiles; without it a
     workgroup per tile, whatever the size (measured faster)."""

@@ -335,6 +335,20 @@ def test_nhwc_input_kernels(oracle, monkeypatch, t, by_lane):
     run_and_compare(oracle, d, x, w, fmts)
 
 
+def test_streamed_nhwc_input(oracle):
+    """Channels-last input of a little more than 32 MB; a ragged last tile and slice."""
+    d = shapes.as_dims((13, 100, 3, 81, 80, 3, 3, 2, 2, 1, 1))
+    x = synth.normal(97, d["mb"] * d["ic"] * d["ih"] * d["iw"]).reshape(
+        d["mb"], d["ih"], d["iw"], d["ic"])
+    x.ravel()[::5] = 0.0
+    x.ravel()[1::7] = -0.0
+    w = synth.normal(98, d["oc"] * d["ic"] * d["kh"] * d["kw"], 0.05).reshape(
+        d["oc"], d["ic"], d["kh"], d["kw"])
+    fmts = (capi.FMT_NHWC, capi.FMT_OIHW, capi.FMT_NCHW)
+    assert make(d, w, fmts).kernel_name(2) == "binarize_nhwc_tiled_kernel<STREAM>"
+    run_and_compare(oracle, d, x, w, fmts)
+
+
 def _random_case(rng):
     kh, kw = int(rng.integers(1, 8)), int(rng.integers(1, 8))
     ph, pw = int(rng.integers(0, 4)), int(rng.integers(0, 4))

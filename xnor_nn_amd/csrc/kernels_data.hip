@@ -17,14 +17,7 @@ namespace {
 constexpr int TILE = 64;       // pixels per workgroup = lanes per wave
 constexpr int MAX_WAVES = 12;  // waves per workgroup
 constexpr int TURN_ROW = 36;   // floats per pixel row of the NHWC turn-around buffer (32 + 4)
-// Cache policy of the NHWC input: the "nt" bit.  Every line is read once and whole, so it need not
-// push out what waits in the caches to be written back.  us a pass without / with it, on changing
-// inputs, on the same one, on one that the kernel before has written: 128 to 256 channels on 32x32,
-// minibatch 100, 42.8 / 40.7, 38.8 / 39.1, 58.4 / 56.2; 256 channels on 56x56, minibatch 64,
-// 111.8 / 104.4, 98.5 / 101.7, 158.7 / 161.5; 384 on 13x13, minibatch 256, 38.1 / 36.1, 34.6 / 34.7,
-// 54.5 / 55.7; 64 on 56x56 28.1 / 26.7, 26.3 / 24.1, 43.7 / 42.7.  Not for NCHW, where neighbouring
-// tiles share lines: 384 channels on 13x13 44.9 / 41.7 on changing inputs, but 35.8 / 39.6 on the same
-// one and 56.2 / 65.1 on one just written, as a network's layers find it.
+// Cache policy of the NHWC input: the "nt" bit, or none (nhwc_streams)
 constexpr int LOAD_STREAMING = 2;
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
@@ -57,7 +50,7 @@ __device__ __forceinline__ uint32_t fbits(float v) { return __float_as_uint(v); 
 // every load instruction reads eight whole cache lines, and turns the block around through
 // LDS into the lane = pixel layout (one lane per pixel straight from memory, 64 partial
 // cache lines per instruction, took 19.7 us where this takes 13.5 us, the NCHW kernel 13.3).
-template <bool NHWC, bool WRITE_BITS, bool WRITE_A>
+template <bool NHWC, bool STREAM, bool WRITE_BITS, bool WRITE_A>
 __device__ __forceinline__
 void binarize_tile(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry &g, const float inv_ic, const int rounds,
@@ -106,7 +99,7 @@ void binarize_tile(const float *__restrict__ x, uint32_t *__restrict__ bits,
                 const uint32_t off = c < g.ic ? qc * (uint32_t)g.ic * 4u + (uint32_t)c * 4u
                                               : 0xFFFFFFF0u;
                 v[i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
-                        src, off, 0, LOAD_STREAMING));
+                        src, off, 0, STREAM ? LOAD_STREAMING : 0));
             }
             float *mine = turn + wave * (32 * TURN_ROW);
 #pragma unroll
@@ -196,7 +189,7 @@ __global__ __launch_bounds__(TILE * 16)
 void binarize_nchw_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry g, const float inv_ic, const int rounds,
         const uint32_t ntiles, const uint32_t tiles_per_xcd) {
-    binarize_tile<false, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
+    binarize_tile<false, false, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
             tiles_per_xcd, blockIdx.x);
 }
 
@@ -215,7 +208,7 @@ void binarize_nchw_and_weights_kernel(const float *__restrict__ x, uint32_t *__r
     extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ Runs runs;
     if (blockIdx.x >= weight_blocks) {
-        binarize_tile<false, true, true>(x, bits, a, g, inv_ic, rounds, ntiles, tiles_per_xcd,
+        binarize_tile<false, false, true, true>(x, bits, a, g, inv_ic, rounds, ntiles, tiles_per_xcd,
                 blockIdx.x - weight_blocks);
         return;
     }
@@ -224,12 +217,12 @@ void binarize_nchw_and_weights_kernel(const float *__restrict__ x, uint32_t *__r
     filter_stage(w, wbits, frag, alpha, opc, g, f, row, runs, blockIdx.x);
 }
 
-template <bool WRITE_BITS, bool WRITE_A>
+template <bool STREAM, bool WRITE_BITS, bool WRITE_A>
 __global__ __launch_bounds__(TILE * 16)
 void binarize_nhwc_tiled_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry g, const float inv_ic, const int rounds,
         const uint32_t ntiles, const uint32_t tiles_per_xcd) {
-    binarize_tile<true, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
+    binarize_tile<true, STREAM, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
             tiles_per_xcd, blockIdx.x);
 }
 
@@ -552,6 +545,27 @@ int tiled_waves(const Plan &g, int *rounds) {
     return (g.xw + *rounds - 1) / *rounds;
 }
 
+// Whether the tiled kernel reads its NHWC input with the "nt" bit: every line is read once and whole, so
+// it need not push out what waits in the caches to be written back.  It pays for inputs above the 32 MB
+// of the eight L2s and up to 104 MB.  Smaller ones may still lie in the L2s, where the bit lets them go;
+// larger ones lose where they have just been written, which is how a network's layers find them.  us a
+// pass with / without it, on changing inputs, on the same one, on one that a kernel has just written, on
+// changing ones just written:
+//   13 MB   256 channels 14x14   14.5 / 14.6   14.0 / 13.0   24.2 / 22.8   19.6 / 19.0
+//   26 MB   64 on 56x56          16.0 / 16.8   14.7 / 13.9   31.0 / 32.4   26.2 / 25.4
+//   38 MB   64 on 56x56          21.6 / 22.6   19.1 / 20.9   35.1 / 38.0   35.7 / 34.3
+//   52 MB   128 on 32x32         37.9 / 39.8   35.6 / 38.1   55.7 / 56.1   56.6 / 55.1
+//   103 MB  128 on 56x56         32.0 / 35.2   29.6 / 30.9   60.0 / 60.4   64.2 / 62.6
+//   128 MB  100 on 40x40         62.4 / 65.9   59.8 / 55.4  112.2 / 100.6 112.6 / 112.8
+//   154 MB  192 on 56x56         57.3 / 62.0   55.9 / 54.5  106.6 / 101.9 110.0 / 103.8
+//   205 MB  256 on 56x56         97.6 / 104.8  94.7 / 90.3  152.4 / 150.1 152.5 / 152.8
+// Not for NCHW, where neighbouring tiles share lines: 384 channels on 13x13 44.9 / 41.7 (without / with)
+// on changing inputs, but 35.8 / 39.6 on the same one and 56.2 / 65.1 on one just written.
+bool nhwc_streams(const Plan &g) {
+    const uint64_t bytes = (uint64_t)g.npix_in * (uint64_t)g.ic * 4u;
+    return bytes > (32u << 20) && bytes <= (104u << 20);
+}
+
 template <bool NHWC, bool WRITE_BITS, bool WRITE_A>
 void launch_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
         const KernelEvents &ev) {
@@ -566,8 +580,10 @@ void launch_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipSt
     size_t lds = sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw);
     if (NHWC) lds = ((lds + 15) & ~(size_t)15) + sizeof(float) * nw * 32 * TURN_ROW;
     if (NHWC)
-        launch_kernel(binarize_nhwc_tiled_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
-                dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
+        launch_kernel(nhwc_streams(g) ? binarize_nhwc_tiled_kernel<true, WRITE_BITS, WRITE_A>
+                                      : binarize_nhwc_tiled_kernel<false, WRITE_BITS, WRITE_A>,
+                dim3(per_xcd * 8), dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic,
+                rounds, ntiles, per_xcd);
     else
         launch_kernel(binarize_nchw_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
                 dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
@@ -691,7 +707,8 @@ const char *binarize_kernel_name(const Plan &g) {
         : split_nchw(g) ? "binarize_nchw_split_kernel"
         : tiled_nchw(g) ? "binarize_nchw_kernel"
         : !vector_nhwc(g) ? "binarize_generic_kernel"
-        : nhwc_by_lane(g) ? "binarize_nhwc_kernel" : "binarize_nhwc_tiled_kernel";
+        : nhwc_by_lane(g) ? "binarize_nhwc_kernel"
+        : nhwc_streams(g) ? "binarize_nhwc_tiled_kernel<STREAM>" : "binarize_nhwc_tiled_kernel";
 }
 
 hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
