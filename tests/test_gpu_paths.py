@@ -561,6 +561,43 @@ def test_k_sums_by_kernel_width(oracle, monkeypatch, blocks, kw):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("t,joined", [
+    ((26, 384, 40, 13, 13, 3, 3, 1, 1, 1, 1), True),
+    ((26, 70, 8, 13, 13, 15, 15, 4, 4, 7, 7), True),      # long filters, few tiles
+    ((75, 64, 8, 88, 88, 3, 3, 4, 4, 1, 1), True),        # 9075 tiles, short filters
+    ((72, 40, 8, 64, 64, 19, 19, 4, 4, 9, 9), False),     # 4608, long filters, few channels
+], ids=str)
+def test_new_weights_join_the_binarize_launch(gpu, t, joined):
+    """Where the filters' LDS leaves the tiles enough workgroups; the same result either way."""
+    import torch
+    d, x, w = problem(t)
+    wt, xt = torch.from_numpy(w).to(gpu), torch.from_numpy(x).to(gpu)
+    conv = make(d, -2 * wt)
+    try:
+        assert conv.kernel_name(0).startswith("conv_mfma_fp4")
+        yt = torch.empty(d["mb"], d["oc"], conv.desc.oh, conv.desc.ow, device=gpu)
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        conv.forward_on_stream(xt, yt, side.cuda_stream, wt)
+        torch.cuda.synchronize()
+        first = yt.clone()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=side):
+            conv.forward_on_stream(xt, yt, side.cuda_stream, wt)
+        nodes = C.c_size_t()
+        assert conv.lib.hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None,
+                                         C.byref(nodes)) == 0
+        assert nodes.value == (2 if joined else 3)
+        conv.change_weights(wt)
+        yt.fill_(float("nan"))
+        torch.cuda.synchronize()
+        conv.forward(xt, yt)
+        torch.cuda.synchronize()
+        assert torch.equal(first, yt)
+    finally:
+        conv.close()
+
+
 @pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
 @pytest.mark.parametrize("t", [
     (26, 384, 40, 13, 13, 3, 3, 1, 1, 1, 1),    # in one launch with twelve waves of input

@@ -747,26 +747,60 @@ hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
     return hipGetLastError();
 }
 
+namespace {
+
+// The grid of binarize_nchw_and_weights_kernel: tiles, and filters ahead of them.
+struct JoinedGrid {
+    int rounds, tile_waves, waves; // of a tile; of any workgroup
+    uint32_t ntiles, per_xcd, weight_blocks;
+    FilterPlan filters;
+    size_t lds;                    // dynamic; every workgroup has `Runs` beside it
+};
+JoinedGrid joined_grid(const Plan &g, bool fragments) {
+    JoinedGrid j{};
+    j.tile_waves = tiled_waves(g, &j.rounds);
+    j.waves = j.tile_waves < FILTER_WAVES ? FILTER_WAVES : j.tile_waves;
+    j.ntiles = (g.npix_in + TILE - 1) / TILE;
+    j.per_xcd = (j.ntiles + 7) / 8;
+    j.filters = filter_plan(g, fragments);
+    j.weight_blocks = (j.filters.workgroups + 7) / 8 * 8;
+    const size_t tile = sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw);
+    j.lds = tile > j.filters.lds ? tile : j.filters.lds;
+    return j;
+}
+
+} // namespace
+
+// A tile of the joined launch takes the LDS of a filter and four waves at least.  Where long filters leave
+// a compute unit fewer workgroups than its 32 waves allow, what the tiles lose grows with their number
+// and what the launch saves does not: joined while there are at most seven tiles for every 32 channels
+// that are under way on a unit.  us of a pass with new weights, joined / in two launches, beside the tiles
+// up to which they are joined (64 filters, planes of 64x64, stride 4):
+//   40 channels 19x19   4480 tiles   4096: 106.4 / 110.2   8192: 124.6 / 119.4   12288: 204.8 / 182.1
+//   64 channels 15x15   7168         4096:  74.9 /  81.2   8192:  99.2 /  99.6   12288: 152.9 / 147.6
+//   96 channels 12x12  10752         4096:  64.3 /  70.6   8192: 119.6 / 122.4   12288: 146.1 / 143.7
+//   128 channels 11x11 14336         8192: 133.3 / 134.4  12288: 186.5 / 196.5   24576: 361.2 / 353.0
+// Nowhere else was joining slower, on 60 layers: 384 channels 3x3 on 13x13, minibatch 64, 20.9 / 26.6, 256
+// channels 7x7 on 14x14, minibatch 128, 54.8 / 58.8, 64 channels 3x3 on 224x224, minibatch 64 (50176
+// tiles, as many workgroups as the waves allow), 273 / 280.
 bool weights_join_binarize(const Plan &g) {
-    return tiled_nchw(g) && !shallow_nchw(g) && !split_nchw(g) && filter_kernel_applies(g);
+    if (!tiled_nchw(g) || shallow_nchw(g) || split_nchw(g) || !filter_kernel_applies(g)) return false;
+    const JoinedGrid j = joined_grid(g, g.use_mfma != 0);
+    const int by_waves = 32 / j.waves, by_lds = (int)(160 * 1024 / (j.lds + sizeof(Runs)));
+    return by_lds >= by_waves
+        || (uint64_t)j.ntiles * 32 <= (uint64_t)7 * by_lds * g.ic * g.cus;
 }
 
 hipError_t launch_binarize_data_and_weights(const Plan &g, const float *x, uint32_t *bits, float *a,
         const float *w, uint32_t *wbits, uint32_t *frag, float *alpha, int32_t *opc, hipStream_t s) {
-    int rounds;
-    const int own = tiled_waves(g, &rounds), nw = own < FILTER_WAVES ? FILTER_WAVES : own;
-    const uint32_t ntiles = (g.npix_in + TILE - 1) / TILE, per_xcd = (ntiles + 7) / 8;
-    const FilterPlan f = filter_plan(g, frag != nullptr);
-    const uint32_t weight_blocks = (f.workgroups + 7) / 8 * 8;
-    const size_t tile = sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw);
-    const size_t lds = tile > f.lds ? tile : f.lds;
+    const JoinedGrid j = joined_grid(g, frag != nullptr);
     static LdsGrant grant;
     const hipError_t e = grant.ask((const void *)binarize_nchw_and_weights_kernel,
-            lds + sizeof(Runs));
+            j.lds + sizeof(Runs));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(binarize_nchw_and_weights_kernel, dim3(weight_blocks + per_xcd * 8),
-            dim3(nw * TILE), lds, s, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd,
-            weight_blocks, w, wbits, frag, alpha, opc, f);
+    hipLaunchKernelGGL(binarize_nchw_and_weights_kernel, dim3(j.weight_blocks + j.per_xcd * 8),
+            dim3(j.waves * TILE), j.lds, s, x, bits, a, geometry(g), 1.f / g.ic, j.rounds, j.ntiles,
+            j.per_xcd, j.weight_blocks, w, wbits, frag, alpha, opc, j.filters);
     return hipGetLastError();
 }
 
