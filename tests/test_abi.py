@@ -6,6 +6,7 @@ import os
 import re
 import subprocess
 
+import numpy as np
 import pytest
 
 from xnor_nn_amd import capi
@@ -402,3 +403,24 @@ def test_weight_stage_kernel_names():
     assert name((1, 8, 1612, 4, 4, 2, 5, 1, 1, 2, 2)) == "binarize_filter_kernel"  # 16120 values
     assert name((1, 8, 1613, 4, 4, 2, 5, 1, 1, 2, 2)) == "pack_weights_kernel"
     assert name((1, 8, 64, 4, 4, 3, 3, 1, 1, 1, 1), capi.FMT_HWIO) == "pack_weights_kernel"
+
+
+def test_only_new_weights_on_the_gpu_are_vouched_for():
+    """forward_on_stream: weights in host memory must not reach a kernel as they are."""
+    import torch
+
+    from xnor_nn_amd.convolution import Convolution
+
+    class OnGpu:
+        is_cuda = True
+        data_ptr = staticmethod(lambda: 64)
+
+    calls = []
+    conv = Convolution.__new__(Convolution)
+    conv.lib, conv.res, conv._desc_at, conv._res_at = None, capi.Resources(), 1, 2
+    conv._forward_pass = lambda *args: calls.append(args) or capi.SUCCESS
+    for weights in (None, OnGpu(), torch.zeros(4), np.zeros(4, np.float32), 4096):
+        conv.forward_on_stream(OnGpu(), OnGpu(), 3, weights)
+    new, vouched = capi.NEW_WEIGHTS | capi.ON_STREAM, capi.DEVICE_POINTERS
+    assert [c[:5] for c in calls] == [(1, 2, 64, 64, 3)] * 5
+    assert [c[5] for c in calls] == [vouched | capi.ON_STREAM, vouched | new, new, new, new]

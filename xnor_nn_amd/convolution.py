@@ -60,12 +60,15 @@ class Convolution:
 
     def forward_on_stream(self, src, dst, stream, new_weights=None):
         """The same on torch tensors on the GPU, on a stream given by its handle; with new_weights
-        (on the GPU too) as after change_weights."""
+        as after change_weights.  Weights that torch does not know to be on the GPU are left to the
+        library, which asks the driver where they are and brings what is in host memory."""
         flags = capi.DEVICE_POINTERS | capi.ON_STREAM
         if new_weights is not None:
             self._weights = new_weights
             self.res[capi.RES_USER_WEIGHTS] = capi.as_pointer(new_weights)
             flags |= capi.NEW_WEIGHTS
+            if not getattr(new_weights, "is_cuda", False):
+                flags &= ~capi.DEVICE_POINTERS
         status = self._forward_pass(self._desc_at, self._res_at, src.data_ptr(), dst.data_ptr(),
                                     stream, flags)
         if status:
