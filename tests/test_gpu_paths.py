@@ -636,3 +636,63 @@ def test_pass_with_new_weights(oracle, gpu, monkeypatch, t, fmts, separate_k):
         assert np.array_equal(conv.forward_popcount(), want["popc"])
     finally:
         conv.close()
+
+
+@pytest.mark.parametrize("t", [
+    (26, 384, 64, 13, 13, 3, 3, 1, 1, 1, 1),    # weights join the binarize launch
+    (2, 64, 64, 7, 7, 3, 3, 1, 1, 1, 1),        # a pass of one launch
+], ids=str)
+@pytest.mark.parametrize("tensors", ["device", "host", "mixed", "timed"])
+@pytest.mark.parametrize("weights", ["device", "host"])
+def test_new_weights_wherever_they_lie(oracle, gpu, t, tensors, weights):
+    """XNOR_NN_HIP_NEW_WEIGHTS and nothing vouched for; "timed": with kernel timing on."""
+    import torch
+    d, x, w = problem(t, zeros=True)
+    s = oracle_shape(oracle, d)
+    want = oracle.forward(s, x, w)
+    conv = make(d, torch.from_numpy(-2 * w).to(gpu))
+    try:
+        xt, wt = (torch.from_numpy(v).to(gpu) for v in (x, w))
+        yt = torch.full(want["dst"].shape, float("nan"), device=gpu)
+        dst = np.full(want["dst"].shape, np.nan, np.float32)
+        torch.cuda.synchronize()
+        src = capi.as_pointer(x if tensors == "host" else xt)
+        to = capi.as_pointer(dst if tensors in ("host", "mixed") else yt)
+        call = lambda src: conv.lib.xnor_nn_hip_forward_pass(
+            C.byref(conv.desc), conv.res, src, to, None, capi.NEW_WEIGHTS)
+        conv.res[capi.RES_USER_WEIGHTS] = None
+        assert call(src) == capi.ERROR_INVALID_INPUT
+        conv.res[capi.RES_USER_WEIGHTS] = capi.as_pointer(wt if weights == "device" else w)
+        assert call(None) == capi.ERROR_INVALID_INPUT
+        if tensors == "timed":
+            conv.time_kernels(8)
+        for _ in range(2):
+            assert call(src) == capi.SUCCESS
+        conv.synchronize()
+        if tensors == "timed":
+            for stage in (capi.OP_BINARIZE_DATA, capi.OP_CONVOLUTION_FORWARD):
+                assert len(conv.kernel_times(stage)) == 2
+        got = dst if tensors in ("host", "mixed") else yt.cpu().numpy()
+        assert same_bits(got, want["dst"])
+        assert same_bits(conv.export_floats(capi.RES_ALPHA), want["alpha"])
+        assert np.array_equal(conv.export_bin_weights(), want["bin_weights"])
+    finally:
+        conv.close()
+
+
+def test_new_weights_in_host_memory_on_a_stream(oracle, gpu):
+    import torch
+    d, x, w = problem((26, 384, 64, 13, 13, 3, 3, 1, 1, 1, 1))
+    want = oracle.forward(oracle_shape(oracle, d), x, w)
+    xt = torch.from_numpy(x).to(gpu)
+    conv = make(d, torch.from_numpy(-2 * w).to(gpu))
+    try:
+        side = torch.cuda.Stream()
+        for weights in (w, torch.from_numpy(w)):
+            yt = torch.full(want["dst"].shape, float("nan"), device=gpu)
+            torch.cuda.synchronize()
+            conv.forward_on_stream(xt, yt, side.cuda_stream, weights)
+            conv.synchronize()
+            assert same_bits(yt.cpu().numpy(), want["dst"])
+    finally:
+        conv.close()
