@@ -244,7 +244,8 @@ void partial_sum_kernel(const float *__restrict__ from, float *__restrict__ part
     const size_t per = (n + PARTS - 1) / PARTS;
     const size_t lo = (size_t)blockIdx.x * per;
     const size_t hi = lo + per < n ? lo + per : n;
-    // a slice is at most 2^31 / 256 values: the buffer ends with it, and +0 past the end changes no sum
+    // the buffer ends with the slice, and +0 past the end changes no sum (its 32-bit sizes hold for slices
+    // below 2^30 values, which is 1 TB of weights, more than the device holds)
     const uint32_t count = lo < hi ? (uint32_t)(hi - lo) : 0u;
     const __amdgpu_buffer_rsrc_t slice = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float *>(from) + lo, 0, (int)(count * 4u), 0x00020000);
