@@ -561,6 +561,19 @@ def test_k_sums_by_kernel_width(oracle, monkeypatch, blocks, kw):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4])
+@pytest.mark.parametrize("ic", [20, 64, 70, 128, 192, 700])
+def test_short_and_long_walks(oracle, monkeypatch, ic, blocks):
+    """Walks of one to fifteen groups of weight fragments, with and without paired taps: fewer than
+    are under way at once, and every remainder of what the loop takes together."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_PS", str(blocks))
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", "0")
+    for kh, kw in [(1, 1), (1, 2), (1, 3), (2, 2), (1, 5), (2, 3), (1, 7), (2, 4), (3, 3), (2, 5),
+                   (1, 11), (3, 4), (1, 13), (2, 7), (3, 5)]:
+        d, x, w = problem((2, ic, 70, 5, 14, kh, kw, 1, 1, kh // 2, kh // 2), zeros=True)
+        run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("t,joined", [
     ((26, 384, 40, 13, 13, 3, 3, 1, 1, 1, 1), True),
     ((26, 70, 8, 13, 13, 15, 15, 4, 4, 7, 7), True),      # long filters, few tiles

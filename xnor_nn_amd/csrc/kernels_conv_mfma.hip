@@ -256,6 +256,16 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     constexpr int HS = PAIR ? KS : (KS > 8 || (KS == 8 && PS == 4)) ? KS / 4
         : (KS % 2 == 0 && KS >= 4 && (PS > 3 || 40 * PS + 16 * KS > 216)) ? KS / 2 : KS;
     constexpr int GROUPS_PER_TAP = KS / HS; // 1, 2 or 4
+    // Where a group is a few matrix instructions, a good deal less than the way to the L2 and back, one
+    // group ahead is not enough: SETS groups are then under way, as many as the registers of
+    // resident_workgroups() allow, and a group is asked for where the one just multiplied lay.  Kernel
+    // alone, us: 48 to 96 channels 11x11 on 100x100 83.3 -> 58.8, 36 to 40 on 83x83
+    // 31.5 -> 20.0, 32 to 64 channels 5x5 on 32x32 10.6 -> 9.8 (a pass 14.3 -> 13.2), 64 channels on 56x56, minibatch 16, 6.7 ->
+    // 6.1, 192 on 14x14 6.0 -> 5.5, 525 to 21 on 49x49 16.6 -> 14.9; on 21 layers of up to 64 channels
+    // 9 % on average, none more than 1 % slower.  With longer groups it is as fast or slower: 384
+    // channels on 13x13, minibatch 256, 23.2 -> 23.7, 256 on 56x56 63 -> 65.
+    constexpr bool RING = HS == 1 || (PS == 1 && HS <= 3);
+    constexpr int SETS = HS == 1 ? (PS == 1 ? 6 : PS == 2 ? 3 : PS == 3 ? 2 : 4) : RING && HS == 2 ? 4 : 2;
 
     int thread = threadIdx.x;
     // PERSIST: a value the compiler cannot see through, so that nothing computed from it
@@ -506,14 +516,18 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     // this group's and of the next group's first step.  In the loops the group after the
     // last one is the last one again: loaded, awaited after the loops and never multiplied.
     // MORE = false (the single group after the paired loop) asks for nothing.
-    auto run_group = [&](auto more, auto newtap, auto p0, auto off, auto noff, int n,
-                         const v4i (&wc)[HS][2], v4i (&wn)[HS][2]) {
+    // RING: wc is wn, and the group asked for, behind the matrix instructions, is SETS groups on.  The
+    // walk goes by UNROLL groups, in which all register sets and all groups of a tap come round; TAIL >= 0:
+    // the TAIL-th of the fewer ones behind, which ask for nothing that would not exist.
+    constexpr int UNROLL = GROUPS_PER_TAP * (SETS * HS % 2 == 0 || GROUPS_PER_TAP % 2 == 0 ? SETS : 2 * SETS);
+    auto run_group = [&](auto more, auto newtap, auto p0, auto off, auto noff, auto tail, int n,
+                         v4i (&wc)[HS][2], v4i (&wn)[HS][2]) {
         constexpr bool MORE = decltype(more)::value, NEWTAP = decltype(newtap)::value;
         constexpr int P0 = decltype(p0)::value, OFF = decltype(off)::value,
-                      NOFF = decltype(noff)::value;
+                      NOFF = decltype(noff)::value, TAIL = decltype(tail)::value;
         uint32_t nextaddr[PS];
         uint32_t nextpair[PAIR ? 2 : 1][PAIR ? PS : 1];
-        const int next_group = min(n + 1, last_group);
+        const int next_group = min(n + (RING ? SETS : 1), last_group);
         if constexpr (MORE) {
             if constexpr (PAIR) {
                 pair_rows(nextpair);
@@ -527,10 +541,14 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
         // Step hs first asks for the two fragments of step hs of the next group, then waits
         // until its own two have arrived: they were asked for one group ago, and the 2*HS
         // loads started since (vector memory returns in order) may still be under way.
-        constexpr int VM = MORE ? 2 * HS : 0;
+        // RING: of the groups younger than this one, as many as there are sets, or the tail has.
+        constexpr int YOUNGER = TAIL < 0 || UNROLL - 2 - TAIL > SETS - 1 ? SETS - 1 : UNROLL - 2 - TAIL;
+        constexpr bool ASKS = RING && (TAIL < 0 || TAIL + SETS <= UNROLL - 2);
         static_for<HS>([&](auto step) {
             constexpr int hs = decltype(step)::value;
-            if constexpr (MORE) request_step(next_group, step, wn);
+            constexpr int VM = ASKS ? 2 * (HS * SETS - 1) : RING ? 2 * (HS * YOUNGER + HS - 1 - hs)
+                : MORE ? 2 * HS : 0;
+            if constexpr (MORE && !RING) request_step(next_group, step, wn);
             if constexpr (hs + 1 < HS || MORE) {
                 constexpr bool SAME = hs + 1 < HS; // the next step belongs to this group
                 constexpr int nhs = SAME ? hs + 1 : 0;
@@ -549,6 +567,7 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
             }
             if constexpr (((P0 + hs) & 1) == 0) mma(wc[hs], b0);
             else mma(wc[hs], b1);
+            if constexpr (ASKS) request_step(next_group, step, wn);
         });
         if constexpr (MORE) {
             if constexpr (PAIR) {
@@ -564,7 +583,8 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
         }
     };
 
-    v4i wa[HS][2], wb[HS][2];
+    v4i w[SETS][HS][2];
+    auto &wa = w[0], &wb = w[1];
     // A wave without filters (fewer than 256 of them in this chunk) leaves here, through a
     // barrier of its own: the barrier counts arrivals, whichever instruction they come from.
     // One test of the condition, ahead of the first hand-issued load, so that no path (of the
@@ -578,7 +598,10 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
         if constexpr (PERSIST) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         return;
     }
-    static_for<HS>([&](auto step) { request_step(0, step, wa); });
+    static_for<RING ? SETS : 1>([&](auto set) {
+        constexpr int i = decltype(set)::value;
+        static_for<HS>([&](auto step) { request_step(min(i, last_group), step, w[i]); });
+    });
     if constexpr (PAIR) {
         pair_rows(pairaddr);
     } else {
@@ -598,53 +621,82 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
         }
     }
     {
+        constexpr int FIRST_WAIT = RING ? 63 : 0;
         if constexpr (PAIR) {
             uint32_t a0[PS];
             pair_addr(std::integral_constant<int, 0>{}, pairaddr, a0);
-            fetch_rows_after<PS, 0, pair_offset(0)>(b0, a0, acc);
+            fetch_rows_after<PS, FIRST_WAIT, pair_offset(0)>(b0, a0, acc);
         } else {
-            fetch_rows_after<PS, 0, 0>(b0, rowaddr, acc);
+            fetch_rows_after<PS, FIRST_WAIT, 0>(b0, rowaddr, acc);
         }
-        wait_all_after<PS>(acc);
+        if constexpr (!RING) wait_all_after<PS>(acc); // (RING: the first step waits for its own)
         constexpr int P1 = HS & 1, OFF1 = GROUPS_PER_TAP == 2 ? HS * 32 : 0;
         using std::integral_constant;
         int n = 0;
-        if constexpr (GROUPS_PER_TAP == 4) { // the four quarters of a tap, wa and wb in turn
+        if constexpr (GROUPS_PER_TAP == 4 && !RING) { // the four quarters of a tap, wa and wb in turn
             for (; n + 3 <= last_group; n += 4) {
                 run_group(std::true_type{}, std::false_type{}, integral_constant<int, 0>{},
-                        integral_constant<int, 0>{}, integral_constant<int, HS * 32>{}, n, wa, wb);
+                        integral_constant<int, 0>{}, integral_constant<int, HS * 32>{},
+                        integral_constant<int, -1>{}, n, wa, wb);
                 run_group(std::true_type{}, std::false_type{}, integral_constant<int, P1>{},
                         integral_constant<int, HS * 32>{}, integral_constant<int, 2 * HS * 32>{},
-                        n + 1, wb, wa);
+                        integral_constant<int, -1>{}, n + 1, wb, wa);
                 run_group(std::true_type{}, std::false_type{}, integral_constant<int, 0>{},
                         integral_constant<int, 2 * HS * 32>{},
-                        integral_constant<int, 3 * HS * 32>{}, n + 2, wa, wb);
+                        integral_constant<int, 3 * HS * 32>{}, integral_constant<int, -1>{},
+                        n + 2, wa, wb);
                 run_group(std::true_type{}, std::true_type{}, integral_constant<int, P1>{},
                         integral_constant<int, 3 * HS * 32>{}, integral_constant<int, 0>{},
-                        n + 3, wb, wa);
+                        integral_constant<int, -1>{}, n + 3, wb, wa);
             }
         }
-        for (; n + 1 <= last_group; n += 2) {
-            run_group(std::true_type{}, integral_constant<bool, GROUPS_PER_TAP == 1>{},
-                    integral_constant<int, 0>{}, integral_constant<int, 0>{},
-                    integral_constant<int, OFF1>{}, n, wa, wb);
-            run_group(std::true_type{}, std::true_type{}, integral_constant<int, P1>{},
-                    integral_constant<int, OFF1>{}, integral_constant<int, 0>{}, n + 1, wb, wa);
+        if constexpr (RING) {
+            auto nth_group = [&](auto nth, auto tail) {
+                constexpr int I = decltype(nth)::value, G = GROUPS_PER_TAP, AT = I % G;
+                run_group(std::true_type{}, integral_constant<bool, AT == G - 1>{},
+                        integral_constant<int, (I * HS) & 1>{}, integral_constant<int, AT * HS * 32>{},
+                        integral_constant<int, (AT + 1) % G * HS * 32>{},
+                        integral_constant<int, decltype(tail)::value ? I : -1>{}, n + I, w[I % SETS],
+                        w[I % SETS]);
+            };
+            for (; n + UNROLL - 1 <= last_group; n += UNROLL)
+                static_for<UNROLL>([&](auto nth) { nth_group(nth, std::false_type{}); });
+            // one inside the other: no path (of those that the walk over the machine code knows) leaves one
+            // out and takes the next
+            auto tail_from = [&](auto self, auto nth) {
+                constexpr int I = decltype(nth)::value;
+                if constexpr (I < UNROLL - 1)
+                    if (n + I <= last_group) { // uniform
+                        nth_group(nth, std::true_type{});
+                        self(self, integral_constant<int, I + 1>{});
+                    }
+            };
+            tail_from(tail_from, integral_constant<int, 0>{});
+        } else {
+            for (; n + 1 <= last_group; n += 2) {
+                run_group(std::true_type{}, integral_constant<bool, GROUPS_PER_TAP == 1>{},
+                        integral_constant<int, 0>{}, integral_constant<int, 0>{},
+                        integral_constant<int, OFF1>{}, integral_constant<int, -1>{}, n, wa, wb);
+                run_group(std::true_type{}, std::true_type{}, integral_constant<int, P1>{},
+                        integral_constant<int, OFF1>{}, integral_constant<int, 0>{},
+                        integral_constant<int, -1>{}, n + 1, wb, wa);
+            }
+            if (n <= last_group) // odd number of groups (only with one group per tap)
+                run_group(std::false_type{}, std::false_type{}, integral_constant<int, 0>{},
+                        integral_constant<int, 0>{}, integral_constant<int, 0>{},
+                        integral_constant<int, -1>{}, n, wa, wb);
         }
-        if (n <= last_group) // odd number of groups (only with one group per tap)
-            run_group(std::false_type{}, std::false_type{}, integral_constant<int, 0>{},
-                    integral_constant<int, 0>{}, integral_constant<int, 0>{}, n, wa, wb);
         // The last group of the loops has asked for fragments that nothing multiplies.  They
-        // are awaited here, and both register sets are named as inputs after the wait: a
+        // are awaited here, and all register sets are named as inputs after the wait: a
         // register that is dead after the loop would otherwise be handed to the epilogue's
         // address arithmetic while its load is still on the way.
         // The same holds for the pixel fragments: the last step has started LDS reads for a
         // step that does not exist.
         wait_all_after<PS>(acc);
-        static_for<HS>([&](auto step) {
-            constexpr int hs = decltype(step)::value;
-            const v4i a0 = wa[hs][0], a1 = wa[hs][1], c0 = wb[hs][0], c1 = wb[hs][1];
-            asm volatile("" : : "v"(a0), "v"(a1), "v"(c0), "v"(c1));
+        static_for<SETS * HS>([&](auto step) {
+            constexpr int set = decltype(step)::value / HS, hs = decltype(step)::value % HS;
+            const v4i a0 = w[set][hs][0], a1 = w[set][hs][1];
+            asm volatile("" : : "v"(a0), "v"(a1));
         });
         static_for<PS>([&](auto block) {
             constexpr int ps = decltype(block)::value;
