@@ -574,6 +574,28 @@ def test_short_and_long_walks(oracle, monkeypatch, ic, blocks):
         run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("t", [
+    (1, 70, 33, 3, 200, 3, 3, 1, 1, 1, 1),      # rows longer than a tile, taps above and below
+    (2, 20, 40, 9, 61, 1, 1, 2, 2, 0, 0),       # one tap, rows and pixels that nothing reads
+    (2, 64, 40, 9, 61, 2, 2, 3, 3, 0, 0),       # gaps between the taps
+    (3, 40, 40, 5, 37, 3, 5, 1, 2, 2, 4),       # taps left and right of the image
+    (2, 96, 300, 1, 90, 1, 7, 1, 1, 3, 3),      # one row; most kernel rows outside
+    (1, 130, 30, 12, 150, 5, 5, 2, 1, 2, 2),
+    (1, 1100, 40, 4, 70, 3, 3, 1, 1, 1, 1),     # channel parts
+    (1, 864, 40, 5, 83, 3, 3, 1, 1, 1, 1),      # more than the LDS if whole rows were staged
+], ids=str)
+@pytest.mark.parametrize("small", ["0", "1"])
+def test_tiles_that_begin_inside_a_row(oracle, monkeypatch, t, small):
+    """The input of a tile runs from its first pixel's first tap to its last pixel's last one."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", small)
+    d, x, w = problem(t, zeros=True)
+    assert make(d, w).kernel_name(0).startswith("conv_mfma_fp4")
+    for blocks in ("1", "2", "3"):
+        if small == "0":
+            monkeypatch.setenv("XNOR_NN_HIP_MFMA_PS", blocks)
+        run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("t,joined", [
     ((26, 384, 40, 13, 13, 3, 3, 1, 1, 1, 1), True),
     ((26, 70, 8, 13, 13, 15, 15, 4, 4, 7, 7), True),      # long filters, few tiles

@@ -90,7 +90,7 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     // buffer ends with the tile's run: with a branch around each load the compiler would wait for one
     // after the other)
     int lo, hi;
-    tile_span(g, p_first, min(p_first + 32u, p_limit), lo, hi);
+    row_span(g, p_first, min(p_first + 32u, p_limit), lo, hi);
     const int nrows = min(hi - lo + 1, s.max_rows), nitems = nrows * g.xw;
     const bool fuse_k = FUSED || a_plane != nullptr; // uniform
     const uint32_t *run = xbits + (size_t)lo * g.xw;
@@ -155,7 +155,7 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
         if (writes) {
             int nlo, nhi;
             w_from = block == 0 ? 0 : lo;
-            if (block + 1 < s.blocks) tile_span(g, p_first + 32u, min(p_first + 64u, p_limit), nlo, nhi);
+            if (block + 1 < s.blocks) row_span(g, p_first + 32u, min(p_first + 64u, p_limit), nlo, nhi);
             else nlo = (int)g.npix_in;
             w_to = nlo;
             from = min(from, w_from);
@@ -372,7 +372,7 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     const uint32_t look = blocks < (uint32_t)g.ohw + 1 ? blocks : (uint32_t)g.ohw + 1;
     auto see = [&](uint32_t b) {
         int lo, hi;
-        tile_span(g, b * 32u, b * 32u + 32u < g.npix_out ? b * 32u + 32u : g.npix_out, lo, hi);
+        row_span(g, b * 32u, b * 32u + 32u < g.npix_out ? b * 32u + 32u : g.npix_out, lo, hi);
         if (hi - lo + 1 > most) most = hi - lo + 1;
     };
     for (uint32_t b = 0; b < look; b++) see(b);
