@@ -445,6 +445,25 @@ def test_few_input_pixels(oracle, monkeypatch, t, separate_k):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("separate_k", [False, True])
+@pytest.mark.parametrize("t", [
+    (1, 2048, 8, 7, 7, 1, 1, 1, 1, 0, 0),      # both places of every loader once
+    (3, 2049, 8, 5, 5, 1, 1, 1, 1, 0, 0),      # a third chunk, of one channel
+    (5, 4095, 8, 9, 7, 1, 1, 1, 1, 0, 0),      # four, all places twice
+    (2, 8160, 8, 3, 11, 1, 1, 1, 1, 0, 0),     # eight: as deep as tiles go
+    (17, 511, 8, 16, 16, 1, 1, 1, 1, 0, 0),    # 68 tiles of 64 pixels, a channel short
+    (17, 512, 8, 16, 16, 1, 1, 1, 1, 0, 0),    # ... and deep enough for tiles of 16
+    (32, 1025, 8, 16, 16, 1, 1, 1, 1, 0, 0),   # 128 tiles: the last that are few
+    (33, 1025, 8, 16, 16, 1, 1, 1, 1, 0, 0),   # 132: too many
+], ids=str)
+def test_deep_input_of_few_pixels(oracle, monkeypatch, t, separate_k):
+    """Parts of chunks are handed to the adding wave and their places given back one by one."""
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
 @pytest.mark.parametrize("t", [
     (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0),         # one value

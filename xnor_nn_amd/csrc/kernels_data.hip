@@ -231,11 +231,16 @@ void binarize_nhwc_tiled_kernel(const float *__restrict__ x, uint32_t *__restric
 // The tiled kernel above walks the running sum from wave to wave, with a barrier at every
 // hand-over, and gives a tile's whole transfer to one compute unit: 2048 channels on 7x7,
 // minibatch 64, were 49 workgroups of 11 waves that took six rounds, 23.6 us.  Here a wave loads
-// four words (128 channels) of 16 pixels at a time, lane = (pixel, word); the loaders pack the
-// sign words and leave the magnitudes in LDS, channel by channel along a pixel's row, and the
+// four words (128 channels) of 16 pixels at a time, lane = (pixel, word); the loaders pack and store
+// the sign words and leave the magnitudes in LDS, channel by channel along a pixel's row, and the
 // last wave of the workgroup adds them, reading 32 values ahead, while the loaders fetch the next
 // chunk.  What bounds it is that chain: one addition per eight cycles and channel, 7 us for 2048
-// channels; 16.4 us in all there.
+// channels.  It must not stand still: no barrier, every loader says by itself that its part of a
+// chunk lies there, and the adding wave takes as many parts in a row as it finds (a part at a time,
+// with the first read of each exposed: 13.9 and 10.6 us below), and frees their places one by one.
+// us for 2048 channels on 7x7, minibatch 64 / 1, and 3000 channels, minibatch 8, with a barrier per
+// chunk of all loaders: 16.3 / 11.6 and 17.5, now 13.4 / 10.0 and 15.0.  Both of the first two
+// chunks asked for at once make the first one come later: 17.0 / 12.3 and 18.7.
 struct SplitPlan {
     uint32_t npix, ihw, ntiles, tiles_per_xcd;
     int ic, xw, loaders, chunks;
@@ -253,8 +258,10 @@ void binarize_nchw_split_kernel(const float *__restrict__ x, uint32_t *__restric
     // a pixel's row in floats: 4 mod 64, so that the 16-byte accesses of both sides spread over
     // the banks
     const int chunk_words = s.loaders * G, row = chunk_words * 32 + 4;
-    // [one or two buffers][T pixels][row], then the packed words [T][xw]
-    uint32_t *stage = reinterpret_cast<uint32_t *>(split_lds + (s.chunks > 1 ? 2 : 1) * T * row);
+    // [one or two buffers][T pixels][row], then the loaders' chunks that lie there, then the number of
+    // loaders' chunks that have been added
+    uint32_t *there = reinterpret_cast<uint32_t *>(split_lds + (s.chunks > 1 ? 2 : 1) * T * row);
+    uint32_t *added = there + SPLIT_LOADERS;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile = (blockIdx.x & 7) * s.tiles_per_xcd + (blockIdx.x >> 3);
     fetch_together(x, a, bits, s.npix, s.ihw, s.ic, s.xw, s.loaders, s.chunks, inv_ic);
@@ -262,7 +269,16 @@ void binarize_nchw_split_kernel(const float *__restrict__ x, uint32_t *__restric
     if (tile >= s.ntiles) return;
     const int lp = lane & (T - 1), lg = lane / T;
     const uint32_t p = tile * T + lp;
-    auto meet = [] { // LDS is in place; loads from memory stay under way
+    if (WRITE_A && wave == s.loaders && lane <= SPLIT_LOADERS) there[lane] = 0; // (`added` as well)
+    auto load_of = [](uint32_t *flag) {
+        return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    // (what this wave read or wrote in LDS before is done)
+    auto say = [](uint32_t *flag, uint32_t value) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    auto flags_are_clear = [] { // loads from memory stay under way
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -290,10 +306,10 @@ void binarize_nchw_split_kernel(const float *__restrict__ x, uint32_t *__restric
             }
         };
         load(0);
+        if (WRITE_A) flags_are_clear();
         for (int k = 0; k < s.chunks; k++) {
             const int j = (k * s.loaders + wave) * G + lg;
             uint32_t neg = 0; // sign bits, first channel ends up in the MSB
-            // (the sum of chunk k - 2, which used this buffer, ended ahead of the last barrier)
             v4f *to = reinterpret_cast<v4f *>(split_lds + ((k & 1) * T + lp) * row
                     + (wave * G + lg) * 32);
 #pragma unroll
@@ -302,52 +318,69 @@ void binarize_nchw_split_kernel(const float *__restrict__ x, uint32_t *__restric
                 t[i] = __fmul_rn(__builtin_fabsf(t[i]), inv_ic);
             }
             if (WRITE_A) {
+                // what chunk k - 2 left here has been added (chunks are added in order, a chunk loader by
+                // loader)
+                if (k >= 2) {
+                    while (load_of(added) < (uint32_t)((k - 2) * s.loaders + wave + 1))
+                        __builtin_amdgcn_s_sleep(1);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                }
 #pragma unroll
                 for (int i = 0; i < 8; i++)
                     to[i] = v4f{t[4 * i], t[4 * i + 1], t[4 * i + 2], t[4 * i + 3]};
+                say(there + wave, k + 1);
             }
-            if (WRITE_BITS && j < s.xw) stage[lp * s.xw + j] = (~neg) & top_bits(s.ic - 32 * j);
+            // (sixteen bytes of a pixel; they meet the next wave's in L2)
+            if (WRITE_BITS && j < s.xw && p < s.npix)
+                bits[(size_t)p * s.xw + j] = (~neg) & top_bits(s.ic - 32 * j);
             if (k + 1 < s.chunks) load(k + 1);
-            meet();
         }
-    } else {
-        // the chain is what the workgroup waits for: ahead of the loaders' packing on its SIMD (2048
-        // channels on 7x7, a pass at minibatch 1 / 64: 17.7 / 24.5 -> 17.0 / 23.7 us)
-        __builtin_amdgcn_s_setprio(3);
-        float sum = 0.f;
-        for (int k = 0; k < s.chunks; k++) {
-            meet();
-            if (!WRITE_A) continue;
-            const int words = min(chunk_words, s.xw - k * chunk_words); // uniform
-            const v4f *at = reinterpret_cast<const v4f *>(split_lds + ((k & 1) * T + lp) * row);
-            v4f u[8], v[8];
-            auto read = [&](v4f (&to)[8], int w) {
+        return;
+    }
+    if (!WRITE_A) return;
+    // the chain is what the workgroup waits for: ahead of the loaders' packing on its SIMD (2048
+    // channels on 7x7, a pass at minibatch 1 / 64: 17.7 / 24.5 -> 17.0 / 23.7 us)
+    flags_are_clear();
+    __builtin_amdgcn_s_setprio(3);
+    float sum = 0.f;
+    v4f u[8], v[8];
+    auto read = [&](v4f (&to)[8], int k, int word) {
+        const v4f *at = reinterpret_cast<const v4f *>(split_lds + ((k & 1) * T + lp) * row) + 8 * word;
 #pragma unroll
-                for (int i = 0; i < 8; i++) to[i] = at[8 * w + i];
-            };
-            auto add = [&](const v4f (&from)[8]) {
+        for (int i = 0; i < 8; i++) to[i] = at[i];
+    };
+    auto add = [&](const v4f (&from)[8]) {
 #pragma unroll
-                for (int i = 0; i < 8; i++)
+        for (int i = 0; i < 8; i++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) sum = __fadd_rn(sum, from[i][e]);
-            };
-            read(u, 0);
-            for (int w = 0; w < words; w += 2) {
-                if (w + 1 < words) read(v, w + 1);
+            for (int e = 0; e < 4; e++) sum = __fadd_rn(sum, from[i][e]);
+    };
+    for (int k = 0; k < s.chunks; k++) {
+        const int words = min(chunk_words, s.xw - k * chunk_words); // uniform
+        for (int w = 0; w < words;) {
+            // the loaders whose chunks lie there, in the order of their channels (a flag that no loader has
+            // stays 0)
+            const uint64_t lie_there = __ballot(load_of(there + (lane & (SPLIT_LOADERS - 1))) > (uint32_t)k);
+            const int ready = __builtin_ctz(~((uint32_t)lie_there & ((1u << SPLIT_LOADERS) - 1)));
+            const int end = min(words, ready * G);
+            if (w >= end) {
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            read(u, k, w);
+            for (; w < end; w += 2) {
+                if (w + 1 < end) read(v, k, w + 1);
                 add(u);
-                if (w + 1 < words) {
-                    if (w + 2 < words) read(u, w + 2);
+                if (w + 1 < end) {
+                    if (w + 2 < end) read(u, k, w + 2);
                     add(v);
                 }
             }
+            if (k + 2 < s.chunks) say(added, k * s.loaders + ready);
         }
-        if (WRITE_A && lane < T && p < s.npix) a[p] = sum;
     }
-    if (!WRITE_BITS) return;
-    meet();
-    const uint32_t first = tile * (uint32_t)(T * s.xw), total = s.npix * (uint32_t)s.xw;
-    for (uint32_t i = threadIdx.x; i < (uint32_t)(T * s.xw); i += blockDim.x)
-        if (first + i < total) bits[first + i] = stage[i];
+    if (lane < T && p < s.npix) a[p] = sum;
 }
 
 // NCHW input of at most 32 channels (one packed word per pixel): a lane takes all channels of U
@@ -594,7 +627,7 @@ size_t split_lds_bytes(const Plan &g, int *loaders, int *chunks) {
     *loaders = sets < SPLIT_LOADERS ? sets : SPLIT_LOADERS;
     *chunks = (sets + *loaders - 1) / *loaders;
     return sizeof(float) * ((*chunks > 1 ? 2 : 1) * SPLIT_TILE * (*loaders * SPLIT_WORDS * 32 + 4)
-            + SPLIT_TILE * (size_t)g.xw);
+            + SPLIT_LOADERS + 1);
 }
 
 template <bool WRITE_BITS, bool WRITE_A>
@@ -670,15 +703,24 @@ static bool shallow_nchw(const Plan &g) {
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < (1ull << 31);
 }
 
-// Up to one tile of 64 pixels for every four compute units: AlexNet conv4 (384 channels) at
-// minibatch 1 / 8 / 32 (3 / 22 / 85 tiles) 4.2 / 4.5 / 5.9 us against 4.6 / 4.7 / 5.3 for the tiled
-// kernel, 1024 channels on 14x14 at minibatch 8 / 32 (25 / 98 tiles) 7.8 / 14.1 against 11.2 / 11.6,
-// 2048 channels on 7x7 at minibatch 1 / 64 (1 / 49 tiles) 10.4 / 16.4 against 18.0 / 23.0: with
-// more tiles the tiled kernel's whole cache lines count for more than the shorter walk.
+static uint32_t pixel_tiles(const Plan &g) { return (g.npix_in + TILE - 1) / TILE; }
+
+// Up to one tile of 64 pixels for every four compute units, one for every two from 512 channels on:
+// us here / by the tiled kernel
+//   384 channels   13x13, minibatch 1 / 8 / 24 (3 / 22 / 64 tiles): 4.1 / 4.3 / 4.7 and 4.6 / 4.7 / 5.0
+//                  9x9, 13x13, 14x14, 27x27, about 85 tiles: 5.4, 5.9, 5.1, 5.4 and 5.6, 5.6, 5.4, 5.5
+//   512 channels   the same: 7.2, 7.0, 6.2, 7.3 and 7.3, 7.3, 7.0, 7.0; 125 tiles 6.4 to 7.2 and 7.2 to 7.7
+//   1024 channels  the same: 10.6, 11.6, 10.4, 10.8 and 11.6, 11.7, 11.6, 11.7; 125 tiles 11.3 to 12.8 and
+//                  13.8 to 15.4
+//   2048 channels  7x7, minibatch 64 / 128 / 160 (49 / 98 / 123 tiles): 13.4 / 24.3 / 27.3 and
+//                  23.0 / 30.8 / 31.6
+//   4000 channels  14x14, 74 / 120 tiles: 38.7 / 43.6 and 55.1 / 57.3
+// With more tiles a compute unit gets a third one of 16 pixels and has LDS for one or two, and the tiled
+// kernel's whole cache lines count for more than the shorter walk: 200 tiles on 14x14, 512 / 1024 / 2048
+// channels 8.6 / 19.6 / 44.7 and 8.2 / 17.3 / 32.7.
 static bool split_nchw(const Plan &g) {
     int loaders, chunks;
-    const uint32_t tiles = (g.npix_in + TILE - 1) / TILE;
-    return tiled_nchw(g) && tiles <= (uint32_t)g.cus / 4
+    return tiled_nchw(g) && pixel_tiles(g) <= (uint32_t)g.cus / (g.ic < 512 ? 4 : 2)
         && split_lds_bytes(g, &loaders, &chunks) <= 160 * 1024;
 }
 
@@ -783,8 +825,11 @@ JoinedGrid joined_grid(const Plan &g, bool fragments) {
 // Nowhere else was joining slower, on 60 layers: 384 channels 3x3 on 13x13, minibatch 64, 20.9 / 26.6, 256
 // channels 7x7 on 14x14, minibatch 128, 54.8 / 58.8, 64 channels 3x3 on 224x224, minibatch 64 (50176
 // tiles, as many workgroups as the waves allow), 273 / 280.
+// Input of at most one tile for every four compute units is left to its own kernel.
 bool weights_join_binarize(const Plan &g) {
-    if (!tiled_nchw(g) || shallow_nchw(g) || split_nchw(g) || !filter_kernel_applies(g)) return false;
+    if (!tiled_nchw(g) || shallow_nchw(g) || pixel_tiles(g) <= (uint32_t)g.cus / 4
+            || !filter_kernel_applies(g))
+        return false;
     const JoinedGrid j = joined_grid(g, g.use_mfma != 0);
     const int by_waves = 32 / j.waves, by_lds = (int)(160 * 1024 / (j.lds + sizeof(Runs)));
     return by_lds >= by_waves
