@@ -464,6 +464,40 @@ def test_deep_input_of_few_pixels(oracle, monkeypatch, t, separate_k):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("separate_k", [False, True])
+@pytest.mark.parametrize("t,name", [
+    ((1, 32, 8, 9, 8, 1, 1, 1, 1, 0, 0), "tiled_kernel"),            # whole pieces, one slice
+    ((2, 6, 8, 9, 8, 3, 3, 1, 1, 1, 1), "generic_kernel"),
+    ((2, 7, 8, 9, 8, 3, 3, 1, 1, 1, 1), "tiled_kernel<RAGGED>"),     # one ragged slice
+    ((1, 31, 8, 13, 5, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"),   # 65 pixels
+    ((1, 31, 8, 8, 8, 1, 1, 1, 1, 0, 0), "generic_kernel"),          # 64
+    ((1, 33, 8, 1, 1, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"),    # one pixel
+    ((3, 130, 8, 9, 7, 3, 3, 1, 1, 1, 1), "tiled_kernel<RAGGED>"),   # tiles across images
+    ((2, 383, 8, 8, 16, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"),  # twelve waves, whole tiles
+    ((1, 385, 8, 9, 9, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"),   # two rounds of seven
+    ((1, 1502, 8, 6, 11, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"), # above 64 KB of LDS
+    ((1, 13535, 1, 9, 8, 1, 1, 1, 1, 0, 0), "tiled_kernel<RAGGED>"), # as deep as LDS goes
+    ((1, 13537, 1, 9, 8, 1, 1, 1, 1, 0, 0), "generic_kernel"),
+    ((1, 2048, 8, 8, 8, 1, 1, 1, 1, 0, 0), "binarize_nhwc_kernel"),  # 64 pixels
+    ((1, 2048, 8, 13, 5, 1, 1, 1, 1, 0, 0), "tiled_kernel"),         # 65
+    ((1, 13536, 1, 9, 8, 1, 1, 1, 1, 0, 0), "tiled_kernel"),
+    ((1, 13540, 1, 9, 8, 1, 1, 1, 1, 0, 0), "binarize_nhwc_kernel"),
+], ids=str)
+def test_channels_last_of_any_count(oracle, gpu, monkeypatch, t, name, separate_k):
+    """Pixels that begin anywhere in a line, and the rule that chooses their kernel on either side of
+    each line."""
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    x, w = in_layout(x, w, NHWC)
+    conv = make(d, w, NHWC)
+    try:
+        assert conv.kernel_name(2).endswith(name)
+    finally:
+        conv.close()
+    run_and_compare(oracle, d, x, w, NHWC, True, gpu)
+
+
 @pytest.mark.parametrize("fmts,separate_k", [(NCHW, False), (NCHW, True), (NHWC, False)])
 @pytest.mark.parametrize("t", [
     (1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0),         # one value

@@ -45,12 +45,17 @@ __device__ __forceinline__ uint32_t fbits(float v) { return __float_as_uint(v); 
 // neighbouring tiles (a channel plane is rarely a multiple of 128 bytes) are fetched into
 // one L2 instead of two.  Workgroup b takes local tile b / 8 of XCD b % 8.
 //
-// NHWC input (channel count a multiple of 4) runs the same tile: the 32 values of a slice are
-// then 128 contiguous bytes of a pixel.  A wave fetches them eight lanes to a pixel, so that
+// NHWC input runs the same tile: the 32 values of a slice are then 128 contiguous bytes of a
+// pixel.  A wave fetches them eight lanes to a pixel, so that
 // every load instruction reads eight whole cache lines, and turns the block around through
 // LDS into the lane = pixel layout (one lane per pixel straight from memory, 64 partial
 // cache lines per instruction, took 19.7 us where this takes 13.5 us, the NCHW kernel 13.3).
-template <bool NHWC, bool STREAM, bool WRITE_BITS, bool WRITE_A>
+// RAGGED: a channel count that is no multiple of 4.  Its whole slices are read the same way, from
+// wherever a pixel begins; in the last one a lane is a channel, since 16 bytes would run into
+// the next pixel (111 channels on 40x40, minibatch 60: 89.8 -> 10.7 us, 4.0 TB/s).  An instantiation of
+// its own, since that slice takes 36 registers more (128 channels on 32x32, minibatch 100: 10.5 -> 11.7),
+// and without the "nt" bit: neighbouring pixels share lines (130 on 40x40, minibatch 60: 18.1, 19.4 with).
+template <bool NHWC, bool STREAM, bool RAGGED, bool WRITE_BITS, bool WRITE_A>
 __device__ __forceinline__
 void binarize_tile(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry &g, const float inv_ic, const int rounds,
@@ -88,8 +93,44 @@ void binarize_tile(const float *__restrict__ x, uint32_t *__restrict__ bits,
             // (32 pixels at a time, rows of 144 bytes so that neither side has bank
             // conflicts) to end up with the lane = pixel layout of the rest of the kernel.
             typedef float v4f __attribute__((ext_vector_type(4)));
+            float *mine = turn + wave * (32 * TURN_ROW);
+            // rows of 32 pixels to lane = pixel
+            auto turn_around = [&](int half) {
+                if ((lane >> 5) != half) return;
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const v4f r = *reinterpret_cast<const v4f *>(
+                            mine + (lane & 31) * TURN_ROW + 4 * u);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t[4 * u + e] = r[e];
+                }
+            };
+            if (RAGGED && c0 + 32 > g.ic) { // uniform
+                // The last slice of a channel count that is no multiple of 4: a channel to a lane, two
+                // pixels per load.
+                const int c = c0 + (lane & 31);
+                // (a pixel past the last one lies outside the buffer, or where nothing is written from)
+                const uint32_t off = ((tile * TILE + (lane >> 5)) * (uint32_t)g.ic + (uint32_t)c) * 4u;
+                float v[32];
+#pragma unroll
+                for (int i = 0; i < 32; i++) v[i] = 0.f;
+                if (c < g.ic) {
+#pragma unroll
+                    for (int i = 0; i < 32; i++)
+                        v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                src, off + (uint32_t)i * (8u * (uint32_t)g.ic), 0, 0));
+                }
+#pragma unroll
+                for (int half = 0; half < 2; half++) {
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        mine[(2 * i + (lane >> 5)) * TURN_ROW + (lane & 31)] = v[16 * half + i];
+                    turn_around(half);
+                }
+                return;
+            }
             const int piece = lane & 7;
-            const int c = c0 + 4 * piece; // IC is a multiple of 4: a piece is inside or outside
+            const int c = c0 + 4 * piece; // a piece is inside or outside
             v4f v[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -101,22 +142,13 @@ void binarize_tile(const float *__restrict__ x, uint32_t *__restrict__ bits,
                 v[i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
                         src, off, 0, STREAM ? LOAD_STREAMING : 0));
             }
-            float *mine = turn + wave * (32 * TURN_ROW);
 #pragma unroll
             for (int half = 0; half < 2; half++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
                     *reinterpret_cast<v4f *>(mine + (8 * i + (lane >> 3)) * TURN_ROW + 4 * piece)
                         = v[4 * half + i];
-                if ((lane >> 5) == half) {
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const v4f r = *reinterpret_cast<const v4f *>(
-                                mine + (lane & 31) * TURN_ROW + 4 * u);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) t[4 * u + e] = r[e];
-                    }
-                }
+                turn_around(half);
             }
             return;
         }
@@ -189,7 +221,7 @@ __global__ __launch_bounds__(TILE * 16)
 void binarize_nchw_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry g, const float inv_ic, const int rounds,
         const uint32_t ntiles, const uint32_t tiles_per_xcd) {
-    binarize_tile<false, false, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
+    binarize_tile<false, false, false, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
             tiles_per_xcd, blockIdx.x);
 }
 
@@ -208,7 +240,7 @@ void binarize_nchw_and_weights_kernel(const float *__restrict__ x, uint32_t *__r
     extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ Runs runs;
     if (blockIdx.x >= weight_blocks) {
-        binarize_tile<false, false, true, true>(x, bits, a, g, inv_ic, rounds, ntiles, tiles_per_xcd,
+        binarize_tile<false, false, false, true, true>(x, bits, a, g, inv_ic, rounds, ntiles, tiles_per_xcd,
                 blockIdx.x - weight_blocks);
         return;
     }
@@ -217,12 +249,12 @@ void binarize_nchw_and_weights_kernel(const float *__restrict__ x, uint32_t *__r
     filter_stage(w, wbits, frag, alpha, opc, g, f, row, runs, blockIdx.x);
 }
 
-template <bool STREAM, bool WRITE_BITS, bool WRITE_A>
+template <bool STREAM, bool RAGGED, bool WRITE_BITS, bool WRITE_A>
 __global__ __launch_bounds__(TILE * 16)
 void binarize_nhwc_tiled_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
         float *__restrict__ a, const Geometry g, const float inv_ic, const int rounds,
         const uint32_t ntiles, const uint32_t tiles_per_xcd) {
-    binarize_tile<true, STREAM, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
+    binarize_tile<true, STREAM, RAGGED, WRITE_BITS, WRITE_A>(x, bits, a, g, inv_ic, rounds, ntiles,
             tiles_per_xcd, blockIdx.x);
 }
 
@@ -434,8 +466,7 @@ void binarize_nchw_shallow_kernel(const float *__restrict__ x, uint32_t *__restr
     }
 }
 
-// Any source layout, one lane per pixel, channels visited in order.  Used for NHWC input
-// (reference src/bcast_binarize_data.cpp:56-57, src/bcast_calculate_k.cpp:59-60).
+// Any source layout, one lane per pixel, channels visited in order (reference src/bcast_binarize_data.cpp:56-57, src/bcast_calculate_k.cpp:59-60).
 template <bool WRITE_BITS, bool WRITE_A>
 __global__ __launch_bounds__(256)
 void binarize_generic_kernel(const float *__restrict__ x, uint32_t *__restrict__ bits,
@@ -467,9 +498,8 @@ void binarize_generic_kernel(const float *__restrict__ x, uint32_t *__restrict__
     if (WRITE_A) a[p] = acc;
 }
 
-// NHWC input with IC a multiple of 4 and too many channels for the tiled kernel's LDS: a lane
-// is a pixel and walks over its channels, which
-// are contiguous, in order, 32 at a time (one packed word): eight 16-byte buffer loads per
+// NHWC input with IC a multiple of 4 that the tiled kernel does not take (nhwc_tiled): a lane
+// is a pixel and walks over its channels, which are contiguous, in order, 32 at a time (one packed word): eight 16-byte buffer loads per
 // word, the loads of the next three words in flight while the current one is folded into
 // the sign word and the running mean|x| (reference src/bcast_binarize_data.cpp:56-57,
 // src/bcast_calculate_k.cpp:59-60).  The lanes of a wave read addresses IC*4 bytes apart,
@@ -599,27 +629,46 @@ bool nhwc_streams(const Plan &g) {
     return bytes > (32u << 20) && bytes <= (104u << 20);
 }
 
-template <bool NHWC, bool WRITE_BITS, bool WRITE_A>
+// At most twelve waves per workgroup, the slices split evenly over the rounds: with more
+// waves the hand-over chain of one workgroup gets long and too few workgroups are
+// resident to cover it (512 input channels: 14.1 us with 16 waves, 10.4 us with 2 x 8;
+// 384 channels: 12 x 1 and 6 x 2 are equal at MB 256, 12 x 1 is 5% faster at MB 1024).
+template <bool WRITE_BITS, bool WRITE_A>
 void launch_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
         const KernelEvents &ev) {
-    // At most twelve waves per workgroup, the slices split evenly over the rounds: with more
-    // waves the hand-over chain of one workgroup gets long and too few workgroups are
-    // resident to cover it (512 input channels: 14.1 us with 16 waves, 10.4 us with 2 x 8;
-    // 384 channels: 12 x 1 and 6 x 2 are equal at MB 256, 12 x 1 is 5% faster at MB 1024).
     int rounds;
     const int nw = tiled_waves(g, &rounds);
     const uint32_t ntiles = (g.npix_in + TILE - 1) / TILE;
     const uint32_t per_xcd = (ntiles + 7) / 8;
-    size_t lds = sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw);
-    if (NHWC) lds = ((lds + 15) & ~(size_t)15) + sizeof(float) * nw * 32 * TURN_ROW;
-    if (NHWC)
-        launch_kernel(nhwc_streams(g) ? binarize_nhwc_tiled_kernel<true, WRITE_BITS, WRITE_A>
-                                      : binarize_nhwc_tiled_kernel<false, WRITE_BITS, WRITE_A>,
-                dim3(per_xcd * 8), dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic,
-                rounds, ntiles, per_xcd);
-    else
-        launch_kernel(binarize_nchw_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
-                dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
+    launch_kernel(binarize_nchw_kernel<WRITE_BITS, WRITE_A>, dim3(per_xcd * 8),
+            dim3(nw * TILE), sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw), s, ev, x, bits, a,
+            geometry(g), 1.f / g.ic, rounds, ntiles, per_xcd);
+}
+
+// LDS of the tiled NHWC kernel: chain, packed words, turn-around rows.
+size_t nhwc_tiled_lds_bytes(const Plan &g, int waves) {
+    const size_t words = sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw);
+    return ((words + 15) & ~(size_t)15) + sizeof(float) * waves * 32 * TURN_ROW;
+}
+
+template <bool WRITE_BITS, bool WRITE_A>
+hipError_t launch_nhwc_tiled(const Plan &g, const float *x, uint32_t *bits, float *a, hipStream_t s,
+        const KernelEvents &ev) {
+    int rounds;
+    const int nw = tiled_waves(g, &rounds);
+    const uint32_t ntiles = (g.npix_in + TILE - 1) / TILE;
+    const uint32_t per_xcd = (ntiles + 7) / 8;
+    const size_t lds = nhwc_tiled_lds_bytes(g, nw);
+    const bool ragged = (g.ic & 3) != 0, streams = nhwc_streams(g);
+    const auto kernel = ragged ? binarize_nhwc_tiled_kernel<false, true, WRITE_BITS, WRITE_A>
+        : streams ? binarize_nhwc_tiled_kernel<true, false, WRITE_BITS, WRITE_A>
+                          : binarize_nhwc_tiled_kernel<false, false, WRITE_BITS, WRITE_A>;
+    static LdsGrant grants[3];
+    const hipError_t e = grants[ragged ? 2 : streams ? 1 : 0].ask((const void *)kernel, lds);
+    if (e != hipSuccess) return e;
+    launch_kernel(kernel, dim3(per_xcd * 8), dim3(nw * TILE), lds, s, ev, x, bits, a, geometry(g),
+            1.f / g.ic, rounds, ntiles, per_xcd);
+    return hipSuccess;
 }
 
 size_t split_lds_bytes(const Plan &g, int *loaders, int *chunks) {
@@ -674,16 +723,6 @@ void launch_shallow_any(const Plan &g, const float *x, uint32_t *bits, float *a,
     else launch_shallow<32, WRITE_BITS, WRITE_A>(g, x, bits, a, s, ev);
 }
 
-// NHWC input runs the tiled kernel unless its LDS (chain, packed words, turn-around rows) would
-// not fit 64 KB (more than about a thousand channels).
-bool nhwc_by_lane(const Plan &g) {
-    if (g.bin_nhwc_lane) return true;
-    const int rounds = (g.xw + MAX_WAVES - 1) / MAX_WAVES;
-    const int nw = (g.xw + rounds - 1) / rounds;
-    return sizeof(uint32_t) * (TILE + (size_t)TILE * g.xw) + 16
-        + sizeof(float) * nw * 32 * TURN_ROW > 64 * 1024;
-}
-
 } // namespace
 
 // The tiled kernel addresses the input with 32-bit byte offsets and stages the packed words
@@ -724,12 +763,36 @@ static bool split_nchw(const Plan &g) {
         && split_lds_bytes(g, &loaders, &chunks) <= 160 * 1024;
 }
 
-// The NHWC kernel reads 16 bytes per load at 32-bit byte offsets (and drops pieces past the
-// last channel the same way).
+// The NHWC kernels read at 32-bit byte offsets (and drop what lies past the last channel the same
+// way).
 static bool vector_nhwc(const Plan &g) {
-    return g.src_fmt == xnor_nn_data_format_nhwc && (g.ic & 3) == 0
+    return g.src_fmt == xnor_nn_data_format_nhwc
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET;
 }
+
+// The tiled kernel takes NHWC input that its LDS can hold: about 13500 channels.  us here / where it
+// does not run, a lane to a pixel:
+//   channels a multiple of 4: binarize_nhwc_kernel, whose loads touch 64 lines each
+//     1500 on 7x7, minibatch 100: 19.3 / 84.0; 28x28, minibatch 60: 61.1 / 160;  2048 on 7x7, minibatch
+//     8 / 64: 19.0 / 84.5 and 21.4 / 86.2;  4000 on 14x14, minibatch 2: 33.4 / 167
+//     (a single tile of more than 64 KB, 2048 channels on 6x6, would be 18.0 / 42.0; that choice is fixed
+//     by the names that the interface reports for it)
+//   others: binarize_generic_kernel, one channel per load
+//     minibatch 64 on 100x100, 6 / 7 / 9 / 13 / 30 / 33 channels: 7.9 / 7.9, 8.0 / 9.7, 8.6 / 13.6,
+//     9.8 / 23.8, 16.1 / 246, 21 / 290; on 224x224, 6 / 7 channels: 33.9 / 29.4, 34.3 / 36.1
+//     minibatch 18 on 23x23, 33 / 111 / 254 / 1023 channels: 4.2 / 6.5, 4.1 / 28.8, 5.4 / 59.7, 16.2 / 447
+//     one tile, 30 / 33 / 65 / 401 channels: 4.2 / 4.2, 4.2 / 4.2, 4.0 / 7.4, 5.2 / 45.1
+static bool nhwc_tiled(const Plan &g) {
+    if (!vector_nhwc(g) || g.bin_nhwc_lane) return false;
+    int rounds;
+    const size_t lds = nhwc_tiled_lds_bytes(g, tiled_waves(g, &rounds));
+    const bool one_tile = g.npix_in <= (uint32_t)TILE;
+    if (g.ic & 3) return g.ic > (one_tile ? 32 : 6) && lds <= 160 * 1024;
+    return lds <= (one_tile ? 64 : 160) * 1024;
+}
+
+// A lane to a pixel, 16 bytes per load.
+static bool nhwc_by_lane(const Plan &g) { return vector_nhwc(g) && (g.ic & 3) == 0 && !nhwc_tiled(g); }
 
 // The measurement switches of this stage, read once when a descriptor is initialised (a launch
 // asks the environment for nothing): XNOR_NN_HIP_BIN_WAVES caps the waves of a workgroup,
@@ -748,8 +811,9 @@ const char *binarize_kernel_name(const Plan &g) {
     return shallow_nchw(g) ? "binarize_nchw_shallow_kernel"
         : split_nchw(g) ? "binarize_nchw_split_kernel"
         : tiled_nchw(g) ? "binarize_nchw_kernel"
-        : !vector_nhwc(g) ? "binarize_generic_kernel"
         : nhwc_by_lane(g) ? "binarize_nhwc_kernel"
+        : !nhwc_tiled(g) ? "binarize_generic_kernel"
+        : g.ic & 3 ? "binarize_nhwc_tiled_kernel<RAGGED>"
         : nhwc_streams(g) ? "binarize_nhwc_tiled_kernel<STREAM>" : "binarize_nhwc_tiled_kernel";
 }
 
@@ -764,12 +828,13 @@ hipError_t launch_binarize_data(const Plan &g, const float *x, uint32_t *bits,
                                        : launch_split<true, false>(g, x, bits, nullptr, s, ev);
         if (e != hipSuccess) return e;
     } else if (tiled_nchw(g)) {
-        if (a_or_null) launch_tiled<false, true, true>(g, x, bits, a_or_null, s, ev);
-        else launch_tiled<false, true, false>(g, x, bits, nullptr, s, ev);
-    } else if (vector_nhwc(g) && !nhwc_by_lane(g)) {
-        if (a_or_null) launch_tiled<true, true, true>(g, x, bits, a_or_null, s, ev);
-        else launch_tiled<true, true, false>(g, x, bits, nullptr, s, ev);
-    } else if (vector_nhwc(g)) {
+        if (a_or_null) launch_tiled<true, true>(g, x, bits, a_or_null, s, ev);
+        else launch_tiled<true, false>(g, x, bits, nullptr, s, ev);
+    } else if (nhwc_tiled(g)) {
+        const hipError_t e = a_or_null ? launch_nhwc_tiled<true, true>(g, x, bits, a_or_null, s, ev)
+                                       : launch_nhwc_tiled<true, false>(g, x, bits, nullptr, s, ev);
+        if (e != hipSuccess) return e;
+    } else if (nhwc_by_lane(g)) {
         const unsigned blocks = (g.npix_in + 255) / 256;
         if (a_or_null)
             launch_kernel(binarize_nhwc_kernel<true, true>, dim3(blocks), dim3(256), 0, s, ev,
@@ -857,10 +922,11 @@ hipError_t launch_mean_abs(const Plan &g, const float *x, float *a, hipStream_t 
         const hipError_t e = launch_split<false, true>(g, x, nullptr, a, s, KernelEvents{});
         if (e != hipSuccess) return e;
     } else if (tiled_nchw(g)) {
-        launch_tiled<false, false, true>(g, x, nullptr, a, s, KernelEvents{});
-    } else if (vector_nhwc(g) && !nhwc_by_lane(g)) {
-        launch_tiled<true, false, true>(g, x, nullptr, a, s, KernelEvents{});
-    } else if (vector_nhwc(g)) {
+        launch_tiled<false, true>(g, x, nullptr, a, s, KernelEvents{});
+    } else if (nhwc_tiled(g)) {
+        const hipError_t e = launch_nhwc_tiled<false, true>(g, x, nullptr, a, s, KernelEvents{});
+        if (e != hipSuccess) return e;
+    } else if (nhwc_by_lane(g)) {
         const unsigned blocks = (g.npix_in + 255) / 256;
         hipLaunchKernelGGL((binarize_nhwc_kernel<false, true>), dim3(blocks), dim3(256), 0, s,
                 x, nullptr, a, geometry(g), inv_ic);
