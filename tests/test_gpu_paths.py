@@ -464,6 +464,18 @@ def test_deep_input_of_few_pixels(oracle, monkeypatch, t, separate_k):
     run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("small", ["0", "1"])
+@pytest.mark.parametrize("kh,kw", [(1, 2), (2, 1), (4, 3), (3, 4), (6, 6), (5, 8), (9, 9), (2, 10),
+                                   (11, 11), (11, 1), (3, 12), (12, 12)])
+@pytest.mark.parametrize("mb,ic,ih,iw", [(1, 16, 1, 1), (1, 16, 2, 1), (2, 40, 1, 3), (3, 70, 13, 12)])
+def test_sums_of_mean_magnitudes_of_any_width(oracle, monkeypatch, mb, ic, ih, iw, kh, kw, small):
+    """K of kernels that are narrower than the rows their sums read, down to images of one pixel."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", small)
+    pad = max(kh, kw) // 2
+    d, x, w = problem((mb, ic, 40, ih, iw, kh, kw, 1, 1, pad, pad), zeros=True)
+    run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("separate_k", [False, True])
 @pytest.mark.parametrize("t,name", [
     ((1, 32, 8, 9, 8, 1, 1, 1, 1, 0, 0), "tiled_kernel"),            # whole pieces, one slice

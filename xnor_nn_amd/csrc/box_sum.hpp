@@ -16,9 +16,13 @@ namespace xnor_hip {
 // row ahead of it is added.  (An address selected per tap took eight.)  A row that has a valid tap
 // begins at -(KW-1) at least and limit-1 at most; others are moved there, so reads reach from
 // KW-1 floats ahead of a to KW-1 floats past a[limit]: LDS of the same workgroup on both sides.
+// A kernel of fewer columns runs the next wider one: a column past its last has no bit in the mask.
 // What it bounds: the end of a tile's staging, which the waves that sum K reach last.  32 to 64
 // channels 5x5 on 32x32, minibatch 100: 3.6 -> 1.1 us of a tile's 10.2 (a pass 17.2 -> 15.3); 3x3: a
-// pass of 64 channels on 56x56, minibatch 4, 9.9 -> 8.6.
+// pass of 64 channels on 56x56, minibatch 4, 9.9 -> 8.6.  Rows of 11 and of even widths (the loop at
+// the end before), us of the kernel: 11x11 stride 4, 16 channels on 83x83, minibatch 64, 20.0 -> 17.2,
+// 48 on 120x120, 30, 44.1 -> 37.4, 16 on 85x86, 3, 12.6 -> 10.1; 8x8, 6x6, 4x4 and 2x2 of 16 channels on
+// 22x22, 3: 8.2 -> 7.0, 7.4 -> 6.2, 5.5 -> 4.9, 4.8 -> 4.5.
 template <int KW>
 __device__ __forceinline__ float box_sum_rows(const float *a, const int first, const int limit,
         const uint32_t rowmask, const uint32_t colmask, const int kh_n, const int iw,
@@ -49,12 +53,11 @@ __device__ __forceinline__ float box_sum_rows(const float *a, const int first, c
 __device__ __forceinline__ float box_sum(const float *a, const int first, const int limit,
         const uint32_t rowmask, const uint32_t colmask, const int kh_n, const int kw_n, const int iw,
         const float inv_khw) {
-    switch (kw_n) { // uniform
-    case 1: return box_sum_rows<1>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
-    case 3: return box_sum_rows<3>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
-    case 5: return box_sum_rows<5>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
-    case 7: return box_sum_rows<7>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
-    }
+    if (kw_n == 1) return box_sum_rows<1>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
+    if (kw_n <= 3) return box_sum_rows<3>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
+    if (kw_n <= 5) return box_sum_rows<5>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
+    if (kw_n <= 7) return box_sum_rows<7>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
+    if (kw_n <= 11) return box_sum_rows<11>(a, first, limit, rowmask, colmask, kh_n, iw, inv_khw);
     // four taps per round, all reads of a round issued before its first addition; a tap outside
     // the image reads the slot past the last pixel, which holds zero
     float sum = 0.f;

@@ -368,7 +368,7 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     const int walk = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
     const bool one_launch = g.xw <= 2 && walk < 16;
     // input pixels a block of 32 output pixels touches at most (blocks start at multiples of 32)
-    int most = 1;
+    int most = g.kw > 7 ? 2 : 1; // (sums of K read up to ten floats ahead of mean|x|: rows lie there)
     const uint32_t look = blocks < (uint32_t)g.ohw + 1 ? blocks : (uint32_t)g.ohw + 1;
     auto see = [&](uint32_t b) {
         int lo, hi;
