@@ -1148,6 +1148,8 @@ int oc_subblocks(const Plan &g) { return ((g.oc + NT - 1) / NT) * (NT / 32); }
 // many (plus the last, possibly short, tile) are enough to look at.
 int max_tile_rows(const Plan &g, uint32_t mt, uint32_t step = 0) {
     if (step == 0) step = mt;
+    for (const auto &known : g.tile_rows)
+        if (known.pixels == mt && known.step == step) return known.rows;
     const uint32_t starts = (g.npix_out + step - 1) / step;
     const uint32_t look = starts < (uint32_t)g.ohw + 1 ? starts : (uint32_t)g.ohw + 1;
     int most = 1;
@@ -1159,6 +1161,7 @@ int max_tile_rows(const Plan &g, uint32_t mt, uint32_t step = 0) {
     };
     for (uint32_t t = 0; t < look; t++) see(t);
     see(starts - 1);
+    g.tile_rows[g.tile_rows_next++ % TILE_ROWS_KNOWN] = {mt, step, most};
     return most;
 }
 
@@ -1459,6 +1462,8 @@ static int stream_output(const Plan &g) {
 }
 
 void mfma_plan(Plan &g) {
+    for (auto &known : g.tile_rows) known = {};
+    g.tile_rows_next = 0;
     g.stream_dst = stream_output(g);
     g.mfma_parts = g.mfma_groups = 1;
     if (shallow_plan(g)) { // (every other mfma_* field stays zero)
