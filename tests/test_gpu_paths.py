@@ -477,6 +477,30 @@ def test_sums_of_mean_magnitudes_of_any_width(oracle, monkeypatch, mb, ic, ih, i
 
 
 @pytest.mark.parametrize("separate_k", [False, True])
+@pytest.mark.parametrize("t,small", [
+    ((1, 256, 112, 41, 61, 5, 5, 1, 1, 2, 2), True),       # 316 pairs of blocks (256 compute units), 100 steps
+    ((1, 256, 192, 42, 60, 5, 5, 1, 1, 2, 2), False),      # 474
+    ((2, 300, 96, 56, 60, 3, 3, 1, 1, 1, 1), False),       # 630, as many steps of nine taps
+    ((1, 64, 40, 47, 45, 5, 5, 1, 1, 2, 2), True),         # 25 steps, two launches of 134
+    ((1, 50, 40, 29, 31, 5, 5, 1, 1, 2, 2), True),         # no more than 1024 words to pack
+    ((1, 1, 33, 24, 25, 11, 11, 1, 1, 5, 5), False),       # (a kernel for few channels)
+    ((1, 70, 33, 9, 9, 9, 9, 1, 1, 4, 4), True),           # the summing wave has no steps
+    ((1, 70, 33, 9, 9, 1, 3, 1, 1, 0, 1), True),           # six steps in four waves
+], ids=str)
+def test_sums_of_k_beside_the_steps(oracle, gpu, t, small, separate_k, monkeypatch):
+    """One wave of the kernel for few tiles sums K and has fewer steps, or none."""
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    conv = make(d, w)
+    try:
+        assert ("small_kernel" in conv.kernel_name(0)) == small
+    finally:
+        conv.close()
+    run_and_compare(oracle, d, x, w, NCHW, True, gpu)
+
+
+@pytest.mark.parametrize("separate_k", [False, True])
 @pytest.mark.parametrize("t,name", [
     ((1, 32, 8, 9, 8, 1, 1, 1, 1, 0, 0), "tiled_kernel"),            # whole pieces, one slice
     ((2, 6, 8, 9, 8, 3, 3, 1, 1, 1, 1), "generic_kernel"),

@@ -83,8 +83,11 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     const uint32_t block = s.subs == 1 ? blockIdx.x : s.div_subs.div(blockIdx.x);
     const int sub = (int)(blockIdx.x - block * (uint32_t)s.subs); // 32-filter block
     const uint32_t p_first = block * 32u, p_limit = g.npix_out;
-    // this wave's share of the steps
-    const int s_lo = (wave * s.nsteps) / WAVES, s_hi = ((wave + 1) * s.nsteps) / WAVES;
+    const bool fuse_k = FUSED || a_plane != nullptr; // uniform
+    // this wave's share of the steps; the last wave sums K as well
+    const int share = s.nsteps + (fuse_k ? s.k_steps : 0);
+    const int s_lo = min((wave * share) / WAVES, s.nsteps);
+    const int s_hi = min(((wave + 1) * share) / WAVES, s.nsteps);
 
     // ---- the input: which pixels the tile touches; their words and mean|x| are asked for first (a
     // buffer ends with the tile's run: with a branch around each load the compiler would wait for one
@@ -92,7 +95,6 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     int lo, hi;
     row_span(g, p_first, min(p_first + 32u, p_limit), lo, hi);
     const int nrows = min(hi - lo + 1, s.max_rows), nitems = nrows * g.xw;
-    const bool fuse_k = FUSED || a_plane != nullptr; // uniform
     const uint32_t *run = xbits + (size_t)lo * g.xw;
     [[maybe_unused]] uint32_t word[4];
     [[maybe_unused]] float a_early = 0.f;
@@ -276,15 +278,17 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
 #pragma unroll
     for (int i = 0; i < 16; i++)
         if (i / KEEP != wave) parts[(wave * 16 + i) * 64 + lane] = acc0[i]; // uniform
-    // ---- K of the lane's pixel (box_sum.hpp), while the other waves finish their steps, unless it
-    // came from the K plane
+    // ---- K of the lane's pixel (box_sum.hpp): the last wave's, where it keeps registers itself
     float kv = k_read;
-    if (fuse_k) {
+    float *k_lds = parts + (WAVES - 1) * (16 + KEEP) * 64;
+    if (fuse_k && wave == WAVES - 1) {
         kv = box_sum(a_lds, in0, s.max_rows, rowmask, colmask, g.kh, g.kw, g.iw, inv_khw);
-        if (sub == 0 && wave == 0 && lane < 32 && live) k_out[pix] = kv;
+        k_lds[lane] = kv;
+        if (sub == 0 && lane < 32 && live) k_out[pix] = kv;
     }
 
     __syncthreads();
+    if (fuse_k) kv = k_lds[lane];
     float sum[KEEP];
 #pragma unroll
     for (int ii = 0; ii < KEEP; ii++) {
@@ -333,6 +337,13 @@ SmallPlan small_plan(const Plan &g, int rows) {
     s.max_rows = rows;
     s.ks = g.mfma_steps;
     s.nsteps = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
+    // The last wave sums K besides its steps, so it gets fewer: by half a step's time per tap, at most by
+    // all that the others can take evenly.  us of the kernel with all waves summing it / one, with as many
+    // steps / one, with fewer: 11x11 stride 4, 16 channels on 85x86, minibatch 3, 10.1 / 8.5 / 7.2; 7x7 of 19
+    // on 36x39 6.2 / 6.3 / 5.5; 5x5 of 208 on 59x59, minibatch 1, 6.4 / 6.6 / 6.0; 3x3 of 384 on 13x13,
+    // minibatch 1, 5.1 / 5.2 / 4.9 (a quarter 5.0, a whole step 4.8), 512 on 28x28 7.5 / 7.3 / 7.0.
+    const int waves = small_waves(g), even = (s.nsteps + waves - 2) / (waves - 1);
+    s.k_steps = (g.kh * g.kw + 1) / 2 < even ? (g.kh * g.kw + 1) / 2 : even;
     s.subs = (g.oc + 31) / 32;
     s.row_bytes = small_row_bytes(g);
     s.blocks = (g.npix_out + 31) / 32;
@@ -343,6 +354,17 @@ SmallPlan small_plan(const Plan &g, int rows) {
     s.div_kw = FastDiv::make((uint32_t)g.kw);
     return s;
 }
+
+// Every filter block repeats the packing of what its pixels touch, `rows` input pixels: in one launch up
+// to 1024 words.  us a pass, one launch / two, on the device and through the torch module, whose host part
+// is 3 us for two launches more than for one (on a machine where two launches are bound by 3.7 and 5.4):
+//   448 words  64 channels 3x3 on 56x56                4.3 / 3.9
+//   588        64 3x3 stride 2 on 42x42, minibatch 4   4.7 / 3.8   4.7 / 5.5
+//   850        64 3x3 stride 2 on 85x85                5.0 / 3.9   5.0 / 5.6
+//   1530       64 7x7 stride 2 on 85x85                5.6 / 4.2   5.6 / 5.5
+//   1932       64 11x11 stride 4 on 42x42, 4           6.7 / 5.0   6.8 / 5.4
+//   3360       64 11x11 stride 4 on 112x112, 4        11.0 / 6.7  10.9 / 6.7
+static bool one_launch_pays(const Plan &g, int rows) { return rows * g.xw <= 1024; }
 
 // Which problems take this kernel: one channel part and so few (pixel block, filter block) pairs,
 // a workgroup each, that the large-launch kernel would leave most of the chip idle.  Both were
@@ -355,6 +377,11 @@ SmallPlan small_plan(const Plan &g, int rows) {
 //   compute unit while a block stages 112 input pixels at most (1000 channels 3x3 on 17x17, 2.0
 //   pairs: 17.7 / 15.5; conv4 of AlexNet, minibatch 12: 7.6 / 7.2 in the kernel; with more to stage
 //   2.0 pairs of 602 channels on 26x26: 19.7 / 20.6, 1.75 of 660 on 45x45: 27.3 / 30.8);
+//   with 48 steps of 25 taps or more 1.75 per compute unit, whatever a block stages: the other waves do
+//   not wait for the sums of K here (us in the kernel, 1.7 pairs: 256 channels 7x7 on 28x28 17.5 / 10.4,
+//   100 on 28x28 10.5 / 8.4, 256 channels 5x5 on 50x50 11.2 / 8.7, 40 channels 11x11 stride 4 on 150x150
+//   19.0 / 16.0, 24 on 227x227 19.4 / 16.4, 48 on 110x110 17.3 / 15.9; 2.2 pairs: 48 channels 7x7 on 19x19
+//   7.8 / 9.7, 100 10.2 / 10.9, 200 channels 5x5 10.6 / 10.5);
 //   with up to 64 channels and a short walk the pass is one launch here, which saves the host
 //   more than the kernel loses (1.1 pairs: 8.6 / 9.4 on the device, 11.4 / 8.5 through the torch
 //   module): 1.5 pairs;
@@ -366,9 +393,8 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     const uint32_t subs = (uint32_t)(g.oc + 31) / 32;
     const uint64_t pairs = (uint64_t)blocks * subs, cus = (uint64_t)g.cus;
     const int walk = (g.mfma_pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw) * g.mfma_steps;
-    const bool one_launch = g.xw <= 2 && walk < 16;
     // input pixels a block of 32 output pixels touches at most (blocks start at multiples of 32)
-    int most = g.kw > 7 ? 2 : 1; // (sums of K read up to ten floats ahead of mean|x|: rows lie there)
+    int most = g.kw > 7 ? 2 : 1; // (the sums of K read up to ten floats ahead of mean|x|: rows lie there)
     const uint32_t look = blocks < (uint32_t)g.ohw + 1 ? blocks : (uint32_t)g.ohw + 1;
     auto see = [&](uint32_t b) {
         int lo, hi;
@@ -377,8 +403,10 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     };
     for (uint32_t b = 0; b < look; b++) see(b);
     see(blocks - 1);
+    const bool one_launch = g.xw <= 2 && walk < 16 && one_launch_pays(g, most);
     bool take = one_launch ? 2 * pairs <= 3 * cus
-        : walk >= 48 && most <= 112 ? pairs <= 2 * cus : walk > 4 && pairs <= cus;
+        : walk >= 48 && most <= 112 ? pairs <= 2 * cus
+        : walk >= 48 && g.kh * g.kw >= 25 ? 4 * pairs <= 7 * cus : walk > 4 && pairs <= cus;
     // paired taps: from packed words only on long walks (160 channels 5x5, 65 steps: 11.2 us a pass
     // against 13.5; 96 channels 3x3, 15 steps: 9.1 against 8.7 in the large kernel)
     if (g.mfma_pair && g.xw > 1 && walk < 24) take = false;
@@ -397,12 +425,12 @@ bool small_kernel_applies(const Plan &g, int *rows_out, uint32_t *lds_out) {
     return true;
 }
 
-// Whether a forward pass on device buffers may run the one-launch form: up to 64 channels, 32-bit
-// offsets into the input (with room for the dropped one).  Measured per pass, device-bound: 32
+// Whether a forward pass on device buffers may run the one-launch form: up to 64 channels, not too much to
+// pack, 32-bit offsets into the input (with room for the dropped one).  Measured per pass, device-bound: 32
 // channels 3x3 on 14x14, minibatch 1: 7.0 us against 8.2 for two launches, 64 channels on 56x56:
 // 8.1 against 8.5; called from Python through the torch module 8.5 against 11.4 (the host's part).
 bool one_launch_applies(const Plan &g) {
-    return g.mfma_small && g.xw <= 2
+    return g.mfma_small && g.xw <= 2 && one_launch_pays(g, g.small.max_rows)
         && (uint64_t)g.npix_in * (uint64_t)g.ic * 4u < XNOR_HIP_DROPPED_OFFSET;
 }
 

@@ -77,6 +77,7 @@ struct Geometry {
 struct SmallPlan {
     int max_rows;     // input pixels a block stages at most
     int ks, nsteps;   // steps per tap (or pair of taps), and in all
+    int k_steps;      // what the sums of K count for where the steps are dealt out
     int subs;         // 32-filter blocks
     int row_bytes;    // of an input pixel's FP4 row in LDS
     uint32_t blocks, wfrag_bytes; // 32-pixel blocks
