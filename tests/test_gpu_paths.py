@@ -672,6 +672,10 @@ def test_short_and_long_walks(oracle, monkeypatch, ic, blocks):
     (1, 130, 30, 12, 150, 5, 5, 2, 1, 2, 2),
     (1, 1100, 40, 4, 70, 3, 3, 1, 1, 1, 1),     # channel parts
     (1, 864, 40, 5, 83, 3, 3, 1, 1, 1, 1),      # more than the LDS if whole rows were staged
+    (2, 96, 40, 9, 32, 3, 3, 1, 1, 1, 1),       # the widest rows that are staged whole,
+    (2, 96, 40, 9, 33, 3, 3, 1, 1, 1, 1),       # one column more,
+    (2, 96, 40, 9, 32, 3, 3, 2, 1, 1, 1),       # and a stride either way
+    (2, 96, 40, 9, 32, 3, 3, 1, 2, 1, 1),
 ], ids=str)
 @pytest.mark.parametrize("small", ["0", "1"])
 def test_tiles_that_begin_inside_a_row(oracle, monkeypatch, t, small):
