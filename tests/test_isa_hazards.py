@@ -365,6 +365,33 @@ def test_lds_direct_loads_count_but_write_no_register():
     assert m0_outside_asm(ok + ["s_mov_b32 m0, s8"]) == ["s_mov_b32 m0, s8"]
 
 
+def kernel_metadata(isa, field):
+    """Demangled kernel name -> a field of its metadata."""
+    counts, name = {}, None
+    for line in isa:
+        line = line.strip()
+        if line.startswith(".name:"):
+            name = line.split()[1]
+        elif line.startswith("." + field + ":") and name:
+            counts[name] = int(line.split()[1])
+    plain = subprocess.run(["c++filt"], input="\n".join(counts), capture_output=True, text=True,
+                           check=True).stdout.split("\n")
+    return dict(zip(plain, counts.values()))
+
+
+def test_tiles_of_two_sizes_spill_no_scalar_registers(conv_isa):
+    """Both tile bodies of a launch with two tile sizes find room for the addresses, the weights'
+    descriptor and the lane masks of the sums of K (scaled output)."""
+    seen = 0
+    for text, spilled in kernel_metadata(conv_isa, "sgpr_spill_count").items():
+        m = re.search(r"conv_mfma_fp4\w*_kernel<(\d+), (\d+), (\d+), (\w+)", text)
+        if not m or m[3] == "0" or m[4] == "true" or "persistent" in text:
+            continue
+        assert spilled == 0, "%s: %d scalar registers" % (text[:80], spilled)
+        seen += 1
+    assert seen >= 18, seen
+
+
 def resident_by_registers(ks, ps):
     """The register half of resident_workgroups() in kernels_conv_mfma.hip, restated."""
     if ps == 3:
