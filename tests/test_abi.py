@@ -298,6 +298,14 @@ def test_kernel_variants_planned_for_known_shapes(monkeypatch):
     assert kernel_names((256,) + conv4)[1] == "conv_xnor_popc_kernel<XW=12,Q=16>"
 
 
+def test_deep_narrow_images_run_on_the_matrix_cores():
+    """A tile stages its taps' span however few columns the image has: with whole rows the tiles of these
+    layers do not fit the LDS, or only one by one."""
+    for t, steps in (((4, 128, 3000, 28, 28, 3, 3, 1, 1, 1, 1), 16), ((8, 128, 4096, 14, 14, 3, 3, 1, 1, 1, 1), 16),
+                     ((2, 128, 2048, 28, 28, 5, 5, 1, 1, 2, 2), 16), ((4, 128, 3000, 28, 33, 3, 3, 1, 1, 1, 1), 16)):
+        assert kernel_names(t)[1].startswith("conv_mfma_fp4_kernel<KS=%d,PS=" % steps), t
+
+
 def test_inputs_that_reach_the_dropped_offset_take_the_generic_kernel():
     """The tiled binarize kernels read a channel past the end of a ragged slice through the
     byte offset 0xFFFFFFF0, which the hardware drops only while it lies outside the buffer.

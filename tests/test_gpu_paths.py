@@ -689,6 +689,24 @@ def test_tiles_that_begin_inside_a_row(oracle, monkeypatch, t, small):
         run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("t", [
+    (1, 3000, 33, 28, 28, 3, 3, 1, 1, 1, 1),    # one tile to a compute unit's LDS
+    (1, 4096, 8, 14, 14, 3, 3, 1, 1, 1, 1),     # four channel parts
+    (1, 2048, 8, 15, 28, 5, 5, 1, 1, 2, 2),
+    (3, 1024, 40, 10, 10, 3, 3, 1, 1, 1, 1),    # tiles across images
+    (9, 1100, 40, 7, 7, 1, 1, 1, 1, 0, 0),      # a tile's pixels and no more
+], ids=str)
+@pytest.mark.parametrize("separate_k", [False, True])
+def test_deep_narrow_images(oracle, monkeypatch, t, separate_k):
+    """Tiles that begin inside a row of a narrow image."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", "0")
+    if separate_k:
+        monkeypatch.setenv("XNOR_NN_HIP_SEPARATE_K", "1")
+    d, x, w = problem(t, zeros=True)
+    assert make(d, w).kernel_name(0).startswith("conv_mfma_fp4_kernel<")
+    run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("t,joined", [
     ((26, 384, 40, 13, 13, 3, 3, 1, 1, 1, 1), True),
     ((26, 70, 8, 13, 13, 15, 15, 4, 4, 7, 7), True),      # long filters, few tiles

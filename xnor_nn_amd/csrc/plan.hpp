@@ -211,10 +211,11 @@ __host__ __device__ inline void row_span(const Geometry &g, uint32_t p_first, ui
 // wide rows of many channels more than the LDS holds.  Kernel alone, whole rows / this, us: 130 to 70
 // channels 3x3 stride 2 on 45x51 6.9 / 6.4 (a pass 11.4 / 11.0), 256 to 128 channels 1x1 stride 2 on
 // 56x56 15.9 / 10.7, 224 channels 5x5 on 78x78 16.0 / 15.2, 156 channels on 101x101 39.7 / 37.8, 864 on
-// 83x83 226 (the popcount kernel) / 65.  Up to 32 columns without a stride there is little between them, and
-// whole rows are never slower (a pass, whole rows / this: 512 channels on 28x28, minibatch 32, behind a
-// rectifier 36.9 / 37.2; fourteen others of 14 to 32 columns within 0.4 % of each other): they stay.
-// Wider, 512 channels on 36x36 40.7 / 40.6, on 44x44 60.9 / 60.3, 128 on 56x56 35.7 / 35.3.
+// 83x83 226 (the popcount kernel) / 65.  Narrow images without a stride alike, us a pass, whole rows /
+// this: 3000 to 128 channels 3x3 on 28x28, minibatch 4, 276.8 (the popcount kernel) / 47.1, 4096 on 14x14,
+// 8, 378.6 / 62.5, 2048 to 512 1x1 on 13x13, 96, 60.7 / 55.6, 1024 to 128 3x3 on 10x10, 256, 51.4 / 47.5,
+// on 28x28, 8, 26.8 / 24.7; where a tile fits either way there is little between them (512 on 28x28, 32,
+// behind a rectifier 38.8 / 38.6; of 155 layers of up to 32 columns one is slower by more than 1.5 %).
 __host__ __device__ inline void tile_span(const Geometry &g, uint32_t p_first, uint32_t p_end,
         int &lo, int &hi) {
     const uint32_t p_last = p_end - 1;
@@ -223,9 +224,8 @@ __host__ __device__ inline void tile_span(const Geometry &g, uint32_t p_first, u
     const int oh0 = (int)g.div_ow.div((uint32_t)rem0), oh1 = (int)g.div_ow.div((uint32_t)rem1);
     int r0 = oh0 * g.sh - g.ph, r1 = oh1 * g.sh - g.ph + g.kh - 1;
     int c0 = (rem0 - oh0 * g.ow) * g.sw - g.pw, c1 = (rem1 - oh1 * g.ow) * g.sw - g.pw + g.kw - 1;
-    const bool whole_rows = g.iw <= 32 && g.sh == 1 && g.sw == 1;
-    if (whole_rows || r0 < 0 || c0 < 0) c0 = 0;
-    if (whole_rows || r1 > g.ih - 1 || c1 > g.iw - 1) c1 = g.iw - 1;
+    if (r0 < 0 || c0 < 0) c0 = 0;
+    if (r1 > g.ih - 1 || c1 > g.iw - 1) c1 = g.iw - 1;
     if (c0 > g.iw - 1) c0 = g.iw - 1;
     if (c1 < 0) c1 = 0;
     if (r0 < 0) r0 = 0;
