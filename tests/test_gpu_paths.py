@@ -689,6 +689,27 @@ def test_tiles_that_begin_inside_a_row(oracle, monkeypatch, t, small):
         run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4])
+@pytest.mark.parametrize("ic", [20, 64, 70, 128, 192])
+def test_walks_with_several_groups_under_way(oracle, monkeypatch, ic, blocks):
+    """... whatever their length: fewer groups than are under way, every remainder, and the lengths on
+    either side of where the rule takes them."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_PS", str(blocks))
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", "0")
+    for long_walk, kernels in (("1", [(1, 1), (1, 2), (2, 2), (1, 5), (2, 3), (1, 7), (2, 4), (3, 3), (2, 5),
+                                      (1, 11), (3, 4), (1, 13), (2, 7)]),
+                               (None, [(1, 7), (2, 4), (3, 5), (3, 6), (4, 5), (3, 13), (5, 8), (6, 13),
+                                       (8, 10), (11, 11)])):
+        if long_walk:
+            monkeypatch.setenv("XNOR_NN_HIP_MFMA_LONG", long_walk)
+        else:
+            monkeypatch.delenv("XNOR_NN_HIP_MFMA_LONG")
+        for kh, kw in kernels:
+            for oc in (70,) if long_walk else (33, 70, 140): # four, two and one pixel groups
+                d, x, w = problem((2, ic, oc, 5, 14, kh, kw, 1, 1, kh // 2, kh // 2), zeros=True)
+                run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("t", [
     (1, 3000, 33, 28, 28, 3, 3, 1, 1, 1, 1),    # one tile to a compute unit's LDS
     (1, 4096, 8, 14, 14, 3, 3, 1, 1, 1, 1),     # four channel parts

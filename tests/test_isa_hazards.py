@@ -266,6 +266,23 @@ def test_no_register_is_touched_while_its_load_is_in_flight(conv_isa):
     assert checked >= EXPECTED_VARIANTS, checked
 
 
+def test_short_walks_ask_for_few_fragments_that_do_not_exist(conv_isa):
+    """The variants of up to three steps per tap that short walks run have asked for two groups of weight
+    fragments at most when they multiply the first (two fragments a step); those of long walks, whose
+    prologue a 1x1 kernel would pay for in full, for more."""
+    seen = [0, 0]
+    for name, body in kernels_of(conv_isa, r"^_ZN\S*conv_mfma_fp4\S*kernel\S*:"):
+        m = re.search(r"conv_mfma_fp4_(kernel|long_kernel)ILi(\d)ELi(\d)ELi0ELb(\d)E", name)
+        if not m or int(m[2]) > 3 or (m[1] == "kernel" and m[4] == "1"):  # (raw accumulators)
+            continue
+        first = next(i for i, l in enumerate(body) if l.startswith("v_mfma"))
+        asked = sum(l.startswith("buffer_load_dwordx4") for l in body[:first])
+        if m[1] == "kernel":
+            assert asked <= 2 * 2 * int(m[2]), (name[:90], asked)
+        seen[m[1] != "kernel"] += 1
+    assert seen[0] >= 20 and seen[1] >= 8, seen
+
+
 def test_no_wide_store_loses_its_data(conv_isa):
     wide = 0
     for name, body in kernels_of(conv_isa, r"^_ZN\S*conv_mfma_fp4\S*kernel\S*:"):

@@ -212,7 +212,8 @@ __device__ __forceinline__ void copy_to_lds_async(const void *src, const int n,
 // PERSIST: the caller loops over tiles (see conv_mfma_fp4_persistent_kernel); `turn` says what
 // is already in LDS and which tile to prefetch.  The LDS layout then has room for four pixel
 // blocks whatever PS is, so that tiles of two sizes can follow each other.
-template <int KS, int PS, bool RAW, bool PAIR, bool DEEP, bool PERSIST = false>
+// LONG: the walk is long enough for several groups of weight fragments under way (long_walk()).
+template <int KS, int PS, bool RAW, bool PAIR, bool DEEP, bool LONG, bool PERSIST = false>
 __device__ __forceinline__
 void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag,
         const float *__restrict__ alpha, const float *__restrict__ kplane,
@@ -258,14 +259,15 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
     constexpr int GROUPS_PER_TAP = KS / HS; // 1, 2 or 4
     // Where a group is a few matrix instructions, a good deal less than the way to the L2 and back, one
     // group ahead is not enough: SETS groups are then under way, as many as the registers of
-    // resident_workgroups() allow, and a group is asked for where the one just multiplied lay.  Kernel
-    // alone, us: 48 to 96 channels 11x11 on 100x100 83.3 -> 58.8, 36 to 40 on 83x83
-    // 31.5 -> 20.0, 32 to 64 channels 5x5 on 32x32 10.6 -> 9.8 (a pass 14.3 -> 13.2), 64 channels on 56x56, minibatch 16, 6.7 ->
-    // 6.1, 192 on 14x14 6.0 -> 5.5, 525 to 21 on 49x49 16.6 -> 14.9; on 21 layers of up to 64 channels
-    // 9 % on average, none more than 1 % slower.  With longer groups it is as fast or slower: 384
-    // channels on 13x13, minibatch 256, 23.2 -> 23.7, 256 on 56x56 63 -> 65.
-    constexpr bool RING = HS == 1 || (PS == 1 && HS <= 3);
-    constexpr int SETS = HS == 1 ? (PS == 1 ? 6 : PS == 2 ? 3 : PS == 3 ? 2 : 4) : RING && HS == 2 ? 4 : 2;
+    // resident_workgroups() allow, and a group is asked for where the one just multiplied lay.  Up to three
+    // steps per tap only on long walks: what is asked for behind the last group, up to SETS groups of
+    // fragments that nothing multiplies, comes on top of a stream that bounds such a tile
+    // (long_walk()).  Kernel alone, us: 48 to 96 channels 11x11 on 100x100 83.3 -> 58.8, 36 to 40 on
+    // 83x83 31.5 -> 20.0.  Twelve steps per tap, a pass: 525 to 64 channels 5x5 on 10x10, minibatch 256,
+    // 40.1 -> 35.0, 576 to 64 3x3 25.9 -> 24.3, 1x1 level.  With longer groups it is as fast or slower:
+    // 384 channels on 13x13, minibatch 256, 23.2 -> 23.7, 256 on 56x56 63 -> 65.
+    constexpr bool RING = (HS == 1 || (PS == 1 && HS <= 3)) && (LONG || KS >= 12);
+    constexpr int SETS = !RING ? 2 : HS == 1 ? (PS == 1 ? 6 : PS == 2 ? 3 : PS == 3 ? 2 : 4) : HS == 2 ? 4 : 2;
 
     int thread = threadIdx.x;
     // PERSIST: a value the compiler cannot see through, so that nothing computed from it
@@ -876,13 +878,13 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
 // order of their index and the matrix pipe serves the older wave of a SIMD first, so on a
 // compute unit that holds two workgroups the one with the small tile is the one that
 // finishes last: its epilogue, the only one nothing overlaps, is the short one.
-template <int KS, int PS, int PSB, bool RAW, bool PAIR, bool DEEP>
-__global__ __launch_bounds__(256, 2)
-void conv_mfma_fp4_kernel(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag,
+template <int KS, int PS, int PSB, bool RAW, bool PAIR, bool DEEP, bool LONG>
+__device__ __forceinline__
+void conv_tile_of(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag,
         const float *__restrict__ alpha, const float *__restrict__ kplane,
         float *__restrict__ dst, int32_t *__restrict__ popc,
-        const Geometry g, const int max_rows, const int oc_chunks, const uint32_t units,
-        const uint32_t units_per_xcd, const FastDiv div_xw, const FastDiv div_chunks,
+        const Geometry &g, const int max_rows, const int oc_chunks, const uint32_t units,
+        const uint32_t units_per_xcd, const FastDiv &div_xw, const FastDiv &div_chunks,
         const float *__restrict__ a_plane,
         float *__restrict__ k_out, const float inv_khw, const int ic_parts,
         const uint32_t wfrag_bytes, const uint32_t big_per_xcd, const uint32_t blocks_per_xcd) {
@@ -896,7 +898,7 @@ void conv_mfma_fp4_kernel(const uint32_t *__restrict__ xbits, const v4i *__restr
         if (unit >= units) return;
         const uint32_t tile = oc_chunks == 1 ? unit : div_chunks.div(unit);
         const int chunk = unit - tile * oc_chunks;
-        conv_tile<KS, PS, RAW, PAIR, DEEP>(xbits, wfrag, alpha, kplane, dst, popc, g, max_rows,
+        conv_tile<KS, PS, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g, max_rows,
                 div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes,
                 tile * (32u * PS * (uint32_t)g.mfma_groups), g.npix_out, chunk);
     } else {
@@ -907,18 +909,42 @@ void conv_mfma_fp4_kernel(const uint32_t *__restrict__ xbits, const v4i *__restr
         if (tile < big_per_xcd) {
             const uint32_t p_first = (first + tile * PS) * 32u;
             if (p_first >= p_limit) return;
-            conv_tile<KS, PS, RAW, PAIR, DEEP>(xbits, wfrag, alpha, kplane, dst, popc, g,
+            conv_tile<KS, PS, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g,
                     max_rows, div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes, p_first,
                     p_limit, chunk);
         } else {
             const uint32_t p_first = (first + big_per_xcd * PS + (tile - big_per_xcd) * PSB) * 32u;
             if (p_first >= p_limit) return;
-            conv_tile<KS, PSB, RAW, PAIR, DEEP>(xbits, wfrag, alpha, kplane, dst, popc, g,
+            conv_tile<KS, PSB, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g,
                     max_rows, div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes, p_first,
                     p_limit, chunk);
         }
     }
 }
+
+#define XNOR_TILE_PARAMETERS const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag, \
+        const float *__restrict__ alpha, const float *__restrict__ kplane, float *__restrict__ dst, \
+        int32_t *__restrict__ popc, const Geometry g, const int max_rows, const int oc_chunks, \
+        const uint32_t units, const uint32_t units_per_xcd, const FastDiv div_xw, \
+        const FastDiv div_chunks, const float *__restrict__ a_plane, float *__restrict__ k_out, \
+        const float inv_khw, const int ic_parts, const uint32_t wfrag_bytes, \
+        const uint32_t big_per_xcd, const uint32_t blocks_per_xcd
+#define XNOR_TILE_ARGUMENTS xbits, wfrag, alpha, kplane, dst, popc, g, max_rows, oc_chunks, units, \
+        units_per_xcd, div_xw, div_chunks, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes, big_per_xcd, \
+        blocks_per_xcd
+template <int KS, int PS, int PSB, bool RAW, bool PAIR, bool DEEP>
+__global__ __launch_bounds__(256, 2)
+void conv_mfma_fp4_kernel(XNOR_TILE_PARAMETERS) {
+    conv_tile_of<KS, PS, PSB, RAW, PAIR, DEEP, false>(XNOR_TILE_ARGUMENTS);
+}
+// The same for long walks of few steps per tap (long_walk()), scaled output.
+template <int KS, int PS, int PSB, bool PAIR>
+__global__ __launch_bounds__(256, 2)
+void conv_mfma_fp4_long_kernel(XNOR_TILE_PARAMETERS) {
+    conv_tile_of<KS, PS, PSB, false, PAIR, false, true>(XNOR_TILE_ARGUMENTS);
+}
+#undef XNOR_TILE_PARAMETERS
+#undef XNOR_TILE_ARGUMENTS
 
 // The same tiles for launches with several rounds of them: two workgroups per compute unit
 // that stay, each walking over its tiles.  Tiles are numbered per XCD as in the two-size
@@ -994,11 +1020,11 @@ void conv_mfma_fp4_persistent_kernel(const uint32_t *__restrict__ xbits,
         turn.next_first = more ? next_first : 0u;
         turn.next_end = more ? end_pixel(next, next_first) : 0u;
         if (tile < big_per_xcd)
-            conv_tile<KS, PS, false, PAIR, false, true>(xbits, wfrag, alpha, kplane, dst, nullptr,
+            conv_tile<KS, PS, false, PAIR, false, false, true>(xbits, wfrag, alpha, kplane, dst, nullptr,
                     g, max_rows, div_xw, a_plane, k_out, inv_khw, 1, wfrag_bytes, p_first,
                     p_limit, chunk, turn);
         else
-            conv_tile<KS, PSB, false, PAIR, false, true>(xbits, wfrag, alpha, kplane, dst,
+            conv_tile<KS, PSB, false, PAIR, false, false, true>(xbits, wfrag, alpha, kplane, dst,
                     nullptr, g, max_rows, div_xw, a_plane, k_out, inv_khw, 1, wfrag_bytes,
                     p_first, p_limit, chunk, turn);
         if (!more) break;
@@ -1255,6 +1281,33 @@ int resident_workgroups(const Plan &g, int ps) {
     return fit < 2 ? 2 : fit; // a tile that runs alone is priced separately
 }
 
+// Whether the walk over the taps (or pairs of taps) of a layer of up to three steps per tap is long enough
+// to have several groups of weight fragments under way (RING in conv_tile).  XNOR_NN_HIP_MFMA_LONG=0|1
+// overrides, for measurements.  A pass with one group ahead / several, on 440 layers; pixel groups are
+// waves that read the same fragments:
+//   one block a tile, 1 group    9 to 25 taps 1.016 to 1.044, 49 1.12, 121 (2 and 3 steps too) 1.13 to 1.24
+//     2 groups                   1 step: 9 taps 1.019, 16 1.026, 25 1.00 to 1.05, 49 1.09, 121 1.23; pairs
+//                                and more steps: 2 to 9 taps 0.97 to 1.00, 13 pairs 0.99, 25 and more 1.00 to 1.06
+//     4 groups                   up to 25 taps 0.96 to 1.00, 49 and more 1.04 to 1.25 (32 to 64 channels 5x5
+//                                on 32x32, minibatch 50, 9.22 / 9.70 us); with more than 32 KB of LDS,
+//                                as strides need, 16 and 25 taps of one or two steps 0.99 to 1.10
+//   more blocks, 1 step          1 tap 0.98, 4 1.005, 9 1.01, 16 and more 1.01 to 1.2; pairs 5 0.997, 8 1.01,
+//                                13 1.01, but 1 group and more workgroups than two to a compute unit 0.98
+bool long_walk(const Plan &g) {
+    const int ks = steps_per_tap(g), groups = g.mfma_groups;
+    const bool pair = pair_taps(g);
+    if (ks > 3 || (ks > 1 && g.mfma_ps > 1)) return false;
+    if (const char *e = getenv("XNOR_NN_HIP_MFMA_LONG")) return e[0] == '1';
+    const int walk = pair ? (g.kh * g.kw + 1) / 2 : g.kh * g.kw;
+    if (g.mfma_ps == 1) {
+        if (groups == 4) return walk >= (!pair && ks <= 2 && g.mfma_lds > 32 * 1024 ? 16 : 40);
+        return walk >= (groups == 2 && (pair || ks > 1) ? 20 : 8);
+    }
+    const uint64_t workgroups = (uint64_t)((g.npix_out + 31) / 32) / (uint32_t)(g.mfma_ps * groups)
+        * ((g.oc + NT - 1) / NT);
+    return walk >= (pair && groups == 1 && workgroups > 2u * (uint32_t)g.cus ? 20 : 8);
+}
+
 int pick_ps(const Plan &g) {
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_PS")) {
         const int v = atoi(e);
@@ -1315,35 +1368,31 @@ hipError_t launch_mfma(const Plan &g, const uint32_t *xbits, const uint32_t *wfr
     const size_t lds = g.mfma_lds;
     const int parts = g.mfma_parts;
     const v4i *wf = reinterpret_cast<const v4i *>(wfrag);
+    auto kernel = popc ? conv_mfma_fp4_kernel<KS, PS, PSB, true, PAIR, DEEP>
+                       : conv_mfma_fp4_kernel<KS, PS, PSB, false, PAIR, DEEP>;
+    int which = popc ? 1 : 0;
+    if constexpr (!DEEP && (KS == 1 || (KS <= 3 && PS == 1 && PSB == 0)))
+        if (g.mfma_long_walk && !popc) {
+            kernel = conv_mfma_fp4_long_kernel<KS, PS, PSB, PAIR>;
+            which = 2;
+        }
     if (lds > (size_t)LDS_DEFAULT) {
         // asked for once per kernel, device and size (what has been granted is remembered)
-        static std::atomic<size_t> granted[2][MAX_DEVICES];
+        static std::atomic<size_t> granted[3][MAX_DEVICES];
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES)
             return hipErrorInvalidDevice;
-        std::atomic<size_t> &have = granted[popc ? 1 : 0][dev];
+        std::atomic<size_t> &have = granted[which][dev];
         if (lds > have.load(std::memory_order_acquire)) {
-            const void *fn = popc
-                ? (const void *)conv_mfma_fp4_kernel<KS, PS, PSB, true, PAIR, DEEP>
-                : (const void *)conv_mfma_fp4_kernel<KS, PS, PSB, false, PAIR, DEEP>;
-            const hipError_t e = hipFuncSetAttribute(fn,
+            const hipError_t e = hipFuncSetAttribute((const void *)kernel,
                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return e;
             have.store(lds, std::memory_order_release);
         }
     }
-    if (popc)
-        launch_kernel(conv_mfma_fp4_kernel<KS, PS, PSB, true, PAIR, DEEP>, grid, block, lds, s,
-                ev, xbits, wf, alpha, k, dst, popc, geometry(g), rows, chunks, units, per_xcd,
-                FastDiv::make((uint32_t)g.xw), FastDiv::make((uint32_t)chunks), a_or_null, k_out,
-                1.f / g.kh / g.kw, parts,
-                g.mfma_wbytes, big, blocks);
-    else
-        launch_kernel(conv_mfma_fp4_kernel<KS, PS, PSB, false, PAIR, DEEP>, grid, block, lds, s,
-                ev, xbits, wf, alpha, k, dst, popc, geometry(g), rows, chunks, units, per_xcd,
-                FastDiv::make((uint32_t)g.xw), FastDiv::make((uint32_t)chunks), a_or_null, k_out,
-                1.f / g.kh / g.kw, parts,
-                g.mfma_wbytes, big, blocks);
+    launch_kernel(kernel, grid, block, lds, s, ev, xbits, wf, alpha, k, dst, popc, geometry(g), rows,
+            chunks, units, per_xcd, FastDiv::make((uint32_t)g.xw), FastDiv::make((uint32_t)chunks),
+            a_or_null, k_out, 1.f / g.kh / g.kw, parts, g.mfma_wbytes, big, blocks);
     return hipGetLastError();
 }
 
@@ -1483,6 +1532,7 @@ void mfma_plan(Plan &g) {
     g.one_launch = 0;
     g.mfma_persist = g.mfma_reverse = 0;
     g.mfma_tiles_per_round = g.mfma_rounds = g.mfma_stagger = 0;
+    g.mfma_long_walk = 0;
     g.mfma_parts = 1;
     g.mfma_lds = g.mfma_wbytes = 0;
     if (!g.use_mfma) return;
@@ -1597,6 +1647,7 @@ void mfma_plan(Plan &g) {
             g.mfma_lds = (uint32_t)lds;
         }
     }
+    g.mfma_long_walk = long_walk(g) ? 1 : 0;
 }
 
 hipError_t launch_mfma_only(int workgroups, int iterations, hipStream_t s) {

@@ -172,6 +172,7 @@ struct Plan : Geometry {
     // per pair of taps), tap pairing, channel parts, input pixels a tile stages at most, LDS
     // bytes per workgroup, bytes of the weight fragments
     int mfma_steps, mfma_pair, mfma_parts, mfma_rows;
+    int mfma_long_walk;         // 1: the variant with several groups of weight fragments under way
     int mfma_small;             // 1: few tiles: the small-problem kernel (kernels_conv_small.hip),
     SmallPlan small;            // its part of the plan
     uint32_t mfma_small_lds;    // and its LDS bytes per workgroup
