@@ -62,6 +62,11 @@ bool layer(int mb, int ih, int iw, int kh, int kw, int sh, int sw, int ph, int p
     return true;
 }
 
+// A launch reads the descriptor's plan from any thread: nothing in it may be written through a const one (a
+// plan with a mutable member is no constant to copy from).
+constexpr Plan PLANNED{};
+[[maybe_unused]] constexpr Plan READ_BY_A_LAUNCH = PLANNED;
+
 } // namespace
 
 int main() {

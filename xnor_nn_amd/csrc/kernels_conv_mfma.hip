@@ -1171,10 +1171,16 @@ int oc_subblocks(const Plan &g) { return ((g.oc + NT - 1) / NT) * (NT / 32); }
 // Largest number of input pixels any tile of mt output pixels touches.  Tiles start at
 // multiples of `step` pixels (their own size for a launch with one tile size, 32 for a launch
 // with two); the offset of a tile within its image repeats after at most OHW starts, so that
-// many (plus the last, possibly short, tile) are enough to look at.
-int max_tile_rows(const Plan &g, uint32_t mt, uint32_t step = 0) {
+// many (plus the last, possibly short, tile) are enough to look at.  The choice of a tile size asks for the
+// same ones again and again: mfma_plan keeps what it has found while it plans (256 channels on 56x56:
+// 580 -> 140 us to initialise a descriptor).
+struct TileRows {
+    struct { uint32_t pixels, step; int rows; } known[8] = {};
+    uint32_t next = 0;
+};
+int max_tile_rows(const Plan &g, TileRows &found, uint32_t mt, uint32_t step = 0) {
     if (step == 0) step = mt;
-    for (const auto &known : g.tile_rows)
+    for (const auto &known : found.known)
         if (known.pixels == mt && known.step == step) return known.rows;
     const uint32_t starts = (g.npix_out + step - 1) / step;
     const uint32_t look = starts < (uint32_t)g.ohw + 1 ? starts : (uint32_t)g.ohw + 1;
@@ -1187,7 +1193,7 @@ int max_tile_rows(const Plan &g, uint32_t mt, uint32_t step = 0) {
     };
     for (uint32_t t = 0; t < look; t++) see(t);
     see(starts - 1);
-    g.tile_rows[g.tile_rows_next++ % TILE_ROWS_KNOWN] = {mt, step, most};
+    found.known[found.next++ % 8] = {mt, step, most};
     return most;
 }
 
@@ -1221,8 +1227,8 @@ size_t lds_bytes_for(const Plan &g, size_t rows, int ps, bool persist = false) {
         bytes = ((bytes + 15) & ~(size_t)15) + 4 * 32 * TURN_ROW * sizeof(float);
     return bytes;
 }
-size_t lds_bytes(const Plan &g, int ps) {
-    return lds_bytes_for(g, (size_t)max_tile_rows(g, 32 * ps * g.mfma_groups), ps);
+size_t lds_bytes(const Plan &g, TileRows &found, int ps) {
+    return lds_bytes_for(g, (size_t)max_tile_rows(g, found, 32 * ps * g.mfma_groups), ps);
 }
 
 // 32-pixel blocks per tile, by a model of the kernel's time in core cycles that was fitted to
@@ -1270,13 +1276,13 @@ bool tile_fits_registers(const Plan &g, int ps) {
 // tap and 184 or more otherwise, two 119 with one step per tap, 135 to 167 with two to four or
 // twelve steps and 188 or more otherwise, one 70 to 118 up to four steps and from twelve, 139
 // or 149 with five or six, 181 with eight; a SIMD holds 512 per lane) and by LDS.
-int resident_workgroups(const Plan &g, int ps) {
+int resident_workgroups(const Plan &g, TileRows &found, int ps) {
     const int ks = steps_per_tap(g);
     int by_regs = 2;
     if (ps == 3) by_regs = ks == 1 ? 3 : 2;
     if (ps == 2) by_regs = ks == 1 ? 4 : (ks <= 4 || ks == 12) ? 3 : 2;
     if (ps == 1) by_regs = (ks <= 4 || ks >= 12) ? 4 : ks <= 6 ? 3 : 2;
-    const int by_lds = (int)((size_t)LDS_LIMIT / lds_bytes(g, ps));
+    const int by_lds = (int)((size_t)LDS_LIMIT / lds_bytes(g, found, ps));
     const int fit = by_regs < by_lds ? by_regs : by_lds;
     return fit < 2 ? 2 : fit; // a tile that runs alone is priced separately
 }
@@ -1308,10 +1314,10 @@ bool long_walk(const Plan &g) {
     return walk >= (pair && groups == 1 && workgroups > 2u * (uint32_t)g.cus ? 20 : 8);
 }
 
-int pick_ps(const Plan &g) {
+int pick_ps(const Plan &g, TileRows &found) {
     if (const char *e = getenv("XNOR_NN_HIP_MFMA_PS")) {
         const int v = atoi(e);
-        if (v >= 1 && v <= 4 && lds_bytes(g, v) <= (size_t)LDS_LIMIT && tile_fits_registers(g, v))
+        if (v >= 1 && v <= 4 && lds_bytes(g, found, v) <= (size_t)LDS_LIMIT && tile_fits_registers(g, v))
             return v;
     }
     const int chunks = (g.oc + NT - 1) / NT;
@@ -1321,7 +1327,7 @@ int pick_ps(const Plan &g) {
     int best = 0;
     double best_cost = 0;
     for (int ps = 4; ps >= 1; ps--) {
-        if (lds_bytes(g, ps) > (size_t)LDS_LIMIT) continue;
+        if (lds_bytes(g, found, ps) > (size_t)LDS_LIMIT) continue;
         if (!tile_fits_registers(g, ps)) continue;
         const uint32_t mt = 32u * ps * g.mfma_groups; // pixels per tile
         const double tiles = (double)((g.npix_out + mt - 1) / mt);
@@ -1330,17 +1336,17 @@ int pick_ps(const Plan &g) {
         const double per_simd = tiles * chunks * 4 / simds;
         const double busiest = per_simd <= 1 ? 1.0
             : per_simd <= 4 ? (double)(long)(per_simd + 0.999999) : per_simd + 0.5;
-        const double words = (double)max_tile_rows(g, mt) * g.xw;
+        const double words = (double)max_tile_rows(g, found, mt) * g.xw;
         const double one_block = g.mfma_groups > 1 && steps_total < 48 ? 1.3 : 2.0;
         const double stream_bound = ps < 2 && per_simd > 1 ? one_block : (double)ps;
         const double wave = 3700.0 + 264.0 * words / 256.0 + 1700.0 * ps
             + (ps == 2 ? 70.4 : 64.0) * steps_total * stream_bound;
-        const int resident = resident_workgroups(g, ps);
+        const int resident = resident_workgroups(g, found, ps);
         const double further = resident >= 4 ? 0.35 : resident == 3 ? 0.5 : 0.75;
         const double together = busiest < resident ? busiest : (double)resident;
         const double waves = busiest < 2 ? 1.0
             : 1.0 + 0.35 * (together - 1.0) + further * (busiest - together);
-        const double alone = lds_bytes(g, ps) > (size_t)LDS_TWO_PER_CU ? 1.15 : 1.0;
+        const double alone = lds_bytes(g, found, ps) > (size_t)LDS_TWO_PER_CU ? 1.15 : 1.0;
         const double cost = wave * waves * alone;
         if (best == 0 || cost < best_cost - 1e-9) { best = ps; best_cost = cost; }
     }
@@ -1475,7 +1481,7 @@ hipError_t launch_mfma_ps(const Plan &g, const uint32_t *xbits, const uint32_t *
 // tile of input rows fits the 160 KB of LDS; everything else runs the XNOR/popcount kernel.
 // XNOR_NN_HIP_CONV=valu forces the latter (used to profile the two side by side).
 // Returns the tile size (32-pixel blocks per workgroup, 1..4) or 0 when not applicable.
-static int mfma_tile_blocks(const Plan &g) {
+static int mfma_tile_blocks(const Plan &g, TileRows &found) {
     if (const char *e = getenv("XNOR_NN_HIP_CONV"))
         if (e[0] == 'v') return 0;
     if ((g.ic + 63) / 64 > 64) return 0;
@@ -1483,7 +1489,7 @@ static int mfma_tile_blocks(const Plan &g) {
     if ((uint64_t)g.npix_out * g.oc * 4u >= 0xFFFFFFF0ull) return 0; // 32-bit output offsets
     if ((uint64_t)g.npix_in * g.xw > 0x7FFFFFFFull) return 0;
     if (mfma_weight_bytes(g) >= 0xFFFFFFF0ull) return 0; // 32-bit fragment offsets
-    return pick_ps(g);
+    return pick_ps(g, found);
 }
 
 size_t mfma_weight_bytes(const Plan &g) {
@@ -1511,8 +1517,7 @@ static int stream_output(const Plan &g) {
 }
 
 void mfma_plan(Plan &g) {
-    for (auto &known : g.tile_rows) known = {};
-    g.tile_rows_next = 0;
+    TileRows found;
     g.stream_dst = stream_output(g);
     g.mfma_parts = g.mfma_groups = 1;
     if (shallow_plan(g)) { // (every other mfma_* field stays zero)
@@ -1521,8 +1526,8 @@ void mfma_plan(Plan &g) {
     }
     // as many pixel groups as idle waves, fewer if even a one-block tile would not fit the LDS
     for (g.mfma_groups = pixel_groups(g); g.mfma_groups > 1; g.mfma_groups /= 2)
-        if (lds_bytes(g, 1) <= (size_t)LDS_LIMIT) break;
-    g.mfma_ps = mfma_tile_blocks(g);
+        if (lds_bytes(g, found, 1) <= (size_t)LDS_LIMIT) break;
+    g.mfma_ps = mfma_tile_blocks(g, found);
     g.use_mfma = g.mfma_ps > 0 ? 1 : 0;
     g.mfma_steps = g.mfma_pair = g.mfma_rows = 0;
     g.mfma_ps_small = 0;
@@ -1539,8 +1544,8 @@ void mfma_plan(Plan &g) {
     g.mfma_steps = steps_per_tap(g);
     g.mfma_pair = pair_taps(g) ? 1 : 0;
     g.mfma_parts = channel_parts(g);
-    g.mfma_rows = max_tile_rows(g, 32 * g.mfma_ps * g.mfma_groups);
-    g.mfma_lds = (uint32_t)lds_bytes(g, g.mfma_ps);
+    g.mfma_rows = max_tile_rows(g, found, 32 * g.mfma_ps * g.mfma_groups);
+    g.mfma_lds = (uint32_t)lds_bytes(g, found, g.mfma_ps);
     g.mfma_wbytes = (uint32_t)mfma_weight_bytes(g);
     // Few tiles: the small-problem kernel takes the scaled output (the raw accumulators still
     // go through the kernel planned below).
@@ -1598,7 +1603,7 @@ void mfma_plan(Plan &g) {
                 || g.mfma_steps >= 16 || (g.mfma_pair && g.xw >= 5) || !tile_fits_registers(g, 4))
             persist = false;
         if (persist) {
-            const int rows = max_tile_rows(g, 32 * 4, 32);
+            const int rows = max_tile_rows(g, found, 32 * 4, 32);
             const size_t lds = lds_bytes_for(g, (size_t)rows, 4, true);
             if (lds <= (size_t)LDS_TWO_PER_CU) {
                 uint32_t best_a = 0, best_total = 0;
@@ -1629,7 +1634,7 @@ void mfma_plan(Plan &g) {
         }
     }
     if (mix || fill) {
-        const int rows = max_tile_rows(g, 32 * 4, 32);
+        const int rows = max_tile_rows(g, found, 32 * 4, 32);
         const size_t lds = lds_bytes_for(g, (size_t)rows, 4);
         if (lds <= (size_t)LDS_TWO_PER_CU) {
             g.mfma_ps = 4;

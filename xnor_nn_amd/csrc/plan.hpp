@@ -145,14 +145,7 @@ __host__ __device__ inline void shallow_product(int j, int n, int row_codes, int
 // What the host adds to it when a descriptor is initialised: which kernels run and with what
 // tiles.  Kernels get the Geometry part (geometry() below) and their own: the argument block is
 // copied on every launch and read by every workgroup.
-constexpr int TILE_ROWS_KNOWN = 8;
 struct Plan : Geometry {
-    // Input pixels that tiles of so many pixels, so far apart, touch at most: a search over the tiles of an
-    // image, and the choice of a tile size asks for the same ones again and again (256 channels on 56x56:
-    // 580 -> 140 us to initialise a descriptor)
-    struct TileRows { uint32_t pixels, step; int rows; };
-    mutable TileRows tile_rows[TILE_ROWS_KNOWN];
-    mutable uint32_t tile_rows_next;
     int bin_waves;              // waves per workgroup of the binarize kernel at most
     int bin_nhwc_lane;          // 1: NHWC input by the one-lane-per-pixel kernel
     int cus;                    // compute units of the device (256 if it cannot be asked)
