@@ -53,11 +53,18 @@ bool layer(int mb, int ih, int iw, int kh, int kw, int sh, int sw, int ph, int p
     g.div_ow = FastDiv::make((uint32_t)g.ow);
     for (uint32_t from = 0; from < g.npix_out; from += tile) {
         const uint32_t end = from + tile < g.npix_out ? from + tile : g.npix_out;
-        int lo, hi;
-        tile_span(g, from, end, lo, hi);
-        for (uint32_t p = from; p < end; p++)
-            if (!walk<false>(g, p, lo, hi - lo + 1, 1) || !walk<true>(g, p, lo, hi - lo + 1, 3))
+        // what the large kernel stages, and whole rows, as the one for few tiles does
+        for (const auto span : {tile_span, row_span}) {
+            int lo, hi;
+            span(g, from, end, lo, hi);
+            if (lo < 0 || hi < lo || (uint32_t)hi >= (uint32_t)(mb * g.ihw)) {
+                printf("%dx%d kernel %dx%d: a tile stages %d to %d\n", ih, iw, kh, kw, lo, hi);
                 return false;
+            }
+            for (uint32_t p = from; p < end; p++)
+                if (!walk<false>(g, p, lo, hi - lo + 1, 1) || !walk<true>(g, p, lo, hi - lo + 1, 3))
+                    return false;
+        }
     }
     return true;
 }
@@ -79,6 +86,12 @@ int main() {
         const int k = from(0, 3) ? from(1, 7) : from(8, 32), p = from(0, k);
         ok = layer(from(1, 2), from(1, 24), from(1, 24), k, from(0, 1) ? k : from(1, 9), from(1, 3),
                 from(1, 3), from(0, 2) ? p : from(0, 3), p, 32u * from(1, 4));
+    }
+    // wide images, whose tiles begin and end inside a row: without a stride between columns, and with one
+    for (int i = 0; ok && i < 200; i++) {
+        const int k = from(0, 3) ? from(1, 7) : from(8, 32);
+        ok = layer(from(1, 2), from(1, 12), from(25, 130), from(0, 1) ? k : from(1, 9), k, from(1, 3),
+                i % 4 ? 1 : from(2, 3), from(0, 3), from(0, k), 32u * from(1, 4));
     }
     if (ok) printf("ok\n");
     return ok ? 0 : 1;
