@@ -1231,38 +1231,28 @@ size_t lds_bytes(const Plan &g, TileRows &found, int ps) {
     return lds_bytes_for(g, (size_t)max_tile_rows(g, found, 32 * ps * g.mfma_groups), ps);
 }
 
-// 32-pixel blocks per tile, by a model of the kernel's time in core cycles that was fitted to
-// measurements on MI355X (conv4 from MB 4 to MB 1024, ResNet 3x3 56x56 MB 1 to 64, VGG 512 MB
-// 1 to 32, the conv2 shape, 64- and 128-channel layers; PS 1/2/3/4 at conv4 MB 256 = 34.7 /
-// 27.0 / 26.6 / 27.5 us, at MB 32 = 8.2 / 9.4 / 11.7 / 13.8 us).
-//   one wave:   staging (set-up, plus 264 cycles per 256 packed words to expand)
-//               + PS x (epilogue 1700 + 64 per step of the main loop)
-//               -- with one pixel block and more than one wave per SIMD a step costs as much
-//               as with two: the weight stream (2 KB per wave and step whatever the tile)
-//               sets its pace, not the matrix instructions; with pixel groups (128 filters or
-//               fewer) two or four waves of a workgroup read the same fragments and it costs
-//               1.3, unless the walk is long (64 to 96 channels 3x3 on 30x30, minibatch 39,
-//               a pass with one / three blocks 12.5 / 14.2 us; 76 to 40 on 59x59 one / two
-//               12.9 / 14.0; but 384 to 64 channels 3x3 on 73x73, 54 steps, one / three 41.8 /
-//               39.7, 192 to 96 channels 5x5, 75 steps, one / two 19.6 / 17.6: on 60 layers of
-//               16 to 128 filters the mean distance from the fastest tile is 2.1 -> 1.0 %);
-//               Tiles of two pixel blocks pay 10 % more per step: their weight stream is
-//               as wide as the vector-memory return path of the CU;
-//   the kernel: one wave's time for the first wave of the busiest SIMD, 0.35 of it more for
-//               every further wave that is resident with it (their phases overlap), and for
-//               every wave beyond the resident ones 0.75 of it with two resident waves per
-//               SIMD, 0.5 with three, 0.35 with four (small tiles of shallow inputs need at
-//               most 168 or 128 registers, so a third or fourth workgroup fits a CU, and a
-//               launch of many rounds of such tiles is faster than one of large tiles:
-//               ResNet 3x3 56x56 MB 64 61.0 against 63.1 us, 128 filters on the same input
-//               32.5 against 38.1, 64 filters 18.0 against 23.5); with few waves per SIMD the
-//               busiest one counts (rounded up), with many the hardware's dynamic
-//               scheduling evens the load out;
-//   a tile that needs more than half the LDS runs alone on its CU: 15 % more.
-// Ties go to the larger tile, which streams fewer weight bytes.
-// Refitted on 56 shapes (13x13 to 112x112 images, 32 to 512 channels, 64 to 512 filters,
-// 1x1 to 5x5 kernels, MB 1 to 1024) with every tile size forced in turn: the choice is the
-// fastest tile on 50 of them and within 3.2 % on the rest.
+// 32-pixel blocks per tile, by a model of the kernel's time in core cycles, fitted to 893 layers of 13 to
+// 2048 channels and 16 to 768 filters (1x1 to 11x11 kernels, 7x7 to 227x227 images, minibatch 1 to 256,
+// NCHW and NHWC) that were run with every tile size in turn.
+//   one wave:   its own work (set-up, 264 cycles per 256 packed words to expand, an epilogue of 1600 per
+//               block), and 64 cycles per step of the main loop and block.  A block alone costs twice that
+//               as soon as a SIMD has more than one wave: the weight stream (2 KB per wave and step
+//               whatever the tile) sets its pace, not the matrix instructions; 1.7 times with one step per
+//               tap and 1.6 with one per pair of taps, whose fragments are asked for further ahead on long
+//               walks, 1.5 with the whole compute unit to itself.  Two blocks cost 10 % more: their weight stream is as wide as the
+//               vector-memory return path;
+//   the kernel: one wave's time for the first wave of the busiest SIMD; for every further wave that is
+//               resident with it 0.22 of its own work and 0.4 of its steps more (their phases overlap, the
+//               matrix pipe is shared), for every wave beyond those 0.44 of both with two resident waves
+//               per SIMD, 0.32 with three, 0.25 with four.  A tile that needs more than half the LDS runs
+//               alone on its compute unit: 0.7 for every wave after the first.  With few waves per SIMD
+//               the busiest one counts (rounded up), with many the hardware's dynamic scheduling evens the
+//               load out.
+// Ties go to the larger tile, which streams fewer weight bytes.  Time of the chosen tile over the fastest
+// one's, the constants from when tiles staged whole rows and one group of fragments was under way / these:
+// mean 1.6 / 0.5 %, more than 3 % on 153 / 43 layers, at most 35 / 18 %; on layers held out of a fit 0.7 %.
+// Smaller spans had let small tiles look resident by fours and win: a pass with the old choice / this, us, 877
+// to 306 channels 3x3 on 13x13, minibatch 163, 87.3 / 64.5, 80 to 64 5x5 on 63x63, 157, 111.4 / 97.6.
 // Four pixel blocks do not fit the register file with 16 steps per tap or with tap pairing
 // over five words (those variants spill), and are not instantiated for channel parts.
 bool tile_fits_registers(const Plan &g, int ps) {
@@ -1337,17 +1327,17 @@ int pick_ps(const Plan &g, TileRows &found) {
         const double busiest = per_simd <= 1 ? 1.0
             : per_simd <= 4 ? (double)(long)(per_simd + 0.999999) : per_simd + 0.5;
         const double words = (double)max_tile_rows(g, found, mt) * g.xw;
-        const double one_block = g.mfma_groups > 1 && steps_total < 48 ? 1.3 : 2.0;
-        const double stream_bound = ps < 2 && per_simd > 1 ? one_block : (double)ps;
-        const double wave = 3700.0 + 264.0 * words / 256.0 + 1700.0 * ps
-            + (ps == 2 ? 70.4 : 64.0) * steps_total * stream_bound;
-        const int resident = resident_workgroups(g, found, ps);
-        const double further = resident >= 4 ? 0.35 : resident == 3 ? 0.5 : 0.75;
+        const bool alone = lds_bytes(g, found, ps) > (size_t)LDS_TWO_PER_CU;
+        const double pace = ps > 1 || per_simd <= 1 ? (double)ps
+            : alone ? 1.5 : steps_per_tap(g) > 1 ? 2.0 : pair_taps(g) ? 1.6 : 1.7;
+        const double own = 4500.0 + 264.0 * words / 256.0 + 1600.0 * ps;
+        const double steps = (ps == 2 ? 70.4 : 64.0) * steps_total * pace;
+        const int resident = alone ? 1 : resident_workgroups(g, found, ps);
+        const double beyond = alone ? 0.7 : resident >= 4 ? 0.25 : resident == 3 ? 0.32 : 0.44;
         const double together = busiest < resident ? busiest : (double)resident;
-        const double waves = busiest < 2 ? 1.0
-            : 1.0 + 0.35 * (together - 1.0) + further * (busiest - together);
-        const double alone = lds_bytes(g, found, ps) > (size_t)LDS_TWO_PER_CU ? 1.15 : 1.0;
-        const double cost = wave * waves * alone;
+        const double rest = beyond * (busiest - together);
+        const double cost = busiest < 2 ? own + steps
+            : own * (1.0 + 0.22 * (together - 1.0) + rest) + steps * (1.0 + 0.4 * (together - 1.0) + rest);
         if (best == 0 || cost < best_cost - 1e-9) { best = ps; best_cost = cost; }
     }
     return best;
