@@ -213,7 +213,8 @@ __device__ __forceinline__ void copy_to_lds_async(const void *src, const int n,
 // is already in LDS and which tile to prefetch.  The LDS layout then has room for four pixel
 // blocks whatever PS is, so that tiles of two sizes can follow each other.
 // LONG: the walk is long enough for several groups of weight fragments under way (long_walk()).
-template <int KS, int PS, bool RAW, bool PAIR, bool DEEP, bool LONG, bool PERSIST = false>
+// MIXED: the kernel holds tiles of two sizes, and has no scalar registers to spare (box_sum.hpp).
+template <int KS, int PS, bool RAW, bool PAIR, bool DEEP, bool LONG, bool MIXED, bool PERSIST = false>
 __device__ __forceinline__
 void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag,
         const float *__restrict__ alpha, const float *__restrict__ kplane,
@@ -414,7 +415,7 @@ void conv_tile(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wfrag
             constexpr int LAST = PS - 1;
             const int second = 2 * q < LAST ? 2 * q + 1 : LAST; // (an odd last block twice)
             const bool upper = lane >= 32;
-            const float sum = box_sum(a_lds, upper ? in0[second] : in0[2 * q], max_rows,
+            const float sum = box_sum<!MIXED>(a_lds, upper ? in0[second] : in0[2 * q], max_rows,
                     upper ? rowmask[second] : rowmask[2 * q],
                     upper ? colmask[second] : colmask[2 * q], g.kh, g.kw, g.iw, inv_khw);
             if (lane < 32 || 2 * q < LAST) {
@@ -898,7 +899,7 @@ void conv_tile_of(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wf
         if (unit >= units) return;
         const uint32_t tile = oc_chunks == 1 ? unit : div_chunks.div(unit);
         const int chunk = unit - tile * oc_chunks;
-        conv_tile<KS, PS, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g, max_rows,
+        conv_tile<KS, PS, RAW, PAIR, DEEP, LONG, false>(xbits, wfrag, alpha, kplane, dst, popc, g, max_rows,
                 div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes,
                 tile * (32u * PS * (uint32_t)g.mfma_groups), g.npix_out, chunk);
     } else {
@@ -909,13 +910,13 @@ void conv_tile_of(const uint32_t *__restrict__ xbits, const v4i *__restrict__ wf
         if (tile < big_per_xcd) {
             const uint32_t p_first = (first + tile * PS) * 32u;
             if (p_first >= p_limit) return;
-            conv_tile<KS, PS, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g,
+            conv_tile<KS, PS, RAW, PAIR, DEEP, LONG, true>(xbits, wfrag, alpha, kplane, dst, popc, g,
                     max_rows, div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes, p_first,
                     p_limit, chunk);
         } else {
             const uint32_t p_first = (first + big_per_xcd * PS + (tile - big_per_xcd) * PSB) * 32u;
             if (p_first >= p_limit) return;
-            conv_tile<KS, PSB, RAW, PAIR, DEEP, LONG>(xbits, wfrag, alpha, kplane, dst, popc, g,
+            conv_tile<KS, PSB, RAW, PAIR, DEEP, LONG, true>(xbits, wfrag, alpha, kplane, dst, popc, g,
                     max_rows, div_xw, a_plane, k_out, inv_khw, ic_parts, wfrag_bytes, p_first,
                     p_limit, chunk);
         }
@@ -1020,11 +1021,11 @@ void conv_mfma_fp4_persistent_kernel(const uint32_t *__restrict__ xbits,
         turn.next_first = more ? next_first : 0u;
         turn.next_end = more ? end_pixel(next, next_first) : 0u;
         if (tile < big_per_xcd)
-            conv_tile<KS, PS, false, PAIR, false, false, true>(xbits, wfrag, alpha, kplane, dst, nullptr,
+            conv_tile<KS, PS, false, PAIR, false, false, true, true>(xbits, wfrag, alpha, kplane, dst, nullptr,
                     g, max_rows, div_xw, a_plane, k_out, inv_khw, 1, wfrag_bytes, p_first,
                     p_limit, chunk, turn);
         else
-            conv_tile<KS, PSB, false, PAIR, false, false, true>(xbits, wfrag, alpha, kplane, dst,
+            conv_tile<KS, PSB, false, PAIR, false, false, true, true>(xbits, wfrag, alpha, kplane, dst,
                     nullptr, g, max_rows, div_xw, a_plane, k_out, inv_khw, 1, wfrag_bytes,
                     p_first, p_limit, chunk, turn);
         if (!more) break;

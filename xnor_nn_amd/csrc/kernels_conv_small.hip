@@ -282,7 +282,7 @@ void conv_mfma_fp4_small_kernel(const uint32_t *__restrict__ xbits, const v4i *_
     float kv = k_read;
     float *k_lds = parts + (WAVES - 1) * (16 + KEEP) * 64;
     if (fuse_k && wave == WAVES - 1) {
-        kv = box_sum(a_lds, in0, s.max_rows, rowmask, colmask, g.kh, g.kw, g.iw, inv_khw);
+        kv = box_sum<true>(a_lds, in0, s.max_rows, rowmask, colmask, g.kh, g.kw, g.iw, inv_khw);
         k_lds[lane] = kv;
         if (sub == 0 && lane < 32 && live) k_out[pix] = kv;
     }
