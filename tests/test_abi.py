@@ -316,6 +316,20 @@ def test_small_tiles_of_long_walks_are_not_chosen_for_their_number():
         assert "PS=%d" % ps in kernel_names(t)[1], (t, kernel_names(t)[1])
 
 
+def test_pixel_groups_leave_no_half_of_the_chip_idle(monkeypatch):
+    """Few filters: the waves without filters take pixel blocks of their own, but not where that leaves half
+    of the 256 compute units without a workgroup."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", "0")
+    for t, groups in (((2, 64, 416, 103, 103, 1, 1, 2, 2, 0, 0), 1),   # 44 workgroups of four groups
+                      ((4, 64, 64, 64, 64, 1, 1, 1, 1, 0, 0), 2),      # 128
+                      ((1, 64, 64, 113, 145, 1, 1, 1, 1, 0, 0), 4),    # 129
+                      ((2, 64, 64, 64, 64, 1, 1, 1, 1, 0, 0), 1),      # 64, 128 of two groups
+                      ((1, 64, 64, 91, 91, 1, 1, 1, 1, 0, 0), 2),      # 65, 130
+                      ((2, 128, 64, 64, 64, 1, 1, 1, 1, 0, 0), 1), ((1, 128, 64, 91, 91, 1, 1, 1, 1, 0, 0), 2)):
+        name = kernel_names(t)[1]
+        assert ("GROUPS=%d" % groups in name) if groups > 1 else "GROUPS" not in name, (t, name)
+
+
 def test_inputs_that_reach_the_dropped_offset_take_the_generic_kernel():
     """The tiled binarize kernels read a channel past the end of a ragged slice through the
     byte offset 0xFFFFFFF0, which the hardware drops only while it lies outside the buffer.

@@ -710,6 +710,21 @@ def test_walks_with_several_groups_under_way(oracle, monkeypatch, ic, blocks):
                 run_and_compare(oracle, d, x, w)
 
 
+@pytest.mark.parametrize("groups", ["1", "2", "4"])
+@pytest.mark.parametrize("t", [
+    (4, 64, 64, 64, 64, 1, 1, 1, 1, 0, 0),      # 128 workgroups of four groups, 256 of two
+    (1, 70, 33, 46, 45, 3, 3, 1, 1, 1, 1),      # a last tile of a few pixels
+    (1, 130, 128, 31, 33, 3, 3, 1, 1, 1, 1),
+    (3, 288, 24, 19, 23, 3, 3, 2, 2, 1, 1),
+], ids=str)
+def test_pixel_groups_of_few_workgroups(oracle, monkeypatch, t, groups):
+    """A layer of few filters and pixels with every number of pixel groups; 1 is what the plan takes."""
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_SMALL", "0")
+    monkeypatch.setenv("XNOR_NN_HIP_MFMA_GROUPS", groups)
+    d, x, w = problem(t, zeros=True)
+    run_and_compare(oracle, d, x, w)
+
+
 @pytest.mark.parametrize("t", [
     (1, 3000, 33, 28, 28, 3, 3, 1, 1, 1, 1),    # one tile to a compute unit's LDS
     (1, 4096, 8, 14, 14, 3, 3, 1, 1, 1, 1),     # four channel parts

@@ -1518,6 +1518,18 @@ void mfma_plan(Plan &g) {
     // as many pixel groups as idle waves, fewer if even a one-block tile would not fit the LDS
     for (g.mfma_groups = pixel_groups(g); g.mfma_groups > 1; g.mfma_groups /= 2)
         if (lds_bytes(g, found, 1) <= (size_t)LDS_LIMIT) break;
+    // ... or if their workgroups would leave half of the compute units idle.  us a pass with groups for all
+    // waves / by this rule: 416 to 64 channels 1x1 stride 2 on 103x103, minibatch 2 (44 workgroups), 19.9 / 12.6,
+    // 345 to 44 3x3 on 56x55, 4 (98), 14.1 / 11.9, 359 to 49 on 22x22, 20 (63), 14.1 / 11.8, 144 to 96 5x5
+    // stride 2 on 60x60, 9 (127), 14.1 / 12.4, 32 to 96 on 50x51, 3 (120), 7.6 / 7.4; 58 layers of up to 128
+    // workgroups 3 to 58 % faster, 10 % on average.  17 layers of 138 to 200: 0.92 to 1.05 times as fast, 0.7
+    // where a tile is alone on its compute unit either way (43 to 94 channels 11x11 on 142x142, minibatch 9).
+    // A tile size asked for by name keeps the groups.
+    if (!getenv("XNOR_NN_HIP_MFMA_GROUPS") && !getenv("XNOR_NN_HIP_MFMA_PS"))
+        for (; g.mfma_groups > 1; g.mfma_groups /= 2) {
+            const uint32_t pixels = 32u * (uint32_t)g.mfma_groups;
+            if (2 * ((g.npix_out + pixels - 1) / pixels) > (uint32_t)g.cus) break;
+        }
     g.mfma_ps = mfma_tile_blocks(g, found);
     g.use_mfma = g.mfma_ps > 0 ? 1 : 0;
     g.mfma_steps = g.mfma_pair = g.mfma_rows = 0;
