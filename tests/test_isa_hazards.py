@@ -449,3 +449,17 @@ def test_the_tile_model_counts_resident_workgroups_as_the_registers_allow(conv_i
         exact += rule == fit
     assert seen >= 40, seen
     assert seen - exact <= 2, (seen, exact)
+
+
+def test_long_walks_leave_room_for_as_many_workgroups(conv_isa):
+    """The variants of long walks keep more groups of weight fragments in registers; the rule counts as many
+    workgroups of them as of the others."""
+    seen = 0
+    for text, registers in kernel_metadata(conv_isa, "vgpr_count").items():
+        m = re.search(r"conv_mfma_fp4_long_kernel<(\d+), (\d+), (\d+), (\w+)>", text)
+        if not m or m[3] != "0":  # two tile sizes
+            continue
+        fit = min(4, 512 // ((registers + 7) // 8 * 8))
+        assert resident_by_registers(int(m[1]), int(m[2])) <= fit, (text[:70], registers)
+        seen += 1
+    assert seen >= 11, seen

@@ -1263,10 +1263,11 @@ bool tile_fits_registers(const Plan &g, int ps) {
 }
 
 // Workgroups of a tile size that fit a compute unit together, two to four: by registers (the
-// counts of the compiled variants: four pixel blocks 199 to 254, three 168 with one step per
-// tap and 184 or more otherwise, two 119 with one step per tap, 135 to 167 with two to four or
-// twelve steps and 188 or more otherwise, one 70 to 118 up to four steps and from twelve, 139
-// or 149 with five or six, 181 with eight; a SIMD holds 512 per lane) and by LDS.
+// counts of the compiled variants with scaled output: four pixel blocks 215 to 252, three 165 or 166 with
+// one step per tap and 183 or more otherwise, two 118 with one step per tap, and 125 or 128, which is all
+// that four workgroups leave, where several groups of fragments are under way (long_walk()); 135 to 167 with
+// two to four or twelve steps and 168 or more otherwise; one 70 to 119 up to four steps and from twelve,
+// 136 or 151 with five or six, 183 with eight; a SIMD holds 512 per lane) and by LDS.
 int resident_workgroups(const Plan &g, TileRows &found, int ps) {
     const int ks = steps_per_tap(g);
     int by_regs = 2;
