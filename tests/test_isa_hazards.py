@@ -36,7 +36,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "xnor_nn_amd", "csrc")
 VM_MAX, LGKM_MAX = 64, 16
 ASM_BEGIN, ASM_END = "#ASMSTART", "#ASMEND"
-EXPECTED_VARIANTS = 141  # kernels the matrix-core file instantiates (9 of them persistent)
+EXPECTED_VARIANTS = 156  # kernels the matrix-core file instantiates (9 of them persistent, 15 for long walks)
 
 
 def vgprs(token):
